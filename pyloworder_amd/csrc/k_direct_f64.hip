@@ -1,0 +1,637 @@
+// FP64 MFMA streaming kernels for narrow operands (at most 64 real columns, or a
+// product whose W fits one CU's LDS): every wave works on its own rows, straight
+// from global memory to MFMA fragments, with no barrier in the row loop.
+//
+// What bounds these sizes is HBM (30 columns: 4 flop / B in P1, the FP64 matrix
+// rate needs 15), so the point is bytes in flight.  Staging 32-row tiles in LDS
+// with two barriers per tile left one 4 KB tile per workgroup in flight; here each
+// of the 8 waves of a workgroup holds its current rows and loads the next ones.
+//
+// v_mfma_f64_16x16x4f64 (wave64, lane l, i = l % 16, g = l / 16):
+//   A (16x4): A[i][g]    B (4x16): B[g][i]    D (16x16), reg r: D[4 r + g][i]
+// Two facts make LDS unnecessary:
+//   - in a Gram both operands of rows k..k+3 are the same fragment Y[k + g][16 J + i];
+//   - the D registers of Z = Y W are themselves such fragments of Z (register r is
+//     rows 4 r .. 4 r + 3), so P2's Gram takes them as they are.
+// Measured (MI355X) against LDS-staged 32-row tiles: 129 x 200,000 x 30 float32
+// (SPOD) P1 1.54 -> 0.91 ms, P2 2.78 -> 1.62 ms, U = Y W 2.47 -> 1.69 ms (3.7 TB/s);
+// 1M x 64 float64 P1 192 -> 132 us, P2 417 -> 222 us, product 279 -> 242 us (4.2 TB/s,
+// a copy reaches 4.7); 8M x 64 by 64 x 256 float32 (reconstruct) 6.46 -> 4.96 ms;
+// A^T B of 700,001 x 64 and x 48 float32 189 -> 108 us.
+//
+// Loads are V elements per lane (V = 1, 2, 4 by alignment).  In the Grams the V
+// elements go to V column blocks (block c V + e holds the physical columns
+// 16 V c + V i + e), undone when the slab is written; in the products they go to V
+// k-steps (a sum over k may take its terms in any order) and W is laid out in LDS
+// to match.
+#include "common.hpp"
+#include "kernels.hpp"
+
+namespace {
+
+typedef double d4 __attribute__((ext_vector_type(4)));
+constexpr int DNT = 512;        // 8 waves
+constexpr int DNW = DNT / 64;
+// Waves that share a row chunk of a Gram over NB columns, 16 rows each per turn.  Up
+// to 32 columns a chunk is one wave's: its rows are summed in ascending order and the
+// slab is written from registers.  (Summing 8 waves' parts through LDS costs a
+// workgroup about as much as 200 rows of 30 columns.)  Wider Grams have few chunks
+// of long rows, so 8 waves share one.
+constexpr int chunk_waves(int NB) { return NB <= 32 ? 1 : 8; }
+
+PC_DEV d4 mfma64(double a, double b, d4 c) { return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0); }
+
+template <class TS, int V>
+PC_DEV void load_vec(const TS* p, TS* o) {
+  if constexpr (V == 1) {
+    o[0] = p[0];
+  } else {
+    typedef TS vt __attribute__((ext_vector_type(V)));
+    const vt q = *reinterpret_cast<const vt*>(p);
+#pragma unroll
+    for (int e = 0; e < V; e++) o[e] = q[e];
+  }
+}
+template <class TO, int V>
+PC_DEV void store_vec(TO* p, const TO* o) {
+  if constexpr (V == 1) {
+    p[0] = o[0];
+  } else {
+    typedef TO vt __attribute__((ext_vector_type(V)));
+    vt q;
+#pragma unroll
+    for (int e = 0; e < V; e++) q[e] = o[e];
+    *reinterpret_cast<vt*>(p) = q;
+  }
+}
+
+template <int CTRL>
+PC_DEV double dpp_move(double x) {
+  const long long b = __builtin_bit_cast(long long, x);
+  const int lo = __builtin_amdgcn_update_dpp(0, int(b), CTRL, 0xF, 0xF, true);
+  const int hi = __builtin_amdgcn_update_dpp(0, int(b >> 32), CTRL, 0xF, 0xF, true);
+  return __builtin_bit_cast(double, (long long)(unsigned)lo | ((long long)hi << 32));
+}
+// sum over the 16 lanes of a DPP row, in every lane
+PC_DEV double row16_sum(double v) {
+  v += dpp_move<0xB1>(v);   // quad_perm [1,0,3,2]
+  v += dpp_move<0x4E>(v);   // quad_perm [2,3,0,1]
+  v += dpp_move<0x141>(v);  // row_half_mirror
+  v += dpp_move<0x140>(v);  // row_mirror
+  return v;
+}
+// s / n with iv = 1 / n: the quotient and one residual step
+PC_DEV double div_n(double s, double n, double iv) {
+  const double q = s * iv;
+  return fma(fma(-n, q, s), iv, q);
+}
+
+// Sum the NBLK accumulators of the 8 waves in wave order through red (two blocks
+// at a time) and hand every entry (block, i, j, value) to `put`.
+template <int NBLK, class Put>
+PC_DEV void sum_waves(const d4* acc, double* red, Put put) {
+  const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
+#pragma unroll
+  for (int b0 = 0; b0 < NBLK; b0 += 2) {
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < 2; u++)
+      if (b0 + u < NBLK)
+#pragma unroll
+        for (int r = 0; r < 4; r++) red[(w * 2 + u) * 256 + r * 64 + l] = acc[b0 + u][r];
+    __syncthreads();
+    const int u = threadIdx.x >> 8, e = threadIdx.x & 255;
+    if (b0 + u < NBLK) {
+      double s = 0.0;
+#pragma unroll
+      for (int q = 0; q < DNW; q++) s += red[(q * 2 + u) * 256 + e];
+      put(b0 + u, 4 * (e >> 6) + ((e >> 4) & 3), e & 15, s);
+    }
+  }
+}
+
+// Upper blocks (I, J) of a chunk's Gram to `put`: from registers, or summed over its 8 waves
+template <int nb, int WPC, class Put>
+PC_DEV void store_gram(const d4* acc, double* red, Put put) {
+  constexpr int NBLK = nb * (nb + 1) / 2;
+  if constexpr (WPC == 1) {
+    const int l = threadIdx.x & 63;
+    int b = 0;
+#pragma unroll
+    for (int I = 0; I < nb; I++)
+#pragma unroll
+      for (int J = I; J < nb; J++, b++)
+#pragma unroll
+        for (int r = 0; r < 4; r++) put(I, J, 4 * r + (l >> 4), l & 15, acc[b][r]);
+  } else {
+    sum_waves<NBLK>(acc, red, [&](int blk, int pi, int pj, double s) {
+      int I = 0, o = 0;
+      while (o + nb - I <= blk) o += nb - I++;
+      put(I, I + blk - o, pi, pj, s);
+    });
+  }
+}
+
+// fragments of 4 RS rows (RS k-steps) of a row-major operand: v[r][c V + e] is row
+// base + 4 r + g, column 16 V c + V i + e.  Rows beyond the range repeat its last
+// row, columns beyond n column 0: masked by the caller.
+template <class TS, int NBF, int V, int RS>
+PC_DEV void load_rows(const TS* __restrict__ X, int64_t ldx, int n, int64_t base, int64_t row1, TS (*v)[NBF]) {
+  const int l = threadIdx.x & 63, i = l & 15, g = l >> 4;
+#pragma unroll
+  for (int r = 0; r < RS; r++) {
+    const int64_t row = base + 4 * r + g;
+    const TS* xr = X + (row < row1 ? row : row1 - 1) * ldx;
+#pragma unroll
+    for (int c = 0; c < NBF / V; c++) {
+      const int col = 16 * V * c + V * i;
+      load_vec<TS, V>(xr + (col < n ? col : 0), &v[r][c * V]);
+    }
+  }
+}
+
+// P1: partial Gram of the (centred) rows of a chunk
+template <class TS, int NB, int V>
+__global__ __launch_bounds__(DNT) void k_dgram_f64(const TS* __restrict__ X, int64_t ldx, int64_t m, int n, int center,
+                                                   double* mean_out, double* var_out, int chunks, int64_t rpc,
+                                                   double* __restrict__ part, int64_t zx, int64_t zb) {
+  X = zoff(X, zx);
+  mean_out = zoff(mean_out, zb);
+  var_out = zoff(var_out, zb);
+  part = zoff(part, zb);
+  constexpr int nb = NB / 16, NBLK = nb * (nb + 1) / 2;
+  constexpr int WPC = chunk_waves(NB);
+  __shared__ double red[WPC > 1 ? DNW * 2 * 256 : 1];
+  const int w = threadIdx.x >> 6, l = threadIdx.x & 63, i = l & 15, g = l >> 4;
+  const int64_t chunk = int64_t(blockIdx.x) * (DNW / WPC) + w / WPC;
+  if (WPC == 1 && chunk >= chunks) return;
+  const int64_t row0 = chunk * rpc;
+  const int64_t row1 = row0 + rpc < m ? row0 + rpc : m;
+  bool cv[nb];
+#pragma unroll
+  for (int b = 0; b < nb; b++) cv[b] = 16 * V * (b / V) + V * i + b % V < n;
+  const double nd = n, inv_n = 1.0 / nd;
+  d4 acc[NBLK];
+#pragma unroll
+  for (int b = 0; b < NBLK; b++) acc[b] = d4{0, 0, 0, 0};
+  TS cur[4][nb], nxt[4][nb];
+  int64_t t = row0 + 16 * (w % WPC);
+  if (t < row1) load_rows<TS, nb, V, 4>(X, ldx, n, t, row1, cur);
+  for (; t < row1; t += 16 * WPC) {
+    if (t + 16 * WPC < row1) load_rows<TS, nb, V, 4>(X, ldx, n, t + 16 * WPC, row1, nxt);
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+      const int64_t row = t + 4 * r + g;
+      const bool rv = row < row1;
+      double f[nb];
+#pragma unroll
+      for (int b = 0; b < nb; b++) f[b] = rv && cv[b] ? double(cur[r][b]) : 0.0;
+      if (center) {
+        double s = 0.0;
+#pragma unroll
+        for (int b = 0; b < nb; b++) s += f[b];
+        const double mu = div_n(row16_sum(s), nd, inv_n);
+#pragma unroll
+        for (int b = 0; b < nb; b++) f[b] = rv && cv[b] ? f[b] - mu : 0.0;
+        if (center == 2) {
+          double s2 = 0.0;
+#pragma unroll
+          for (int b = 0; b < nb; b++) s2 += f[b] * f[b];
+          const double var = div_n(row16_sum(s2), nd, inv_n);
+#pragma unroll
+          for (int b = 0; b < nb; b++) f[b] = rv && cv[b] ? f[b] / var : 0.0;
+          if (rv && i == 0) var_out[row] = var;
+        }
+        if (rv && i == 0) mean_out[row] = mu;
+      }
+      int b = 0;
+#pragma unroll
+      for (int I = 0; I < nb; I++)
+#pragma unroll
+        for (int J = I; J < nb; J++, b++) acc[b] = mfma64(f[I], f[J], acc[b]);
+    }
+#pragma unroll
+    for (int r = 0; r < 4; r++)
+#pragma unroll
+      for (int b = 0; b < nb; b++) cur[r][b] = nxt[r][b];
+  }
+  double* P = part + chunk * NB * NB;
+  auto put = [&](int I, int J, int pi, int pj, double s) {
+    const int pr = 16 * V * (I / V) + V * pi + I % V, pc = 16 * V * (J / V) + V * pj + J % V;
+    if (I == J && pr > pc) return;
+    P[int64_t(pr < pc ? pr : pc) * NB + (pr < pc ? pc : pr)] = s;
+  };
+  store_gram<nb, WPC>(acc, red, put);
+}
+
+// A fragments of 16 rows for the products: a[c V + e] is row base + i, column
+// 4 V c + V g + e (k-step c V + e)
+template <class TS, int KS, int V>
+PC_DEV void load_afrag(const TS* __restrict__ X, int64_t ldx, int n, int64_t row, int64_t row1, TS* a) {
+  const int g = (threadIdx.x & 63) >> 4;
+  const TS* xr = X + (row < row1 ? row : row1 - 1) * ldx;
+#pragma unroll
+  for (int c = 0; c < KS / V; c++) {
+    const int col = 4 * V * c + V * g;
+    if (4 * V * c < n) load_vec<TS, V>(xr + (col < n ? col : 0), a + c * V);  // uniform: whole k-steps beyond n stay out
+  }
+}
+template <class TS, int V>
+PC_DEV double afrag_value(TS x, int st, int n, bool rv, int center, double mu, double var) {
+  const int g = (threadIdx.x & 63) >> 4;
+  double v = double(x);
+  if (center) v = center == 2 ? (v - mu) / var : v - mu;
+  return rv && 4 * V * (st / V) + V * g + st % V < n ? v : 0.0;
+}
+// W (ld ldw) into LDS in B-fragment order: Wl[(st nbl + J) 64 + l] is row
+// 4 V (st / V) + V g + st % V, column col0 + colmap(J, i); zero beyond n rows / ldw columns
+template <int KS, int NBL, int V, class Map>
+PC_DEV void stage_w(const double* __restrict__ W, int n, int ldw, int col0, double* Wl, Map colmap) {
+  for (int idx = threadIdx.x; idx < KS * NBL * 64; idx += DNT) {
+    const int lane = idx & 63, sj = idx >> 6, st = sj / NBL, J = sj - st * NBL;
+    const int k = 4 * V * (st / V) + V * (lane >> 4) + st % V, col = col0 + colmap(J, lane & 15);
+    Wl[idx] = k < n && col < ldw ? W[int64_t(k) * ldw + col] : 0.0;
+  }
+}
+
+// P2: Z = Yc W in registers, then its Gram.  W upper triangular when `upper`:
+// column block J takes the k-steps below 16 (J + 1) only (the rest are exact zeros).
+template <class TS, int NB, int V>
+__global__ __launch_bounds__(DNT) void k_dzgram_f64(const TS* __restrict__ X, int64_t ldx, int64_t m, int n, int center,
+                                                    const double* mean_in, const double* var_in,
+                                                    const double* __restrict__ W, int upper, int chunks, int64_t rpc,
+                                                    double* __restrict__ part, int64_t zx, int64_t zb) {
+  X = zoff(X, zx);
+  mean_in = zoff(mean_in, zb);
+  var_in = zoff(var_in, zb);
+  W = zoff(W, zb);
+  part = zoff(part, zb);
+  constexpr int nb = NB / 16, NBLK = nb * (nb + 1) / 2, KS = NB / 4;
+  constexpr int WPC = chunk_waves(NB);
+  constexpr int WL = KS * nb * 64, RL = WPC > 1 ? DNW * 2 * 256 : 1;
+  __shared__ double sm[WL > RL ? WL : RL];  // W fragments, then the waves' partial Grams
+  const int w = threadIdx.x >> 6, l = threadIdx.x & 63, i = l & 15;
+  stage_w<KS, nb, V>(W, n, NB, 0, sm, [](int J, int j) { return 16 * J + j; });
+  const int64_t chunk = int64_t(blockIdx.x) * (DNW / WPC) + w / WPC;
+  const int64_t row0 = chunk * rpc;
+  const int64_t row1 = WPC == 1 && chunk >= chunks ? row0 : row0 + rpc < m ? row0 + rpc : m;
+  d4 acc[NBLK];
+#pragma unroll
+  for (int b = 0; b < NBLK; b++) acc[b] = d4{0, 0, 0, 0};
+  TS cur[KS] = {}, nxt[KS] = {};
+  double mu = 0.0, var = 1.0, mu_n = 0.0, var_n = 1.0;
+  auto load = [&](int64_t t, TS* a, double& mu_, double& var_) {
+    const int64_t row = t + i, rc = row < row1 ? row : row1 - 1;
+    load_afrag<TS, KS, V>(X, ldx, n, row, row1, a);
+    if (center) mu_ = mean_in[rc];
+    if (center == 2) var_ = var_in[rc];
+  };
+  int64_t t = row0 + 16 * (w % WPC);
+  if (t < row1) load(t, cur, mu, var);
+  __syncthreads();
+  for (; t < row1; t += 16 * WPC) {
+    if (t + 16 * WPC < row1) load(t + 16 * WPC, nxt, mu_n, var_n);
+    const bool rv = t + i < row1;
+    asm volatile("" ::: "memory");  // keep W's fragments in LDS: hoisted into registers they spill
+    d4 z[nb];
+#pragma unroll
+    for (int J = 0; J < nb; J++) z[J] = d4{0, 0, 0, 0};
+#pragma unroll
+    for (int st = 0; st < KS; st++) {
+      const double a = afrag_value<TS, V>(cur[st], st, n, rv, center, mu, var);
+#pragma unroll
+      for (int J = 0; J < nb; J++)
+        if (!upper || 4 * V * (st / V) < 16 * (J + 1)) z[J] = mfma64(a, sm[(st * nb + J) * 64 + l], z[J]);
+    }
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+      int b = 0;
+#pragma unroll
+      for (int I = 0; I < nb; I++)
+#pragma unroll
+        for (int J = I; J < nb; J++, b++) acc[b] = mfma64(z[I][r], z[J][r], acc[b]);
+    }
+#pragma unroll
+    for (int st = 0; st < KS; st++) cur[st] = nxt[st];
+    mu = mu_n;
+    var = var_n;
+  }
+  if (WPC == 1 && chunk >= chunks) return;
+  double* P = part + chunk * NB * NB;
+  store_gram<nb, WPC>(acc, sm, [&](int I, int J, int pi, int pj, double s) {
+    if (I == J && pi > pj) return;
+    P[int64_t(16 * I + pi) * NB + 16 * J + pj] = s;
+  });
+}
+
+// C = Yc W, W (KB x ldw, at most 128 KB of it per column slice) resident in LDS.
+// A wave takes R 16-row blocks per turn, every k in registers, and writes CV
+// consecutive columns per lane.  blockIdx.y: column slice of NCB.
+template <class TS, class TO, int KB, int NCB, int V, int CV>
+__global__ __launch_bounds__(DNT) void k_dgemm_f64(const TS* __restrict__ X, int64_t ldx, int64_t m, int n, int center,
+                                                   const double* mean_in, const double* var_in,
+                                                   const double* __restrict__ W, int ldw, int nc,
+                                                   TO* __restrict__ C, int64_t ldc, int64_t zx, int64_t zb,
+                                                   int64_t zc) {
+  X = zoff(X, zx);
+  mean_in = zoff(mean_in, zb);
+  var_in = zoff(var_in, zb);
+  W = zoff(W, zb);
+  C = zoff(C, zc);
+  constexpr int KS = KB / 4, nbl = NCB / 16, R = KB > 64 ? 1 : 2;
+  __shared__ double Wl[KS * nbl * 64];
+  const int w = threadIdx.x >> 6, l = threadIdx.x & 63, i = l & 15, g = l >> 4;
+  const int col0 = blockIdx.y * NCB;
+  stage_w<KS, nbl, V>(W, n, ldw, col0, Wl, [](int J, int j) { return 16 * CV * (J / CV) + CV * j + J % CV; });
+  const int64_t step = int64_t(gridDim.x) * DNW * 16 * R;
+  TS cur[R][KS] = {}, nxt[R][KS] = {};
+  double mu[R] = {}, var[R], mu_n[R] = {}, var_n[R];
+#pragma unroll
+  for (int q = 0; q < R; q++) var[q] = var_n[q] = 1.0;
+  auto load = [&](int64_t t, TS (*a)[KS], double* mu_, double* var_) {
+#pragma unroll
+    for (int q = 0; q < R; q++) {
+      const int64_t row = t + 16 * q + i, rc = row < m ? row : m - 1;
+      load_afrag<TS, KS, V>(X, ldx, n, row, m, a[q]);
+      if (center) mu_[q] = mean_in[rc];
+      if (center == 2) var_[q] = var_in[rc];
+    }
+  };
+  int64_t t = (int64_t(blockIdx.x) * DNW + w) * 16 * R;
+  if (t < m) load(t, cur, mu, var);
+  __syncthreads();
+  for (; t < m; t += step) {
+    if (t + step < m) load(t + step, nxt, mu_n, var_n);
+    double a[R][KS];
+#pragma unroll
+    for (int q = 0; q < R; q++)
+#pragma unroll
+      for (int st = 0; st < KS; st++)
+        a[q][st] = afrag_value<TS, V>(cur[q][st], st, n, t + 16 * q + i < m, center, mu[q], var[q]);
+#pragma unroll 1
+    for (int q0 = 0; q0 < nbl / CV; q0++) {
+      if (col0 + 16 * CV * q0 >= nc) break;
+      d4 z[R][CV];
+#pragma unroll
+      for (int q = 0; q < R; q++)
+#pragma unroll
+        for (int u = 0; u < CV; u++) z[q][u] = d4{0, 0, 0, 0};
+      const double* wq = Wl + q0 * CV * 64 + l;
+#pragma unroll
+      for (int st = 0; st < KS; st++) {
+        if (4 * V * (st / V) < n) {
+#pragma unroll
+          for (int u = 0; u < CV; u++) {
+            const double b = wq[(st * nbl + u) * 64];
+#pragma unroll
+            for (int q = 0; q < R; q++) z[q][u] = mfma64(a[q][st], b, z[q][u]);
+          }
+        }
+      }
+      const int col = col0 + 16 * CV * q0 + CV * i;
+#pragma unroll
+      for (int q = 0; q < R; q++)
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+          const int64_t row = t + 16 * q + 4 * r + g;
+          TO o[CV];
+#pragma unroll
+          for (int u = 0; u < CV; u++) o[u] = TO(z[q][u][r]);
+          if (row < m && col < nc) store_vec<TO, CV>(C + row * ldc + col, o);
+        }
+    }
+#pragma unroll
+    for (int q = 0; q < R; q++) {
+#pragma unroll
+      for (int st = 0; st < KS; st++) cur[q][st] = nxt[q][st];
+      mu[q] = mu_n[q];
+      var[q] = var_n[q];
+    }
+  }
+}
+
+// cross product of a chunk's rows: A^T B, both at most 64 columns
+template <class TS, int PB, int QB, int V>
+__global__ __launch_bounds__(DNT) void k_dxgram_f64(const TS* __restrict__ A, int64_t lda, int p,
+                                                    const TS* __restrict__ B, int64_t ldb, int q, int64_t m,
+                                                    int64_t rpc, double* __restrict__ part) {
+  constexpr int pb = PB / 16, qb = QB / 16, NBLK = pb * qb;
+  // k-steps per turn: current and next rows beside the accumulators in 256 registers
+  constexpr int RS = (pb + qb) * int(sizeof(TS)) * 2 + NBLK * 8 > 200 ? 2 : 4;
+  constexpr int unit = DNW * 4 * RS;
+  __shared__ double red[DNW * 2 * 256];
+  const int w = threadIdx.x >> 6, l = threadIdx.x & 63, i = l & 15, g = l >> 4;
+  const int64_t row0 = int64_t(blockIdx.x) * rpc;
+  const int64_t row1 = row0 + rpc < m ? row0 + rpc : m;
+  bool ca[pb], cb[qb];
+#pragma unroll
+  for (int b = 0; b < pb; b++) ca[b] = 16 * V * (b / V) + V * i + b % V < p;
+#pragma unroll
+  for (int b = 0; b < qb; b++) cb[b] = 16 * V * (b / V) + V * i + b % V < q;
+  d4 acc[NBLK];
+#pragma unroll
+  for (int b = 0; b < NBLK; b++) acc[b] = d4{0, 0, 0, 0};
+  TS xa[RS][pb], xb[RS][qb], na[RS][pb], nq[RS][qb];
+  int64_t t = row0 + 4 * RS * w;
+  if (t < row1) {
+    load_rows<TS, pb, V, RS>(A, lda, p, t, row1, xa);
+    load_rows<TS, qb, V, RS>(B, ldb, q, t, row1, xb);
+  }
+  for (; t < row1; t += unit) {
+    if (t + unit < row1) {
+      load_rows<TS, pb, V, RS>(A, lda, p, t + unit, row1, na);
+      load_rows<TS, qb, V, RS>(B, ldb, q, t + unit, row1, nq);
+    }
+#pragma unroll
+    for (int r = 0; r < RS; r++) {
+      const bool rv = t + 4 * r + g < row1;
+      double fa[pb], fb[qb];
+#pragma unroll
+      for (int b = 0; b < pb; b++) fa[b] = rv && ca[b] ? double(xa[r][b]) : 0.0;
+#pragma unroll
+      for (int b = 0; b < qb; b++) fb[b] = rv && cb[b] ? double(xb[r][b]) : 0.0;
+#pragma unroll
+      for (int I = 0; I < pb; I++)
+#pragma unroll
+        for (int J = 0; J < qb; J++) acc[I * qb + J] = mfma64(fa[I], fb[J], acc[I * qb + J]);
+    }
+#pragma unroll
+    for (int r = 0; r < RS; r++) {
+#pragma unroll
+      for (int b = 0; b < pb; b++) xa[r][b] = na[r][b];
+#pragma unroll
+      for (int b = 0; b < qb; b++) xb[r][b] = nq[r][b];
+    }
+  }
+  double* P = part + int64_t(blockIdx.x) * PB * QB;
+  sum_waves<NBLK>(acc, red, [&](int blk, int pi, int pj, double s) {
+    const int I = blk / qb, J = blk - I * qb;
+    P[int64_t(16 * V * (I / V) + V * pi + I % V) * QB + 16 * V * (J / V) + V * pj + J % V] = s;
+  });
+}
+
+template <int N> using Int = std::integral_constant<int, N>;
+
+template <class F>
+int with_nb(int n, F&& f) {
+  if (n <= 16) return f(Int<16>{});
+  if (n <= 32) return f(Int<32>{});
+  if (n <= 48) return f(Int<48>{});
+  if (n <= 64) return f(Int<64>{});
+  return -1;
+}
+
+// widest vector (4, 2, 1 elements, at most 16 bytes) that n columns, the leading
+// dimension and the base address allow; max: the caller's limit
+template <class TS>
+int vec_width(const void* p, int64_t ld, int64_t n, int64_t zstride, int max) {
+  for (int v = int(16 / sizeof(TS)); v > 1; v /= 2)
+    if (v <= max && n % v == 0 && ld % v == 0 && reinterpret_cast<uintptr_t>(p) % (v * sizeof(TS)) == 0 &&
+        zstride % int64_t(v * sizeof(TS)) == 0)
+      return v;
+  return 1;
+}
+template <class TS, class F>
+int with_vec(int v, F&& f) {
+  if constexpr (sizeof(TS) == 4)
+    if (v >= 4) return f(Int<4>{});
+  if (v >= 2) return f(Int<2>{});
+  return f(Int<1>{});
+}
+
+template <class TS>
+int dgram_t(hipStream_t st, const TS* X, int64_t ldx, int64_t m, int n, int center, const double* mean_in,
+            const double* var_in, double* mean_out, double* var_out, const double* W, int chunks, int64_t tpc,
+            double* part, const PassBatch& bz, bool upper) {
+  const int64_t rpc = tpc * (n <= 32 ? 32 : 128);
+  return with_nb(n, [&](auto nbc) {
+    constexpr int NB = decltype(nbc)::value;
+    const dim3 g(unsigned(ceil_div(chunks, DNW / chunk_waves(NB))), 1, unsigned(bz.nz));
+    // the Gram's V column blocks have to exist: 48 columns are three blocks; up to 32
+    // columns Z's k-steps stay in ascending order
+    const int vmax = W ? (NB <= 32 ? 1 : 4) : NB == 64 ? 4 : NB == 32 ? 2 : 1;
+    return with_vec<TS>(vec_width<TS>(X, ldx, n, bz.zx, vmax), [&](auto vc) {
+      constexpr int V = decltype(vc)::value;
+      if (W) {
+        if constexpr (NB > 32 || V == 1)
+          hipLaunchKernelGGL((k_dzgram_f64<TS, NB, V>), g, dim3(DNT), 0, st, X, ldx, m, n, center, mean_in, var_in, W,
+                             upper ? 1 : 0, chunks, rpc, part, bz.zx, bz.zb);
+      } else {
+        if constexpr ((NB / 16) % V == 0)
+          hipLaunchKernelGGL((k_dgram_f64<TS, NB, V>), g, dim3(DNT), 0, st, X, ldx, m, n, center, mean_out, var_out,
+                             chunks, rpc, part, bz.zx, bz.zb);
+      }
+      return 0;
+    });
+  });
+}
+
+template <class TS, class TO>
+int dgemm_t(hipStream_t st, const TS* X, int64_t ldx, int64_t m, int n, int center, const double* mean_in,
+            const double* var_in, const double* W, int ldw, int nc, int chunks, TO* C, int64_t ldc,
+            const PassBatch& bz) {
+  const int vx = vec_width<TS>(X, ldx, n, bz.zx, 4), vc = vec_width<TO>(C, ldc, nc, bz.zc, 4);
+  auto go = [&](auto kc, auto ncc) {
+    constexpr int KB = decltype(kc)::value, NCB = decltype(ncc)::value;
+    return with_vec<TS>(vx, [&](auto v_) {
+      return with_vec<TO>(NCB / 16 < vc ? NCB / 16 : vc, [&](auto c_) {
+        constexpr int V = decltype(v_)::value, CV = decltype(c_)::value;
+        if constexpr ((NCB / 16) % CV == 0)
+          hipLaunchKernelGGL((k_dgemm_f64<TS, TO, KB, NCB, V, CV>),
+                             dim3(unsigned(chunks), unsigned(ceil_div(nc, NCB)), unsigned(bz.nz)), dim3(DNT), 0, st, X,
+                             ldx, m, n, center, mean_in, var_in, W, ldw, nc, C, ldc, bz.zx, bz.zb, bz.zc);
+        return 0;
+      });
+    });
+  };
+  auto cols = [&](auto kc) {
+    constexpr int KB = decltype(kc)::value;
+    if (nc <= 16) return go(kc, Int<16>{});
+    if (nc <= 32) return go(kc, Int<32>{});
+    if (nc <= 64) return go(kc, Int<64>{});
+    if (KB > 64 || nc <= 128) return go(kc, Int<128>{});
+    if constexpr (KB <= 64) return go(kc, Int<256>{});
+    return -1;
+  };
+  if (n <= 16) return cols(Int<16>{});
+  if (n <= 32) return cols(Int<32>{});
+  if (n <= 64) return cols(Int<64>{});
+  if (n <= 128) return cols(Int<128>{});
+  return -1;
+}
+
+template <class TS>
+int dxgram_t(hipStream_t st, const TS* A, int64_t lda, int p, const TS* B, int64_t ldb, int q, int64_t m, int chunks,
+             int64_t tpc, double* part) {
+  return with_nb(p, [&](auto pc_) {
+    return with_nb(q, [&](auto qc_) {
+      constexpr int PB = decltype(pc_)::value, QB = decltype(qc_)::value;
+      constexpr int VM = PB == 64 && QB == 64 ? 4 : PB % 32 == 0 && QB % 32 == 0 ? 2 : 1;
+      const int va = vec_width<TS>(A, lda, p, 0, VM), vb = vec_width<TS>(B, ldb, q, 0, VM);
+      return with_vec<TS>(va < vb ? va : vb, [&](auto vc) {
+        constexpr int V = decltype(vc)::value;
+        if constexpr (V <= VM)
+          hipLaunchKernelGGL((k_dxgram_f64<TS, PB, QB, V>), dim3(unsigned(chunks)), dim3(DNT), 0, st, A, lda, p, B,
+                             ldb, q, m, tpc * 128, part);
+        return 0;
+      });
+    });
+  });
+}
+
+}  // namespace
+
+// Row chunks of the direct Grams, from m and the columns alone; *tpc: turns of 32
+// rows (up to 32 columns, one wave per chunk) or of 128 (at most 512 chunks, two
+// workgroups per CU, of at least 256 rows: a 64-column slab is 32 KB to write and sum)
+int d64_gram_chunks(int64_t m, int n, int64_t* tpc) {
+  int64_t tiles, per;
+  if (n <= 32) {
+    tiles = ceil_div(m, 32);
+    per = ceil_div(tiles, stream_chunks(m, 32));
+  } else {
+    tiles = ceil_div(m, 128);
+    per = ceil_div(tiles, 512);
+    if (per < 2) per = 2;
+  }
+  *tpc = per;
+  return int(ceil_div(tiles, per));
+}
+// Workgroups of the direct product: enough to fill the CUs at the LDS its W takes,
+// no more than there are turns of work.
+int d64_gemm_chunks(int64_t m, int n, int nc) {
+  const int64_t turns = ceil_div(m, DNW * (n > 64 ? 16 : 32));
+  const int kb = n <= 16 ? 16 : n <= 32 ? 32 : n <= 64 ? 64 : 128;
+  const int64_t lds = int64_t(kb) * 8 * (nc <= 16 ? 16 : nc <= 32 ? 32 : nc <= 64 ? 64 : nc <= 128 || n > 64 ? 128 : 256);
+  const int64_t fit = lds > 80 * 1024 ? 1 : lds > 40 * 1024 ? 2 : 4;
+  const int64_t want = 256 * fit;
+  return int(turns < want ? turns : want);
+}
+
+// row chunks of the direct cross products, turns of 128 rows
+int d64_xgram_chunks(int64_t m, int64_t* tpc) { return d64_gram_chunks(m, kDirectGram, tpc); }
+
+int launch_d64_gram(hipStream_t st, pc_dtype dt, const void* X, int64_t ldx, int64_t m, int n, int center,
+                    const double* mean_in, const double* var_in, double* mean_out, double* var_out, const double* W,
+                    int chunks, int64_t tpc, double* part, const PassBatch& bz, bool upper) {
+  if (dt == PC_F64)
+    return dgram_t<double>(st, (const double*)X, ldx, m, n, center, mean_in, var_in, mean_out, var_out, W, chunks, tpc,
+                           part, bz, upper);
+  return dgram_t<float>(st, (const float*)X, ldx, m, n, center, mean_in, var_in, mean_out, var_out, W, chunks, tpc,
+                        part, bz, upper);
+}
+int launch_d64_gemm(hipStream_t st, pc_dtype dt, const void* X, int64_t ldx, int64_t m, int n, int center,
+                    const double* mean_in, const double* var_in, const double* W, int ldw, int nc, int chunks, void* C,
+                    int64_t ldc, const PassBatch& bz) {
+  if (dt == PC_F64)
+    return dgemm_t<double, double>(st, (const double*)X, ldx, m, n, center, mean_in, var_in, W, ldw, nc, chunks,
+                                   (double*)C, ldc, bz);
+  return dgemm_t<float, float>(st, (const float*)X, ldx, m, n, center, mean_in, var_in, W, ldw, nc, chunks, (float*)C,
+                               ldc, bz);
+}
+int launch_d64_xgram(hipStream_t st, pc_dtype dt, const void* A, int64_t lda, int p, const void* B, int64_t ldb, int q,
+                     int64_t m, int chunks, int64_t tpc, double* part) {
+  if (dt == PC_F64)
+    return dxgram_t<double>(st, (const double*)A, lda, p, (const double*)B, ldb, q, m, chunks, tpc, part);
+  return dxgram_t<float>(st, (const float*)A, lda, p, (const float*)B, ldb, q, m, chunks, tpc, part);
+}

@@ -1,4 +1,6 @@
-// FP64 MFMA streaming kernels (v_mfma_f64_16x16x4f64) of the plain POD path.
+// FP64 MFMA streaming kernels (v_mfma_f64_16x16x4f64) of the plain POD path, for
+// operands wider than k_direct_f64.hip takes (Grams over 64 columns, products over
+// more than 128 inputs).
 //
 // A pass over the tall matrix A (m x n, row-major, n <= NB) is split into
 // `chunks` contiguous row ranges, one workgroup each (8 waves).  Each
@@ -383,6 +385,7 @@ template <class F>
 int dispatch_nb(int n, F&& f) {
   if (n <= 16) return f(std::integral_constant<int, 16>{});
   if (n <= 32) return f(std::integral_constant<int, 32>{});
+  if (n <= 48) return f(std::integral_constant<int, 48>{});
   if (n <= 64) return f(std::integral_constant<int, 64>{});
   if (n <= 128) return f(std::integral_constant<int, 128>{});
   if (n <= 256) return f(std::integral_constant<int, 256>{});
@@ -391,8 +394,28 @@ int dispatch_nb(int n, F&& f) {
 
 }  // namespace
 
-int f64_nb(int n) { return n <= 16 ? 16 : n <= 32 ? 32 : n <= 64 ? 64 : n <= 128 ? 128 : n <= 256 ? 256 : -1; }
-int f64_tile_rows() { return TR; }
+int f64_nb(int n) {
+  return n <= 16 ? 16 : n <= 32 ? 32 : n <= 48 ? 48 : n <= 64 ? 64 : n <= 128 ? 128 : n <= 256 ? 256 : -1;
+}
+// row chunks of the Gram passes over n columns (k_direct_f64.hip up to 64)
+int f64_gram_chunks(int64_t m, int n, int64_t* tpc) {
+  if (n <= kDirectGram) return d64_gram_chunks(m, n, tpc);
+  const int c = stream_chunks(m, TR);
+  *tpc = ceil_div(ceil_div(m, TR), c);
+  return c;
+}
+// cross products take the direct kernel when both operands are narrow
+int f64_xgram_chunks(int64_t m, int p, int q, int64_t* tpc) {
+  if (p <= kDirectGram && q <= kDirectGram) return d64_xgram_chunks(m, tpc);
+  const int c = stream_chunks(m, TR);
+  *tpc = ceil_div(ceil_div(m, TR), c);
+  return c;
+}
+// rows of one turn of a product pass over n inputs, and its workgroups
+int f64_gemm_rows(int n) { return n > kDirectProduct ? TR : n > 64 ? 128 : 256; }
+int f64_gemm_chunks(int64_t m, int n, int nc) {
+  return n > kDirectProduct ? stream_chunks(m, TR) : d64_gemm_chunks(m, n, nc);
+}
 
 // P1 / P2 launchers -----------------------------------------------------------
 template <class TS>
@@ -401,20 +424,26 @@ static int launch_gram_t(hipStream_t st, const TS* X, int64_t ldx, int64_t m, in
                          const double* W, int chunks, int64_t tpc, double* part, const PassBatch& bz, bool upper) {
   return dispatch_nb(n, [&](auto nbc) {
     constexpr int NB = decltype(nbc)::value;
-    const dim3 g(unsigned(chunks), 1, unsigned(bz.nz));
-    if (W)
-      hipLaunchKernelGGL((k_gram_f64<TS, NB, true>), g, dim3(NTH), 0, st, X, ldx, m, n, center, stats_in, mean_in,
-                         var_in, mean_out, var_out, W, tpc, part, upper ? 1 : 0, bz.zx, bz.zb);
-    else
-      hipLaunchKernelGGL((k_gram_f64<TS, NB, false>), g, dim3(NTH), 0, st, X, ldx, m, n, center, stats_in, mean_in,
-                         var_in, mean_out, var_out, W, tpc, part, 0, bz.zx, bz.zb);
-    return 0;
+    if constexpr (NB > kDirectGram) {
+      const dim3 g(unsigned(chunks), 1, unsigned(bz.nz));
+      if (W)
+        hipLaunchKernelGGL((k_gram_f64<TS, NB, true>), g, dim3(NTH), 0, st, X, ldx, m, n, center, stats_in, mean_in,
+                           var_in, mean_out, var_out, W, tpc, part, upper ? 1 : 0, bz.zx, bz.zb);
+      else
+        hipLaunchKernelGGL((k_gram_f64<TS, NB, false>), g, dim3(NTH), 0, st, X, ldx, m, n, center, stats_in, mean_in,
+                           var_in, mean_out, var_out, W, tpc, part, 0, bz.zx, bz.zb);
+      return 0;
+    }
+    return -1;
   });
 }
 
 int launch_gram_f64(hipStream_t st, pc_dtype dt, const void* X, int64_t ldx, int64_t m, int n, int center,
                     int stats_in, const double* mean_in, const double* var_in, double* mean_out, double* var_out,
                     const double* W, int chunks, int64_t tpc, double* part, const PassBatch& bz, bool upper) {
+  if (n <= kDirectGram)
+    return launch_d64_gram(st, dt, X, ldx, m, n, center, mean_in, var_in, mean_out, var_out, W, chunks, tpc, part, bz,
+                           upper);
   if (dt == PC_F64)
     return launch_gram_t<double>(st, (const double*)X, ldx, m, n, center, stats_in, mean_in, var_in, mean_out, var_out,
                                  W, chunks, tpc, part, bz, upper);
@@ -429,18 +458,23 @@ static int launch_gemm_t(hipStream_t st, const TS* X, int64_t ldx, int64_t m, in
   int ncb = f64_nb(nc);
   return dispatch_nb(n, [&](auto nbc) {
     constexpr int NB = decltype(nbc)::value;
-    return dispatch_nb(ncb, [&](auto ncc) {
-      constexpr int NCB = decltype(ncc)::value;
-      hipLaunchKernelGGL((k_gemm_f64<TS, TO, NB, NCB>), dim3(unsigned(chunks), 1, unsigned(bz.nz)), dim3(NTH), 0, st,
-                         X, ldx, m, n, center, mean_in, var_in, W, nc, tpc, C, ldc, bz.zx, bz.zb, bz.zc);
-      return 0;
-    });
+    if constexpr (NB > kDirectProduct) {
+      return dispatch_nb(ncb, [&](auto ncc) {
+        constexpr int NCB = decltype(ncc)::value;
+        hipLaunchKernelGGL((k_gemm_f64<TS, TO, NB, NCB>), dim3(unsigned(chunks), 1, unsigned(bz.nz)), dim3(NTH), 0, st,
+                           X, ldx, m, n, center, mean_in, var_in, W, nc, tpc, C, ldc, bz.zx, bz.zb, bz.zc);
+        return 0;
+      });
+    }
+    return -1;
   });
 }
 
 int launch_gemm_f64(hipStream_t st, pc_dtype dt, const void* X, int64_t ldx, int64_t m, int n, int center,
                     const double* mean_in, const double* var_in, const double* W, int nc, int chunks, int64_t tpc,
                     void* C, int64_t ldc, const PassBatch& bz) {
+  if (n <= kDirectProduct)
+    return launch_d64_gemm(st, dt, X, ldx, m, n, center, mean_in, var_in, W, f64_nb(nc), nc, chunks, C, ldc, bz);
   if (dt == PC_F64)
     return launch_gemm_t<double, double>(st, (const double*)X, ldx, m, n, center, mean_in, var_in, W, nc, chunks, tpc,
                                          (double*)C, ldc, bz);
@@ -458,7 +492,7 @@ static int launch_xgram_t(hipStream_t st, const T* A, int64_t lda, int p, const 
     constexpr int PB = decltype(pc_)::value;
     return dispatch_nb(qb, [&](auto qc_) {
       constexpr int QB = decltype(qc_)::value;
-      if constexpr (PB * QB <= 128 * 256) {
+      if constexpr (PB * QB <= 128 * 256 && (PB > kDirectGram || QB > kDirectGram)) {
         hipLaunchKernelGGL((k_xgram_f64<T, T, PB, QB>), dim3(chunks), dim3(NTH), 0, st, A, lda, p, B, ldb, q, m, tpc,
                            part);
         return 0;
@@ -471,6 +505,8 @@ static int launch_xgram_t(hipStream_t st, const T* A, int64_t lda, int p, const 
 
 int launch_xgram_f64(hipStream_t st, pc_dtype dt, const void* A, int64_t lda, int p, const void* B, int64_t ldb, int q,
                      int64_t m, int chunks, int64_t tpc, double* part) {
+  if (p <= kDirectGram && q <= kDirectGram)
+    return launch_d64_xgram(st, dt, A, lda, p, B, ldb, q, m, chunks, tpc, part);
   if (dt == PC_F64)
     return launch_xgram_t<double>(st, (const double*)A, lda, p, (const double*)B, ldb, q, m, chunks, tpc, part);
   return launch_xgram_t<float>(st, (const float*)A, lda, p, (const float*)B, ldb, q, m, chunks, tpc, part);

@@ -63,19 +63,21 @@ PC_DEV double block_max(double v, double* sh) {
 //   Re G_ab = P[2a][2b] + P[2a+1][2b+1], Im G_ab = P[2a][2b+1] - P[2a+1][2b].
 // Summation over chunks is in a fixed order (deterministic).
 // ---------------------------------------------------------------------------
-// Chunk sum of the partial slabs, in place into chunk 0, for the entries
-// i <= j < nr of the NB x NB slab.  A workgroup owns 64 consecutive entries
+// Chunk sum of the partial slabs (row stride ld), in place into chunk 0, for the
+// entries i < rows, j < cols (UPPER: and i <= j).  A workgroup owns 64 consecutive entries
 // and 16 chunk lanes; lane k sums chunks k, k+16, ... in four interleaved
 // accumulators combined in a fixed order, then lane 0 adds the 16 lane sums in
-// order: the summation order depends only on (chunks, NB), so results are
+// order: the summation order depends only on (chunks, ld), so results are
 // deterministic.  Entry e is read and written only by its own workgroup.
-__global__ __launch_bounds__(1024) void k_reduce_slab(double* P, int chunks, int64_t pstride, int NB, int nr, int64_t zb = 0) {
+template <bool UPPER>
+__global__ __launch_bounds__(1024) void k_reduce_slab(double* P, int chunks, int64_t pstride, int ld, int rows,
+                                                      int cols, int64_t zb = 0) {
   P = zoff(P, zb);
   __shared__ double red[16][65];
   const int le = threadIdx.x & 63, k = threadIdx.x >> 6;
   const int e = blockIdx.x * 64 + le;
-  const int i = e / NB, j = e - i * NB;
-  const bool use = e < NB * NB && i <= j && j < nr;
+  const int i = e / ld, j = e - i * ld;
+  const bool use = i < rows && j < cols && (!UPPER || i <= j);
   double s = 0.0;
   if (use) {
     const double* p = P + e;

@@ -4,7 +4,12 @@
 
 // FP64 MFMA streaming kernels (k_mfma_f64.hip); return 0, or -1 when n is too large
 int f64_nb(int n);
-int f64_tile_rows();
+// partition of the passes, from the sizes alone: row chunks of a Gram (tpc: turns
+// per chunk), rows of a product's turn and its workgroups
+int f64_gram_chunks(int64_t m, int n, int64_t* tpc);
+int f64_xgram_chunks(int64_t m, int p, int q, int64_t* tpc);
+int f64_gemm_rows(int n);
+int f64_gemm_chunks(int64_t m, int n, int nc);
 // Batched streaming passes: nz problems in one launch (blockIdx.z), the input
 // moving by zx bytes, the workspace operands by zb and the output by zc.
 struct PassBatch {
@@ -21,6 +26,23 @@ int launch_gemm_f64(hipStream_t st, pc_dtype dt, const void* X, int64_t ldx, int
                     const double* mean_in, const double* var_in, const double* W, int nc, int chunks, int64_t tpc,
                     void* C, int64_t ldc, const PassBatch& bz = PassBatch());
 int launch_xgram_f64(hipStream_t st, pc_dtype dt, const void* A, int64_t lda, int p, const void* B, int64_t ldb, int q,
+                     int64_t m, int chunks, int64_t tpc, double* part);
+
+// FP64 kernels for narrow operands (k_direct_f64.hip), reached through the launchers
+// above: Grams and cross products of at most kDirectGram real columns (their
+// fragments fit one wave's registers), products of at most kDirectProduct inputs
+// (W fits one CU's LDS in slices of 128 columns)
+constexpr int kDirectGram = 64, kDirectProduct = 128;
+int d64_gram_chunks(int64_t m, int n, int64_t* tpc);
+int d64_xgram_chunks(int64_t m, int64_t* tpc);
+int d64_gemm_chunks(int64_t m, int n, int nc);
+int launch_d64_gram(hipStream_t st, pc_dtype dt, const void* X, int64_t ldx, int64_t m, int n, int center,
+                    const double* mean_in, const double* var_in, double* mean_out, double* var_out, const double* W,
+                    int chunks, int64_t tpc, double* part, const PassBatch& bz, bool upper);
+int launch_d64_gemm(hipStream_t st, pc_dtype dt, const void* X, int64_t ldx, int64_t m, int n, int center,
+                    const double* mean_in, const double* var_in, const double* W, int ldw, int nc, int chunks, void* C,
+                    int64_t ldc, const PassBatch& bz);
+int launch_d64_xgram(hipStream_t st, pc_dtype dt, const void* A, int64_t lda, int p, const void* B, int64_t ldb, int q,
                      int64_t m, int chunks, int64_t tpc, double* part);
 
 // mixed (fp16 split) MFMA streaming kernels (k_mfma_mx2.hip): 8 waves, W operand in registers

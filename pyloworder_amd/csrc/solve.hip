@@ -450,8 +450,7 @@ int make_plan(pc_ctx* ctx, pc_dtype dt, int64_t m, int64_t n, int precision, Pla
     p.tr3 = mx2_tile_rows(p.nr);
   } else {
     p.NB = f64_nb(p.nr);
-    p.tr = f64_tile_rows();
-    p.tr3 = f64_tile_rows();
+    p.tr3 = f64_gemm_rows(p.nr);
   }
   p.wide = false;
   if (p.NB < 0 && p.mixed)
@@ -476,6 +475,15 @@ int make_plan(pc_ctx* ctx, pc_dtype dt, int64_t m, int64_t n, int precision, Pla
     p.nparts = p.chunks;
     return PC_OK;
   }
+  if (!p.mixed) {
+    p.chunks = f64_gram_chunks(m, p.nr, &p.tpc);
+    p.chunks3 = f64_gemm_chunks(m, p.nr, p.nr);
+    p.tpc3 = ceil_div(ceil_div(m, p.tr3), p.chunks3);
+    p.chunks2 = p.chunks;
+    p.tpc2 = p.tpc;
+    p.nparts = p.chunks;
+    return PC_OK;
+  }
   p.chunks = stream_chunks(m, p.tr);
   // mixed P1 and P2: at most 512 chunks (two workgroups per CU in turn for
   // long inputs), half the partial slabs to write and sum
@@ -483,11 +491,11 @@ int make_plan(pc_ctx* ctx, pc_dtype dt, int64_t m, int64_t n, int precision, Pla
     const int c512 = int(ceil_div(tiles, ceil_div(tiles, 512)));
     return c512 < c ? c512 : c;
   };
-  if (p.mixed) p.chunks = cap512(ceil_div(m, p.tr), p.chunks);
+  p.chunks = cap512(ceil_div(m, p.tr), p.chunks);
   p.tpc = ceil_div(ceil_div(m, p.tr), p.chunks);
   p.chunks3 = stream_chunks(m, p.tr3);
   p.tpc3 = ceil_div(ceil_div(m, p.tr3), p.chunks3);
-  p.chunks2 = p.mixed ? cap512(ceil_div(m, p.tr3), p.chunks3) : p.chunks3;
+  p.chunks2 = cap512(ceil_div(m, p.tr3), p.chunks3);
   p.tpc2 = ceil_div(ceil_div(m, p.tr3), p.chunks2);
   p.nparts = p.chunks;
   return PC_OK;
@@ -943,8 +951,8 @@ static void reduce_gram(hipStream_t st, const Plan& p, const double* part, int n
 // chunk 0 is unpacked into the symmetric / Hermitian n x n Gram
 static void reduce_slab(hipStream_t st, const Plan& p, const double* part, int nparts, int nz, int64_t zb) {
   const int64_t e = int64_t(p.NB) * p.NB;
-  hipLaunchKernelGGL(k_reduce_slab, dim3(unsigned(ceil_div(e, 64)), 1, nz), dim3(1024), 0, st,
-                     const_cast<double*>(part), nparts, e, p.NB, p.nr, zb);
+  hipLaunchKernelGGL(k_reduce_slab<true>, dim3(unsigned(ceil_div(e, 64)), 1, nz), dim3(1024), 0, st,
+                     const_cast<double*>(part), nparts, e, p.NB, p.nr, p.nr, zb);
 }
 template <>
 void reduce_gram<double>(hipStream_t st, const Plan& p, const double* part, int nparts, double* G, int nz,
