@@ -418,6 +418,8 @@ __global__ __launch_bounds__(256) void k_gemm_small(int opA, int opB, int M, int
 // inter-workgroup waiting is involved; the stream orders the launches.
 //   state: [0] done, [1 + s] rotated-in-sweep-s flags;  dstate[0] = negligible
 //   squared column norm (eps^2 rows ||H||_F^2).
+// Complex problems; real ones take the Gram-driven steps of k_jacobi.hip, which
+// keep G scaled by the power of two dstate[1] and dstate[0] with it.
 // ---------------------------------------------------------------------------
 constexpr int BJ_LDS = 131072;
 
@@ -440,11 +442,22 @@ __global__ __launch_bounds__(NT) void k_bjac_init(const T* H, int ldh, int rows,
     f += abs2_(H[int64_t(k) * ldh + i]);
   }
   f = block_sum(f, sh);
-  if (threadIdx.x == 0) dstate[0] = 2.220446049250313e-16 * 2.220446049250313e-16 * double(rows) * f;
+  if (threadIdx.x == 0) {
+    double sc = 1.0;
+    if constexpr (std::is_same<T, double>::value) {
+      if (f > 0.0 && isfinite(f)) sc = ldexp(1.0, min(96 - ilogb(f), 1000));  // H^T H sc: trace about 2^96
+      dstate[1] = sc;
+    }
+    dstate[0] = 2.220446049250313e-16 * 2.220446049250313e-16 * double(rows) * (f * sc);
+  }
 }
 
-// player sitting at slot k of step s in the circle schedule of N players
-PC_DEV int rr_player(int k, int s, int N) { return k == 0 ? 0 : 1 + ((k - 1 + s) % (N - 1)); }
+// player sitting at slot k < N of step s < N - 1 in the circle schedule of N players:
+// 0 for slot 0, else 1 + (k - 1 + s) mod (N - 1), the sum below 2 (N - 1)
+PC_DEV int rr_player(int k, int s, int N) {
+  const int x = k + s;
+  return k == 0 ? 0 : x >= N ? x - (N - 1) : x;
+}
 
 template <class T>
 __global__ __launch_bounds__(NT) void k_bjac_step(T* H, int ldh, int rows, int cols, T* J, int ldj, int b, int nb2,
@@ -549,362 +562,8 @@ __global__ void k_bjac_check(int* state, int sweep, int64_t zb = 0) {
   if (threadIdx.x == 0 && !state[0] && state[1 + sweep] == 0) state[0] = 1;
 }
 
-// ---------------------------------------------------------------------------
-// Block step of the real one-sided Jacobi driven by the Gram of the block
-// pair (rows <= 256, blocks of GB = 16 columns).  Per launch and workgroup:
-//   1. stage the pair's 32 columns of H in LDS;
-//   2. G = Hs^T Hs with v_mfma_f64_16x16x4f64 (split over the rows, partial
-//      sums added in a fixed order);
-//   3. if no pair (u, v) of G has |G_uv| > tol sqrt(G_uu G_vv) the columns are
-//      already orthogonal to the test's accuracy: nothing is written and the
-//      sweep flag stays clear;
-//   4. otherwise cyclic two-sided Jacobi sweeps on G (16 disjoint rotations per
-//      round) accumulate the orthogonal Q, and H[:, pair] <- Hs Q and
-//      J[:, pair] <- J[:, pair] Q are formed with MFMA.
-// The rotation of columns (u, v) is the one-sided Jacobi rotation of the
-// columns themselves (same angle formula); the test in 3. always uses a Gram
-// freshly computed from the current columns, so convergence is decided by
-// the one-sided criterion.
-// ---------------------------------------------------------------------------
-constexpr int GB = 16;
-constexpr int GC = 2 * GB;
-constexpr int GLD = GC + 1;
-constexpr int GROWS = 256;
-// dstate layout of the Gram-driven steps: [0] negligible squared norm, then
-// from kBjacQOff the nb2 / 2 pair rotations (GC x GC each) and their flags
-constexpr int kBjacQOff = 4;
-constexpr int kBjacDstate = kBjacQOff + (GROWS / GB / 2) * GC * GC + GROWS / GB / 2;
-// dstate length for an n-column problem (at least kBjacDstate)
-inline int64_t bjac_dstate_len(int n) {
-  int64_t nb2 = (int64_t(n) + GB - 1) / GB;
-  nb2 += nb2 & 1;
-  const int64_t len = kBjacQOff + (nb2 / 2) * GC * GC + nb2 / 2;
-  return len > kBjacDstate ? len : kBjacDstate;
-}
-
 typedef double d4s __attribute__((ext_vector_type(4)));
 PC_DEV d4s mfma64s(double a, double b, d4s c) { return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0); }
-
-// FUSED: the step also forms H[:, pair] Q and J[:, pair] Q itself, on its one
-// workgroup (one launch per step, for solves that share the GPU with other
-// streams; rows <= GROWS); otherwise it stores Q for k_bjac_apply.  Both
-// form the same products in the same k order, so H and J do not depend on
-// the choice.  Unfused, the pair's Gram is summed over row chunks of GROWS
-// staged in turn, so any number of rows is taken (one chunk up to GROWS).
-template <bool FUSED>
-__global__ __launch_bounds__(NT) void k_bjac_gstep(double* H, int ldh, int rows, int cols, double* J, int ldj,
-                                                   int nb2, int step, int sweep, int* state, double* dstate,
-                                                   double tol, int max_inner) {
-  __shared__ double Hs[GC * (GROWS + 1)];
-  __shared__ double G[GC * GLD], G2[GC * GLD];
-  __shared__ double Q[GC * GLD], Q2[GC * GLD];
-  __shared__ double Pp[3 * 4 * 256];
-  __shared__ int need;
-  const int RP = (rows + 15) & ~15;
-  const int ld = RP + 1;
-  // the launch holds 8 workgroups per pair and only every eighth works:
-  // workgroup x runs on XCD x mod 8, so the working ones share one L2
-  if (blockIdx.x & 7) return;
-  const int p = blockIdx.x >> 3;
-  const int bi = rr_player(p, step, nb2), bj = rr_player(nb2 - 1 - p, step, nb2);
-  const int w = threadIdx.x >> 6, l = threadIdx.x & 63, lr = l & 15, lk = l >> 4;
-  auto gcol = [&](int lc) { return lc < GB ? bi * GB + lc : bj * GB + (lc - GB); };
-  // Stage row chunk c (rows c GROWS ... of the pair's columns) into Hs with
-  // leading dimension RPc + 1.  Every load is issued before the first LDS
-  // store, and those of chunk 0 together with the done flag (a converged
-  // iteration discards them): false when the iteration has converged.
-  const int nch = FUSED ? 1 : (rows + GROWS - 1) / GROWS;
-  auto chunk_rows = [&](int c) { const int rc = rows - c * GROWS; return rc < GROWS ? rc : GROWS; };
-  auto stage = [&](int c) {
-    constexpr int KL = GC * GROWS / NT;
-    const int rc = chunk_rows(c), RPc = (rc + 15) & ~15, ldc = RPc + 1;
-    const int64_t r0 = int64_t(c) * GROWS;
-    double hv[KL];
-#pragma unroll
-    for (int k = 0; k < KL; k++) {
-      const int idx = threadIdx.x + k * NT, lc = idx / RPc, i = idx - lc * RPc, gc = gcol(lc);
-      hv[k] = (idx < GC * RPc && gc < cols && i < rc) ? H[int64_t(gc) * ldh + r0 + i] : 0.0;
-    }
-    if (c == 0 && state[0]) return false;
-#pragma unroll
-    for (int k = 0; k < KL; k++) {
-      const int idx = threadIdx.x + k * NT, lc = idx / RPc, i = idx - lc * RPc;
-      if (idx < GC * RPc) Hs[lc * ldc + i] = hv[k];
-    }
-    return true;
-  };
-  if (!stage(0)) return;
-  const double negl = dstate[0];
-  if (threadIdx.x == 0) need = 0;
-  __syncthreads();
-  // G = Hs^T Hs, symmetric: waves w < 12 form the upper 16 x 16 tiles
-  // t = w >> 2 ((0,0), (0,1), (1,1)) over row quarter q = w & 3 of each
-  // chunk, and tile (0,1) is mirrored into (1,0)
-  {
-    const int t = w >> 2, q = w & 3, bI = t == 2 ? 1 : 0, bJ = t == 0 ? 0 : 1;
-    d4s acc = {0.0, 0.0, 0.0, 0.0};
-    for (int c = 0; c < nch; c++) {
-      if (c > 0) {
-        __syncthreads();  // the previous chunk is read
-        stage(c);
-        __syncthreads();
-      }
-      const int RPc = (chunk_rows(c) + 15) & ~15, ldc = RPc + 1;
-      const int kq = RPc / 4;
-      const double* ca = Hs + (16 * bI + lr) * ldc;
-      const double* cb = Hs + (16 * bJ + lr) * ldc;
-      if (t < 3) {
-        // the quarter's operands (kq / 4 <= GROWS / 16 k-steps) are read from
-        // LDS before the products, so the products do not wait on each read
-        constexpr int KS = GROWS / 16;
-        double xa[KS], xb[KS];
-#pragma unroll
-        for (int k = 0; k < KS; k++) {
-          const int k0 = q * kq + 4 * k;
-          xa[k] = 4 * k < kq ? ca[k0 + lk] : 0.0;
-          xb[k] = 4 * k < kq ? cb[k0 + lk] : 0.0;
-        }
-#pragma unroll
-        for (int k = 0; k < KS; k++)
-          if (4 * k < kq) acc = mfma64s(xa[k], xb[k], acc);
-      }
-    }
-    if (t < 3 && q > 0)
-      for (int r = 0; r < 4; r++) Pp[((q - 1) * 3 + t) * 256 + r * 64 + l] = acc[r];
-    __syncthreads();
-    if (t < 3 && q == 0) {
-      for (int q2 = 0; q2 < 3; q2++)
-        for (int r = 0; r < 4; r++) acc[r] += Pp[(q2 * 3 + t) * 256 + r * 64 + l];
-      for (int r = 0; r < 4; r++) {
-        G[(16 * bI + 4 * r + lk) * GLD + 16 * bJ + lr] = acc[r];
-        if (t == 1) G[(16 + lr) * GLD + 4 * r + lk] = acc[r];
-      }
-    }
-  }
-  __syncthreads();
-  // The first step of a sweep rotates every pair of its 2 GB columns (GC - 1
-  // rounds); later steps only the GB^2 pairs across the two blocks (GB
-  // rounds): every block meets its own columns in the first step, so a sweep
-  // still rotates each pair of columns once, in n - 1 rounds in all.
-  const bool full = step == 0;
-  for (int idx = threadIdx.x; idx < GC * GC; idx += NT) {
-    int u = idx / GC, v = idx - u * GC;
-    Q[u * GLD + v] = u == v ? 1.0 : 0.0;
-    if (u < v && (full || (u < GB && v >= GB))) {
-      double a = G[u * GLD + u], bb = G[v * GLD + v], c = G[u * GLD + v];
-      if (a > negl && bb > negl && fabs(c) > tol * sqrt(a) * sqrt(bb)) need = 1;
-    }
-  }
-  __syncthreads();
-  double* qout = dstate + kBjacQOff + int64_t(p) * GC * GC;
-  double* qflag = dstate + kBjacQOff + int64_t(nb2 / 2) * GC * GC + p;
-  if (!need) {
-    if (!FUSED && threadIdx.x == 0) *qflag = 0.0;  // k_bjac_apply leaves this pair as it is
-    return;
-  }
-  if (threadIdx.x == 0) atomicOr(&state[1 + sweep], 1);
-  // k-th pair (u < v) of round s
-  auto pair_of = [&](int k, int s, int& u, int& v) {
-    if (full) {
-      u = rr_player(k, s, GC);
-      v = rr_player(GC - 1 - k, s, GC);
-      if (u > v) { int t = u; u = v; v = t; }
-    } else {
-      u = k;
-      v = GB + (k + s) % GB;
-    }
-  };
-  // Each round applies GB disjoint rotations as G <- R^T G R and Q <- Q R:
-  // GB threads form the rotations; thread (bp, bq) of the first GB * GB then
-  // updates the 2 x 2 blocks of G and Q at rows {u_bp, v_bp} and columns
-  // {u_bq, v_bq} from the old buffers into the other ones.  The rotation of
-  // pair (u, v) zeroes G_uv: column u of R is cs e_u - sn e_v, column v is
-  // sn e_u + cs e_v, tan(2 theta) = 2 G_uv / (G_vv - G_uu), |theta| <= pi/4.
-  // Square roots and reciprocals come from the hardware estimates refined by
-  // Newton steps (one for the angle, two for cs, which fixes cs^2 + sn^2 = 1
-  // to rounding); the angle itself only steers convergence.
-  static_assert(GB * GB <= NT, "one thread per 2 x 2 block of the pair's Gram");
-  __shared__ double rc[GB], rs[GB];
-  const int bp = threadIdx.x / GB, bq = threadIdx.x % GB;
-  const int rounds = full ? GC - 1 : GB;
-  for (int inner = 0; inner < max_inner; inner++) {
-    int rotated = 0;
-    for (int s = 0; s < rounds; s++) {
-      const double* Gc = (s & 1) ? G2 : G;
-      double* Gn = (s & 1) ? G : G2;
-      const double* Qc = (s & 1) ? Q2 : Q;
-      double* Qn = (s & 1) ? Q : Q2;
-      if (threadIdx.x < GB) {
-        int u, v;
-        pair_of(threadIdx.x, s, u, v);
-        const double a = Gc[u * GLD + u], bb = Gc[v * GLD + v], c = Gc[u * GLD + v];
-        const double d = bb - a, e = 2.0 * fabs(c);
-        const double mde = fmax(fabs(d), e);
-        const int k = mde > 0.0 ? ilogb(mde) : 0;
-        const double ds = ldexp(d, -k), es = ldexp(e, -k);   // max(|ds|, es) in [1, 2)
-        const double x = ds * ds + es * es;
-        double y = __builtin_amdgcn_rsq(x);
-        y = y * (1.5 - 0.5 * x * y * y);
-        const double den = fabs(ds) + x * y;                  // |d| + hypot(d, e), scaled
-        double r = __builtin_amdgcn_rcp(den);
-        r = r * (2.0 - den * r);
-        const double t = es * r;                              // tan(theta) in [0, 1]
-        const double z = 1.0 + t * t;
-        double cs = __builtin_amdgcn_rsq(z);
-        cs = cs * (1.5 - 0.5 * z * cs * cs);
-        cs = cs * (1.5 - 0.5 * z * cs * cs);
-        double sn = cs * t;
-        if ((d < 0) != (c < 0)) sn = -sn;
-        const bool act = a > negl && bb > negl && fabs(c) > tol * sqrt(a) * sqrt(bb);
-        rc[threadIdx.x] = act ? cs : 1.0;
-        rs[threadIdx.x] = act ? sn : 0.0;
-        rotated |= act;
-      }
-      __syncthreads();
-      if (threadIdx.x < GB * GB) {
-        int up, vp, uq, vq;
-        pair_of(bp, s, up, vp);
-        pair_of(bq, s, uq, vq);
-        const double cp = rc[bp], sp = rs[bp], cq = rc[bq], sq = rs[bq];
-        const double g_uu = Gc[up * GLD + uq], g_uv = Gc[up * GLD + vq];
-        const double g_vu = Gc[vp * GLD + uq], g_vv = Gc[vp * GLD + vq];
-        const double q_uu = Qc[up * GLD + uq], q_uv = Qc[up * GLD + vq];
-        const double q_vu = Qc[vp * GLD + uq], q_vv = Qc[vp * GLD + vq];
-        // columns by pair bq, then rows by pair bp
-        const double x_uu = cq * g_uu - sq * g_uv, x_uv = sq * g_uu + cq * g_uv;
-        const double x_vu = cq * g_vu - sq * g_vv, x_vv = sq * g_vu + cq * g_vv;
-        Gn[up * GLD + uq] = cp * x_uu - sp * x_vu;
-        Gn[up * GLD + vq] = cp * x_uv - sp * x_vv;
-        Gn[vp * GLD + uq] = sp * x_uu + cp * x_vu;
-        Gn[vp * GLD + vq] = sp * x_uv + cp * x_vv;
-        Qn[up * GLD + uq] = cq * q_uu - sq * q_uv;
-        Qn[up * GLD + vq] = sq * q_uu + cq * q_uv;
-        Qn[vp * GLD + uq] = cq * q_vu - sq * q_vv;
-        Qn[vp * GLD + vq] = sq * q_vu + cq * q_vv;
-      }
-      __syncthreads();
-    }
-    // an odd number of rounds leaves the result in the second buffers
-    if (rounds & 1) {
-      for (int idx = threadIdx.x; idx < GC * GC; idx += NT) {
-        int u = idx / GC, v = idx - u * GC;
-        G[u * GLD + v] = G2[u * GLD + v];
-        Q[u * GLD + v] = Q2[u * GLD + v];
-      }
-    }
-    if (!__syncthreads_or(rotated)) break;
-  }
-  if constexpr (!FUSED) {
-    // the pair's rotation Q (row-major) for k_bjac_apply, which forms
-    // H[:, pair] Q and J[:, pair] Q over many workgroups
-    for (int idx = threadIdx.x; idx < GC * GC; idx += NT) qout[idx] = Q[(idx / GC) * GLD + idx % GC];
-    if (threadIdx.x == 0) *qflag = 1.0;
-    return;
-  }
-  // H[:, pair] = Hs Q  (row blocks of 16 rows, one wave each)
-  for (int rb = w; rb < RP / 16; rb += NT / 64) {
-    for (int cB = 0; cB < 2; cB++) {
-      d4s acc = {0.0, 0.0, 0.0, 0.0};
-      for (int k0 = 0; k0 < GC; k0 += 4)
-        acc = mfma64s(Hs[(k0 + lk) * ld + 16 * rb + lr], Q[(k0 + lk) * GLD + 16 * cB + lr], acc);
-      const int gc = gcol(16 * cB + lr);
-      for (int r = 0; r < 4; r++) {
-        const int row = 16 * rb + 4 * r + lk;
-        if (row < rows && gc < cols) H[int64_t(gc) * ldh + row] = acc[r];
-      }
-    }
-  }
-  // J[:, pair] = J[:, pair] Q  (J is cols x cols, column-major)
-  const int CP = (cols + 15) & ~15;
-  for (int rb = w; rb < CP / 16; rb += NT / 64) {
-    double av[GC / 4];
-    const int row = 16 * rb + lr;
-    for (int kk = 0; kk < GC / 4; kk++) {
-      const int gc = gcol(4 * kk + lk);
-      av[kk] = (gc < cols && row < cols) ? J[int64_t(gc) * ldj + row] : 0.0;
-    }
-    d4s acc[2];
-    for (int cB = 0; cB < 2; cB++) {
-      acc[cB] = d4s{0.0, 0.0, 0.0, 0.0};
-      for (int kk = 0; kk < GC / 4; kk++) acc[cB] = mfma64s(av[kk], Q[(4 * kk + lk) * GLD + 16 * cB + lr], acc[cB]);
-    }
-    for (int cB = 0; cB < 2; cB++) {
-      const int gc = gcol(16 * cB + lr);
-      for (int r = 0; r < 4; r++) {
-        const int orow = 16 * rb + 4 * r + lk;
-        if (orow < cols && gc < cols) J[int64_t(gc) * ldj + orow] = acc[cB][r];
-      }
-    }
-  }
-}
-
-// ---------------------------------------------------------------------------
-// Second half of a block step of k_bjac_gstep: H[:, pair] <- H[:, pair] Q and
-// J[:, pair] <- J[:, pair] Q with the pair's rotation Q from dstate.  One
-// workgroup per (pair, 32-row slice), so the FP64 MFMA work of the step is
-// spread over 8 (nb2 / 2) workgroups per pair instead of one; every slice
-// reads and writes only its own rows, and the products are the ones the
-// single-workgroup version formed (same k order).  nsl slices per pair
-// cover max(rows, cols) (kBjacSlices up to GROWS).
-// ---------------------------------------------------------------------------
-constexpr int kBjacSlices = GROWS / 32;
-__global__ __launch_bounds__(256) void k_bjac_apply(double* H, int ldh, int rows, int cols, double* J, int ldj,
-                                                    int nb2, int step, int sweep, int* state, const double* dstate,
-                                                    int nsl) {
-  __shared__ double Qs[GC * GLD];
-  const int p = blockIdx.x / nsl, sl = blockIdx.x % nsl;
-  const int bi = rr_player(p, step, nb2), bj = rr_player(nb2 - 1 - p, step, nb2);
-  auto gcol = [&](int lc) { return lc < GB ? bi * GB + lc : bj * GB + (lc - GB); };
-  const int w = threadIdx.x >> 6, l = threadIdx.x & 63, lr = l & 15, lk = l >> 4;
-  // wave w: matrix w >> 1 (0 H, 1 J), 16-row block w & 1 of the slice, both
-  // 16-column blocks of the pair.  Every global read (flags, Q, the slice)
-  // is issued before the first test, so the launch waits on memory once.
-  double* M = (w >> 1) ? J : H;
-  const int ld = (w >> 1) ? ldj : ldh, nr = (w >> 1) ? cols : rows;
-  const int row = 32 * sl + 16 * (w & 1);
-  const double* qin = dstate + kBjacQOff + int64_t(p) * GC * GC;
-  double av[GC / 4], qv[GC * GC / 256];
-#pragma unroll
-  for (int kk = 0; kk < GC / 4; kk++) {
-    const int gc = gcol(4 * kk + lk);
-    av[kk] = (gc < cols && row + lr < nr) ? M[int64_t(gc) * ld + row + lr] : 0.0;
-  }
-#pragma unroll
-  for (int t = 0; t < GC * GC / 256; t++) qv[t] = qin[threadIdx.x + 256 * t];
-  const int done = state[0];
-  const double rot = dstate[kBjacQOff + int64_t(nb2 / 2) * GC * GC + p];
-  // the last step of a sweep also closes it (k_bjac_check's test): every
-  // step's k_bjac_gstep has set its rotation flag by now
-  if (step == nb2 - 2 && blockIdx.x == 0 && threadIdx.x == 0 && !done && state[1 + sweep] == 0) state[0] = 1;
-  if (done || rot == 0.0) return;
-#pragma unroll
-  for (int t = 0; t < GC * GC / 256; t++) {
-    const int idx = threadIdx.x + 256 * t;
-    Qs[(idx / GC) * GLD + idx % GC] = qv[t];
-  }
-  __syncthreads();
-  double q0[GC / 4], q1[GC / 4];
-#pragma unroll
-  for (int kk = 0; kk < GC / 4; kk++) {
-    q0[kk] = Qs[(4 * kk + lk) * GLD + lr];
-    q1[kk] = Qs[(4 * kk + lk) * GLD + 16 + lr];
-  }
-  d4s acc[2] = {{0.0, 0.0, 0.0, 0.0}, {0.0, 0.0, 0.0, 0.0}};
-#pragma unroll
-  for (int kk = 0; kk < GC / 4; kk++) {
-    acc[0] = mfma64s(av[kk], q0[kk], acc[0]);
-    acc[1] = mfma64s(av[kk], q1[kk], acc[1]);
-  }
-#pragma unroll
-  for (int cB = 0; cB < 2; cB++) {
-    const int gc = gcol(16 * cB + lr);
-#pragma unroll
-    for (int r = 0; r < 4; r++) {
-      const int orow = row + 4 * r + lk;
-      if (orow < nr && gc < cols) M[int64_t(gc) * ld + orow] = acc[cB][r];
-    }
-  }
-}
 
 // One-sided Jacobi of a small problem held by a single block pair (2b <= 32
 // columns, rows <= 64), on one wavefront: 4 lanes per column pair, every

@@ -23,6 +23,7 @@
 #include "common.hpp"
 #include "kernels.hpp"
 #include "k_small.hip"
+#include "k_jacobi.hip"
 #include "k_dense.hip"
 #include "k_mwg.hip"
 
@@ -50,91 +51,111 @@ __global__ void k_status_copy(const int* src, int* dst, int64_t zs = 0, int64_t 
 }
 constexpr double kJacTolMx = 1e-8;  // Jacobi orthogonality tolerance, mixed path
 
-// One-sided block Jacobi on H (rows x cols, column-major) with J accumulated:
-// one launch per round-robin step of a sweep, a check launch per sweep.  After
-// convergence every remaining launch exits immediately.
-// Block layout of the one-sided Jacobi of a rows x cols problem: real FP64
-// with rows <= 256 takes Gram-driven MFMA steps on 16-column blocks, other
-// problems column-pair rotations staged in LDS.  b = block width, nb2 = even
+// One-sided block Jacobi on H (n x n, column-major) with J accumulated.  Block layout:
+// real problems take the Gram-driven steps of k_jacobi.hip on 16-column blocks,
+// complex ones column-pair rotations staged in LDS.  b = block width, nb2 = even
 // number of blocks (>= 2); nb2 == 2 means one block pair holds every column.
-// Gram-driven steps for real problems
 template <class T>
-void jacobi_blocks(int rows, int cols, bool& gram_steps, int& b, int& nb2) {
-  gram_steps = std::is_same<T, double>::value;
-  b = gram_steps ? GB : bjac_width(std::max(rows, cols), int(sizeof(T)));
-  nb2 = int(ceil_div(cols, b));
+void jacobi_blocks(int n, int& b, int& nb2) {
+  b = std::is_same<T, double>::value ? GB : bjac_width(n, int(sizeof(T)));
+  nb2 = int(ceil_div(n, b));
   nb2 += nb2 & 1;
   if (nb2 < 2) nb2 = 2;
 }
 
-template <class T>
-void launch_block_jacobi(pc_ctx* ctx, T* H, int ldh, int rows, int cols, T* J, int ldj, double* sig, int* state,
-                         double* dstate, int* status, double min_tol, int nz = 1, int64_t zb = 0) {
+// Sweeps are queued in batches: after the first batch the host reads the done flag
+// and stops queueing once the iteration has converged (typically after ~10 sweeps at
+// n = 256).  Under stream capture no host read is possible, so every sweep is
+// queued; converged sweeps then return at once.
+struct SweepChecks {
+  static constexpr int kFirst = 8, kNext = 2;
+  pc_ctx* ctx;
+  bool host;
+  int next = kFirst;
+  explicit SweepChecks(pc_ctx* c) : ctx(c) {
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    (void)hipStreamIsCapturing(c->stream, &cap);
+    host = cap == hipStreamCaptureStatusNone;
+  }
+  bool converged(int s, const int* state) {
+    if (!host || s != next) return false;
+    next += kNext;
+    return hipMemcpyAsync(ctx->hflag + 8, state, sizeof(int), hipMemcpyDeviceToHost, ctx->stream) == hipSuccess &&
+           hipStreamSynchronize(ctx->stream) == hipSuccess && ctx->hflag[8];
+  }
+};
+
+// real sweeps (k_jacobi.hip); Ga, Gb: two n x n buffers
+void real_sweeps(pc_ctx* ctx, double* H, int ldh, int n, double* J, int ldj, int* state, double* dstate, double tol,
+                 double* Ga, double* Gb, int nb2) {
   hipStream_t st = ctx->stream;
-  bool gram_steps;
+  const double tol2 = tol * tol;
+  if (nb2 == 2) {
+    hipLaunchKernelGGL(k_bjac_one, dim3(1), dim3(256), 0, st, H, ldh, n, J, ldj, state, (const double*)dstate, tol2,
+                       60);
+    return;
+  }
+  SweepChecks chk(ctx);
+  const int nt = int(ceil_div(n, 16)), np = nb2 / 2;
+  double* Qg = dstate + kBjacQOff;
+  for (int s = 0; s < kBjacMaxSweeps && !chk.converged(s, state); s++) {
+    hipLaunchKernelGGL(k_bjac_gram, dim3(nt * (nt + 1) / 2), dim3(256), 0, st, (const double*)H, ldh, n, nt, Ga, s,
+                       state, (const double*)dstate, tol2);
+    for (int step = 0; step < nb2 - 1; step++) {
+      auto launch = [&](auto mode, int wgs) {
+        constexpr int M = decltype(mode)::value;
+        if (step == 0)
+          hipLaunchKernelGGL((k_bjac_pair<M, true>), dim3(wgs), dim3(512), 0, st, H, ldh, n, J, ldj, (const double*)Ga,
+                             Gb, nb2, step, s, state, (const double*)dstate, Qg, tol2);
+        else
+          hipLaunchKernelGGL((k_bjac_pair<M, false>), dim3(wgs), dim3(512), 0, st, H, ldh, n, J, ldj,
+                             (const double*)Ga, Gb, nb2, step, s, state, (const double*)dstate, Qg, tol2);
+      };
+      if (n <= kJacFused) {
+        launch(std::integral_constant<int, 0>{}, np * np);
+      } else {
+        launch(std::integral_constant<int, 1>{}, (np + 1) / 2);
+        launch(std::integral_constant<int, 2>{}, np * np);
+      }
+      std::swap(Ga, Gb);
+    }
+  }
+}
+
+// Ga, Gb: two n x n buffers (real problems of more than one block pair)
+template <class T>
+void launch_block_jacobi(pc_ctx* ctx, T* H, int ldh, int n, T* J, int ldj, double* sig, int* state, double* dstate,
+                         int* status, double min_tol, T* Ga, T* Gb, int nz = 1, int64_t zb = 0) {
+  hipStream_t st = ctx->stream;
   int b, nb2;
-  // a context that shares the GPU with other streams (grouped solve) takes
-  // the one-launch steps (they hold the pair's rows in LDS: up to GROWS):
-  // there the launch count costs more than the one-CU step time the split
-  // steps save.  Both forms give the same H and J.
-  const bool fused = ctx->concurrent && rows <= GROWS;
-  jacobi_blocks<T>(rows, cols, gram_steps, b, nb2);
-  // row slices of the apply launch
-  const int nsl = std::max(kBjacSlices, int(ceil_div(std::max(rows, cols), 32)));
-  hipLaunchKernelGGL((k_bjac_init<T>), dim3(1, 1, nz), dim3(1024), 0, st, H, ldh, rows, cols, J, ldj, state, dstate,
+  jacobi_blocks<T>(n, b, nb2);
+  hipLaunchKernelGGL((k_bjac_init<T>), dim3(1, 1, nz), dim3(1024), 0, st, H, ldh, n, n, J, ldj, state, dstate,
                      kBjacMaxSweeps + 1, zb);
-  // one block pair (all columns in one workgroup): each launch iterates to
-  // convergence on its own, so a short fixed run of sweeps is queued and the
-  // host never waits; several pairs: sweeps in host-checked batches
-  const bool one_pair = nb2 == 2;
-  int max_inner = one_pair ? 60 : gram_steps ? 1 : 3;
   // relative orthogonality test |h_p^H h_q| <= tol ||h_p|| ||h_q||: the dot
   // product itself carries ~eps sqrt(rows) rounding, so tol grows with rows
-  double tol = std::max(2.220446049250313e-16 * std::max(rows, 16), min_tol);
-  // Sweeps are queued in batches: after the first batch the host reads the
-  // done flag and stops queueing once the iteration has converged (typically
-  // after ~10 sweeps at n = 256).  Under stream capture no host read is
-  // possible, so every sweep is queued; converged sweeps then return at once.
-  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-  (void)hipStreamIsCapturing(st, &cap);
-  const bool host_checks = cap == hipStreamCaptureStatusNone && !one_pair;
-  constexpr int kFirstBatch = 8, kNextBatch = 2, kOnePairSweeps = 6;
-  int next_check = kFirstBatch;
-  const int sweeps = one_pair ? kOnePairSweeps : kBjacMaxSweeps;
-  for (int s = 0; s < sweeps; s++) {
-    if (host_checks && s == next_check) {
-      next_check += kNextBatch;
-      if (hipMemcpyAsync(ctx->hflag + 8, state, sizeof(int), hipMemcpyDeviceToHost, st) == hipSuccess &&
-          hipStreamSynchronize(st) == hipSuccess && ctx->hflag[8])
-        break;
-    }
-    for (int step = 0; step < nb2 - 1; step++) {
-      if constexpr (std::is_same<T, double>::value) {
-        if (gram_steps) {
-          if (fused) {
-            hipLaunchKernelGGL(k_bjac_gstep<true>, dim3(nb2 / 2 * 8), dim3(1024), 0, st, H, ldh, rows, cols, J, ldj,
-                               nb2, step, s, state, dstate, tol, max_inner);
-            continue;
-          }
-          hipLaunchKernelGGL(k_bjac_gstep<false>, dim3(nb2 / 2 * 8), dim3(1024), 0, st, H, ldh, rows, cols, J, ldj,
-                             nb2, step, s, state, dstate, tol, max_inner);
-          hipLaunchKernelGGL(k_bjac_apply, dim3(nb2 / 2 * nsl), dim3(256), 0, st, H, ldh, rows, cols, J, ldj, nb2,
-                             step, s, state, (const double*)dstate, nsl);
-          continue;
-        }
+  const double tol = std::max(2.220446049250313e-16 * std::max(n, 16), min_tol);
+  if constexpr (std::is_same<T, double>::value) {
+    real_sweeps(ctx, H, ldh, n, J, ldj, state, dstate, tol, Ga, Gb, nb2);
+  } else {
+    // one block pair (all columns in one workgroup): each launch iterates to
+    // convergence on its own, so a short fixed run of sweeps is queued and the
+    // host never waits; several pairs: sweeps in host-checked batches
+    const bool one_pair = nb2 == 2;
+    SweepChecks chk(ctx);
+    const int sweeps = one_pair ? 6 : kBjacMaxSweeps;
+    for (int s = 0; s < sweeps && !(!one_pair && chk.converged(s, state)); s++) {
+      for (int step = 0; step < nb2 - 1; step++) {
+        if (one_pair && n <= 64 && 2 * b <= 32)
+          hipLaunchKernelGGL((k_bjac_small<T>), dim3(1, 1, nz), dim3(64), 0, st, H, ldh, n, n, J, ldj, b, s, state,
+                             dstate, tol, 60, zb);
+        else
+          hipLaunchKernelGGL((k_bjac_step<T>), dim3(nb2 / 2), dim3(1024), 0, st, H, ldh, n, n, J, ldj, b, nb2, step, s,
+                             state, dstate, tol, one_pair ? 60 : 3);
       }
-      if (one_pair && rows <= 64 && 2 * b <= 32) {
-        hipLaunchKernelGGL((k_bjac_small<T>), dim3(1, 1, nz), dim3(64), 0, st, H, ldh, rows, cols, J, ldj, b, s, state,
-                           dstate, tol, max_inner, zb);
-        continue;
-      }
-      hipLaunchKernelGGL((k_bjac_step<T>), dim3(nb2 / 2), dim3(1024), 0, st, H, ldh, rows, cols, J, ldj, b, nb2, step,
-                         s, state, dstate, tol, max_inner);
-    }
-    if (!(std::is_same<T, double>::value && gram_steps && !fused))  // else the sweep closes in k_bjac_apply
       hipLaunchKernelGGL(k_bjac_check, dim3(1, 1, nz), dim3(64), 0, st, state, s, zb);
+    }
   }
-  hipLaunchKernelGGL((k_bjac_norms<T>), dim3(1, 1, nz), dim3(1024), 0, st, H, ldh, rows, cols, sig, state, status, zb);
+  hipLaunchKernelGGL((k_bjac_norms<T>), dim3(1, 1, nz), dim3(1024), 0, st, H, ldh, n, n, sig, state, status, zb);
 }
 
 
@@ -517,7 +538,7 @@ int64_t carve(WsCursor& c, const Plan& p, SmallBufs<T>& b, double** mean, double
   b.status = c.take<int>(4);
   b.perm3 = c.take<int>(n); b.rank3 = c.take<int>(4);
   b.jstate = c.take<int>(kBjacMaxSweeps + 8);
-  b.jdstate = c.take<double>(bjac_dstate_len(n));  // [0] negligible norm, then the Gram steps' pair rotations
+  b.jdstate = c.take<double>(bjac_dstate_len(n));  // k_bjac_init, k_jacobi.hip
   b.dsc = c.take<double>(4);
   b.Wpad = c.take<double>(int64_t(p.NB) * p.NB);
   int ncand = int(std::min<int64_t>(p.m, 4 * int64_t(n) + 16));
@@ -1232,15 +1253,14 @@ static int core_t(pc_ctx* ctx, const Plan& p, const void* A, int64_t lda, int ce
       return pc_fail(ctx, PC_ERR_UNSUPPORTED, "randomized through the factor: float32 storage only");
   }
   int nc = n;
-  bool gram_steps_;
   int jb_, jnb2_;
-  jacobi_blocks<T>(n, n, gram_steps_, jb_, jnb2_);
+  jacobi_blocks<T>(n, jb_, jnb2_);
   if (mode == CORE_SVD && jnb2_ == 2) {
     // every column fits one block pair: the Jacobi launch iterates to
     // convergence on its own, so M (Hc, column-major) is rotated directly and
     // V = J; no preconditioner is needed
-    launch_block_jacobi<T>(ctx, b.Hc, n, n, n, b.J, n, b.sig, b.jstate, b.jdstate, b.status,
-                           p.mixed ? kJacTolMx : 0.0);
+    launch_block_jacobi<T>(ctx, b.Hc, n, n, b.J, n, b.sig, b.jstate, b.jdstate, b.status,
+                           p.mixed ? kJacTolMx : 0.0, b.G1, b.R1);
     hipLaunchKernelGGL(k_sort_desc, dim3(1), dim3(1024), 0, st, b.sig, n, b.order);
     hipLaunchKernelGGL((k_svd_finish<T, ST, typename VtType<T, ST>::type>), dim3(nblk(nn)), dim3(256), 0, st, b.Hc,
                        n, n, n, b.sig, b.order, b.J, n, p.mixed ? kNullMx : kNullF64, (const int*)b.rank,
@@ -1263,9 +1283,10 @@ static int core_t(pc_ctx* ctx, const Plan& p, const void* A, int64_t lda, int ce
     hipLaunchKernelGGL((k_gemm_small<T>), gg, dim3(256), 0, st, 0, 0, n, n, n, T(1.0), b.tmp, n, (const int*)nullptr,
                        b.Awk, n, (const int*)nullptr, T(0.0), b.Hc, n, 1);
     // mixed precision: the factor carries ~1e-7 relative data error, so the
-    // columns need only be orthogonal to 1e-8 (sigma errs by O(tol^2))
-    launch_block_jacobi<T>(ctx, b.Hc, n, n, n, b.J, n, b.sig, b.jstate, b.jdstate, b.status,
-                           p.mixed ? kJacTolMx : 0.0);
+    // columns need only be orthogonal to 1e-8 (sigma errs by O(tol^2)).  G1 and R1
+    // (R4 and R3) are not read again
+    launch_block_jacobi<T>(ctx, b.Hc, n, n, b.J, n, b.sig, b.jstate, b.jdstate, b.status,
+                           p.mixed ? kJacTolMx : 0.0, b.G1, b.R1);
     // V = V0 J (column-major like J)
     hipLaunchKernelGGL((k_gemm_small<T>), gg, dim3(256), 0, st, 0, 1, n, n, n, T(1.0), b.Awk, n, (const int*)nullptr,
                        b.J, n, (const int*)nullptr, T(0.0), b.tmp, n, 1);
@@ -1342,9 +1363,8 @@ inline int64_t byte_diff(const void* a, const void* b) {
 static bool batch_eligible(pc_dtype dt, const pc_problem* pr, int64_t count, BatchDesc& d) {
   if (count < 2 || count > 65535 || !dtype_complex(dt)) return false;
   const pc_problem& q = pr[0];
-  bool gs;
   int jb, jnb2;
-  jacobi_blocks<cdouble>(int(q.n), int(q.n), gs, jb, jnb2);
+  jacobi_blocks<cdouble>(int(q.n), jb, jnb2);
   if (!(jnb2 == 2 && q.n <= 64 && 2 * jb <= 32)) return false;
   d.zA = byte_diff(pr[1].A, q.A);
   d.zU = byte_diff(pr[1].U, q.U);
@@ -1401,8 +1421,8 @@ static int core_batch_t(pc_ctx* ctx, const Plan& p, const pc_problem* pr, int64_
     hipLaunchKernelGGL((k_center_right<T>), dim3(nblk(n), 1, z), dim3(256), 0, st, b.Hc, n, n, zb);
   hipLaunchKernelGGL((k_pad_identity<T>), dim3(1, 1, z), dim3(256), 0, st, b.R2, n, n, b.rank, zb);
   run_trinv<T>(st, b.R2, n, b.R2i, nz, zb);
-  launch_block_jacobi<T>(ctx, b.Hc, n, n, n, b.J, n, b.sig, b.jstate, b.jdstate, b.status,
-                         p.mixed ? kJacTolMx : 0.0, nz, zb);
+  launch_block_jacobi<T>(ctx, b.Hc, n, n, b.J, n, b.sig, b.jstate, b.jdstate, b.status,
+                         p.mixed ? kJacTolMx : 0.0, nullptr, nullptr, nz, zb);
   hipLaunchKernelGGL(k_sort_desc, dim3(1, 1, z), dim3(1024), 0, st, b.sig, n, b.order, zb);
   hipLaunchKernelGGL((k_svd_finish<T, ST, typename VtType<T, ST>::type>), dim3(nblk(nn), 1, z), dim3(256), 0, st,
                      b.Hc, n, n, n, b.sig, b.order, b.J, n, p.mixed ? kNullMx : kNullF64, (const int*)b.rank,
