@@ -313,8 +313,10 @@ __global__ __launch_bounds__(NT) void k_pchol_fast(const double* __restrict__ G,
   __syncthreads();
   if (tid == 0) {
     int k = rank;
+    // every index not pivoted (-2), one whose diagonal is NaN included: perm is a
+    // permutation whatever the input, since it is used to address
     for (int q = 0; q < n; q++)
-      if (dg[q] >= 0.0 && k < n) perm[k++] = q;
+      if (dg[q] != -2.0 && k < n) perm[k++] = q;
     rank_out[0] = rank;
   }
   __syncthreads();
