@@ -25,11 +25,11 @@
 // k-steps (a sum over k may take its terms in any order) and W is laid out in LDS
 // to match.
 #include "common.hpp"
+#include "f64_common.hpp"
 #include "kernels.hpp"
 
 namespace {
 
-typedef double d4 __attribute__((ext_vector_type(4)));
 constexpr int DNT = 512;        // 8 waves
 constexpr int DNW = DNT / 64;
 // Waves that share a row chunk of a Gram over NB columns, 16 rows each per turn.  Up
@@ -38,8 +38,6 @@ constexpr int DNW = DNT / 64;
 // workgroup about as much as 200 rows of 30 columns.)  Wider Grams have few chunks
 // of long rows, so 8 waves share one.
 constexpr int chunk_waves(int NB) { return NB <= 32 ? 1 : 8; }
-
-PC_DEV d4 mfma64(double a, double b, d4 c) { return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0); }
 
 template <class TS, int V>
 PC_DEV void load_vec(const TS* p, TS* o) {
@@ -63,27 +61,6 @@ PC_DEV void store_vec(TO* p, const TO* o) {
     for (int e = 0; e < V; e++) q[e] = o[e];
     *reinterpret_cast<vt*>(p) = q;
   }
-}
-
-template <int CTRL>
-PC_DEV double dpp_move(double x) {
-  const long long b = __builtin_bit_cast(long long, x);
-  const int lo = __builtin_amdgcn_update_dpp(0, int(b), CTRL, 0xF, 0xF, true);
-  const int hi = __builtin_amdgcn_update_dpp(0, int(b >> 32), CTRL, 0xF, 0xF, true);
-  return __builtin_bit_cast(double, (long long)(unsigned)lo | ((long long)hi << 32));
-}
-// sum over the 16 lanes of a DPP row, in every lane
-PC_DEV double row16_sum(double v) {
-  v += dpp_move<0xB1>(v);   // quad_perm [1,0,3,2]
-  v += dpp_move<0x4E>(v);   // quad_perm [2,3,0,1]
-  v += dpp_move<0x141>(v);  // row_half_mirror
-  v += dpp_move<0x140>(v);  // row_mirror
-  return v;
-}
-// s / n with iv = 1 / n: the quotient and one residual step
-PC_DEV double div_n(double s, double n, double iv) {
-  const double q = s * iv;
-  return fma(fma(-n, q, s), iv, q);
 }
 
 // Sum the NBLK accumulators of the 8 waves in wave order through red (two blocks
@@ -198,8 +175,9 @@ __global__ __launch_bounds__(DNT) void k_dgram_f64(const TS* __restrict__ X, int
 #pragma unroll
           for (int b = 0; b < nb; b++) s2 += f[b] * f[b];
           const double var = div_n(row16_sum(s2), nd, inv_n);
+          divide_rows<nb>(f, var);
 #pragma unroll
-          for (int b = 0; b < nb; b++) f[b] = rv && cv[b] ? f[b] / var : 0.0;
+          for (int b = 0; b < nb; b++) f[b] = rv && cv[b] ? f[b] : 0.0;
           if (rv && i == 0) var_out[row] = var;
         }
         if (rv && i == 0) mean_out[row] = mu;
@@ -236,12 +214,15 @@ PC_DEV void load_afrag(const TS* __restrict__ X, int64_t ldx, int n, int64_t row
     if (4 * V * c < n) load_vec<TS, V>(xr + (col < n ? col : 0), a + c * V);  // uniform: whole k-steps beyond n stay out
   }
 }
-template <class TS, int V>
-PC_DEV double afrag_value(TS x, int st, int n, bool rv, int center, double mu, double var) {
+// their values: centred, zero beyond the rows and columns
+template <class TS, int KS, int V>
+PC_DEV void afrag_values(const TS* x, double* a, int n, bool rv, int center, double mu, double var) {
   const int g = (threadIdx.x & 63) >> 4;
-  double v = double(x);
-  if (center) v = center == 2 ? (v - mu) / var : v - mu;
-  return rv && 4 * V * (st / V) + V * g + st % V < n ? v : 0.0;
+#pragma unroll
+  for (int st = 0; st < KS; st++) a[st] = center ? double(x[st]) - mu : double(x[st]);
+  if (center == 2) divide_rows<KS>(a, var);
+#pragma unroll
+  for (int st = 0; st < KS; st++) a[st] = rv && 4 * V * (st / V) + V * g + st % V < n ? a[st] : 0.0;
 }
 // W (ld ldw) into LDS in B-fragment order: Wl[(st nbl + J) 64 + l] is row
 // 4 V (st / V) + V g + st % V, column col0 + colmap(J, i); zero beyond n rows / ldw columns
@@ -254,12 +235,12 @@ PC_DEV void stage_w(const double* __restrict__ W, int n, int ldw, int col0, doub
   }
 }
 
-// P2: Z = Yc W in registers, then its Gram.  W upper triangular when `upper`:
-// column block J takes the k-steps below 16 (J + 1) only (the rest are exact zeros).
+// P2: Z = Yc W in registers, then its Gram.  W is upper triangular: column block J
+// takes the k-steps below 16 (J + 1) only (the rest are exact zeros).
 template <class TS, int NB, int V>
 __global__ __launch_bounds__(DNT) void k_dzgram_f64(const TS* __restrict__ X, int64_t ldx, int64_t m, int n, int center,
                                                     const double* mean_in, const double* var_in,
-                                                    const double* __restrict__ W, int upper, int chunks, int64_t rpc,
+                                                    const double* __restrict__ W, int chunks, int64_t rpc,
                                                     double* __restrict__ part, int64_t zx, int64_t zb) {
   X = zoff(X, zx);
   mean_in = zoff(mean_in, zb);
@@ -296,12 +277,13 @@ __global__ __launch_bounds__(DNT) void k_dzgram_f64(const TS* __restrict__ X, in
     d4 z[nb];
 #pragma unroll
     for (int J = 0; J < nb; J++) z[J] = d4{0, 0, 0, 0};
+    double a[KS];
+    afrag_values<TS, KS, V>(cur, a, n, rv, center, mu, var);
 #pragma unroll
     for (int st = 0; st < KS; st++) {
-      const double a = afrag_value<TS, V>(cur[st], st, n, rv, center, mu, var);
 #pragma unroll
       for (int J = 0; J < nb; J++)
-        if (!upper || 4 * V * (st / V) < 16 * (J + 1)) z[J] = mfma64(a, sm[(st * nb + J) * 64 + l], z[J]);
+        if (4 * V * (st / V) < 16 * (J + 1)) z[J] = mfma64(a[st], sm[(st * nb + J) * 64 + l], z[J]);
     }
 #pragma unroll
     for (int r = 0; r < 4; r++) {
@@ -365,9 +347,7 @@ __global__ __launch_bounds__(DNT) void k_dgemm_f64(const TS* __restrict__ X, int
     double a[R][KS];
 #pragma unroll
     for (int q = 0; q < R; q++)
-#pragma unroll
-      for (int st = 0; st < KS; st++)
-        a[q][st] = afrag_value<TS, V>(cur[q][st], st, n, t + 16 * q + i < m, center, mu[q], var[q]);
+      afrag_values<TS, KS, V>(cur[q], a[q], n, t + 16 * q + i < m, center, mu[q], var[q]);
 #pragma unroll 1
     for (int q0 = 0; q0 < nbl / CV; q0++) {
       if (col0 + 16 * CV * q0 >= nc) break;
@@ -502,7 +482,7 @@ int with_vec(int v, F&& f) {
 template <class TS>
 int dgram_t(hipStream_t st, const TS* X, int64_t ldx, int64_t m, int n, int center, const double* mean_in,
             const double* var_in, double* mean_out, double* var_out, const double* W, int chunks, int64_t tpc,
-            double* part, const PassBatch& bz, bool upper) {
+            double* part, const PassBatch& bz) {
   const int64_t rpc = tpc * (n <= 32 ? 32 : 128);
   return with_nb(n, [&](auto nbc) {
     constexpr int NB = decltype(nbc)::value;
@@ -515,7 +495,7 @@ int dgram_t(hipStream_t st, const TS* X, int64_t ldx, int64_t m, int n, int cent
       if (W) {
         if constexpr (NB > 32 || V == 1)
           hipLaunchKernelGGL((k_dzgram_f64<TS, NB, V>), g, dim3(DNT), 0, st, X, ldx, m, n, center, mean_in, var_in, W,
-                             upper ? 1 : 0, chunks, rpc, part, bz.zx, bz.zb);
+                             chunks, rpc, part, bz.zx, bz.zb);
       } else {
         if constexpr ((NB / 16) % V == 0)
           hipLaunchKernelGGL((k_dgram_f64<TS, NB, V>), g, dim3(DNT), 0, st, X, ldx, m, n, center, mean_out, var_out,
@@ -613,12 +593,12 @@ int d64_xgram_chunks(int64_t m, int64_t* tpc) { return d64_gram_chunks(m, kDirec
 
 int launch_d64_gram(hipStream_t st, pc_dtype dt, const void* X, int64_t ldx, int64_t m, int n, int center,
                     const double* mean_in, const double* var_in, double* mean_out, double* var_out, const double* W,
-                    int chunks, int64_t tpc, double* part, const PassBatch& bz, bool upper) {
+                    int chunks, int64_t tpc, double* part, const PassBatch& bz) {
   if (dt == PC_F64)
     return dgram_t<double>(st, (const double*)X, ldx, m, n, center, mean_in, var_in, mean_out, var_out, W, chunks, tpc,
-                           part, bz, upper);
+                           part, bz);
   return dgram_t<float>(st, (const float*)X, ldx, m, n, center, mean_in, var_in, mean_out, var_out, W, chunks, tpc,
-                        part, bz, upper);
+                        part, bz);
 }
 int launch_d64_gemm(hipStream_t st, pc_dtype dt, const void* X, int64_t ldx, int64_t m, int n, int center,
                     const double* mean_in, const double* var_in, const double* W, int ldw, int nc, int chunks, void* C,

@@ -4,6 +4,7 @@
 
 // FP64 MFMA streaming kernels (k_mfma_f64.hip); return 0, or -1 when n is too large
 int f64_nb(int n);
+int f64_xnb(int n);  // of a cross product's operand
 // partition of the passes, from the sizes alone: row chunks of a Gram (tpc: turns
 // per chunk), rows of a product's turn and its workgroups
 int f64_gram_chunks(int64_t m, int n, int64_t* tpc);
@@ -16,15 +17,17 @@ struct PassBatch {
   int nz = 1;
   int64_t zx = 0, zb = 0, zc = 0;
 };
-// W non-null: the second pass, Gram of Z = Y W; upper: W is upper triangular
-// (zero-padded), so Z skips the k-steps where W is zero
+// W non-null: the second pass, Gram of Z = Y W, W (n x n, padded to f64_nb) upper
+// triangular: Z skips the products with its zero blocks
 int launch_gram_f64(hipStream_t st, pc_dtype dt, const void* X, int64_t ldx, int64_t m, int n, int center,
-                    int stats_in, const double* mean_in, const double* var_in, double* mean_out, double* var_out,
-                    const double* W, int chunks, int64_t tpc, double* part, const PassBatch& bz = PassBatch(),
-                    bool upper = false);
+                    const double* mean_in, const double* var_in, double* mean_out, double* var_out, const double* W,
+                    int chunks, int64_t tpc, double* part, const PassBatch& bz = PassBatch());
+// C (m x nc) = Yc W, any n and nc; W FP64, rows padded with zeros to a multiple of 16
+// (n > kDirectProduct).  out_f64: C is FP64 whatever the storage; upper: W is upper
+// triangular (both n > kDirectProduct only)
 int launch_gemm_f64(hipStream_t st, pc_dtype dt, const void* X, int64_t ldx, int64_t m, int n, int center,
-                    const double* mean_in, const double* var_in, const double* W, int nc, int chunks, int64_t tpc,
-                    void* C, int64_t ldc, const PassBatch& bz = PassBatch());
+                    const double* mean_in, const double* var_in, const double* W, int64_t ldw, int nc, int chunks,
+                    void* C, int64_t ldc, const PassBatch& bz = PassBatch(), bool out_f64 = false, bool upper = false);
 int launch_xgram_f64(hipStream_t st, pc_dtype dt, const void* A, int64_t lda, int p, const void* B, int64_t ldb, int q,
                      int64_t m, int chunks, int64_t tpc, double* part);
 
@@ -38,7 +41,7 @@ int d64_xgram_chunks(int64_t m, int64_t* tpc);
 int d64_gemm_chunks(int64_t m, int n, int nc);
 int launch_d64_gram(hipStream_t st, pc_dtype dt, const void* X, int64_t ldx, int64_t m, int n, int center,
                     const double* mean_in, const double* var_in, double* mean_out, double* var_out, const double* W,
-                    int chunks, int64_t tpc, double* part, const PassBatch& bz, bool upper);
+                    int chunks, int64_t tpc, double* part, const PassBatch& bz);
 int launch_d64_gemm(hipStream_t st, pc_dtype dt, const void* X, int64_t ldx, int64_t m, int n, int center,
                     const double* mean_in, const double* var_in, const double* W, int ldw, int nc, int chunks, void* C,
                     int64_t ldc, const PassBatch& bz);
@@ -73,13 +76,10 @@ int launch_pack_w_mx(hipStream_t st, const double* W, int ldw, int n, int nc, in
 // count float32 / float64 values (k_rng.hip); -1 for other dtypes
 int launch_mt_omega(hipStream_t st, uint32_t seed, int64_t count, pc_dtype dt, void* out);
 // wide problems (256 < real columns <= 2048), FP64 MFMA (k_wide.hip): stripe-pair
-// Gram into NBp x NBp slabs per row chunk, and the K-looped tall product
+// Gram into NBp x NBp slabs per row chunk
 int wide_stripe();
 int wide_tile_rows();
 int launch_wgram_f64(hipStream_t st, pc_dtype dt, const void* X, int64_t ldx, int64_t m, int n, int center,
                      const double* mean, const double* var, int chunks, int64_t tpc, double* part, int NBp);
-int launch_wgemm_f64(hipStream_t st, pc_dtype dt, const void* X, int64_t ldx, int64_t m, int K, int center,
-                     const double* mean, const double* var, const double* W, int64_t ldw, int N, int chunks,
-                     int64_t tpc, void* C, int64_t ldc, int out_f64);
 int launch_wxgram_f64(hipStream_t st, pc_dtype dt, const void* A, int64_t lda, int p, const void* B, int64_t ldb,
                       int q, int64_t m, int chunks, int64_t tpc, double* part, int PBp, int QBp);

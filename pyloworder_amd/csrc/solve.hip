@@ -485,11 +485,12 @@ int make_plan(pc_ctx* ctx, pc_dtype dt, int64_t m, int64_t n, int precision, Pla
     // chunk count still depends on (m, n) only)
     p.wide = true;
     p.NB = int(round_up(p.nr, wide_stripe()));
-    p.tr = p.tr3 = wide_tile_rows();
+    p.tr = wide_tile_rows();
+    p.tr3 = f64_gemm_rows(p.nr);
     const int64_t cap = std::max<int64_t>(1, kWideSlabBytes / (int64_t(p.NB) * p.NB * 8));
     p.chunks = int(std::min<int64_t>(stream_chunks(m, p.tr), cap));
     p.tpc = ceil_div(ceil_div(m, p.tr), p.chunks);
-    p.chunks3 = stream_chunks(m, p.tr3);
+    p.chunks3 = f64_gemm_chunks(m, p.nr, p.nr);
     p.tpc3 = ceil_div(ceil_div(m, p.tr3), p.chunks3);
     p.chunks2 = p.chunks3;
     p.tpc2 = p.tpc3;
@@ -934,8 +935,8 @@ static int launch_streams(pc_ctx* ctx, const Plan& p, const void* A, int64_t lda
     if (pass == 1) {
       rc = launch_wgram_f64(st, sdt, A, ldr, p.m, p.nr, center, mean, var, p.chunks, p.tpc, part, p.NB);
     } else {
-      rc = launch_wgemm_f64(st, sdt, A, ldr, p.m, p.nr, center, mean, var, b.Wpad, p.NB, p.nr, p.chunks3, p.tpc3,
-                            b.Zw, b.ldz, 1);
+      rc = launch_gemm_f64(st, sdt, A, ldr, p.m, p.nr, center, mean, var, b.Wpad, p.NB, p.nr, p.chunks3, b.Zw, b.ldz,
+                           PassBatch(), /*out_f64=*/true, /*upper: W1 = R1^-1, zero-padded*/ true);
       if (rc == 0)
         rc = launch_wgram_f64(st, PC_F64, b.Zw, b.ldz, p.m, p.nr, 0, nullptr, nullptr, p.chunks, p.tpc, part, p.NB);
     }
@@ -953,11 +954,11 @@ static int launch_streams(pc_ctx* ctx, const Plan& p, const void* A, int64_t lda
                             p.tpc2, part, bz, /*upper: W1 = R1^-1, zero-padded*/ true);
   } else {
     if (pass == 1)
-      rc = launch_gram_f64(st, sdt, A, ldr, p.m, p.nr, center, 0, nullptr, nullptr, center ? mean : nullptr,
+      rc = launch_gram_f64(st, sdt, A, ldr, p.m, p.nr, center, nullptr, nullptr, center ? mean : nullptr,
                            center == 2 ? var : nullptr, nullptr, p.chunks, p.tpc, part, bz);
     else
-      rc = launch_gram_f64(st, sdt, A, ldr, p.m, p.nr, center, 1, mean, var, nullptr, nullptr, b.Wpad, p.chunks,
-                           p.tpc, part, bz, /*upper: W1 = R1^-1, zero-padded*/ true);
+      rc = launch_gram_f64(st, sdt, A, ldr, p.m, p.nr, center, mean, var, nullptr, nullptr, b.Wpad, p.chunks, p.tpc,
+                           part, bz);
   }
   if (rc != 0) return pc_fail(ctx, PC_ERR_SHAPE, "streaming kernel has no variant for n = %d", p.n);
   PC_HIP(ctx, hipGetLastError());
@@ -1056,14 +1057,10 @@ static int launch_p3(pc_ctx* ctx, const Plan& p0, const void* A, int64_t lda, in
   int64_t ldu = p0.cplx ? 2 * out.ldu : out.ldu;
   Plan p = p0;
   auto launch = [&](int chunks, int64_t tpc) {
-    if (p.wide)
-      return launch_wgemm_f64(st, sdt, A, ldr, p.m, p.nr, center, mean, var, b.Wpad, p.NB, p.nr, chunks, tpc, out.U,
-                              ldu, 0);
     if (p.mixed)
       return launch_gemm_mx2(st, (const float*)A, ldr, p.m, p.nr, center, mean, var, b.Wh, b.Wl, b.wscale, p.nr,
                              chunks, tpc, (float*)out.U, ldu, bz);
-    return launch_gemm_f64(st, sdt, A, ldr, p.m, p.nr, center, mean, var, b.Wpad, p.nr, chunks, tpc, out.U, ldu,
-                           bz);
+    return launch_gemm_f64(st, sdt, A, ldr, p.m, p.nr, center, mean, var, b.Wpad, p.NB, p.nr, chunks, out.U, ldu, bz);
   };
   const int64_t tiles = ceil_div(p.m, p.tr3);
   auto geometry = [&](int chunks) {
