@@ -1,10 +1,8 @@
-// FP64 dense kernels for real n x n matrices, n <= 256 (the small dense
-// stage of the POD core).  Shifted Cholesky, pivoted Cholesky and Householder
-// QR with explicit Q are blocked single-workgroup factorizations (1024
-// threads): matrices live in global memory (L2-resident at these sizes),
-// 32-column panels are staged in LDS and every rank-32 update runs on
-// v_mfma_f64_16x16x4f64.  The triangular inverse is n independent column
-// back-substitutions, one wavefront each.
+// FP64 dense kernels for real n x n matrices (the small dense stage of the POD
+// core): shifted Cholesky, pivoted Cholesky and the triangular inverse for n <= 512,
+// Householder QR with explicit Q for n <= 256.  The factorisations are blocked, on
+// one workgroup: matrices live in global memory (L2-resident at these sizes), panels
+// are staged in LDS and the updates run on v_mfma_f64_16x16x4f64.
 //
 // f64 MFMA 16x16x4 lane layout (wave64): lane l holds A[l % 16][l / 16] and
 // B[l / 16][l % 16]; accumulator register r holds D[4 r + l / 16][l % 16].
@@ -14,15 +12,8 @@ namespace dense {
 
 constexpr int PW = 32;           // panel width
 constexpr int PLD = 257;         // LDS leading dimension of panels (odd: no bank conflicts)
-constexpr int NMAX = 256;
-
-// (I, J), I <= J, of the t-th upper tile of an nt x nt tile grid
-PC_DEV void upper_tile(int t, int nt, int& I, int& J) {
-  int i = 0;
-  while (t >= nt - i) { t -= nt - i; i++; }
-  I = i;
-  J = i + t;
-}
+constexpr int NMAX = 256;        // of the Householder QR
+constexpr int DMAX = 512;        // of the Cholesky factorisations and the triangular inverse
 
 // DPP move of a double (both 32-bit halves), lanes that the row mask leaves
 // out return `old`
@@ -52,35 +43,115 @@ PC_DEV double wave_sum_dpp(double v) {
   v += dpp_f64<0x143, 0xC>(v, 0.0);  // row_bcast:31 into rows 2, 3
   return readlane63_f64(v);
 }
-// Maximum over the 64 lanes (NaN-free input), returned to every lane
-PC_DEV double wave_max_dpp(double v) {
-  v = fmax(v, dpp_f64<0xB1, 0xF>(v, v));
-  v = fmax(v, dpp_f64<0x4E, 0xF>(v, v));
-  v = fmax(v, dpp_f64<0x124, 0xF>(v, v));
-  v = fmax(v, dpp_f64<0x128, 0xF>(v, v));
-  v = fmax(v, dpp_f64<0x142, 0xA>(v, v));
-  v = fmax(v, dpp_f64<0x143, 0xC>(v, v));
-  return readlane63_f64(v);
+// Maximum over the 64 lanes, returned to every lane
+PC_DEV int wave_max_dpp_i32(int v) {
+  v = max(v, __builtin_amdgcn_update_dpp(v, v, 0xB1, 0xF, 0xF, false));
+  v = max(v, __builtin_amdgcn_update_dpp(v, v, 0x4E, 0xF, 0xF, false));
+  v = max(v, __builtin_amdgcn_update_dpp(v, v, 0x124, 0xF, 0xF, false));
+  v = max(v, __builtin_amdgcn_update_dpp(v, v, 0x128, 0xF, 0xF, false));
+  v = max(v, __builtin_amdgcn_update_dpp(v, v, 0x142, 0xA, 0xF, false));
+  v = max(v, __builtin_amdgcn_update_dpp(v, v, 0x143, 0xC, 0xF, false));
+  return __builtin_amdgcn_readlane(v, 63);
+}
+// x of lane i (wave-uniform), to every lane
+PC_DEV double lane_read_f64(double x, int i) {
+  const long long b = __builtin_bit_cast(long long, x);
+  const int lo = __builtin_amdgcn_readlane(int(b), i), hi = __builtin_amdgcn_readlane(int(b >> 32), i);
+  return __builtin_bit_cast(double, (long long)(unsigned)lo | ((long long)hi << 32));
+}
+// 1 / sqrt(d), d > 0: the hardware's estimate (2^-24) and two Newton steps
+PC_DEV double rsqrt_f64(double d) {
+  double y = __builtin_amdgcn_rsq(d);
+#pragma unroll
+  for (int k = 0; k < 2; k++) y = fma(0.5 * y, fma(-d * y, y, 1.0), y);
+  return y;
+}
+// r = sqrt(d) from y = 1 / sqrt(d), and x / r = q + (x - q r) y, q = x y: each result
+// corrected by its residual, as a square root and a division would round it
+PC_DEV double sqrt_from(double d, double y) {
+  const double r = d * y;
+  return fma(0.5 * y, fma(-r, r, d), r);
+}
+PC_DEV double div_by(double x, double r, double y) {
+  const double q = x * y;
+  return fma(fma(-q, r, x), y, q);
+}
+// LDS and memory accesses of one wave in program order across its lanes
+PC_DEV void wave_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+// The upper tiles of any grid, numbered from its last one: tile k is e / 256 rows and
+// e % 256 columns before the last, e = tab[k]
+constexpr int kMaxTiles = (DMAX / 16) * (DMAX / 16 + 1) / 2;
+PC_DEV void tile_table(unsigned short* tab, int nt, int tid, int nth) {
+  for (int e = tid; e < nt * nt; e += nth) {
+    const int b = e / nt, a = e % nt;
+    if (a <= b) tab[b * (b + 1) / 2 + a] = (unsigned short)(256 * b + a);
+  }
+}
+// f(I, J, acc) over a wave's upper tiles of an nt x nt grid, acc loaded by g(I, J, acc),
+// BATCH tiles at a time: their loads are waited for once, before the first of the
+// batch's stores (the counter of outstanding accesses covers both, so a wait between
+// them would be one for the stores).  g and f keep clear of branches for the same
+// reason, and because a branch costs as much as a tile's product.
+template <int NW, int BATCH, class L, class F>
+PC_DEV void fold_tiles(int w, int nt, const unsigned short* tab, L g, F f) {
+  const int count = nt * (nt + 1) / 2;
+  for (int t = w; t < count; t += NW * BATCH) {
+    int I[BATCH], J[BATCH];
+    d4s acc[BATCH];
+#pragma unroll
+    for (int d = 0; d < BATCH; d++) {
+      const int e = __builtin_amdgcn_readfirstlane(tab[min(t + d * NW, count - 1)]);
+      I[d] = nt - 1 - (e >> 8);
+      J[d] = nt - 1 - (e & 255);
+    }
+#pragma unroll
+    for (int d = 0; d < BATCH; d++) g(I[d], J[d], acc[d]);
+#pragma unroll
+    for (int d = 0; d < BATCH; d++) asm volatile("" : "+v"(acc[d][0]), "+v"(acc[d][1]), "+v"(acc[d][2]), "+v"(acc[d][3]));
+#pragma unroll
+    for (int d = 0; d < BATCH; d++)
+      if (t + d * NW < count) f(I[d], J[d], acc[d]);
+  }
 }
 
 }  // namespace dense
 
 // ---------------------------------------------------------------------------
-// Shifted Cholesky, real: R upper with R^T R = G + tau I, tau = shift_rel *
-// max G_ii.  Right-looking with 32-wide panels; a pivot below tau/2 (rounding
-// made G indefinite at that scale) restarts with tau *= 8.
+// Shifted Cholesky, real (n <= DMAX): R upper with R^T R = G + tau I, tau =
+// shift_rel * max G_ii.  Right-looking with 16-wide panels; a pivot below tau/2
+// (rounding made G indefinite at that scale) restarts with tau *= 8.
 // status[0] = 1 on a non-finite Gram or when 20 restarts did not suffice.
+//
+// What bounds it is the chain of pivots, so wave 0 alone factors each 16 x 16
+// diagonal block, lane c holding column c in registers: a pivot and its row reach
+// the other lanes by lane reads, no barrier and no LDS in the chain (four waves a
+// SIMD sharing it, each step behind three barriers: 460 us at n = 256, now 165).  The
+// panel's rows are one forward substitution per thread in registers, the trailing
+// update MFMA tiles loaded four at a time.  CN: columns P has room for.
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(NT) void k_chol_fast(const double* __restrict__ G, int ldg, int n, double shift_rel,
-                                                  double* __restrict__ R, int ldr, int* status) {
+constexpr int kCholThreads = 512;
+constexpr int CW = 16;  // panel width: at 32 the factorisation of a block is 60 KB of unrolled code, fetched anew for each
+template <int CN>
+__global__ __launch_bounds__(kCholThreads) void k_chol_fast(const double* G, int ldg, int n, double shift_rel,
+                                                            double* R, int ldr, int* status) {
   using namespace dense;
-  __shared__ double D[PW * (PW + 1)];
-  __shared__ double P[PW * PLD];
+  constexpr int NW = kCholThreads / 64, LD = CN + 1, DLD = CW + 2;
+  static_assert(CN - CW <= kCholThreads, "one thread per panel column");
+  __shared__ double P[CW * LD];
+  __shared__ __attribute__((aligned(16))) double Dt[CW * DLD];  // column i of the factored block at Dt[i * DLD]
+  __shared__ double Ds[CW * DLD];                               // the block to be factored
+  __shared__ double ri_s[CW];
+  __shared__ unsigned short tab[kMaxTiles];
   __shared__ double sh[32];
   __shared__ int restart;
-  const int tid = threadIdx.x, w = tid >> 6, l = tid & 63, lr = l & 15, lk = l >> 4;
+  const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), l = tid & 63, lr = l & 15, lk = l >> 4;
+  tile_table(tab, (n + 15) >> 4, tid, kCholThreads);
   double dmax = 0.0;
-  for (int i = tid; i < n; i += NT) dmax = fmax(dmax, G[int64_t(i) * ldg + i]);
+  for (int i = tid; i < n; i += kCholThreads) dmax = fmax(dmax, G[int64_t(i) * ldg + i]);
   dmax = block_max(dmax, sh);
   if (!isfinite(dmax)) {
     if (tid == 0) status[0] = 1;
@@ -89,87 +160,116 @@ __global__ __launch_bounds__(NT) void k_chol_fast(const double* __restrict__ G, 
   double tau = shift_rel * dmax;
   if (!(tau > 0.0)) tau = 1.0;
   for (int attempt = 0; attempt < 20; attempt++) {
-    for (int i = w; i < n; i += NT / 64)
-      for (int j = l; j < n; j += 64) {
-        double v = i <= j ? G[int64_t(i) * ldg + j] : 0.0;
-        if (i == j) v += tau;
-        R[int64_t(i) * ldr + j] = v;
-      }
     if (tid == 0) restart = 0;
+    for (int e = tid; e < CW * CW; e += kCholThreads) {
+      const int i = e >> 4, j = e & 15;
+      Ds[i * DLD + j] = i < n && j < n ? G[int64_t(i) * ldg + j] + (i == j ? tau : 0.0) : 0.0;
+    }
     __syncthreads();
-    for (int k0 = 0; k0 < n; k0 += PW) {
-      const int bs = min(PW, n - k0);
-      for (int idx = tid; idx < PW * PW; idx += NT) {
-        int i = idx >> 5, j = idx & 31;
-        D[i * (PW + 1) + j] = (i < bs && j < bs && i <= j) ? R[int64_t(k0 + i) * ldr + k0 + j] : 0.0;
+    for (int k0 = 0; k0 < n; k0 += CW) {
+      const int bs = min(CW, n - k0);
+      // the first panel reads G, the later ones the trailing block left in R
+      const double* A = k0 ? R : G;
+      const int64_t lda = k0 ? ldr : ldg;
+      const double add = k0 ? 0.0 : tau;  // the shift of the diagonal (the update adds it for the later panels)
+      const int c1 = k0 + bs, nt = n - c1, ntl = (nt + 15) >> 4;
+      // this thread's column of the panel, on its way while the block is factored
+      double x[CW];
+      const bool own = tid < 16 * ntl, in = tid < nt;
+      if (own) {
+        const double* src = A + int64_t(k0) * lda + (in ? c1 + tid : 0);
+#pragma unroll
+        for (int i = 0; i < CW; i++) x[i] = src[int64_t(i) * lda];  // nt > 0: bs = CW
       }
-      __syncthreads();
-      for (int j = 0; j < bs; j++) {
-        if (tid == 0) {
-          double d = D[j * (PW + 1) + j];
-          if (!isfinite(d)) { status[0] = 1; d = tau; }
-          else if (d < 0.5 * tau) { restart = 1; d = tau; }
-          D[j * (PW + 1) + j] = sqrt(d);
+      if (w == 0) {
+        const int c = l & 15;
+        double a[CW], ri = 1.0;
+#pragma unroll
+        for (int i = 0; i < CW; i++) {
+          const double v = Ds[i * DLD + c];
+          a[i] = c < bs ? (i <= c ? v : 0.0) : (i == c ? 1.0 : 0.0);
         }
-        __syncthreads();
-        if (restart) break;
-        const double r = D[j * (PW + 1) + j];
-        if (tid > j && tid < bs) D[j * (PW + 1) + tid] /= r;
-        __syncthreads();
-        {
-          int i = tid >> 5, c = tid & 31;
-          if (i > j && i <= c && c < bs) D[i * (PW + 1) + c] -= D[j * (PW + 1) + i] * D[j * (PW + 1) + c];
-        }
-        __syncthreads();
-      }
-      if (restart) break;
-      for (int idx = tid; idx < PW * PW; idx += NT) {
-        int i = idx >> 5, j = idx & 31;
-        if (i < bs && j < bs && i <= j) R[int64_t(k0 + i) * ldr + k0 + j] = D[i * (PW + 1) + j];
-      }
-      // panel: rows k0..k0+bs-1 of R right of the block, D^T X = A
-      const int c1 = k0 + bs, nt = n - c1;
-      // (each thread owns one column of the panel; its column of P is its scratch)
-      for (int c = tid; c < nt; c += NT) {
-        for (int i = 0; i < PW; i++) {
-          double s = 0.0;
-          if (i < bs) {
-            s = R[int64_t(k0 + i) * ldr + c1 + c];
-            for (int t = 0; t < i; t++) s -= D[t * (PW + 1) + i] * P[t * PLD + c];
-            s /= D[i * (PW + 1) + i];
-            R[int64_t(k0 + i) * ldr + c1 + c] = s;
+        bool bad = false, low = false;
+#pragma unroll
+        for (int j = 0; j < CW; j++) {
+          double d = lane_read_f64(a[j], j);
+          if (!isfinite(d)) {
+            bad = bad || !low;  // what follows a failed pivot may well overflow
+            d = tau;
+          } else if (j < bs && d < 0.5 * tau) {
+            low = true;
+            d = tau;
           }
-          P[i * PLD + c] = s;
+          const double y = rsqrt_f64(d);
+          const double r = sqrt_from(d, y);
+          a[j] = c == j ? r : div_by(a[j], r, y);
+          if (c == j) ri = y;
+#pragma unroll
+          for (int i = j + 1; i < CW; i++) a[i] = fma(-lane_read_f64(a[j], i), a[j], a[i]);
+        }
+        if (l < CW) {
+          ri_s[c] = ri;
+#pragma unroll
+          for (int i = 0; i < CW; i++) Dt[c * DLD + i] = i <= c ? a[i] : 0.0;
+        }
+        if (l == 0) {
+          if (bad) status[0] = 1;
+          if (low) restart = 1;
         }
       }
       __syncthreads();
-      // trailing update (upper tiles): A[c1:, c1:] -= P^T P
-      const int ntl = (nt + 15) >> 4;
-      for (int t = w; t < ntl * (ntl + 1) / 2; t += NT / 64) {
-        int I, J;
-        upper_tile(t, ntl, I, J);
-        const int col = 16 * J + lr;
-        d4s acc;
+      if (restart) break;
+      for (int e = tid; e < CW * CW; e += kCholThreads) {
+        const int i = e >> 4, j = e & 15;
+        if (i < bs && j < bs) R[int64_t(k0 + i) * ldr + k0 + j] = Dt[j * DLD + i];
+      }
+      // panel: rows k0..k0+bs-1 of R right of the block, D^T X = A, a column per thread
+      if (own) {
 #pragma unroll
-        for (int r = 0; r < 4; r++) {
-          int row = 16 * I + 4 * r + lk;
-          acc[r] = (row < nt && col < nt) ? -R[int64_t(c1 + row) * ldr + c1 + col] : 0.0;
-        }
+        for (int i = 0; i < CW; i++) {
+          double s = in ? x[i] : 0.0;
 #pragma unroll
-        for (int k = 0; k < PW; k += 4) acc = mfma64s(P[(k + lk) * PLD + 16 * I + lr], P[(k + lk) * PLD + col], acc);
-#pragma unroll
-        for (int r = 0; r < 4; r++) {
-          int row = 16 * I + 4 * r + lk;
-          if (row < nt && col < nt) R[int64_t(c1 + row) * ldr + c1 + col] = -acc[r];
+          for (int t = 0; t < i; t++) s = fma(-Dt[i * DLD + t], x[t], s);
+          x[i] = div_by(s, Dt[i * DLD + i], ri_s[i]);
+          P[i * LD + tid] = x[i];
+          if (in) R[int64_t(k0 + i) * ldr + c1 + tid] = x[i];
         }
       }
+      __syncthreads();
+      // trailing update (upper tiles): A[c1:, c1:] -= P^T P; the next panel's block also to LDS
+      fold_tiles<NW, 4>(
+          w, ntl, tab,
+          [&](int I, int J, d4s& acc) {
+            const double* src = A + int64_t(c1) * lda + c1 + min(16 * J + lr, nt - 1);
+#pragma unroll
+            for (int r = 0; r < 4; r++) acc[r] = src[min(16 * I + 4 * r + lk, nt - 1) * int(lda)];
+          },
+          [&](int I, int J, d4s acc) {
+#pragma unroll
+            for (int r = 0; r < 4; r++) acc[r] = -(I == J && 4 * r + lk == lr ? acc[r] + add : acc[r]);
+#pragma unroll
+            for (int k = 0; k < CW; k += 4)
+              acc = mfma64s(P[(k + lk) * LD + 16 * I + lr], P[(k + lk) * LD + 16 * J + lr], acc);
+            double* dst = R + (c1 + 16 * I + lk) * ldr + c1 + 16 * J + lr;
+            if (J == 0) {
+#pragma unroll
+              for (int r = 0; r < 4; r++) Ds[(4 * r + lk) * DLD + lr] = -acc[r];
+            } else if (16 * J + 16 <= nt) {  // I <= J: all rows too
+#pragma unroll
+              for (int r = 0; r < 4; r++) dst[4 * r * ldr] = -acc[r];
+            } else {
+#pragma unroll
+              for (int r = 0; r < 4; r++)
+                if (16 * I + 4 * r + lk < nt && 16 * J + lr < nt) dst[4 * r * ldr] = -acc[r];
+            }
+          });
       __syncthreads();
     }
-    int again = restart;
+    const int again = restart;
     __syncthreads();
     if (!again) {
       // strictly lower part
-      for (int i = w; i < n; i += NT / 64)
+      for (int i = w; i < n; i += NW)
         for (int j = l; j < i; j += 64) R[int64_t(i) * ldr + j] = 0.0;
       return;
     }
@@ -179,160 +279,288 @@ __global__ __launch_bounds__(NT) void k_chol_fast(const double* __restrict__ G, 
 }
 
 // ---------------------------------------------------------------------------
-// Pivoted Cholesky with rank detection, real (n <= 256): P^T G P = R^T R.
-// The factorisation runs in physical (unpermuted) column indices, so nothing
-// is swapped: row j of R picks the unpivoted index p with the largest Schur
-// diagonal, R_phys[j][q] = (A[p][q] - sum_{t in panel, t<j} R_phys[t][p]
-// R_phys[t][q]) / sqrt(d_p); earlier panels are folded into A by MFMA rank-32
-// updates.  At the end R[t][c] = R_phys[t][perm[c]].  Stops when the largest
-// remaining diagonal is <= tol * max(diag G) (rank); rows >= rank are zero and
-// perm[rank..] lists the unpivoted indices in increasing order.
-// A: n x n workspace (upper triangle used, physical indices).
+// Pivoted Cholesky with rank detection, real (n <= 256 C): P^T G P = R^T R.  Row j
+// of R picks the unpivoted column p with the largest Schur diagonal (ties to the
+// lower index), R[j][q] = (A[p][q] - sum_{t in panel, t < j} R[t][p] R[t][q]) /
+// sqrt(d_p); after 32 rows they are folded into A.  Stops when the largest
+// remaining diagonal is <= tol * max(diag G) (rank); perm[rank..] lists the
+// unpivoted columns in increasing order.
+//
+// The pivot steps form one chain: largest diagonal, its row of A from L2, new row,
+// diagonals.  One wave per SIMD, thread t owning columns t + 256 c: with 16 waves
+// the chain's scalar work was issued four times per SIMD (2.0 us a step), with one
+// wave its LDS traffic and selections came one after the other (1.7 us).  A thread
+// reads its own columns of the panel while the pivot is being found, those of column
+// p by one LDS read, entry t on lane t, and lane reads, while A's row comes.  One
+// barrier per step, over which the waves exchange their largest diagonals.
+// The fold runs on MFMA and writes the Schur complement of the remaining columns
+// only, compacted (in increasing order) into the other of two buffers: a third of
+// the products that a fold of all columns does.  n = 256: 568 -> 310 us (1,800
+// cycles a step, a quarter of the time in the folds).
+//
+// A, B: n x n workspaces.  R leaves with its columns in G's order (R[t][q], only
+// the columns unpivoted before row t's panel written); k_pchol_cols permutes them.
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(NT) void k_pchol_fast(const double* __restrict__ G, int ldg, int n, double tol,
-                                                   double* __restrict__ A, double* __restrict__ R, int ldr,
-                                                   int* __restrict__ perm, int* __restrict__ rank_out,
-                                                   int* __restrict__ status) {
+constexpr int kPcholThreads = 256;
+template <int C>
+__global__ __launch_bounds__(kPcholThreads) void k_pchol_fast(const double* G, int ldg, int n, double tol, double* A,
+                                                              double* B, double* R, int ldr, int* perm, int* rank_out,
+                                                              int* status) {
   using namespace dense;
-  __shared__ double P[PW * PLD];
-  __shared__ double dg[NMAX];
-  __shared__ double wv_best[2 * (NT / 64)];
-  __shared__ int wv_idx[2 * (NT / 64)];
+  constexpr int NTH = kPcholThreads, NW = NTH / 64, N = NTH * C, LD = PW + 2;
+  __shared__ double P[N * LD];       // entry t of column q at P[q * LD + t]
+  __shared__ double dgs[N];          // diagonals, compacted
+  __shared__ short id[N], al[N];     // column of a position; its position before the fold
+  __shared__ short prm[N];           // the pivots
+  __shared__ double cand_v[2][NW];   // the waves' largest diagonals and their positions
+  __shared__ int cand_p[2][NW];
+  __shared__ int kept[NW * C];
+  __shared__ unsigned short tab[kMaxTiles];
   __shared__ double sh[32];
-  const int tid = threadIdx.x, w = tid >> 6, l = tid & 63, lr = l & 15, lk = l >> 4;
-  for (int i = w; i < n; i += NT / 64)
-    for (int j = l; j < n; j += 64) A[int64_t(i) * n + j] = i <= j ? G[int64_t(i) * ldg + j] : 0.0;
-  for (int q = tid; q < n; q += NT) dg[q] = G[int64_t(q) * ldg + q];
+  const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), l = tid & 63, lr = l & 15, lk = l >> 4;
+  tile_table(tab, (n + 15) >> 4, tid, NTH);
   double dmax = 0.0;
-  for (int q = tid; q < n; q += NT) dmax = fmax(dmax, G[int64_t(q) * ldg + q]);
+  for (int q = tid; q < n; q += NTH) {
+    const double d = G[int64_t(q) * ldg + q];
+    dmax = fmax(dmax, d);
+    dgs[q] = d;
+    id[q] = short(q);
+  }
+  for (int e = tid; e < N * LD; e += NTH) P[e] = 0.0;
   dmax = block_max(dmax, sh);
   if (!(dmax > 0.0) || !isfinite(dmax)) {
-    for (int i = w; i < n; i += NT / 64)
-      for (int j = l; j < n; j += 64) R[int64_t(i) * ldr + j] = 0.0;
-    for (int q = tid; q < n; q += NT) perm[q] = q;
-    if (tid == 0) { rank_out[0] = 0; if (!isfinite(dmax)) atomicOr(status, 16); }
+    for (int q = tid; q < n; q += NTH) perm[q] = q;
+    if (tid == 0) {
+      rank_out[0] = 0;
+      if (!isfinite(dmax)) atomicOr(status, 16);
+    }
     return;
   }
   const double thr = tol * dmax;
-  int rank = n;
-  // Each of the first n threads owns one index q = tid and keeps its Schur
-  // diagonal dq in a register (-2 once pivoted, -3 for threads beyond n).
-  // A pivot step is one barrier: the owners form their entry of the new row
-  // and update dq, and every wave leaves its (max dq, lowest index at that
-  // max) in one of two LDS slots, read by all threads after the barrier to
-  // pick the next pivot (largest dq, ties to the lower index).
-  const int nw = (n + 63) >> 6;
-  const bool own = tid < n;
-  double dq = own ? dg[tid] : -3.0;
-  auto wave_argmax = [&](int slot) {
-    const double m = wave_max_dpp(dq);
-    const uint64_t at = __ballot(dq == m);
-    if (l == 0) {
-      wv_best[slot * (NT / 64) + w] = m;
-      wv_idx[slot * (NT / 64) + w] = 64 * w + (at ? __builtin_ctzll(at) : 63);
-    }
-  };
-  wave_argmax(0);
-  __syncthreads();
-  int slot = 0;
+  const double* S = G;  // Schur complement of the na remaining columns
+  int64_t lds = ldg;
+  int na = n, rank = n;
   for (int k0 = 0; k0 < n; k0 += PW) {
     const int bs = min(PW, n - k0);
+    // dq: the Schur diagonal, -2 once pivoted, -1 if NaN (never a pivot), -3 beyond na
+    double dq[C];
+#pragma unroll
+    for (int c = 0; c < C; c++) {
+      const int q = tid + NTH * c;
+      const double d = q < na ? dgs[q] : -3.0;
+      dq[c] = d == d ? d : -1.0;
+#pragma unroll
+      for (int t = 0; t < PW; t++) P[q * LD + t] = 0.0;
+    }
+    // The wave's largest diagonal (lowest position of several) into slot sl, by the high
+    // words, which order non-negative doubles and put the negative marks last; the
+    // low words only if several lanes share the highest.
+    auto offer = [&](int sl) {
+      double v = dq[0];
+      int q = tid;
+#pragma unroll
+      for (int c = 1; c < C; c++)
+        if (dq[c] > v) {
+          v = dq[c];
+          q = tid + NTH * c;
+        }
+      const int hi = __double2hiint(v), lo = __double2loint(v);
+      const int hm = wave_max_dpp_i32(hi);
+      uint64_t at = __ballot(hi == hm);
+      if (at & (at - 1)) {
+        const int lm = wave_max_dpp_i32(hi == hm ? int(unsigned(lo) >> 1) : 0);  // 31 bits: signed order
+        const bool top = hi == hm && int(unsigned(lo) >> 1) == lm;
+        at = __ballot(top && (lo & 1));
+        if (!at) at = __ballot(top);
+        if (C > 1 && (at & (at - 1))) {  // equal: the lowest position, not the lowest lane
+          int best = 1 << 30;
+          for (uint64_t m = at; m; m &= m - 1) best = min(best, __builtin_amdgcn_readlane(q, __builtin_ctzll(m)));
+          at = __ballot(q == best && ((at >> l) & 1));
+        }
+      }
+      if (l == __builtin_ctzll(at)) {
+        cand_v[sl][w] = v;
+        cand_p[sl][w] = q;
+      }
+    };
+    offer(0);
+    __syncthreads();
     int jj = 0;
     for (; jj < bs; jj++) {
-      const int j = k0 + jj;
-      // all candidates are read at once (n <= 256: at most four waves own indices)
-      double cb[NMAX / 64];
-      int ci[NMAX / 64];
+      const int sl = jj & 1;
+      double bk[NW];
+      int pk[NW];
 #pragma unroll
-      for (int q = 0; q < NMAX / 64; q++) {
-        cb[q] = wv_best[slot * (NT / 64) + q];
-        ci[q] = wv_idx[slot * (NT / 64) + q];
+      for (int k = 0; k < NW; k++) {
+        bk[k] = cand_v[sl][k];
+        pk[k] = cand_p[sl][k];
       }
-      double b = cb[0];
-      int p = ci[0];
+      // this thread's columns of the panel (zero from entry jj on) come from LDS while
+      // the pivot is being found; jd hides jj, or the compiler makes a loop of its own
+      // for each group of entries (32 KB of code)
+      int jd = jj;
+      asm volatile("" : "+s"(jd));
+      double pr[C][PW];
 #pragma unroll
-      for (int q = 1; q < NMAX / 64; q++)
-        if (q < nw && cb[q] > b) { b = cb[q]; p = ci[q]; }
-      if (!(b > thr) || p >= n) break;  // the same decision in every thread
-      if (tid == 0) perm[j] = p;
-      if (own) {
-        const int q = tid;
-        double v;
-        const double r = sqrt(b);
-        if (q == p) v = r;
-        else if (dq < 0.0) v = 0.0;  // already pivoted
-        else {
-          double sacc = p <= q ? A[int64_t(p) * n + q] : A[int64_t(q) * n + p];
-#pragma unroll 8
-          for (int t = 0; t < jj; t++) sacc -= P[t * PLD + p] * P[t * PLD + q];
-          v = sacc / r;
+      for (int t0 = 0; t0 < PW; t0 += 8)
+        if (t0 < jd) {
+#pragma unroll
+          for (int t = t0; t < t0 + 8; t++)
+#pragma unroll
+            for (int c = 0; c < C; c++) pr[c][t] = P[(tid + NTH * c) * LD + t];
         }
-        P[jj * PLD + q] = v;
-        if (q == p) dq = -2.0;
-        else if (dq >= 0.0) dq = fmax(dq - v * v, 0.0);
+      double b = bk[0];
+      int p = pk[0];
+#pragma unroll
+      for (int k = 1; k < NW; k++) {
+        const bool up = bk[k] > b || (C > 1 && bk[k] == b && pk[k] < p);
+        b = up ? bk[k] : b;
+        p = up ? pk[k] : p;
       }
-      slot ^= 1;
-      wave_argmax(slot);
+      p = __builtin_amdgcn_readfirstlane(p);
+      if (__ballot(b > thr) == 0) break;
+      const double prow = P[p * LD + (l & (PW - 1))];
+      double x[C], s[C][4];
+#pragma unroll
+      for (int c = 0; c < C; c++) {
+        const int q = tid + NTH * c;
+        x[c] = S[int64_t(p) * lds + (q < na ? q : 0)];
+        s[c][0] = s[c][1] = s[c][2] = s[c][3] = 0.0;
+      }
+      const double y = rsqrt_f64(b), r = sqrt_from(b, y);
+#pragma unroll
+      for (int t0 = 0; t0 < PW; t0 += 8)
+        if (t0 < jd) {
+#pragma unroll
+          for (int t = t0; t < t0 + 8; t++) {
+            const double pt = lane_read_f64(prow, t);
+#pragma unroll
+            for (int c = 0; c < C; c++) s[c][t & 3] = fma(pt, pr[c][t], s[c][t & 3]);
+          }
+        }
+      if (tid == 0) prm[k0 + jj] = short(p);  // as positions until the panel's end
+#pragma unroll
+      for (int c = 0; c < C; c++) {
+        const int q = tid + NTH * c;
+        double v = div_by(x[c] - ((s[c][0] + s[c][1]) + (s[c][2] + s[c][3])), r, y);
+        double d = fmax(fma(-v, v, dq[c]), 0.0);
+        asm volatile("" : "+v"(v), "+v"(d));  // selections, no branches around them
+        v = q == p ? r : dq[c] <= -2.0 ? 0.0 : v;
+        dq[c] = q == p ? -2.0 : dq[c] >= 0.0 ? d : dq[c];
+        P[q * LD + jj] = v;
+      }
+      offer(sl ^ 1);
       __syncthreads();
     }
-    if (jj < bs) rank = k0 + jj;
-    // rows of this panel (zero beyond the rows computed)
-    for (int t = w; t < PW; t += NT / 64)
-      for (int q = l; q < n; q += 64) {
-        if (t >= jj) P[t * PLD + q] = 0.0;
-        if (t < bs) R[int64_t(k0 + t) * ldr + q] = t < jj ? P[t * PLD + q] : 0.0;
-      }
+    // the remaining columns, in order, move up
+    int mine[C];
+#pragma unroll
+    for (int c = 0; c < C; c++) {
+      const uint64_t m = __ballot(dq[c] > -2.0);
+      mine[c] = __builtin_popcountll(m & ((uint64_t(1) << l) - 1));
+      if (l == 0) kept[c * NW + w] = __builtin_popcountll(m);
+    }
     __syncthreads();
-    if (jj < bs) break;
-    // fold this panel into A (upper tiles, physical indices)
-    const int ntl = (n + 15) >> 4;
-    for (int t = w; t < ntl * (ntl + 1) / 2; t += NT / 64) {
-      int I, J;
-      upper_tile(t, ntl, I, J);
-      const int col = 16 * J + lr;
-      d4s acc;
+    int nr = 0;
 #pragma unroll
-      for (int r4 = 0; r4 < 4; r4++) {
-        int row = 16 * I + 4 * r4 + lk;
-        acc[r4] = (row < n && col < n) ? -A[int64_t(row) * n + col] : 0.0;
+    for (int k = 0; k < NW * C; k++) {
+#pragma unroll
+      for (int c = 0; c < C; c++)
+        if (k < c * NW + w) mine[c] += kept[k];
+      nr += kept[k];
+    }
+#pragma unroll
+    for (int c = 0; c < C; c++)
+      if (dq[c] > -2.0) {
+        al[mine[c]] = short(tid + NTH * c);
+        dgs[mine[c]] = dq[c];
       }
+    if (tid < jj) prm[k0 + tid] = id[prm[k0 + tid]];
 #pragma unroll
-      for (int k = 0; k < PW; k += 4) acc = mfma64s(P[(k + lk) * PLD + 16 * I + lr], P[(k + lk) * PLD + col], acc);
-#pragma unroll
-      for (int r4 = 0; r4 < 4; r4++) {
-        int row = 16 * I + 4 * r4 + lk;
-        if (row < n && col < n) A[int64_t(row) * n + col] = -acc[r4];
+    for (int c = 0; c < C; c++) {
+      const int q = tid + NTH * c;
+      if (q < na) {
+        double* o = R + int64_t(k0) * ldr + id[q];
+        for (int t = 0; t < jj; t++) o[int64_t(t) * ldr] = P[q * LD + t];
       }
     }
     __syncthreads();
-  }
-  // rows at and beyond the rank are zero; perm completes with the unpivoted indices
-  for (int t = rank + w; t < n; t += NT / 64)
-    for (int q = l; q < n; q += 64) R[int64_t(t) * ldr + q] = 0.0;
-  if (own) dg[tid] = dq;
-  __syncthreads();
-  if (tid == 0) {
-    int k = rank;
-    // every index not pivoted (-2), one whose diagonal is NaN included: perm is a
-    // permutation whatever the input, since it is used to address
-    for (int q = 0; q < n; q++)
-      if (dg[q] != -2.0 && k < n) perm[k++] = q;
-    rank_out[0] = rank;
-  }
-  __syncthreads();
-  // R[t][c] = R_phys[t][perm[c]] for c >= t, in chunks of 32 rows through LDS
-  for (int t0 = 0; t0 < rank; t0 += PW) {
-    for (int t = w; t < PW; t += NT / 64)
-      for (int q = l; q < n; q += 64) P[t * PLD + q] = (t0 + t < rank) ? R[int64_t(t0 + t) * ldr + q] : 0.0;
+    short nid[C];  // columns of this thread's positions after the fold
+#pragma unroll
+    for (int c = 0; c < C; c++) nid[c] = tid + NTH * c < nr ? id[al[tid + NTH * c]] : short(0);
+    if (jj < bs || k0 + bs >= n) {
+      rank = k0 + jj;
+#pragma unroll
+      for (int c = 0; c < C; c++)
+        if (tid + NTH * c < nr) prm[rank + tid + NTH * c] = nid[c];
+      break;
+    }
+    // fold the panel into the remaining columns (upper tiles, mirrored)
+    double* D = S == A ? B : A;
+    fold_tiles<NW, 6>(
+        w, (nr + 15) >> 4, tab,
+        [&](int I, int J, d4s& acc) {
+          const double* src = S + al[min(16 * J + lr, nr - 1)];
+#pragma unroll
+          for (int r = 0; r < 4; r++) acc[r] = src[al[min(16 * I + 4 * r + lk, nr - 1)] * int(lds)];
+        },
+        [&](int I, int J, d4s acc) {
+          acc = -acc;
+          const int pi = al[min(16 * I + lr, nr - 1)] * LD + lk, pj = al[min(16 * J + lr, nr - 1)] * LD + lk;
+#pragma unroll
+          for (int k = 0; k < PW; k += 4) acc = mfma64s(P[pi + k], P[pj + k], acc);
+          const int row = 16 * I + lk, col = 16 * J + lr;
+          double *d0 = D + row * n + col, *d1 = D + col * n + row;
+          if (16 * J + 16 <= nr) {  // I <= J: all rows too; a diagonal tile is its own mirror
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+              d0[4 * r * n] = -acc[r];
+              d1[4 * r] = -acc[r];
+            }
+          } else {
+#pragma unroll
+            for (int r = 0; r < 4; r++)
+              if (row + 4 * r < nr && col < nr) {
+                d0[4 * r * n] = -acc[r];
+                d1[4 * r] = -acc[r];
+              }
+          }
+        });
     __syncthreads();
-    for (int t = w; t < PW && t0 + t < rank; t += NT / 64)
-      for (int c = l; c < n; c += 64) {
-        int pc = perm[c];
-        pc = pc < 0 ? 0 : (pc >= n ? n - 1 : pc);
-        R[int64_t(t0 + t) * ldr + c] = c >= t0 + t ? P[t * PLD + pc] : 0.0;
-      }
+#pragma unroll
+    for (int c = 0; c < C; c++)
+      if (tid + NTH * c < nr) id[tid + NTH * c] = nid[c];
+    S = D;
+    lds = n;
+    na = nr;
     __syncthreads();
   }
+  __syncthreads();
+  for (int q = tid; q < n; q += NTH) perm[q] = prm[q];
+  if (tid == 0) rank_out[0] = rank;
+}
+
+// R[t][c] <- R[t][perm[c]] (c >= t, t < rank), 0 elsewhere; one wave per row
+template <int C>
+__global__ __launch_bounds__(256) void k_pchol_cols(double* R, int ldr, int n, const int* perm, const int* rank) {
+  const int t = blockIdx.x * 4 + (threadIdx.x >> 6), l = threadIdx.x & 63;
+  if (t >= n) return;
+  double* r = R + int64_t(t) * ldr;
+  const bool in = t < rank[0];
+  double v[C];
+#pragma unroll
+  for (int c = 0; c < C; c++) {
+    const int q = l + 64 * c, p = q < n ? perm[q] : 0;
+    const double x = r[p >= 0 && p < n ? p : 0];
+    v[c] = in && q >= t ? x : 0.0;
+  }
+  // a lane's stores come after every lane's loads
+#pragma unroll
+  for (int c = 0; c < C; c++) asm volatile("" : "+v"(v[c]));
+  dense::wave_fence();
+#pragma unroll
+  for (int c = 0; c < C; c++)
+    if (l + 64 * c < n) r[l + 64 * c] = v[c];
 }
 
 // ---------------------------------------------------------------------------
@@ -876,67 +1104,84 @@ __global__ __launch_bounds__(256) void k_hqr_rq(int n, const double* __restrict_
   Q[int64_t(i) * ldq + j] = i == j ? 1.0 : 0.0;
 }
 
-// W = R^-1 for an upper triangular R (n <= 256, row-major), one wavefront per
-// column j of W: the back substitution R w = e_j runs from i = j down to 0
-// with the right-hand side r in registers (lane l owns rows l + 64 q):
+// W = R^-1 for an upper triangular R (n <= 64 C, row-major, zeros below), one
+// wavefront per column j of W: the back substitution R w = e_j runs from i = j down
+// to 0 with the right-hand side r in registers (lane l owns rows l + 64 q):
 //   w_i = r_i / R_ii,   r_k -= R_ki w_i  (k < i).
-// The columns of R a stretch of 64 steps needs are staged in LDS, rows
-// padded to 65 doubles so that the lanes of a wave read one column without
-// bank conflicts.  The n columns are independent solves, one workgroup each.
-__global__ __launch_bounds__(64) void k_trinv_cols(const double* __restrict__ R, int ldr, int n,
-                                                   double* __restrict__ W, int ldw) {
-  __shared__ double Rs[dense::NMAX * 65];
-  const int j = blockIdx.x, l = threadIdx.x;
-  auto wave_sync = [] {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-  };
-  double r[4], w[4];
+// The columns of R a stretch of ST steps needs are staged in LDS, rows padded to an
+// odd number of doubles so that the lanes of a wave read one column without bank
+// conflicts.  A workgroup's four waves solve four neighbouring columns on the same
+// stretches, so the staging, which took 85 % of the time of a lone wave, has four
+// times the loads in flight and is done once for the four (n = 256: 97 -> 27 us).
+// The chain of a step is two lane reads and four FMAs (125 cycles): the row block
+// that holds r_i is known when the code is compiled and rows at or below i, which
+// nothing reads again, are updated with the others, so no selection or mask is in it.
+template <int C>
+__global__ __launch_bounds__(256) void k_trinv_cols(const double* __restrict__ R, int ldr, int n,
+                                                    double* __restrict__ W, int ldw) {
+  constexpr int ST = C <= 4 ? 64 : 32, LD = ST + 1, PER = 64 / ST;
+  __shared__ double Rs[64 * C * LD];
+  const int jw = n - 1 - 4 * int(blockIdx.x);  // the workgroup's last column; the longest go first
+  const int j = jw - int(threadIdx.x >> 6), l = threadIdx.x & 63;
+  double r[C], w[C];
 #pragma unroll
-  for (int q = 0; q < 4; q++) {
+  for (int q = 0; q < C; q++) {
     r[q] = (l + 64 * q == j) ? 1.0 : 0.0;
     w[q] = 0.0;
   }
-  for (int g = j >> 6; g >= 0; --g) {
-    const int c0 = 64 * g;
-    const int cl = j - c0 < 63 ? j - c0 : 63;  // last column of the stretch
-    const int rows = c0 + cl + 1;              // rows 0 .. c0 + cl hold the upper triangle
-    wave_sync();  // the previous stretch has been read
-    if (l <= cl) {
+#pragma unroll
+  for (int g = C - 1; g >= 0; g--)  // rows 64 g .. 64 g + 63
+#pragma unroll
+    for (int h = PER - 1; h >= 0; h--) {
+      const int c0 = 64 * g + ST * h;
+      if (c0 > jw) continue;
+      // always whole stretches (a constant trip count): below row j (i > j) the
+      // right-hand side is zero and the diagonal counts as 1, so those steps do nothing
+      const int cl = j - c0 < ST - 1 ? j - c0 : ST - 1;
+      __syncthreads();  // the previous stretch has been read
+      {
+        constexpr int ROWS = 256 / ST;  // rows a pass of the workgroup loads
+        const int lc = threadIdx.x % ST, r0 = threadIdx.x / ST;
+        const bool ok = c0 + lc < n;
+        const double* src = R + (ok ? c0 + lc : 0);
+        double v[64 * C / ROWS];
+#pragma unroll
+        for (int u = 0; u < 64 * (g + 1) / ROWS; u++) {
+          const int k = r0 + ROWS * u;
+          v[u] = src[k < n ? int64_t(k) * ldr : 0];
+        }
+#pragma unroll
+        for (int u = 0; u < 64 * (g + 1) / ROWS; u++) {
+          const int k = r0 + ROWS * u;
+          Rs[k * LD + lc] = ok && k < n ? v[u] : 0.0;
+        }
+      }
+      __syncthreads();
+      // The stretch's diagonal and its reciprocals, one division per lane in
+      // parallel.  A step's quotient is then q0 = r y refined by one residual
+      // step, q0 + (r - d q0) y (the last step of Newton-Markstein division),
+      // so the division leaves the step's dependency chain.
+      const int ld = l % ST;
+      const double dgl = ld <= cl ? Rs[(c0 + ld) * LD + ld] : 1.0;
+      const double dl = 1.0 / dgl;
 #pragma unroll 8
-      for (int k = 0; k < rows; k++) Rs[k * 65 + l] = R[int64_t(k) * ldr + c0 + l];
-    }
-    wave_sync();
-    // The stretch's diagonal and its reciprocals, one division per lane in
-    // parallel.  A step's quotient is then q0 = r y refined by one residual
-    // step, q0 + (r - d q0) y (the last step of Newton-Markstein division),
-    // so the division leaves the step's dependency chain.
-    const double dgl = l <= cl ? Rs[(c0 + l) * 65 + l] : 1.0;
-    const double dl = 1.0 / dgl;
-    auto lane_read = [](double v, int t) {  // t is wave-uniform: a lane read, not a shuffle
-      const long long b = __builtin_bit_cast(long long, v);
-      return __builtin_bit_cast(double, (long long)(unsigned)__builtin_amdgcn_readlane(int(b), t) |
-                                            ((long long)__builtin_amdgcn_readlane(int(b >> 32), t) << 32));
-    };
-    for (int t = cl; t >= 0; --t) {
-      const int i = c0 + t;
-      double rv = r[0];
+      for (int t = ST - 1; t >= 0; --t) {
+        double rk[C];
 #pragma unroll
-      for (int q = 1; q < 4; q++) rv = g == q ? r[q] : rv;
-      const double rt = lane_read(rv, t), d = lane_read(dgl, t), y = lane_read(dl, t);
-      const double q0 = rt * y;
-      const double wi = fma(fma(-d, q0, rt), y, q0);
+        for (int q = 0; q <= g; q++) rk[q] = Rs[(l + 64 * q) * LD + t];
+        const int tl = ST * h + t;  // the lane of row c0 + t
+        const double rt = dense::lane_read_f64(r[g], tl), d = dense::lane_read_f64(dgl, t),
+                     y = dense::lane_read_f64(dl, t);
+        const double q0 = rt * y;
+        const double wi = fma(fma(-d, q0, rt), y, q0);
+        w[g] = l == tl ? wi : w[g];
 #pragma unroll
-      for (int q = 0; q < 4; q++) {
-        if (g == q && l == t) w[q] = wi;
-        const int k = l + 64 * q;
-        if (k < i) r[q] -= Rs[k * 65 + t] * wi;
+        for (int q = 0; q <= g; q++) r[q] = fma(-rk[q], wi, r[q]);
       }
     }
-  }
+  if (j < 0) return;
 #pragma unroll
-  for (int q = 0; q < 4; q++) {
+  for (int q = 0; q < C; q++) {
     const int k = l + 64 * q;
     if (k < n) W[int64_t(k) * ldw + j] = k <= j ? w[q] : 0.0;
   }

@@ -159,13 +159,25 @@ void launch_block_jacobi(pc_ctx* ctx, T* H, int ldh, int n, T* J, int ldj, doubl
 }
 
 
-// Small dense factorisations: blocked MFMA kernels for real n <= 256 (one
-// workgroup), one launch per step over many workgroups for larger single
-// problems (k_mwg.hip), the generic single-workgroup kernels otherwise
+// Small dense factorisations: blocked MFMA kernels for real n <= 512 (one
+// workgroup; at 512 the Cholesky factorisations' products reach about half of one
+// CU's MFMA rate and the chain of pivots costs as much again, still 10 to 30 times
+// less than a launch per step), one launch per step over many workgroups for larger
+// single problems (k_mwg.hip), the generic single-workgroup kernels otherwise
 // (complex n <= 128, batched groups).
 template <class T>
-inline bool use_fast(int n, int nz) { return std::is_same<T, double>::value && n <= dense::NMAX && nz == 1; }
+inline bool use_fast(int n, int nz) { return std::is_same<T, double>::value && n <= dense::DMAX && nz == 1; }
 inline bool use_mw(int n, int nz) { return n > 128 && nz == 1; }
+// f(C): kernels with 64 C >= n columns on the lanes of a wave
+template <class F>
+void with_cols(int n, F f) {
+  if (n <= 64) f(std::integral_constant<int, 1>{});
+  else if (n <= 128) f(std::integral_constant<int, 2>{});
+  else if (n <= 192) f(std::integral_constant<int, 3>{});
+  else if (n <= 256) f(std::integral_constant<int, 4>{});
+  else if (n <= 384) f(std::integral_constant<int, 6>{});
+  else f(std::integral_constant<int, 8>{});
+}
 
 // work: n x n of T, dsc: 1 double, flag: 1 int (multi-workgroup path only)
 template <class T>
@@ -173,7 +185,8 @@ void run_chol_shift(hipStream_t st, const T* G, int n, double shift, T* R, int* 
                     T* work = nullptr, double* dsc = nullptr, int* flag = nullptr) {
   if constexpr (std::is_same<T, double>::value)
     if (use_fast<T>(n, nz)) {
-      hipLaunchKernelGGL(k_chol_fast, dim3(1), dim3(NT), 0, st, G, n, n, shift, R, n, status);
+      const auto k = n <= 256 ? k_chol_fast<256> : k_chol_fast<dense::DMAX>;
+      hipLaunchKernelGGL(k, dim3(1), dim3(kCholThreads), 0, st, G, n, n, shift, R, n, status);
       return;
     }
   if (use_mw(n, nz) && work && dsc && flag) {
@@ -198,7 +211,9 @@ template <class T>
 void run_trinv(hipStream_t st, const T* R, int n, T* W, int nz = 1, int64_t zb = 0) {
   if constexpr (std::is_same<T, double>::value)
     if (use_fast<T>(n, nz)) {
-      hipLaunchKernelGGL(k_trinv_cols, dim3(n), dim3(64), 0, st, R, n, n, W, n);
+      with_cols(n, [&](auto c) {
+        hipLaunchKernelGGL(k_trinv_cols<decltype(c)::value>, dim3(unsigned(ceil_div(n, 4))), dim3(256), 0, st, R, n, n, W, n);
+      });
       return;
     }
   if (use_mw(n, nz)) {  // columns spread over the workgroups
@@ -208,13 +223,19 @@ void run_trinv(hipStream_t st, const T* R, int n, T* W, int nz = 1, int64_t zb =
   }
   hipLaunchKernelGGL((k_trinv_upper<T>), dim3(1, 1, nz), dim3(NT), 0, st, R, n, n, W, n, zb);
 }
-// state: 1 int (multi-workgroup path)
+// A, A2: n x n workspaces (A2: real n <= 512 only); state: 1 int (multi-workgroup path)
 template <class T>
-void run_pchol(hipStream_t st, const T* G, int n, double tol, T* A, T* R, int* perm, int* rank, int* status,
+void run_pchol(hipStream_t st, const T* G, int n, double tol, T* A, T* A2, T* R, int* perm, int* rank, int* status,
                int nz = 1, int64_t zb = 0, int* state = nullptr) {
   if constexpr (std::is_same<T, double>::value)
     if (use_fast<T>(n, nz)) {
-      hipLaunchKernelGGL(k_pchol_fast, dim3(1), dim3(NT), 0, st, G, n, n, tol, A, R, n, perm, rank, status);
+      with_cols(n, [&](auto c) {
+        constexpr int C = decltype(c)::value;
+        hipLaunchKernelGGL(k_pchol_fast<(C > 4 ? 2 : 1)>, dim3(1), dim3(kPcholThreads), 0, st, G, n, n, tol, A, A2, R,
+                           n, perm, rank, status);
+        hipLaunchKernelGGL(k_pchol_cols<C>, dim3(unsigned(ceil_div(n, 4))), dim3(256), 0, st, R, n, n,
+                           (const int*)perm, (const int*)rank);
+      });
       return;
     }
   if (use_mw(n, nz) && state) {
@@ -1229,7 +1250,8 @@ static int core_t(pc_ctx* ctx, const Plan& p, const void* A, int64_t lda, int ce
   }
   PC_CHECK(ctx, launch_streams<T>(ctx, p, A, lda, center, mean, var, part, b, 2));
   reduce_gram<T>(st, p, part, p.mixed ? p.chunks2 : p.chunks, b.G2);
-  run_pchol<T>(st, b.G2, n, p.mixed ? kTolMx : kTolF64, b.Awk, b.R2, b.perm, b.rank, b.status, 1, 0, b.rank + 1);
+  run_pchol<T>(st, b.G2, n, p.mixed ? kTolMx : kTolF64, b.Awk, b.UM, b.R2, b.perm, b.rank, b.status, 1, 0,
+               b.rank + 1);
   // M = R2 (rows < rank) * R1h[perm, :], stored column-major into Hc
   dim3 gg(unsigned(ceil_div(n, 32)), unsigned(ceil_div(n, 32)));
   hipLaunchKernelGGL((k_gemm_small<T>), gg, dim3(256), 0, st, 0, 0, n, n, n, T(1.0), b.R2, n, (const int*)nullptr,
@@ -1272,7 +1294,7 @@ static int core_t(pc_ctx* ctx, const Plan& p, const void* A, int64_t lda, int ce
     hipLaunchKernelGGL((k_copy2d<T>), dim3(nblk(nn)), dim3(256), 0, st, b.Hc, n, n, n, b.tmp, n, 1);
     hipLaunchKernelGGL((k_gemm_small<T>), gg, dim3(256), 0, st, 2, 0, n, n, n, T(1.0), b.tmp, n, (const int*)nullptr,
                        b.tmp, n, (const int*)nullptr, T(0.0), b.G1, n, 0);
-    run_pchol<T>(st, b.G1, n, 1e-30, b.Awk, b.R1, b.perm3, b.rank3, b.status, 1, 0, b.rank3 + 1);
+    run_pchol<T>(st, b.G1, n, 1e-30, b.Awk, b.UM, b.R1, b.perm3, b.rank3, b.status, 1, 0, b.rank3 + 1);
     hipLaunchKernelGGL((k_copy2d<T>), dim3(nblk(nn)), dim3(256), 0, st, b.R1, n, n, n, b.Awk, n, 2);
     run_house_qr_sq<T>(st, b.Awk, n, b.UM, b.G1, nwork, ctx->concurrent);
     hipLaunchKernelGGL((k_permute_rows<T>), dim3(nblk(nn)), dim3(256), 0, st, b.UM, n, n, (const int*)b.perm3, b.Awk,
@@ -1410,7 +1432,7 @@ static int core_batch_t(pc_ctx* ctx, const Plan& p, const pc_problem* pr, int64_
   // ---- P2
   PC_CHECK(ctx, launch_streams<T>(ctx, p, pr[0].A, lda, center, mean, var, part, b, 2, pb));
   reduce_gram<T>(st, p, part, p.mixed ? p.chunks2 : p.chunks, b.G2, nz, zb);
-  run_pchol<T>(st, b.G2, n, p.mixed ? kTolMx : kTolF64, b.Awk, b.R2, b.perm, b.rank, b.status, nz, zb);
+  run_pchol<T>(st, b.G2, n, p.mixed ? kTolMx : kTolF64, b.Awk, (T*)nullptr, b.R2, b.perm, b.rank, b.status, nz, zb);
   dim3 gg(unsigned(ceil_div(n, 32)), unsigned(ceil_div(n, 32)), z);
   hipLaunchKernelGGL((k_gemm_small<T>), gg, dim3(256), 0, st, 0, 0, n, n, n, T(1.0), b.R2, n, (const int*)nullptr,
                      b.R1h, n, (const int*)b.perm, T(0.0), b.Hc, n, 1, zb);

@@ -1,0 +1,53 @@
+"""Dense factorisations of the small stage (k_dense.hip) at the edges of their panels, lane columns and size
+classes, through the solves that run them.  A = Q diag(s) V^T has exact singular values; the FP64 solve's error
+is a small multiple of n u times the largest one (1e-13 n gives it 40 times n u sigma_1 of room at any n here)."""
+import numpy as np
+import pytest
+import torch
+
+import pyloworder_amd as pl
+
+pytestmark = pytest.mark.gpu
+EDGES = [1, 2, 3, 15, 16, 17, 31, 32, 33, 63, 64, 65, 127, 128, 129, 192, 193, 255, 256, 257, 320, 384, 385, 511, 512,
+         513]
+
+
+def _orth(rng, m, n):
+    return np.linalg.qr(rng.standard_normal((m, n)))[0]
+
+
+@pytest.mark.parametrize("n", EDGES)
+@pytest.mark.parametrize("rank", ["full", "half"])
+def test_factor_sizes(n, rank):
+    rng = np.random.default_rng(n)
+    m, k = 2 * n + 40, n if rank == "full" else (n + 1) // 2
+    s = np.linspace(2.0, 1.0, k)
+    A = (_orth(rng, m, k) * s) @ _orth(rng, n, k).T
+    U, S, VT = (x.cpu().numpy() for x in pl.math.tsqr_svd(torch.from_numpy(A).cuda()))
+    tol = 1e-13 * max(n, 10)
+    assert np.abs(S[:k] - s).max() <= tol and (k == n or S[k:].max() <= tol)
+    assert np.abs((U * S) @ VT - A).max() <= tol
+    assert np.abs(U.T @ U - np.eye(n)).max() <= tol and np.abs(VT @ VT.T - np.eye(n)).max() <= tol
+    Q, R = (x.cpu().numpy() for x in pl.math.tsqr(torch.from_numpy(A).cuda()))
+    assert np.abs(Q @ R - A).max() <= tol and np.abs(Q.T @ Q - np.eye(n)).max() <= tol
+
+
+@pytest.mark.parametrize("n", [33, 64, 200, 300])
+def test_equal_diagonals(n):
+    """An orthonormal input: every pivot of the second factorisation ties with the others up to rounding."""
+    Q = _orth(np.random.default_rng(7), 4 * n, n)
+    U, S, VT = (x.cpu().numpy() for x in pl.math.tsqr_svd(torch.from_numpy(Q).cuda()))
+    assert np.abs(S - 1).max() <= 1e-13 * n and np.abs((U * S) @ VT - Q).max() <= 1e-13 * n
+
+
+@pytest.mark.parametrize("n,r", [(256, 74), (200, 17), (64, 33)])
+def test_restarted_shift(n, r):
+    """Sketches after power steps are so ill-conditioned that the shifted factorisation restarts with a larger
+    shift, some pivots in: the result is orthonormal and holds A's leading part all the same."""
+    rng = np.random.default_rng(r)
+    s = 1e3 * 0.8 ** np.arange(n)
+    A = (_orth(rng, 4 * n, n) * s) @ _orth(rng, n, n).T
+    U, S, VT = (x.cpu().numpy() for x in pl.math.randomized_svd(torch.from_numpy(A).cuda(), r, 3, seed=5))
+    assert np.abs(U.T @ U - np.eye(r)).max() <= 1e-13 * n
+    # three power steps and a gap of 0.8 per mode: what is lost is far below the first mode left out's energy
+    assert np.linalg.norm(A - (U * S) @ VT, 2) <= 2 * s[r]
