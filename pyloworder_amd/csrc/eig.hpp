@@ -17,8 +17,12 @@
 // imaginary part first (as ?geev).  The order within T depends on the
 // deflation sequence, so it can differ from LAPACK's for the same matrix.
 //
-// Plain scalar code, __host__ __device__: one GPU thread runs it (n is the
-// truncated DMD rank, small).  Work arrays are the caller's.
+// __host__ __device__; work arrays are the caller's.  The lanes L of one group run it
+// together: every scalar of the iteration is formed by all of them from the same
+// values, rows, columns and vectors are dealt to them, and sync() orders their
+// accesses.  Serial is one lane; on the GPU one wave, with the arrays in LDS where
+// they fit (n is the truncated DMD rank, small): one thread on arrays in memory spent
+// its time on the latency of one access after the other, 1.6 ms at n = 12.
 #pragma once
 #include <cmath>
 
@@ -31,6 +35,11 @@
 #endif
 
 namespace eig {
+
+struct Serial {
+  static constexpr int id = 0, count = 1;
+  PC_EIG_HD void sync() const {}
+};
 
 PC_EIG_HD inline double dabs(double x) { return x < 0 ? -x : x; }
 PC_EIG_HD inline double dmax(double a, double b) { return a > b ? a : b; }
@@ -50,53 +59,67 @@ PC_EIG_HD inline void cdiv(double ar, double ai, double br, double bi, double& c
 
 // H (n x n, row-major, ld n) is overwritten; Z (n x n) receives the Schur
 // vectors and then the (real-packed) eigenvectors; wr / wi the eigenvalues;
-// ort (n) work.  Returns 0, or -1 when the QR iteration did not converge.
-PC_EIG_HD inline int real_eig(double* H, double* Z, double* wr, double* wi, double* ort, int nn) {
+// E (n x n) and ort (n) work.  Returns 0, or -1 when the QR iteration did not converge.
+template <class L>
+PC_EIG_HD inline int real_eig(const L& lanes, double* H, double* Z, double* E, double* wr, double* wi, double* ort,
+                              int nn) {
+#define Em(i, j) E[(i) * nn + (j)]
 #define Hm(i, j) H[(i) * nn + (j)]
 #define Zm(i, j) Z[(i) * nn + (j)]
   const double eps = 2.220446049250313e-16;
   const int low = 0, high = nn - 1;
+  const int me = lanes.id, step = lanes.count;
   // ---- 1. Hessenberg reduction
   for (int m = low + 1; m <= high - 1; m++) {
     double scale = 0.0;
     for (int i = m; i <= high; i++) scale += dabs(Hm(i, m - 1));
     if (scale != 0.0) {
       double h = 0.0;
-      for (int i = high; i >= m; i--) {
-        ort[i] = Hm(i, m - 1) / scale;
-        h += ort[i] * ort[i];
-      }
+      for (int i = m + me; i <= high; i += step) ort[i] = Hm(i, m - 1) / scale;
+      lanes.sync();
+      for (int i = high; i >= m; i--) h += ort[i] * ort[i];
       double g = sqrt(h);
-      if (ort[m] > 0) g = -g;
-      h -= ort[m] * g;
-      ort[m] -= g;
-      for (int j = m; j < nn; j++) {
+      const double om = ort[m];
+      if (om > 0) g = -g;
+      h -= om * g;
+      lanes.sync();
+      if (me == 0) ort[m] = om - g;
+      lanes.sync();
+      for (int j = m + me; j < nn; j += step) {
         double f = 0.0;
         for (int i = high; i >= m; i--) f += ort[i] * Hm(i, j);
         f /= h;
         for (int i = m; i <= high; i++) Hm(i, j) -= f * ort[i];
       }
-      for (int i = 0; i <= high; i++) {
+      lanes.sync();
+      for (int i = me; i <= high; i += step) {
         double f = 0.0;
         for (int j = high; j >= m; j--) f += ort[j] * Hm(i, j);
         f /= h;
         for (int j = m; j <= high; j++) Hm(i, j) -= f * ort[j];
       }
-      ort[m] = scale * ort[m];
-      Hm(m, m - 1) = scale * g;
+      lanes.sync();
+      if (me == 0) {
+        ort[m] = scale * (om - g);
+        Hm(m, m - 1) = scale * g;
+      }
+      lanes.sync();
     }
   }
-  for (int i = 0; i < nn; i++)
+  for (int i = me; i < nn; i += step)
     for (int j = 0; j < nn; j++) Zm(i, j) = (i == j ? 1.0 : 0.0);
+  lanes.sync();
   for (int m = high - 1; m >= low + 1; m--) {
     if (Hm(m, m - 1) != 0.0) {
-      for (int i = m + 1; i <= high; i++) ort[i] = Hm(i, m - 1);
-      for (int j = m; j <= high; j++) {
+      for (int i = m + 1 + me; i <= high; i += step) ort[i] = Hm(i, m - 1);
+      lanes.sync();
+      for (int j = m + me; j <= high; j += step) {
         double g = 0.0;
         for (int i = m; i <= high; i++) g += ort[i] * Zm(i, j);
         g = (g / ort[m]) / Hm(m, m - 1);  // two divisions: no underflow of the product
         for (int i = m; i <= high; i++) Zm(i, j) += g * ort[i];
       }
+      lanes.sync();
     }
   }
   // ---- 2. Francis double-shift QR
@@ -115,9 +138,12 @@ PC_EIG_HD inline int real_eig(double* H, double* Z, double* wr, double* wi, doub
       l--;
     }
     if (l == n) {  // one root
-      Hm(n, n) = Hm(n, n) + exshift;
-      wr[n] = Hm(n, n);
-      wi[n] = 0.0;
+      if (me == 0) {
+        Hm(n, n) = Hm(n, n) + exshift;
+        wr[n] = Hm(n, n);
+        wi[n] = 0.0;
+      }
+      lanes.sync();
       n--;
       iter = 0;
     } else if (l == n - 1) {  // two roots
@@ -125,16 +151,21 @@ PC_EIG_HD inline int real_eig(double* H, double* Z, double* wr, double* wi, doub
       p = (Hm(n - 1, n - 1) - Hm(n, n)) / 2.0;
       q = p * p + w;
       z = sqrt(dabs(q));
-      Hm(n, n) = Hm(n, n) + exshift;
-      Hm(n - 1, n - 1) = Hm(n - 1, n - 1) + exshift;
-      x = Hm(n, n);
+      x = Hm(n, n) + exshift;
+      lanes.sync();
+      if (me == 0) {
+        Hm(n, n) = x;
+        Hm(n - 1, n - 1) = Hm(n - 1, n - 1) + exshift;
+      }
+      lanes.sync();
       if (q >= 0) {  // real pair: rotate the 2x2 block to upper triangular
         z = (p >= 0) ? p + z : p - z;
-        wr[n - 1] = x + z;
-        wr[n] = wr[n - 1];
-        if (z != 0.0) wr[n] = x - w / z;
-        wi[n - 1] = 0.0;
-        wi[n] = 0.0;
+        if (me == 0) {
+          wr[n - 1] = x + z;
+          wr[n] = z != 0.0 ? x - w / z : x + z;
+          wi[n - 1] = 0.0;
+          wi[n] = 0.0;
+        }
         x = Hm(n, n - 1);
         s = dabs(x) + dabs(z);
         p = x / s;
@@ -142,22 +173,24 @@ PC_EIG_HD inline int real_eig(double* H, double* Z, double* wr, double* wi, doub
         r = sqrt(p * p + q * q);
         p /= r;
         q /= r;
-        for (int j = n - 1; j < nn; j++) {
+        for (int j = n - 1 + me; j < nn; j += step) {
           z = Hm(n - 1, j);
           Hm(n - 1, j) = q * z + p * Hm(n, j);
           Hm(n, j) = q * Hm(n, j) - p * z;
         }
-        for (int i = 0; i <= n; i++) {
+        lanes.sync();
+        for (int i = me; i <= n; i += step) {
           z = Hm(i, n - 1);
           Hm(i, n - 1) = q * z + p * Hm(i, n);
           Hm(i, n) = q * Hm(i, n) - p * z;
         }
-        for (int i = low; i <= high; i++) {
+        for (int i = low + me; i <= high; i += step) {
           z = Zm(i, n - 1);
           Zm(i, n - 1) = q * z + p * Zm(i, n);
           Zm(i, n) = q * Zm(i, n) - p * z;
         }
-      } else {  // complex pair
+        lanes.sync();
+      } else if (me == 0) {  // complex pair
         wr[n - 1] = x + p;
         wr[n] = x + p;
         wi[n - 1] = z;
@@ -175,7 +208,9 @@ PC_EIG_HD inline int real_eig(double* H, double* Z, double* wr, double* wi, doub
       }
       if (iter == 10) {  // exceptional shift (Wilkinson)
         exshift += x;
-        for (int i = low; i <= n; i++) Hm(i, i) -= x;
+        lanes.sync();
+        for (int i = low + me; i <= n; i += step) Hm(i, i) -= x;
+        lanes.sync();
         s = dabs(Hm(n, n - 1)) + dabs(Hm(n - 1, n - 2));
         x = y = 0.75 * s;
         w = -0.4375 * s * s;
@@ -187,7 +222,9 @@ PC_EIG_HD inline int real_eig(double* H, double* Z, double* wr, double* wi, doub
           s = sqrt(s);
           if (y < x) s = -s;
           s = x - w / ((y - x) / 2.0 + s);
-          for (int i = low; i <= n; i++) Hm(i, i) -= s;
+          lanes.sync();
+          for (int i = low + me; i <= n; i += step) Hm(i, i) -= s;
+          lanes.sync();
           exshift += s;
           x = y = w = 0.964;
         }
@@ -212,17 +249,21 @@ PC_EIG_HD inline int real_eig(double* H, double* Z, double* wr, double* wi, doub
           break;
         m--;
       }
-      for (int i = m + 2; i <= n; i++) {
+      lanes.sync();
+      for (int i = m + 2 + me; i <= n; i += step) {
         Hm(i, i - 2) = 0.0;
         if (i > m + 2) Hm(i, i - 3) = 0.0;
       }
+      lanes.sync();
       for (int k = m; k <= n - 1; k++) {  // chase the bulge
         const bool notlast = (k != n - 1);
+        lanes.sync();
         if (k != m) {
           p = Hm(k, k - 1);
           q = Hm(k + 1, k - 1);
           r = notlast ? Hm(k + 2, k - 1) : 0.0;
           x = dabs(p) + dabs(q) + dabs(r);
+          lanes.sync();
           if (x == 0.0) continue;
           p /= x;
           q /= x;
@@ -231,15 +272,17 @@ PC_EIG_HD inline int real_eig(double* H, double* Z, double* wr, double* wi, doub
         s = sqrt(p * p + q * q + r * r);
         if (p < 0) s = -s;
         if (s != 0) {
-          if (k != m) Hm(k, k - 1) = -s * x;
-          else if (l != m) Hm(k, k - 1) = -Hm(k, k - 1);
+          if (me == 0) {  // read by every lane above, and not again in this step
+            if (k != m) Hm(k, k - 1) = -s * x;
+            else if (l != m) Hm(k, k - 1) = -Hm(k, k - 1);
+          }
           p += s;
           x = p / s;
           y = q / s;
           z = r / s;
           q /= p;
           r /= p;
-          for (int j = k; j < nn; j++) {
+          for (int j = k + me; j < nn; j += step) {
             p = Hm(k, j) + q * Hm(k + 1, j);
             if (notlast) {
               p += r * Hm(k + 2, j);
@@ -249,7 +292,8 @@ PC_EIG_HD inline int real_eig(double* H, double* Z, double* wr, double* wi, doub
             Hm(k + 1, j) -= p * y;
           }
           const int ilim = n < k + 3 ? n : k + 3;
-          for (int i = 0; i <= ilim; i++) {
+          lanes.sync();
+          for (int i = me; i <= ilim; i += step) {
             p = x * Hm(i, k) + y * Hm(i, k + 1);
             if (notlast) {
               p += z * Hm(i, k + 2);
@@ -258,7 +302,7 @@ PC_EIG_HD inline int real_eig(double* H, double* Z, double* wr, double* wi, doub
             Hm(i, k) -= p;
             Hm(i, k + 1) -= p * q;
           }
-          for (int i = low; i <= high; i++) {
+          for (int i = low + me; i <= high; i += step) {
             p = x * Zm(i, k) + y * Zm(i, k + 1);
             if (notlast) {
               p += z * Zm(i, k + 2);
@@ -269,55 +313,58 @@ PC_EIG_HD inline int real_eig(double* H, double* Z, double* wr, double* wi, doub
           }
         }
       }
+      lanes.sync();
     }
   }
-  // ---- 3. eigenvectors of the quasi-triangular form, then back-transformed
+  // ---- 3. eigenvectors of the quasi-triangular form (into E, a vector per lane), then
+  // back-transformed
+  lanes.sync();
   if (norm == 0.0) return 0;
-  for (n = nn - 1; n >= 0; n--) {
+  for (n = nn - 1 - me; n >= 0; n -= step) {
     p = wr[n];
     q = wi[n];
     if (q == 0) {  // real vector
       int l = n;
-      Hm(n, n) = 1.0;
+      Em(n, n) = 1.0;
       for (int i = n - 1; i >= 0; i--) {
         w = Hm(i, i) - p;
         r = 0.0;
-        for (int j = l; j <= n; j++) r += Hm(i, j) * Hm(j, n);
+        for (int j = l; j <= n; j++) r += Hm(i, j) * Em(j, n);
         if (wi[i] < 0.0) {
           z = w;
           s = r;
         } else {
           l = i;
           if (wi[i] == 0.0) {
-            Hm(i, n) = (w != 0.0) ? -r / w : -r / (eps * norm);
+            Em(i, n) = (w != 0.0) ? -r / w : -r / (eps * norm);
           } else {  // the 2x2 block of a conjugate pair above
             x = Hm(i, i + 1);
             y = Hm(i + 1, i);
             q = (wr[i] - p) * (wr[i] - p) + wi[i] * wi[i];
             t = (x * s - z * r) / q;
-            Hm(i, n) = t;
-            Hm(i + 1, n) = (dabs(x) > dabs(z)) ? (-r - w * t) / x : (-s - y * t) / z;
+            Em(i, n) = t;
+            Em(i + 1, n) = (dabs(x) > dabs(z)) ? (-r - w * t) / x : (-s - y * t) / z;
           }
-          t = dabs(Hm(i, n));
+          t = dabs(Em(i, n));
           if ((eps * t) * t > 1)
-            for (int j = i; j <= n; j++) Hm(j, n) /= t;
+            for (int j = i; j <= n; j++) Em(j, n) /= t;
         }
       }
     } else if (q < 0) {  // complex vector: real part in column n-1, imaginary in column n
       int l = n - 1;
       if (dabs(Hm(n, n - 1)) > dabs(Hm(n - 1, n))) {
-        Hm(n - 1, n - 1) = q / Hm(n, n - 1);
-        Hm(n - 1, n) = -(Hm(n, n) - p) / Hm(n, n - 1);
+        Em(n - 1, n - 1) = q / Hm(n, n - 1);
+        Em(n - 1, n) = -(Hm(n, n) - p) / Hm(n, n - 1);
       } else {
-        cdiv(0.0, -Hm(n - 1, n), Hm(n - 1, n - 1) - p, q, Hm(n - 1, n - 1), Hm(n - 1, n));
+        cdiv(0.0, -Hm(n - 1, n), Hm(n - 1, n - 1) - p, q, Em(n - 1, n - 1), Em(n - 1, n));
       }
-      Hm(n, n - 1) = 0.0;
-      Hm(n, n) = 1.0;
+      Em(n, n - 1) = 0.0;
+      Em(n, n) = 1.0;
       for (int i = n - 2; i >= 0; i--) {
         double ra = 0.0, sa = 0.0, vr, vi;
         for (int j = l; j <= n; j++) {
-          ra += Hm(i, j) * Hm(j, n - 1);
-          sa += Hm(i, j) * Hm(j, n);
+          ra += Hm(i, j) * Em(j, n - 1);
+          sa += Hm(i, j) * Em(j, n);
         }
         w = Hm(i, i) - p;
         if (wi[i] < 0.0) {
@@ -327,56 +374,60 @@ PC_EIG_HD inline int real_eig(double* H, double* Z, double* wr, double* wi, doub
         } else {
           l = i;
           if (wi[i] == 0) {
-            cdiv(-ra, -sa, w, q, Hm(i, n - 1), Hm(i, n));
+            cdiv(-ra, -sa, w, q, Em(i, n - 1), Em(i, n));
           } else {
             x = Hm(i, i + 1);
             y = Hm(i + 1, i);
             vr = (wr[i] - p) * (wr[i] - p) + wi[i] * wi[i] - q * q;
             vi = (wr[i] - p) * 2.0 * q;
             if (vr == 0.0 && vi == 0.0) vr = eps * norm * (dabs(w) + dabs(q) + dabs(x) + dabs(y) + dabs(z));
-            cdiv(x * r - z * ra + q * sa, x * s - z * sa - q * ra, vr, vi, Hm(i, n - 1), Hm(i, n));
+            cdiv(x * r - z * ra + q * sa, x * s - z * sa - q * ra, vr, vi, Em(i, n - 1), Em(i, n));
             if (dabs(x) > (dabs(z) + dabs(q))) {
-              Hm(i + 1, n - 1) = (-ra - w * Hm(i, n - 1) + q * Hm(i, n)) / x;
-              Hm(i + 1, n) = (-sa - w * Hm(i, n) - q * Hm(i, n - 1)) / x;
+              Em(i + 1, n - 1) = (-ra - w * Em(i, n - 1) + q * Em(i, n)) / x;
+              Em(i + 1, n) = (-sa - w * Em(i, n) - q * Em(i, n - 1)) / x;
             } else {
-              cdiv(-r - y * Hm(i, n - 1), -s - y * Hm(i, n), z, q, Hm(i + 1, n - 1), Hm(i + 1, n));
+              cdiv(-r - y * Em(i, n - 1), -s - y * Em(i, n), z, q, Em(i + 1, n - 1), Em(i + 1, n));
             }
           }
-          t = dmax(dabs(Hm(i, n - 1)), dabs(Hm(i, n)));
+          t = dmax(dabs(Em(i, n - 1)), dabs(Em(i, n)));
           if ((eps * t) * t > 1)
             for (int j = i; j <= n; j++) {
-              Hm(j, n - 1) /= t;
-              Hm(j, n) /= t;
+              Em(j, n - 1) /= t;
+              Em(j, n) /= t;
             }
         }
       }
     }
   }
-  for (int j = nn - 1; j >= low; j--)
-    for (int i = low; i <= high; i++) {
+  lanes.sync();
+  for (int i = low + me; i <= high; i += step)
+    for (int j = nn - 1; j >= low; j--) {
       z = 0.0;
-      for (int k = low; k <= (j < high ? j : high); k++) z += Zm(i, k) * Hm(k, j);
+      for (int k = low; k <= j; k++) z += Zm(i, k) * Em(k, j);
       Zm(i, j) = z;
     }
+  lanes.sync();
+#undef Em
 #undef Hm
 #undef Zm
   return 0;
 }
 
 // ?geev's normalisation of the packed real vectors in Z into complex vectors
-// V (n x n, interleaved re/im, row-major): a real eigenvalue's column scaled
+// V (n x n, interleaved re/im, row-major, ld ldv): a real eigenvalue's column scaled
 // to unit 2-norm; a pair (j, j+1) (wi[j] > 0) gives v_j = (z_j + i z_{j+1})
 // scaled to unit norm and rotated so that its largest-modulus component is
 // real with the sign of its real part, and v_{j+1} = conj(v_j).
-PC_EIG_HD inline void normalise(const double* Z, const double* wi, int nn, double* V) {
-  for (int j = 0; j < nn; j++) {
+template <class L>
+PC_EIG_HD inline void normalise(const L& lanes, const double* Z, const double* wi, int nn, double* V, long long ldv) {
+  for (int j = lanes.id; j < nn; j += lanes.count) {
     if (wi[j] == 0.0) {
       double s = 0.0;
       for (int i = 0; i < nn; i++) s += Z[i * nn + j] * Z[i * nn + j];
       s = s > 0 ? 1.0 / sqrt(s) : 1.0;
       for (int i = 0; i < nn; i++) {
-        V[2 * (i * nn + j)] = Z[i * nn + j] * s;
-        V[2 * (i * nn + j) + 1] = 0.0;
+        V[2 * (i * ldv + j)] = Z[i * nn + j] * s;
+        V[2 * (i * ldv + j) + 1] = 0.0;
       }
     } else if (wi[j] > 0.0 && j + 1 < nn) {
       double s = 0.0, best = -1.0;
@@ -394,12 +445,11 @@ PC_EIG_HD inline void normalise(const double* Z, const double* wi, int nn, doubl
       for (int i = 0; i < nn; i++) {
         const double a = Z[i * nn + j] * s, b = Z[i * nn + j + 1] * s;
         const double re = c * a + sn * b, im = c * b - sn * a;
-        V[2 * (i * nn + j)] = re;
-        V[2 * (i * nn + j) + 1] = i == kb ? 0.0 : im;
-        V[2 * (i * nn + j + 1)] = re;
-        V[2 * (i * nn + j + 1) + 1] = i == kb ? 0.0 : -im;
+        V[2 * (i * ldv + j)] = re;
+        V[2 * (i * ldv + j) + 1] = i == kb ? 0.0 : im;
+        V[2 * (i * ldv + j + 1)] = re;
+        V[2 * (i * ldv + j + 1) + 1] = i == kb ? 0.0 : -im;
       }
-      j++;
     }
   }
 }

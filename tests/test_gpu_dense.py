@@ -51,3 +51,28 @@ def test_restarted_shift(n, r):
     assert np.abs(U.T @ U - np.eye(r)).max() <= 1e-13 * n
     # three power steps and a gap of 0.8 per mode: what is lost is far below the first mode left out's energy
     assert np.linalg.norm(A - (U * S) @ VT, 2) <= 2 * s[r]
+
+
+@pytest.mark.parametrize("n", [1, 2, 3, 5, 12, 31, 64, 65, 72, 73, 100])
+@pytest.mark.parametrize("kind", ["random", "rotations"])
+def test_eig_sizes(n, kind):
+    """Eigenpairs by their residual (n u ||A|| of the backward-stable QR iteration, with room) and trace; below and
+    above one lane per column and the size whose arrays fit in LDS. Rotations: every eigenvalue in a pair of modulus 1
+    (and one 1), none of which the iteration may split into reals."""
+    rng = np.random.default_rng(n)
+    A = rng.standard_normal((n, n))
+    if kind == "rotations":
+        Q = _orth(rng, n, n)
+        th = np.linspace(0.3, 2.8, n // 2)
+        D = np.eye(n)
+        for i, t in enumerate(th):
+            D[2 * i:2 * i + 2, 2 * i:2 * i + 2] = [[np.cos(t), -np.sin(t)], [np.sin(t), np.cos(t)]]
+        A = Q @ D @ Q.T
+    wr, wi, V = (x.cpu().numpy() for x in pl.math.eigen(torch.from_numpy(A).cuda()))
+    w = wr + 1j * wi
+    tol = 1e-13 * max(n, 10) * np.linalg.norm(A, 2)
+    assert np.abs(A @ V - V * w).max() <= tol
+    assert abs(w.sum() - np.trace(A)) <= tol * n
+    assert np.abs(np.linalg.norm(V, axis=0) - 1).max() <= 1e-13
+    if kind == "rotations":
+        assert np.abs(np.abs(w) - 1).max() <= tol and (np.abs(wi) > 0.1).sum() == 2 * (n // 2)
