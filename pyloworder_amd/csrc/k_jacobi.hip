@@ -94,8 +94,11 @@ struct JacPair {
 // both side by side, through LDS) before the 16 rounds of pairs across them, in which
 // round s pairs u_k with v_{k+s}: u's data stay with their thread, v's move on by one
 // pair per round, along bq by DPP, along bp through LDS.  One barrier per round.
+// players < 16 (even): no column beyond the first `players` exists, so players - 1
+// rounds meet every pair.
 template <bool FULL>
-PC_DEV void jac_rounds(JacPair<FULL>& S, int t, double negl, double tol2, const double (&g)[4], double (&q)[4]) {
+PC_DEV void jac_rounds(JacPair<FULL>& S, int t, double negl, double tol2, const double (&g)[4], double (&q)[4],
+                       int players = GB, bool cross = true) {
   const int bp = t >> 4, bq = t & 15;
   double guu = g[0], guv = g[1], gvu = g[2], gvv = g[3];
   q[0] = 2 * bp == bq ? 1.0 : 0.0;
@@ -112,18 +115,21 @@ PC_DEV void jac_rounds(JacPair<FULL>& S, int t, double negl, double tol2, const 
     S.Q[0][(2 * bp + 1) * GLD + bq] = q[2];
     S.Q[0][(2 * bp + 1) * GLD + GB + bq] = q[3];
     // Positions, not columns: the players of each block's circle schedule sit at
-    // positions 0..15, pair k of block k / 8 at positions k & 7 and 15 - (k & 7), and
-    // every result is stored where its player sits in the next round (slot k moves to
-    // k - 1, slot 1 to 15, slot 0 stays), so a thread's addresses never change.  After
-    // 15 rounds everybody is back.
-    auto next = [](int k) { return k == 0 ? 0 : k == 1 ? GB - 1 : k - 1; };
+    // positions 0..players - 1, pair k of block k / 8 at positions k & 7 and players - 1 -
+    // (k & 7), and every result is stored where its player sits in the next round (slot
+    // k moves to k - 1, slot 1 to the last, slot 0 stays), so a thread's addresses never
+    // change.  After players - 1 rounds everybody is back.  The (empty) positions
+    // beyond pair up among themselves and stay.
+    auto first = [&](int k) { return 2 * k < players ? k : 2 * k; };
+    auto second = [&](int k) { return 2 * k < players ? players - 1 - k : 2 * k + 1; };
+    auto next = [&](int k) { return k == 0 || k >= players ? k : k == 1 ? players - 1 : k - 1; };
     const int ob = 2 * (bp & 8), oq = 2 * (bq & 8);
-    const int up = ob + (bp & 7), vp = ob + GB - 1 - (bp & 7), uq = oq + (bq & 7), vq = oq + GB - 1 - (bq & 7);
-    const int upn = ob + next(bp & 7), vpn = ob + next(GB - 1 - (bp & 7));
-    const int uqn = oq + next(bq & 7), vqn = oq + next(GB - 1 - (bq & 7));
+    const int up = ob + first(bp & 7), vp = ob + second(bp & 7), uq = oq + first(bq & 7), vq = oq + second(bq & 7);
+    const int upn = ob + next(up - ob), vpn = ob + next(vp - ob);
+    const int uqn = oq + next(uq - oq), vqn = oq + next(vq - oq);
     __syncthreads();
 #pragma unroll 2
-    for (int s = 0; s < GB - 1; s++) {
+    for (int s = 0; s < players - 1; s++) {
       const double *G0 = S.G[s & 1], *Q0 = S.Q[s & 1];
       double *G1 = S.G[~s & 1], *Q1 = S.Q[~s & 1];
       double cq, sq;
@@ -154,6 +160,7 @@ PC_DEV void jac_rounds(JacPair<FULL>& S, int t, double negl, double tol2, const 
     q[2] = S.Q[last][(2 * bp + 1) * GLD + bq];
     q[3] = S.Q[last][(2 * bp + 1) * GLD + GB + bq];
   }
+  if (!cross) return;
   // Round s's rotation k needs G_uu, G_vv, G_uv of pair k: the last two are the
   // diagonals of what moved in the round before (G_uv as its mirror G_vu), the first
   // every thread carries along for its own k = bq.
@@ -409,7 +416,8 @@ __global__ __launch_bounds__(512) void k_bjac_pair(double* __restrict__ H, int l
   }
 }
 
-// n <= 32: every column in one pair, iterated to convergence on one workgroup
+// n <= 32: every column in one pair, iterated to convergence on one workgroup.  A sweep
+// is n - 1 rounds (n even) up to 16 columns, 31 beyond: n = 8 76 -> 31 us.
 __global__ __launch_bounds__(256) void k_bjac_one(double* __restrict__ H, int ldh, int n, double* __restrict__ J,
                                                   int ldj, int* state, const double* dstate, double tol2,
                                                   int max_sweeps) {
@@ -452,7 +460,7 @@ __global__ __launch_bounds__(256) void k_bjac_one(double* __restrict__ H, int ld
       break;
     }
     double qq[4];
-    jac_rounds<true>(S, t, negl, tol2, gg, qq);
+    jac_rounds<true>(S, t, negl, tol2, gg, qq, n <= GB ? (n < 2 ? 2 : (n + 1) & ~1) : GB, n > GB);
     double* o = Qs + 2 * bp * GLD;
     o[bq] = qq[0];
     o[GB + bq] = qq[1];
