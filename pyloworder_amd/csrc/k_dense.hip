@@ -1,8 +1,8 @@
 // FP64 dense kernels for real n x n matrices (the small dense stage of the POD
-// core): shifted Cholesky, pivoted Cholesky and the triangular inverse for n <= 512,
-// Householder QR with explicit Q for n <= 256.  The factorisations are blocked, on
-// one workgroup: matrices live in global memory (L2-resident at these sizes), panels
-// are staged in LDS and the updates run on v_mfma_f64_16x16x4f64.
+// core), n <= 512: shifted Cholesky, pivoted Cholesky, the triangular inverse and
+// Householder QR with explicit Q.  The factorisations are blocked, the Cholesky ones
+// on one workgroup: matrices live in global memory (L2-resident at these sizes),
+// panels in LDS or registers, and the updates run on v_mfma_f64_16x16x4f64.
 //
 // f64 MFMA 16x16x4 lane layout (wave64): lane l holds A[l % 16][l / 16] and
 // B[l / 16][l % 16]; accumulator register r holds D[4 r + l / 16][l % 16].
@@ -11,9 +11,7 @@
 namespace dense {
 
 constexpr int PW = 32;           // panel width
-constexpr int PLD = 257;         // LDS leading dimension of panels (odd: no bank conflicts)
-constexpr int NMAX = 256;        // of the Householder QR
-constexpr int DMAX = 512;        // of the Cholesky factorisations and the triangular inverse
+constexpr int DMAX = 512;        // widest matrix
 
 // DPP move of a double (both 32-bit halves), lanes that the row mask leaves
 // out return `old`
@@ -81,6 +79,14 @@ PC_DEV void wave_fence() {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+// f(I), f(I + 1), ... f(N - 1), the number a constant
+template <int I, int N, class F>
+PC_DEV void static_for(F f) {
+  if constexpr (I < N) {
+    f(std::integral_constant<int, I>{});
+    static_for<I + 1, N>(f);
+  }
 }
 // The upper tiles of any grid, numbered from its last one: tile k is e / 256 rows and
 // e % 256 columns before the last, e = tab[k]
@@ -564,532 +570,337 @@ __global__ __launch_bounds__(256) void k_pchol_cols(double* R, int ldr, int n, c
 }
 
 // ---------------------------------------------------------------------------
-// Householder QR of a real n x n matrix (n <= 256) in one launch on one
-// workgroup: the same panels, block reflectors and MFMA sequence as the
-// launch sequence below (k_hqr_panel / k_hqr_strip / k_hqr_rq), so Q and R
-// are the same; it serves solves that share the GPU with other streams,
-// where one launch costs less than the sequence's 3 npan launches.
+// Householder QR of a real n x n matrix (n <= 64 RW), A = Q R, Q explicit.
 // LAPACK conventions (beta = -sign(alpha) ||x||, tau = (beta - alpha) / beta).
-// work: n*n (the factored matrix) + n (tau) + 32*32*ceil(n/32) (T).  The
-// K-loops over global memory load eight k-steps ahead of their products.
+// Panels of 32 columns are factored on one workgroup (k_hqr_panel: the column loop,
+// V^T V, T of the compact WY form); the block reflector I - V T V^T updates the
+// trailing columns after each panel, and Q, accumulated backwards, one workgroup per
+// 32-column strip (k_hqr_strip).  work: n*n (the factored matrix) + n (tau) +
+// 32*32*ceil(n/32) (T).
+//
+// The column loop is a chain (norm, reflector, its products with the other columns),
+// so the panel lives in the registers of one wave per SIMD, wave w holding columns
+// w + 4 k, lane l rows l + 64 q: only the reflector goes through LDS, one barrier per
+// column, and a wave reduces its columns' dot products together.  n = 256: a panel 69
+// -> 29 us (on 16 waves, each forming the reflector and summing its columns' products
+// one after the other), a strip 9 to 25 -> 10 us.
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(NT) void k_house_qr_fast(const double* __restrict__ A, int lda, int n,
-                                                      double* __restrict__ Q, int ldq, double* __restrict__ R,
-                                                      int ldr, double* __restrict__ work) {
+// d[v] summed over the 64 lanes, in the lanes l with l % 4 = v % 4 of set[v / 4]
+template <int CNT>
+PC_DEV void wave_sums(const double (&d)[CNT], double (&set)[(CNT + 3) / 4]) {
   using namespace dense;
-  __shared__ double Pn[PW * PLD];  // panel columns (column c at Pn[c * PLD], rows relative to the panel start)
-  __shared__ double Xs[PW * PLD];  // X = V^T A_t (row i at Xs[i * PLD]); also V^T V
-  __shared__ double Ts[PW * (PW + 1)];
-  __shared__ double tau_s[PW], sc_s[PW], beta_s[PW];
-  constexpr int NW = NT / 64;
-  const int tid = threadIdx.x, w = tid >> 6, l = tid & 63, lr = l & 15, lk = l >> 4;
-  double* Wm = work;
-  double* tau = work + int64_t(n) * n;
-  double* Tg = tau + n;
-  for (int i = w; i < n; i += NW)
-    for (int j = l; j < n; j += 64) Wm[int64_t(i) * n + j] = A[int64_t(i) * lda + j];
-  __syncthreads();
-  const int npan = (n + PW - 1) / PW;
-  // V element (row i of the panel, column c), unit diagonal, zero above
-  auto vget = [&](int i, int c) -> double { return i < c ? 0.0 : (i == c ? 1.0 : Pn[c * PLD + i]); };
-  // X = V^T B for a K = mr tall B (row k, column col at B[k * ldb]), two
-  // tile rows of 16 x ntl tiles, KD k-steps of loads ahead of the products
-  constexpr int KD = 4;
-  auto vt_times = [&](const double* B, int64_t ldb, int mr, int bs, int ncols, int ntl) {
-    for (int t = w; t < 2 * ntl; t += NW) {
-      const int I = t / ntl, J = t % ntl, col = 16 * J + lr, ca = 16 * I + lr;
-      d4s acc = {0.0, 0.0, 0.0, 0.0};
-      const double* Bc = B + col;
-      for (int k0 = 0; k0 < mr; k0 += 4 * KD) {
-        double bv[KD];
+  const bool b0 = threadIdx.x & 1, b1 = threadIdx.x & 2;
+  constexpr int HALF = (CNT + 1) / 2;
+  double h[HALF];
 #pragma unroll
-        for (int u = 0; u < KD; u++) {
-          const int k = k0 + 4 * u + lk;
-          bv[u] = (k < mr && col < ncols) ? Bc[int64_t(k) * ldb] : 0.0;
-        }
-#pragma unroll
-        for (int u = 0; u < KD; u++) {
-          const int k = k0 + 4 * u + lk;
-          acc = mfma64s((k < mr && ca < bs) ? vget(k, ca) : 0.0, bv[u], acc);
-        }
-      }
-#pragma unroll
-      for (int r = 0; r < 4; r++) Xs[(16 * I + 4 * r + lk) * PLD + col] = acc[r];
-    }
-  };
-  // X <- T^T X (trans) or T X, on MFMA; every wave holds its (at most two)
-  // result tiles in registers until all have read X
-  auto t_times = [&](bool trans, int ntl) {
-    d4s y[2];
-#pragma unroll
-    for (int u = 0; u < 2; u++) {
-      const int t = w + u * NW;
-      y[u] = d4s{0.0, 0.0, 0.0, 0.0};
-      if (t < 2 * ntl) {
-        const int I = t / ntl, J = t % ntl, col = 16 * J + lr, i = 16 * I + lr;
-#pragma unroll
-        for (int k0 = 0; k0 < PW; k0 += 4) {
-          const int k = k0 + lk;
-          const double tv = trans ? Ts[k * (PW + 1) + i] : Ts[i * (PW + 1) + k];
-          y[u] = mfma64s(tv, Xs[k * PLD + col], y[u]);
-        }
-      }
-    }
-    __syncthreads();
-#pragma unroll
-    for (int u = 0; u < 2; u++) {
-      const int t = w + u * NW;
-      if (t < 2 * ntl) {
-        const int I = t / ntl, J = t % ntl, col = 16 * J + lr;
-#pragma unroll
-        for (int r = 0; r < 4; r++) Xs[(16 * I + 4 * r + lk) * PLD + col] = y[u][r];
-      }
-    }
-    __syncthreads();
-  };
-  // C -= V X for an mr x ncols block C (row-major, ldc), two tiles per wave
-  // at a time: both tiles' loads go out before their products
-  auto minus_vx = [&](double* C, int64_t ldc, int mr, int bs, int ncols, int nml, int ntl) {
-    const int ntiles = nml * ntl;
-    for (int t = w; t < ntiles; t += 2 * NW) {
-      d4s acc[2];
-#pragma unroll
-      for (int u = 0; u < 2; u++) {
-        const int tt = t + u * NW, I = tt / ntl, J = tt % ntl, col = 16 * J + lr;
-#pragma unroll
-        for (int r = 0; r < 4; r++) {
-          const int row = 16 * I + 4 * r + lk;
-          acc[u][r] = (tt < ntiles && row < mr && col < ncols) ? -C[int64_t(row) * ldc + col] : 0.0;
-        }
-      }
-#pragma unroll
-      for (int u = 0; u < 2; u++) {
-        const int tt = t + u * NW, I = tt / ntl, J = tt % ntl, col = 16 * J + lr, arow = 16 * I + lr;
-        if (tt < ntiles) {
-#pragma unroll
-          for (int k0 = 0; k0 < PW; k0 += 4) {
-            const int kc = k0 + lk;
-            const double av = (arow < mr && kc < bs) ? vget(arow, kc) : 0.0;
-            acc[u] = mfma64s(av, Xs[kc * PLD + col], acc[u]);
-          }
-        }
-      }
-#pragma unroll
-      for (int u = 0; u < 2; u++) {
-        const int tt = t + u * NW, I = tt / ntl, J = tt % ntl, col = 16 * J + lr;
-        if (tt < ntiles) {
-#pragma unroll
-          for (int r = 0; r < 4; r++) {
-            const int row = 16 * I + 4 * r + lk;
-            if (row < mr && col < ncols) C[int64_t(row) * ldc + col] = -acc[u][r];
-          }
-        }
-      }
-    }
-  };
-  for (int pp = 0; pp < npan; pp++) {
-    const int c0 = pp * PW, bs = min(PW, n - c0), mr = n - c0;
-    for (int c = w; c < PW; c += NW)
-      for (int i = l; i < PLD; i += 64) Pn[c * PLD + i] = (c < bs && i < mr) ? Wm[int64_t(c0 + i) * n + c0 + c] : 0.0;
-    __syncthreads();
-    for (int j = 0; j < bs; j++) {
-      // every wave forms the reflector of column j itself (same arithmetic, same result)
-      double s = 0.0;
-      for (int i = j + 1 + l; i < mr; i += 64) s += Pn[j * PLD + i] * Pn[j * PLD + i];
-      s = wave_sum_dpp(s);
-      const double al = Pn[j * PLD + j];
-      double tj, sc, beta;
-      if (s == 0.0) {
-        tj = 0.0; sc = 0.0; beta = al;
-      } else {
-        double anorm = sqrt(al * al + s);
-        beta = al >= 0 ? -anorm : anorm;
-        tj = (beta - al) / beta;
-        sc = 1.0 / (al - beta);
-      }
-      if (tid == 0) { tau_s[j] = tj; sc_s[j] = sc; beta_s[j] = beta; }
-      // apply H_j to the panel columns c > j (column j itself is read, not written)
-      for (int c = j + 1 + w; c < bs; c += NW) {
-        double d = 0.0;
-        for (int i = j + l; i < mr; i += 64) {
-          double v = i == j ? 1.0 : Pn[j * PLD + i] * sc;
-          d += v * Pn[c * PLD + i];
-        }
-        d = wave_sum_dpp(d);
-        double f = tj * d;
-        for (int i = j + l; i < mr; i += 64) {
-          double v = i == j ? 1.0 : Pn[j * PLD + i] * sc;
-          Pn[c * PLD + i] -= v * f;
-        }
-      }
-      __syncthreads();
-    }
-    // the panel's reflectors in place: v below the diagonal, beta on it
-    for (int c = w; c < bs; c += NW) {
-      const double sc = sc_s[c];
-      for (int i = c + 1 + l; i < mr; i += 64) Pn[c * PLD + i] *= sc;
-      if (l == 0) Pn[c * PLD + c] = beta_s[c];
-    }
-    __syncthreads();
-    // V^T V (bs x bs) into Xs: four 16 x 16 tiles, one wave each, two
-    // accumulators over alternating k-steps
-    if (w < 4) {
-      const int I = w >> 1, J = w & 1, ca = 16 * I + lr, cb = 16 * J + lr;
-      d4s a0 = {0.0, 0.0, 0.0, 0.0}, a1 = {0.0, 0.0, 0.0, 0.0};
-      for (int k0 = 0; k0 < mr; k0 += 8) {
-        const int k = k0 + lk, k2 = k0 + 4 + lk;
-        const double x0 = (k < mr && ca < bs) ? vget(k, ca) : 0.0;
-        const double y0 = (k < mr && cb < bs) ? vget(k, cb) : 0.0;
-        const double x1 = (k2 < mr && ca < bs) ? vget(k2, ca) : 0.0;
-        const double y1 = (k2 < mr && cb < bs) ? vget(k2, cb) : 0.0;
-        a0 = mfma64s(x0, y0, a0);
-        a1 = mfma64s(x1, y1, a1);
-      }
-#pragma unroll
-      for (int r = 0; r < 4; r++) Xs[(16 * I + 4 * r + lk) * PLD + cb] = a0[r] + a1[r];
-    }
-    __syncthreads();
-    // T of the compact WY form.  T^-1 = diag(1 / tau) + strictly upper
-    // (V^T V) (Puglisi 1992), so in 16 x 16 blocks T11 and T22 come from back
-    // substitution, one lane per column in registers: T_jj = tau_j,
-    // T_ij = -tau_i sum_{k = i+1..j} (V^T V)_ik T_kj; multiplying by tau_i
-    // (not dividing by 1 / tau_i) keeps a trivial reflector (tau_i = 0) exact,
-    // its row and column of T zero.  Then T12 = -T11 (V^T V)_12 T22 on MFMA.
-    if (w == 0) {
-      auto wave_sync = [] {
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-      };
-      {
-        // lane jl of half-wave `base / 16` owns column jl of block (base, base);
-        // its column lives in Ts (row stride PW + 1), rows from the bottom up
-        const int base = 16 * ((l >> 4) & 1), jl = l & 15;
-        double* tc = Ts + base * (PW + 1) + base + jl;
-#pragma unroll 1
-        for (int i = 15; i >= 0; i--) {
-          double acc = 0.0;
-#pragma unroll
-          for (int k = 0; k < 16; k++)
-            if (k > i && k <= jl) acc += Xs[(base + i) * PLD + base + k] * tc[k * (PW + 1)];
-          const double ti = base + i < bs ? tau_s[base + i] : 0.0;
-          const double v = i == jl ? ti : (i < jl ? -ti * acc : 0.0);
-          if (l < 32) tc[i * (PW + 1)] = v;
-        }
-        if (l < 16)
-          for (int i = 0; i < 16; i++) Ts[(16 + i) * (PW + 1) + jl] = 0.0;
-      }
-      wave_sync();
-      // W = (V^T V)_12 T22 into the lower-left block of Xs (not read again)
-      d4s acc = {0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-      for (int k0 = 0; k0 < 16; k0 += 4)
-        acc = mfma64s(Xs[lr * PLD + 16 + k0 + lk], Ts[(16 + k0 + lk) * (PW + 1) + 16 + lr], acc);
-#pragma unroll
-      for (int r = 0; r < 4; r++) Xs[(16 + 4 * r + lk) * PLD + lr] = acc[r];
-      wave_sync();
-      acc = d4s{0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-      for (int k0 = 0; k0 < 16; k0 += 4)
-        acc = mfma64s(Ts[lr * (PW + 1) + k0 + lk], Xs[(16 + k0 + lk) * PLD + lr], acc);
-#pragma unroll
-      for (int r = 0; r < 4; r++) Ts[(4 * r + lk) * (PW + 1) + 16 + lr] = -acc[r];
-    }
-    __syncthreads();
-    // store the panel (R part and V) and T
-    for (int c = w; c < bs; c += NW)
-      for (int i = l; i < mr; i += 64) Wm[int64_t(c0 + i) * n + c0 + c] = Pn[c * PLD + i];
-    for (int idx = tid; idx < PW * PW; idx += NT) Tg[int64_t(pp) * PW * PW + idx] = Ts[(idx >> 5) * (PW + 1) + (idx & 31)];
-    if (tid < bs) tau[c0 + tid] = tau_s[tid];
-    // trailing update of columns c1.. (rows c0..)
-    const int c1 = c0 + bs, nt = n - c1;
-    if (nt > 0) {
-      const int ntl = (nt + 15) >> 4, nml = (mr + 15) >> 4;
-      vt_times(Wm + int64_t(c0) * n + c1, n, mr, PW, nt, ntl);
-      __syncthreads();
-      t_times(true, ntl);
-      minus_vx(Wm + int64_t(c0) * n + c1, n, mr, PW, nt, nml, ntl);
-    }
-    __syncthreads();
+  for (int k = 0; k < HALF; k++) {
+    const double x = d[2 * k], y = 2 * k + 1 < CNT ? d[2 * k + 1] : d[2 * k];
+    h[k] = (b0 ? y : x) + dpp_f64<0xB1, 0xF>(b0 ? x : y, 0.0);  // lane l ^ 1
   }
-  // R
-  for (int i = w; i < n; i += NW)
-    for (int j = l; j < n; j += 64) R[int64_t(i) * ldr + j] = i <= j ? Wm[int64_t(i) * n + j] : 0.0;
-  // Q = H_0 ... H_{n-1} I, accumulated backwards over the panels
-  for (int i = w; i < n; i += NW)
-    for (int j = l; j < n; j += 64) Q[int64_t(i) * ldq + j] = i == j ? 1.0 : 0.0;
-  __syncthreads();
-  for (int pp = npan - 1; pp >= 0; pp--) {
-    const int c0 = pp * PW, bs = min(PW, n - c0), mr = n - c0, nq = n - c0;
-    for (int c = w; c < PW; c += NW)
-      for (int i = l; i < PLD; i += 64)
-        Pn[c * PLD + i] = (c < bs && i < mr && i > c) ? Wm[int64_t(c0 + i) * n + c0 + c] : 0.0;
-    for (int idx = tid; idx < PW * PW; idx += NT) Ts[(idx >> 5) * (PW + 1) + (idx & 31)] = Tg[int64_t(pp) * PW * PW + idx];
-    __syncthreads();
-    const int ntl = (nq + 15) >> 4, nml = (mr + 15) >> 4;
-    double* Qs = Q + int64_t(c0) * ldq + c0;
-    vt_times(Qs, ldq, mr, bs, nq, ntl);
-    __syncthreads();
-    t_times(false, ntl);
-    minus_vx(Qs, ldq, mr, bs, nq, nml, ntl);
-    __syncthreads();
+#pragma unroll
+  for (int k = 0; k < (CNT + 3) / 4; k++) {
+    const double x = h[2 * k], y = 2 * k + 1 < HALF ? h[2 * k + 1] : h[2 * k];
+    double v = (b1 ? y : x) + dpp_f64<0x4E, 0xF>(b1 ? x : y, 0.0);  // lane l ^ 2
+    v += dpp_f64<0x124, 0xF>(v, 0.0);                               // row_ror:4
+    v += dpp_f64<0x128, 0xF>(v, 0.0);                               // row_ror:8
+    // rows 0 and 1, 2 and 3, then the halves: the swaps leave both terms in every lane
+    auto both = [](double u, auto swap) {
+      const long long bits = __builtin_bit_cast(long long, u);
+      const auto lo = swap(unsigned(bits)), hi = swap(unsigned(bits >> 32));
+      return __builtin_bit_cast(double, (long long)lo[0] | ((long long)hi[0] << 32)) +
+             __builtin_bit_cast(double, (long long)lo[1] | ((long long)hi[1] << 32));
+    };
+    v = both(v, [](unsigned x) { return __builtin_amdgcn_permlane16_swap(x, x, false, false); });
+    v = both(v, [](unsigned x) { return __builtin_amdgcn_permlane32_swap(x, x, false, false); });
+    set[k] = v;
   }
 }
 
-// ---------------------------------------------------------------------------
-// Householder QR of a real n x n matrix (n <= 256), A = Q R, Q explicit.
-// LAPACK conventions (beta = -sign(alpha) ||x||, tau = (beta - alpha) / beta).
-// Panels of 32 columns are factored in LDS; the block reflector
-// I - V T V^T (compact WY, T upper) updates the trailing columns with MFMA
-// (X = V^T A_t, X <- T^T X, A_t -= V X); Q is accumulated backwards the
-// same way.  Latency is what costs in the panel (one workgroup): wave sums
-// use DPP, a column of the panel costs one barrier (its scaling waits for
-// the panel's end), V^T V and T's off-diagonal block run on MFMA.
-// The factorisation runs in launches that spread its FP64 MFMA work: the
-// panels are factored on one workgroup (k_hqr_panel: the column loop, V^T V,
-// T), while the block-reflector updates, of the trailing columns after each
-// panel and of Q (accumulated backwards) afterwards, run one workgroup per
-// 32-column strip (k_hqr_strip, the strip of B staged in LDS).  A panel's
-// update is ~3,800 FP64 MFMAs at 64 cycles each per SIMD, about 25 us on one
-// CU.  The strips form the same tiles with the same MFMA sequence as one
-// workgroup doing the whole update would, so Q and R do not depend on the
-// split.  work: n*n (the factored matrix) + n (tau) + 32*32*ceil(n/32) (T).
-// ---------------------------------------------------------------------------
-__global__ __launch_bounds__(NT) void k_hqr_panel(const double* __restrict__ A, int lda, int n, int pp,
-                                                  double* __restrict__ work) {
+constexpr int kHqrThreads = 256;
+template <int RW>
+__global__ __launch_bounds__(kHqrThreads) void k_hqr_panel(const double* __restrict__ A, int lda, int n, int pp,
+                                                           double* __restrict__ work) {
   using namespace dense;
-  __shared__ double Pn[PW * PLD];  // panel columns (column c at Pn[c * PLD], rows relative to the panel start)
-  __shared__ double Xs[PW * PLD];  // V^T V
+  constexpr int NW = kHqrThreads / 64, K = PW / NW, LD = 64 * RW + 1;
+  __shared__ double Pn[PW * LD];  // panel columns (column c at Pn[c * LD], rows relative to the panel start)
+  __shared__ double Xs[PW * (PW + 1)];  // V^T V
   __shared__ double Ts[PW * (PW + 1)];
-  __shared__ double tau_s[PW], sc_s[PW], beta_s[PW];
-  constexpr int NW = NT / 64;
-  const int tid = threadIdx.x, w = tid >> 6, l = tid & 63, lr = l & 15, lk = l >> 4;
+  __shared__ double vb[2][64 * RW], tau_s[PW];
+  const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), l = tid & 63, lr = l & 15, lk = l >> 4;
   double* Wm = work;
   double* tau = work + int64_t(n) * n;
   double* Tg = tau + n;
-  if (pp == 0) {
-    for (int i = w; i < n; i += NW)
-      for (int j = l; j < n; j += 64) Wm[int64_t(i) * n + j] = A[int64_t(i) * lda + j];
-    __syncthreads();
-  }
-  auto vget = [&](int i, int c) -> double { return i < c ? 0.0 : (i == c ? 1.0 : Pn[c * PLD + i]); };
-  {
-    const int c0 = pp * PW, bs = min(PW, n - c0), mr = n - c0;
-    for (int c = w; c < PW; c += NW)
-      for (int i = l; i < PLD; i += 64) Pn[c * PLD + i] = (c < bs && i < mr) ? Wm[int64_t(c0 + i) * n + c0 + c] : 0.0;
-    __syncthreads();
-    for (int j = 0; j < bs; j++) {
-      // every wave forms the reflector of column j itself (same arithmetic, same result)
-      double s = 0.0;
-#pragma unroll
-      for (int q = 0; q < NMAX / 64; q++) {  // rows j + 1 + l + 64 q < mr: the reads go out together
-        const int i = j + 1 + l + 64 * q;
-        if (i < mr) s += Pn[j * PLD + i] * Pn[j * PLD + i];
-      }
-      s = wave_sum_dpp(s);
-      const double al = Pn[j * PLD + j];
-      double tj, sc, beta;
-      if (s == 0.0) {
-        tj = 0.0; sc = 0.0; beta = al;
-      } else {
-        double anorm = sqrt(al * al + s);
-        beta = al >= 0 ? -anorm : anorm;
-        tj = (beta - al) / beta;
-        sc = 1.0 / (al - beta);
-      }
-      if (tid == 0) { tau_s[j] = tj; sc_s[j] = sc; beta_s[j] = beta; }
-      // apply H_j to the panel columns c > j (column j itself is read, not written)
-      for (int c = j + 1 + w; c < bs; c += NW) {
-        double d = 0.0;
-#pragma unroll
-        for (int q = 0; q < NMAX / 64; q++) {
-          const int i = j + l + 64 * q;
-          if (i < mr) {
-            double v = i == j ? 1.0 : Pn[j * PLD + i] * sc;
-            d += v * Pn[c * PLD + i];
-          }
-        }
-        d = wave_sum_dpp(d);
-        double f = tj * d;
-#pragma unroll
-        for (int q = 0; q < NMAX / 64; q++) {
-          const int i = j + l + 64 * q;
-          if (i < mr) {
-            double v = i == j ? 1.0 : Pn[j * PLD + i] * sc;
-            Pn[c * PLD + i] -= v * f;
-          }
-        }
-      }
-      __syncthreads();
-    }
-    // the panel's reflectors in place: v below the diagonal, beta on it
-    for (int c = w; c < bs; c += NW) {
-      const double sc = sc_s[c];
-      for (int i = c + 1 + l; i < mr; i += 64) Pn[c * PLD + i] *= sc;
-      if (l == 0) Pn[c * PLD + c] = beta_s[c];
-    }
-    __syncthreads();
-    // V^T V (bs x bs) into Xs: four 16 x 16 tiles, one wave each, two
-    // accumulators over alternating k-steps
-    if (w < 4) {
-      const int I = w >> 1, J = w & 1, ca = 16 * I + lr, cb = 16 * J + lr;
-      d4s a0 = {0.0, 0.0, 0.0, 0.0}, a1 = {0.0, 0.0, 0.0, 0.0};
-      for (int k0 = 0; k0 < mr; k0 += 8) {
-        const int k = k0 + lk, k2 = k0 + 4 + lk;
-        const double x0 = (k < mr && ca < bs) ? vget(k, ca) : 0.0;
-        const double y0 = (k < mr && cb < bs) ? vget(k, cb) : 0.0;
-        const double x1 = (k2 < mr && ca < bs) ? vget(k2, ca) : 0.0;
-        const double y1 = (k2 < mr && cb < bs) ? vget(k2, cb) : 0.0;
-        a0 = mfma64s(x0, y0, a0);
-        a1 = mfma64s(x1, y1, a1);
-      }
-  #pragma unroll
-      for (int r = 0; r < 4; r++) Xs[(16 * I + 4 * r + lk) * PLD + cb] = a0[r] + a1[r];
-    }
-    __syncthreads();
-    // T of the compact WY form.  T^-1 = diag(1 / tau) + strictly upper
-    // (V^T V) (Puglisi 1992), so in 16 x 16 blocks T11 and T22 come from back
-    // substitution, one lane per column in registers: T_jj = tau_j,
-    // T_ij = -tau_i sum_{k = i+1..j} (V^T V)_ik T_kj; multiplying by tau_i
-    // (not dividing by 1 / tau_i) keeps a trivial reflector (tau_i = 0) exact,
-    // its row and column of T zero.  Then T12 = -T11 (V^T V)_12 T22 on MFMA.
-    if (w == 0) {
-      auto wave_sync = [] {
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-      };
-      {
-        // lane jl of half-wave `base / 16` owns column jl of block (base, base);
-        // its column lives in Ts (row stride PW + 1), rows from the bottom up
-        const int base = 16 * ((l >> 4) & 1), jl = l & 15;
-        double* tc = Ts + base * (PW + 1) + base + jl;
-  #pragma unroll 1
-        for (int i = 15; i >= 0; i--) {
-          double acc = 0.0;
-  #pragma unroll
-          for (int k = 0; k < 16; k++)
-            if (k > i && k <= jl) acc += Xs[(base + i) * PLD + base + k] * tc[k * (PW + 1)];
-          const double ti = base + i < bs ? tau_s[base + i] : 0.0;
-          const double v = i == jl ? ti : (i < jl ? -ti * acc : 0.0);
-          if (l < 32) tc[i * (PW + 1)] = v;
-        }
-        if (l < 16)
-          for (int i = 0; i < 16; i++) Ts[(16 + i) * (PW + 1) + jl] = 0.0;
-      }
-      wave_sync();
-      // W = (V^T V)_12 T22 into the lower-left block of Xs (not read again)
-      d4s acc = {0.0, 0.0, 0.0, 0.0};
-  #pragma unroll
-      for (int k0 = 0; k0 < 16; k0 += 4)
-        acc = mfma64s(Xs[lr * PLD + 16 + k0 + lk], Ts[(16 + k0 + lk) * (PW + 1) + 16 + lr], acc);
-  #pragma unroll
-      for (int r = 0; r < 4; r++) Xs[(16 + 4 * r + lk) * PLD + lr] = acc[r];
-      wave_sync();
-      acc = d4s{0.0, 0.0, 0.0, 0.0};
-  #pragma unroll
-      for (int k0 = 0; k0 < 16; k0 += 4)
-        acc = mfma64s(Ts[lr * (PW + 1) + k0 + lk], Xs[(16 + k0 + lk) * PLD + lr], acc);
-  #pragma unroll
-      for (int r = 0; r < 4; r++) Ts[(4 * r + lk) * (PW + 1) + 16 + lr] = -acc[r];
-    }
-    __syncthreads();
-    // store the panel (R part and V) and T
-    for (int c = w; c < bs; c += NW)
-      for (int i = l; i < mr; i += 64) Wm[int64_t(c0 + i) * n + c0 + c] = Pn[c * PLD + i];
-    for (int idx = tid; idx < PW * PW; idx += NT) Tg[int64_t(pp) * PW * PW + idx] = Ts[(idx >> 5) * (PW + 1) + (idx & 31)];
-    if (tid < bs) tau[c0 + tid] = tau_s[tid];
-  }
-}
-
-// one workgroup per 32-column strip: qmode 0 updates the trailing columns of
-// Wm after panel pp, qmode 1 applies panel pp's block reflector to Q
-__global__ __launch_bounds__(256) void k_hqr_strip(int n, int pp, int qmode, double* __restrict__ work,
-                                                   double* __restrict__ Q, int ldq) {
-  using namespace dense;
-  constexpr int NWS = 4, XLD = PW + 1, BLD = PW + 1;
-  __shared__ double Pn[PW * PLD];
-  __shared__ double Bs[NMAX * BLD];  // the strip of B (rows relative to the panel start)
-  __shared__ double Xs[PW * XLD];
-  __shared__ double Ts[PW * (PW + 1)];
-  const int tid = threadIdx.x, w = tid >> 6, l = tid & 63, lr = l & 15, lk = l >> 4;
-  double* Wm = work;
-  const double* Tg = work + int64_t(n) * n + n;
   const int c0 = pp * PW, bs = min(PW, n - c0), mr = n - c0;
-  const int cst = qmode ? c0 : c0 + bs;        // first column of the updated block
+  {
+    const double* src = pp ? Wm + int64_t(c0) * n + c0 : A;  // the first panel comes from A
+    const int lds = pp ? n : lda, c = tid & 31, i0 = tid >> 5;
+    constexpr int PER = 64 * RW / (kHqrThreads / 32);
+    double v[PER];
+#pragma unroll
+    for (int u = 0; u < PER; u++) v[u] = src[min(i0 + 8 * u, mr - 1) * lds + min(c, bs - 1)];
+#pragma unroll
+    for (int u = 0; u < PER; u++) Pn[c * LD + i0 + 8 * u] = c < bs && i0 + 8 * u < mr ? v[u] : 0.0;
+  }
+  if (tid < PW) tau_s[tid] = 0.0;
+  __syncthreads();
+  double a[K][RW];  // column w + NW k, row l + 64 q
+#pragma unroll
+  for (int k = 0; k < K; k++)
+#pragma unroll
+    for (int q = 0; q < RW; q++) a[k][q] = Pn[(w + NW * k) * LD + l + 64 * q];
+  static_for<0, K>([&](auto kc) {
+    constexpr int k = decltype(kc)::value;
+#pragma unroll 1
+    for (int o = 0; o < NW; o++) {
+      const int j = NW * k + o;
+      if (j >= bs) break;
+      double* v_s = vb[o & 1];
+      if (w == o) {
+        // rows above j are R's; s: the squares below
+        double s = l > j ? a[k][0] * a[k][0] : 0.0;
+#pragma unroll
+        for (int q = 1; q < RW; q++) s = fma(a[k][q], a[k][q], s);
+        s = wave_sum_dpp(s);
+        const double al = lane_read_f64(a[k][0], j);
+        double tj = 0.0, sc = 0.0, beta = al;
+        if (s != 0.0) {
+          const double anorm = sqrt(al * al + s);
+          beta = al >= 0 ? -anorm : anorm;
+          tj = (beta - al) / beta;
+          sc = 1.0 / (al - beta);
+        }
+#pragma unroll
+        for (int q = 0; q < RW; q++) {
+          const bool below = q > 0 || l > j;
+          const double v = a[k][q] * sc;
+          a[k][q] = below ? v : l == j ? beta : a[k][q];
+          v_s[l + 64 * q] = below ? v : l == j ? 1.0 : 0.0;
+        }
+        if (l == 0) tau_s[j] = tj;
+      }
+      __syncthreads();
+      double v[RW], d[K - k], set[(K - k + 3) / 4];
+#pragma unroll
+      for (int q = 0; q < RW; q++) v[q] = v_s[l + 64 * q];
+      const double tj = tau_s[j];
+#pragma unroll
+      for (int x = k; x < K; x++) {
+        d[x - k] = v[0] * a[x][0];
+#pragma unroll
+        for (int q = 1; q < RW; q++) d[x - k] = fma(v[q], a[x][q], d[x - k]);
+      }
+      wave_sums<K - k>(d, set);
+#pragma unroll
+      for (int x = k; x < K; x++) {
+        double f = tj * lane_read_f64(set[(x - k) / 4], (x - k) % 4);
+        if (x == k && w <= o) f = 0.0;  // columns up to j are done
+#pragma unroll
+        for (int q = 0; q < RW; q++) a[x][q] = fma(-v[q], f, a[x][q]);
+      }
+    }
+  });
+#pragma unroll
+  for (int k = 0; k < K; k++)
+#pragma unroll
+    for (int q = 0; q < RW; q++) Pn[(w + NW * k) * LD + l + 64 * q] = a[k][q];
+  __syncthreads();
+  // V: unit diagonal, zero above
+  auto vget = [&](int i, int c) -> double {
+    const double v = Pn[c * LD + i];
+    return i < c ? 0.0 : (i == c ? 1.0 : v);
+  };
+  // V^T V into Xs: four 16 x 16 tiles, one wave each, two accumulators over alternating
+  // k-steps (rows beyond mr are zero, and so are columns beyond bs below the diagonal)
+  {
+    const int I = w >> 1, J = w & 1, ca = 16 * I + lr, cb = 16 * J + lr;
+    d4s a0 = {0.0, 0.0, 0.0, 0.0}, a1 = {0.0, 0.0, 0.0, 0.0};
+    const int kend = min(64 * RW, (mr + 7) & ~7);
+#pragma unroll 4
+    for (int k0 = 0; k0 < kend; k0 += 8) {
+      a0 = mfma64s(vget(k0 + lk, ca), vget(k0 + lk, cb), a0);
+      a1 = mfma64s(vget(k0 + 4 + lk, ca), vget(k0 + 4 + lk, cb), a1);
+    }
+#pragma unroll
+    for (int r = 0; r < 4; r++) Xs[(16 * I + 4 * r + lk) * (PW + 1) + cb] = a0[r] + a1[r];
+  }
+  __syncthreads();
+  // T of the compact WY form.  T^-1 = diag(1 / tau) + strictly upper
+  // (V^T V) (Puglisi 1992), so in 16 x 16 blocks T11 and T22 come from back
+  // substitution, one lane per column in registers: T_jj = tau_j,
+  // T_ij = -tau_i sum_{k = i+1..j} (V^T V)_ik T_kj; multiplying by tau_i
+  // (not dividing by 1 / tau_i) keeps a trivial reflector (tau_i = 0) exact,
+  // its row and column of T zero.  Then T12 = -T11 (V^T V)_12 T22 on MFMA.
+  // The other waves store the panel meanwhile.
+  if (w == 0) {
+    {
+      // lane jl of half-wave `base / 16` owns column jl of block (base, base)
+      const int base = 16 * ((l >> 4) & 1), jl = l & 15;
+      double tc[16];
+#pragma unroll
+      for (int i = 15; i >= 0; i--) {
+        double acc = 0.0;
+#pragma unroll
+        for (int k = i + 1; k < 16; k++) acc += Xs[(base + i) * (PW + 1) + base + k] * tc[k];
+        const double ti = tau_s[base + i];
+        tc[i] = i == jl ? ti : (i < jl ? -ti * acc : 0.0);
+      }
+      if (l < 32) {
+#pragma unroll
+        for (int i = 0; i < 16; i++) Ts[(base + i) * (PW + 1) + base + jl] = tc[i];
+      }
+      if (l < 16)
+        for (int i = 0; i < 16; i++) Ts[(16 + i) * (PW + 1) + jl] = 0.0;
+    }
+    wave_fence();
+    // W = (V^T V)_12 T22 into the lower-left block of Xs (not read again)
+    d4s acc = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int k0 = 0; k0 < 16; k0 += 4)
+      acc = mfma64s(Xs[lr * (PW + 1) + 16 + k0 + lk], Ts[(16 + k0 + lk) * (PW + 1) + 16 + lr], acc);
+#pragma unroll
+    for (int r = 0; r < 4; r++) Xs[(16 + 4 * r + lk) * (PW + 1) + lr] = acc[r];
+    wave_fence();
+    acc = d4s{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int k0 = 0; k0 < 16; k0 += 4)
+      acc = mfma64s(Ts[lr * (PW + 1) + k0 + lk], Xs[(16 + k0 + lk) * (PW + 1) + lr], acc);
+#pragma unroll
+    for (int r = 0; r < 4; r++) Ts[(4 * r + lk) * (PW + 1) + 16 + lr] = -acc[r];
+    wave_fence();
+    for (int e = l; e < PW * PW; e += 64) Tg[int64_t(pp) * PW * PW + e] = Ts[(e >> 5) * (PW + 1) + (e & 31)];
+    if (l < bs) tau[c0 + l] = tau_s[l];
+  } else {
+    const int c = tid & 31;
+    if (c < bs)
+      for (int i = (tid - 64) >> 5; i < mr; i += 6) Wm[int64_t(c0 + i) * n + c0 + c] = Pn[c * LD + i];
+  }
+}
+
+// One workgroup per 32-column strip: qmode 0 updates the trailing columns of Wm after
+// panel pp (those of the first panel come from A), qmode 1 applies panel pp's block
+// reflector to Q.  A wave holds the strip's rows 16 (w + 4 u) .. + 15 in registers in the
+// products' accumulator layout, which is the right operand's of X = V^T B: entry r of
+// tile u is row 4 r + lk of the tile, the four rows of one k-step.  X is the sum of the
+// waves' parts, Y = T^T X or T X, and the same registers are the accumulators of
+// B - V Y, so B is read and written once and never staged.
+template <int RW>
+__global__ __launch_bounds__(kHqrThreads) void k_hqr_strip(const double* A, int lda, int n, int pp, int qmode,
+                                                           double* work, double* Q, int ldq) {
+  using namespace dense;
+  constexpr int NW = kHqrThreads / 64, LD = 64 * RW + 1, XLD = PW + 1;
+  __shared__ double Pn[PW * LD];
+  __shared__ double Xs[NW - 1][PW * XLD];
+  const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), l = tid & 63, lr = l & 15, lk = l >> 4;
+  double* Wm = work;
+  const double* T = work + int64_t(n) * n + n + int64_t(pp) * PW * PW;
+  const int c0 = pp * PW, bs = min(PW, n - c0), mr = n - c0;
+  const int cst = qmode ? c0 : c0 + bs;  // first column of the updated block
   const int ncols = n - cst, s0 = 32 * blockIdx.x;
   if (s0 >= ncols) return;
   double* B = qmode ? Q + int64_t(c0) * ldq + cst : Wm + int64_t(c0) * n + cst;
-  const int64_t ldb = qmode ? ldq : n;
-  const int bsv = qmode ? bs : PW;             // reflector columns the products read
-  // stage V (below the diagonal), T and the strip of B: every load of a
-  // thread is issued before its first LDS store
+  const int ldb = qmode ? ldq : n;
+  const double* Bin = !qmode && pp == 0 ? A + cst : B;
+  const int ldi = !qmode && pp == 0 ? lda : ldb;
+  // V below the diagonal (its diagonal is 1), the strip and this wave's tile of T: every
+  // load goes out before the first is waited for
+  const int ti = w >> 1, tj = w & 1;  // this wave's tile of Y
+  d4s b[RW][2];
+  double tv[PW / 4];
   {
-    constexpr int PER = PW * NMAX / 256;  // 32 elements of V and of B per thread
-    double vv[PER], bb[PER];
+    const int c = tid & 31, i0 = tid >> 5;
+    constexpr int PER = 64 * RW / (kHqrThreads / 32);
+    double v[PER];
 #pragma unroll
-    for (int q = 0; q < PER; q++) {
-      const int idx = tid + 256 * q, i = idx >> 5, c = idx & 31;  // row i, column c
-      vv[q] = (c < bs && i < mr && i > c) ? Wm[int64_t(c0 + i) * n + c0 + c] : 0.0;
-      bb[q] = (i < mr && s0 + c < ncols) ? B[int64_t(i) * ldb + s0 + c] : 0.0;
-    }
-    for (int idx = tid; idx < PW * PW; idx += 256) Ts[(idx >> 5) * (PW + 1) + (idx & 31)] = Tg[int64_t(pp) * PW * PW + idx];
+    for (int u = 0; u < PER; u++) v[u] = Wm[(c0 + min(i0 + 8 * u, mr - 1)) * n + c0 + min(c, bs - 1)];
 #pragma unroll
-    for (int q = 0; q < PER; q++) {
-      const int idx = tid + 256 * q, i = idx >> 5, c = idx & 31;
-      Pn[c * PLD + i] = vv[q];
-      Bs[i * BLD + c] = bb[q];
+    for (int u = 0; u < RW; u++)
+#pragma unroll
+      for (int h = 0; h < 2; h++)
+#pragma unroll
+        for (int r = 0; r < 4; r++)
+          b[u][h][r] = Bin[min(16 * (w + NW * u) + 4 * r + lk, mr - 1) * ldi + min(s0 + 16 * h + lr, ncols - 1)];
+#pragma unroll
+    for (int k = 0; k < PW / 4; k++) {
+      const int i = 16 * ti + lr, x = 4 * k + lk;
+      tv[k] = qmode ? T[i * PW + x] : T[x * PW + i];
     }
+#pragma unroll
+    for (int u = 0; u < PER; u++) {
+      const int i = i0 + 8 * u;
+      Pn[c * LD + i] = i < mr && c < bs && i >= c ? (i == c ? 1.0 : v[u]) : 0.0;
+    }
+#pragma unroll
+    for (int u = 0; u < RW; u++)
+#pragma unroll
+      for (int h = 0; h < 2; h++)
+#pragma unroll
+        for (int r = 0; r < 4; r++)
+          if (16 * (w + NW * u) + 4 * r + lk >= mr) b[u][h][r] = 0.0;
   }
   __syncthreads();
-  auto vget = [&](int i, int c) -> double { return i < c ? 0.0 : (i == c ? 1.0 : Pn[c * PLD + i]); };
-  // X = V^T B for the strip: wave w forms tile (I, Jl) = (w >> 1, w & 1)
-  {
-    const int I = w >> 1, Jl = w & 1, cl = 16 * Jl + lr, ca = 16 * I + lr;
-    d4s acc = {0.0, 0.0, 0.0, 0.0};
-    for (int k0 = 0; k0 < mr; k0 += 4) {
-      const int k = k0 + lk;
-      acc = mfma64s((k < mr && ca < bsv) ? vget(k, ca) : 0.0, k < mr ? Bs[k * BLD + cl] : 0.0, acc);
-    }
+  d4s x[2][2] = {};
 #pragma unroll
-    for (int r = 0; r < 4; r++) Xs[(16 * I + 4 * r + lk) * XLD + cl] = acc[r];
+  for (int u = 0; u < RW; u++)
+    if (16 * (w + NW * u) < mr) {
+#pragma unroll
+      for (int r = 0; r < 4; r++)
+#pragma unroll
+        for (int I = 0; I < 2; I++) {
+          const double v = Pn[(16 * I + lr) * LD + 16 * (w + NW * u) + 4 * r + lk];
+#pragma unroll
+          for (int h = 0; h < 2; h++) x[I][h] = mfma64s(v, b[u][h][r], x[I][h]);
+        }
+    }
+  if (w > 0) {
+#pragma unroll
+    for (int I = 0; I < 2; I++)
+#pragma unroll
+      for (int h = 0; h < 2; h++)
+#pragma unroll
+        for (int r = 0; r < 4; r++) Xs[w - 1][(16 * I + 4 * r + lk) * XLD + 16 * h + lr] = x[I][h][r];
   }
   __syncthreads();
-  // X <- T^T X (trailing) or T X (Q)
+  if (w == 0) {
+#pragma unroll
+    for (int I = 0; I < 2; I++)
+#pragma unroll
+      for (int h = 0; h < 2; h++)
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+          const int e = (16 * I + 4 * r + lk) * XLD + 16 * h + lr;
+          Xs[0][e] = (x[I][h][r] + Xs[0][e]) + (Xs[1][e] + Xs[2][e]);
+        }
+  }
+  __syncthreads();
   {
-    const int I = w >> 1, Jl = w & 1, i = 16 * I + lr;
     d4s y = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
-    for (int k0 = 0; k0 < PW; k0 += 4) {
-      const int k = k0 + lk;
-      const double tv = qmode ? Ts[i * (PW + 1) + k] : Ts[k * (PW + 1) + i];
-      y = mfma64s(tv, Xs[k * XLD + 16 * Jl + lr], y);
-    }
-    __syncthreads();
+    for (int k = 0; k < PW / 4; k++) y = mfma64s(tv[k], Xs[0][(4 * k + lk) * XLD + 16 * tj + lr], y);
 #pragma unroll
-    for (int r = 0; r < 4; r++) Xs[(16 * I + 4 * r + lk) * XLD + 16 * Jl + lr] = y[r];
+    for (int r = 0; r < 4; r++) Xs[1][(16 * ti + 4 * r + lk) * XLD + 16 * tj + lr] = -y[r];
   }
   __syncthreads();
-  // B -= V X: tiles (row block I, column block Jl) of the strip, B from LDS
-  const int nml = (mr + 15) >> 4, ntiles = nml * 2;
-  for (int t = w; t < ntiles; t += NWS) {
-    const int I = t >> 1, Jl = t & 1, cl = 16 * Jl + lr, col = s0 + cl, arow = 16 * I + lr;
-    d4s acc;
+  double yv[PW / 4][2];
 #pragma unroll
-    for (int r = 0; r < 4; r++) {
-      const int row = 16 * I + 4 * r + lk;
-      acc[r] = row < mr ? -Bs[row * BLD + cl] : 0.0;
-    }
+  for (int k = 0; k < PW / 4; k++)
 #pragma unroll
-    for (int k0 = 0; k0 < PW; k0 += 4) {
-      const int kc = k0 + lk;
-      const double av = (arow < mr && kc < bsv) ? vget(arow, kc) : 0.0;
-      acc = mfma64s(av, Xs[kc * XLD + cl], acc);
-    }
+    for (int h = 0; h < 2; h++) yv[k][h] = Xs[1][(4 * k + lk) * XLD + 16 * h + lr];
 #pragma unroll
-    for (int r = 0; r < 4; r++) {
-      const int row = 16 * I + 4 * r + lk;
-      if (row < mr && col < ncols) B[int64_t(row) * ldb + col] = -acc[r];
+  for (int u = 0; u < RW; u++) {
+    const int i0 = 16 * (w + NW * u);
+    if (i0 < mr) {
+#pragma unroll
+      for (int k = 0; k < PW / 4; k++) {
+        const double v = Pn[(4 * k + lk) * LD + i0 + lr];
+#pragma unroll
+        for (int h = 0; h < 2; h++) b[u][h] = mfma64s(v, yv[k][h], b[u][h]);
+      }
+#pragma unroll
+      for (int h = 0; h < 2; h++)
+#pragma unroll
+        for (int r = 0; r < 4; r++)
+          if (i0 + 4 * r + lk < mr && s0 + 16 * h + lr < ncols)
+            B[int64_t(i0 + 4 * r + lk) * ldb + s0 + 16 * h + lr] = b[u][h][r];
     }
   }
 }

@@ -252,30 +252,26 @@ void run_pchol(hipStream_t st, const T* G, int n, double tol, T* A, T* A2, T* R,
   }
   hipLaunchKernelGGL((k_pchol<T>), dim3(1, 1, nz), dim3(NT), 0, st, G, n, n, tol, A, R, n, perm, rank, status, zb);
 }
-// square Householder QR (n x n), Q and R explicit; work: 2 n^2 + n of T.
-// fused: one launch (k_house_qr_fast) instead of the panel / strip sequence,
-// for contexts that share the GPU with other streams; same Q and R.
+// square Householder QR (n x n), Q and R explicit; work: 2 n^2 + n of T
 template <class T>
-void run_house_qr_sq(hipStream_t st, const T* A, int n, T* Q, T* R, T* work, bool fused = false) {
+void run_house_qr_sq(hipStream_t st, const T* A, int n, T* Q, T* R, T* work) {
   if constexpr (std::is_same<T, double>::value)
-    if (n <= dense::NMAX && fused) {
-      hipLaunchKernelGGL(k_house_qr_fast, dim3(1), dim3(NT), 0, st, A, n, n, Q, n, R, n, work);
-      return;
-    }
-  if constexpr (std::is_same<T, double>::value)
-    if (n <= dense::NMAX) {
+    if (use_fast<T>(n, 1)) {
       // panels on one workgroup, the block-reflector updates on one
       // workgroup per 32-column strip
       const int npan = (n + dense::PW - 1) / dense::PW;
+      const auto panel = n <= 256 ? k_hqr_panel<4> : k_hqr_panel<8>;
+      const auto strip = n <= 256 ? k_hqr_strip<4> : k_hqr_strip<8>;
       for (int pp = 0; pp < npan; pp++) {
-        hipLaunchKernelGGL(k_hqr_panel, dim3(1), dim3(NT), 0, st, A, n, n, pp, work);
+        hipLaunchKernelGGL(panel, dim3(1), dim3(kHqrThreads), 0, st, A, n, n, pp, work);
         const int nt = n - std::min(n, (pp + 1) * dense::PW);
-        if (nt > 0) hipLaunchKernelGGL(k_hqr_strip, dim3((nt + 31) / 32), dim3(256), 0, st, n, pp, 0, work, Q, n);
+        if (nt > 0)
+          hipLaunchKernelGGL(strip, dim3((nt + 31) / 32), dim3(kHqrThreads), 0, st, A, n, n, pp, 0, work, Q, n);
       }
       hipLaunchKernelGGL(k_hqr_rq, dim3(nblk(int64_t(n) * n)), dim3(256), 0, st, n, (const double*)work, R, n, Q, n);
       for (int pp = npan - 1; pp >= 0; pp--)
-        hipLaunchKernelGGL(k_hqr_strip, dim3((n - pp * dense::PW + 31) / 32), dim3(256), 0, st, n, pp, 1, work, Q,
-                           n);
+        hipLaunchKernelGGL(strip, dim3((n - pp * dense::PW + 31) / 32), dim3(kHqrThreads), 0, st, A, n, n, pp, 1, work,
+                           Q, n);
       return;
     }
   if (use_mw(n, 1)) {
@@ -1296,7 +1292,7 @@ static int core_t(pc_ctx* ctx, const Plan& p, const void* A, int64_t lda, int ce
                        b.tmp, n, (const int*)nullptr, T(0.0), b.G1, n, 0);
     run_pchol<T>(st, b.G1, n, 1e-30, b.Awk, b.UM, b.R1, b.perm3, b.rank3, b.status, 1, 0, b.rank3 + 1);
     hipLaunchKernelGGL((k_copy2d<T>), dim3(nblk(nn)), dim3(256), 0, st, b.R1, n, n, n, b.Awk, n, 2);
-    run_house_qr_sq<T>(st, b.Awk, n, b.UM, b.G1, nwork, ctx->concurrent);
+    run_house_qr_sq<T>(st, b.Awk, n, b.UM, b.G1, nwork);
     hipLaunchKernelGGL((k_permute_rows<T>), dim3(nblk(nn)), dim3(256), 0, st, b.UM, n, n, (const int*)b.perm3, b.Awk,
                        n);
     hipLaunchKernelGGL((k_gemm_small<T>), gg, dim3(256), 0, st, 0, 0, n, n, n, T(1.0), b.tmp, n, (const int*)nullptr,
@@ -1316,7 +1312,7 @@ static int core_t(pc_ctx* ctx, const Plan& p, const void* A, int64_t lda, int ce
   } else {
     // QR of M (n x n, rows >= rank zero): M = Q_M R_M;  R output, UM := Q_M
     hipLaunchKernelGGL((k_copy2d<T>), dim3(nblk(nn)), dim3(256), 0, st, b.Hc, n, n, n, b.tmp, n, 1);
-    run_house_qr_sq<T>(st, b.tmp, n, b.UM, b.J, nwork, ctx->concurrent);
+    run_house_qr_sq<T>(st, b.tmp, n, b.UM, b.J, nwork);
     // diag(R) real and non-negative (the phases go to Q_M's columns); tmp is free here
     hipLaunchKernelGGL((k_qr_phase<T>), dim3(nblk(n)), dim3(256), 0, st, b.J, n, n, b.tmp);
     hipLaunchKernelGGL((k_qr_apply_phase<T>), dim3(nblk(nn)), dim3(256), 0, st, b.J, n, b.UM, n, n,
