@@ -12,6 +12,9 @@ namespace {
 
 constexpr int NT = 1024;
 
+typedef double d4s __attribute__((ext_vector_type(4)));
+PC_DEV d4s mfma64s(double a, double b, d4s c) { return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0); }
+
 PC_DEV double wave_sum(double v) {
   for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
   return v;
@@ -341,6 +344,11 @@ __global__ __launch_bounds__(NT) void k_pchol(const T* G, int ldg, int n, double
 //   op(B)[k][j] uses row brow[k] of B (op = none) when brow != NULL.
 // opA/opB: 0 none, 1 transpose, 2 conjugate transpose.  If ctrans, C is
 // stored transposed (C^T, column-major result).  32x32 tiles, 256 threads.
+//
+// Real products: a 16 x 16 MFMA tile per wave, its operands straight from memory, 16
+// k-steps of loads on their way while the 16 before are multiplied.  One wave covers a
+// row of 64 k-steps in 2 us of MFMA; through LDS tiles with two barriers for every 32 k a
+// product of n = 256 took 26 us.
 // ---------------------------------------------------------------------------
 template <class T>
 __global__ __launch_bounds__(256) void k_gemm_small(int opA, int opB, int M, int N, int K, T alpha, const T* A,
@@ -351,6 +359,58 @@ __global__ __launch_bounds__(256) void k_gemm_small(int opA, int opB, int M, int
   B = zoff(B, zb);
   brow = zoff(brow, zb);
   C = zoff(C, zb);
+  if constexpr (std::is_same<T, double>::value) {
+    const int w = threadIdx.x >> 6, lr = threadIdx.x & 15, lk = (threadIdx.x >> 4) & 3;
+    const int i0 = blockIdx.y * 32 + 16 * (w >> 1), j0 = blockIdx.x * 32 + 16 * (w & 1);
+    if (i0 >= M || j0 >= N) return;
+    // element (i, k) of op(A) at A[i ai + k ak], (k, j) of op(B) at B[k bk + j bj]
+    const int ak = opA ? lda : 1, bk = opB ? 1 : ldb;
+    const double* a = A + min(i0 + lr, M - 1) * int64_t(opA ? 1 : lda);
+    const double* b = B + min(j0 + lr, N - 1) * int64_t(opB ? ldb : 1);
+    constexpr int U = 16;
+    double av[U], bv[U];
+    auto fetch = [&](int k0) {
+      int ka[U], kb[U];
+#pragma unroll
+      for (int u = 0; u < U; u++) ka[u] = kb[u] = min(k0 + 4 * u + lk, K - 1);
+      if (acol && !opA) {
+#pragma unroll
+        for (int u = 0; u < U; u++) ka[u] = acol[ka[u]];
+      }
+      if (brow && !opB) {
+#pragma unroll
+        for (int u = 0; u < U; u++) kb[u] = brow[kb[u]];
+      }
+#pragma unroll
+      for (int u = 0; u < U; u++) {
+        av[u] = a[int64_t(ka[u]) * ak];
+        bv[u] = b[int64_t(kb[u]) * bk];
+      }
+    };
+    d4s acc = {0.0, 0.0, 0.0, 0.0};
+    if (K > 0) fetch(0);
+    for (int k0 = 0; k0 < K; k0 += 4 * U) {
+      double x[U], y[U];
+#pragma unroll
+      for (int u = 0; u < U; u++) {
+        const bool in = k0 + 4 * u + lk < K;
+        x[u] = in ? av[u] : 0.0;
+        y[u] = in ? bv[u] : 0.0;
+      }
+      fetch(k0 + 4 * U);
+#pragma unroll
+      for (int u = 0; u < U; u++) acc = mfma64s(x[u], y[u], acc);
+    }
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+      const int i = i0 + 4 * r + lk, j = j0 + lr;
+      if (i < M && j < N) {
+        double* c = C + (ctrans ? int64_t(j) * ldc + i : int64_t(i) * ldc + j);
+        *c = beta == 0.0 ? alpha * acc[r] : alpha * acc[r] + beta * *c;
+      }
+    }
+    return;
+  }
   __shared__ T As[32][33];
   __shared__ T Bs[32][33];
   int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;  // ty 0..7
@@ -431,15 +491,18 @@ __global__ __launch_bounds__(NT) void k_bjac_init(const T* H, int ldh, int rows,
   state = zoff(state, zb);
   dstate = zoff(dstate, zb);
   __shared__ double sh[32];
-  for (int i = threadIdx.x; i < nflags; i += NT) state[i] = 0;
-  for (int64_t idx = threadIdx.x; idx < int64_t(cols) * cols; idx += NT) {
-    int j = int(idx / cols), i = int(idx % cols);  // consecutive threads, consecutive addresses
-    J[int64_t(j) * ldj + i] = T(i == j ? 1.0 : 0.0);
-  }
+  if (blockIdx.x == 0)
+    for (int i = threadIdx.x; i < nflags; i += NT) state[i] = 0;
+  // the columns of J, one wave each, over all workgroups
+  const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
+  for (int j = blockIdx.x * (NT / 64) + w; j < cols; j += gridDim.x * (NT / 64))
+    for (int i = l; i < cols; i += 64) J[int64_t(j) * ldj + i] = T(i == j ? 1.0 : 0.0);
+  if (blockIdx.x > 0) return;
   double f = 0.0;
-  for (int64_t idx = threadIdx.x; idx < int64_t(cols) * rows; idx += NT) {
-    int k = int(idx / rows), i = int(idx % rows);
-    f += abs2_(H[int64_t(k) * ldh + i]);
+  for (int k = w; k < cols; k += NT / 64) {
+    const T* h = H + int64_t(k) * ldh;
+#pragma unroll 4
+    for (int i = l; i < rows; i += 64) f += abs2_(h[i]);
   }
   f = block_sum(f, sh);
   if (threadIdx.x == 0) {
@@ -562,8 +625,6 @@ __global__ void k_bjac_check(int* state, int sweep, int64_t zb = 0) {
   if (threadIdx.x == 0 && !state[0] && state[1 + sweep] == 0) state[0] = 1;
 }
 
-typedef double d4s __attribute__((ext_vector_type(4)));
-PC_DEV d4s mfma64s(double a, double b, d4s c) { return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0); }
 
 // One-sided Jacobi of a small problem held by a single block pair (2b <= 32
 // columns, rows <= 64), on one wavefront: 4 lanes per column pair, every
@@ -685,7 +746,7 @@ __global__ __launch_bounds__(NT) void k_bjac_norms(const T* H, int ldh, int rows
   state = zoff(state, zb);
   status = zoff(status, zb);
   int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  for (int k = wv; k < cols; k += NT / 64) {
+  for (int k = blockIdx.x * (NT / 64) + wv; k < cols; k += gridDim.x * (NT / 64)) {
     double s = 0;
     const T* hk = H + int64_t(k) * ldh;
     for (int i = lane; i < rows; i += 64) s += abs2_(hk[i]);
@@ -695,7 +756,7 @@ __global__ __launch_bounds__(NT) void k_bjac_norms(const T* H, int ldh, int rows
       if (!isfinite(s)) atomicOr(status, 8);
     }
   }
-  if (threadIdx.x == 0 && !state[0]) atomicOr(status, 2);
+  if (blockIdx.x == 0 && threadIdx.x == 0 && !state[0]) atomicOr(status, 2);
 }
 
 // block width of the block Jacobi for an n x n problem with element size esz:
@@ -714,14 +775,27 @@ __global__ __launch_bounds__(NT) void k_sort_desc(const double* sig, int n, int*
   order = zoff(order, zb);
   // NaN keys rank as -inf, ties by index: the ranks always form a permutation,
   // so every order[] entry is written with a valid column index.
-  for (int i = threadIdx.x; i < n; i += NT) {
-    double v = key_desc(sig[i]);
+  // The keys are compared from LDS, KEYS of them at a time (256 keys: 19 -> 6 us)
+  constexpr int KEYS = 2048;
+  __shared__ double key[KEYS];
+  for (int i0 = 0; i0 < n; i0 += NT) {
+    const int i = i0 + threadIdx.x;
+    const double v = key_desc(sig[i < n ? i : 0]);
     int rnk = 0;
-    for (int j = 0; j < n; j++) {
-      double u = key_desc(sig[j]);
-      rnk += (u > v) || (u == v && j < i);
+    for (int j0 = 0; j0 < n; j0 += KEYS) {
+      const int m = n - j0 < KEYS ? n - j0 : KEYS;
+      __syncthreads();
+      for (int j = threadIdx.x; j < m; j += NT) key[j] = key_desc(sig[j0 + j]);
+      __syncthreads();
+      if (i < n) {  // waves beyond the keys would take the others' issue slots
+#pragma unroll 8
+        for (int j = 0; j < m; j++) {
+          const double u = key[j];
+          rnk += (u > v) || (u == v && j0 + j < i);
+        }
+      }
     }
-    order[rnk] = i;
+    if (i < n) order[rnk] = i;
   }
 }
 
@@ -879,13 +953,13 @@ __global__ __launch_bounds__(256) void k_svd_finish(const T* Hc, int ldh, int ro
   int64_t idx = int64_t(blockIdx.x) * 256 + threadIdx.x;
   double smax = sig[order[0]];
   int rk = rank_in ? rank_in[0] : n;
-  if (idx == 0) {
+  if (blockIdx.x == 0) {
     int c = 0;
-    for (int k = 0; k < n; k++) {
-      double s = sig[order[k]];
-      if (!(s > null_tol * smax) || k >= rk) c++;
+    for (int k0 = 0; k0 < n; k0 += 256) {
+      const int k = k0 + threadIdx.x;
+      c += __syncthreads_count(k < n && (!(sig[order[k < n ? k : 0]] > null_tol * smax) || k >= rk));
     }
-    nnull[0] = c;
+    if (threadIdx.x == 0) nnull[0] = c;
   }
   if (idx < n) {
     double s = sig[order[idx]];

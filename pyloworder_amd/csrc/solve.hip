@@ -129,7 +129,8 @@ void launch_block_jacobi(pc_ctx* ctx, T* H, int ldh, int n, T* J, int ldj, doubl
   hipStream_t st = ctx->stream;
   int b, nb2;
   jacobi_blocks<T>(n, b, nb2);
-  hipLaunchKernelGGL((k_bjac_init<T>), dim3(1, 1, nz), dim3(1024), 0, st, H, ldh, n, n, J, ldj, state, dstate,
+  const unsigned gc = unsigned(ceil_div(n, 1024 / 64));  // a wave per column
+  hipLaunchKernelGGL((k_bjac_init<T>), dim3(gc, 1, nz), dim3(1024), 0, st, H, ldh, n, n, J, ldj, state, dstate,
                      kBjacMaxSweeps + 1, zb);
   // relative orthogonality test |h_p^H h_q| <= tol ||h_p|| ||h_q||: the dot
   // product itself carries ~eps sqrt(rows) rounding, so tol grows with rows
@@ -155,7 +156,7 @@ void launch_block_jacobi(pc_ctx* ctx, T* H, int ldh, int n, T* J, int ldj, doubl
       hipLaunchKernelGGL(k_bjac_check, dim3(1, 1, nz), dim3(64), 0, st, state, s, zb);
     }
   }
-  hipLaunchKernelGGL((k_bjac_norms<T>), dim3(1, 1, nz), dim3(1024), 0, st, H, ldh, n, n, sig, state, status, zb);
+  hipLaunchKernelGGL((k_bjac_norms<T>), dim3(gc, 1, nz), dim3(1024), 0, st, H, ldh, n, n, sig, state, status, zb);
 }
 
 
@@ -698,15 +699,61 @@ __global__ __launch_bounds__(1024) void k_null_build(int64_t m, int n, const int
   int* pick = reinterpret_cast<int*>(keys + ncand);
   for (int c = threadIdx.x; c < ncand; c += 1024) keys[c] = key_asc(lev[c]);
   __syncthreads();
-  // rank candidates by leverage (ties by index), keep the first d
-  for (int c = threadIdx.x; c < ncand; c += 1024) {
-    double v = keys[c];
-    int r = 0;
-    for (int e = 0; e < ncand; e++) {
-      double u = keys[e];
-      r += (u < v) || (u == v && e < c);
+  // the d candidates of the lowest leverage (ties by index).  Few, the usual case (row
+  // centring leaves one null direction): the next one after the last pick, d times, and
+  // below one wave per sum; n = 256, d = 1: 118 -> 25 us.  Many: by their ranks.
+  const bool few = d <= 4;
+  const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  __shared__ double best_v[16];
+  __shared__ int best_c[16];
+  if (few) {
+    double lv = -1e308;
+    int lc = -1;
+    for (int a = 0; a < d; a++) {
+      double v = 0.0;
+      int at = -1;
+      for (int c = threadIdx.x; c < ncand; c += 1024) {
+        const double u = keys[c];
+        if ((lc < 0 || u > lv || (u == lv && c > lc)) && (at < 0 || u < v)) {
+          v = u;
+          at = c;
+        }
+      }
+      for (int o = 32; o > 0; o >>= 1) {
+        const double u = __shfl_xor(v, o);
+        const int c = __shfl_xor(at, o);
+        if (c >= 0 && (at < 0 || u < v || (u == v && c < at))) {
+          v = u;
+          at = c;
+        }
+      }
+      if (lane == 0) {
+        best_v[wv] = v;
+        best_c[wv] = at;
+      }
+      __syncthreads();
+      v = best_v[0];
+      at = best_c[0];
+      for (int k = 1; k < 16; k++)
+        if (best_c[k] >= 0 && (at < 0 || best_v[k] < v || (best_v[k] == v && best_c[k] < at))) {
+          v = best_v[k];
+          at = best_c[k];
+        }
+      lv = v;
+      lc = at;
+      if (threadIdx.x == 0) pick[a] = at;
+      __syncthreads();
     }
-    if (r < d) pick[r] = c;
+  } else {
+    for (int c = threadIdx.x; c < ncand; c += 1024) {
+      double v = keys[c];
+      int r = 0;
+      for (int e = 0; e < ncand; e++) {
+        double u = keys[e];
+        r += (u < v) || (u == v && e < c);
+      }
+      if (r < d) pick[r] = c;
+    }
   }
   __syncthreads();
   for (int a = threadIdx.x; a < d; a += 1024) {
@@ -717,13 +764,17 @@ __global__ __launch_bounds__(1024) void k_null_build(int64_t m, int n, const int
   // Md (d x d) in work, row-major
   T* Md = work;
   T* Rd = work + int64_t(d) * d;
-  for (int64_t idx = threadIdx.x; idx < int64_t(d) * d; idx += 1024) {
+  // lanes of a wave (few) or one thread share a sum
+  const int step = few ? 64 : 1, first = few ? lane : 0;
+  auto total = [&](T v) { return few ? group_sum_t(v, 64) : v; };
+  for (int64_t idx = few ? wv : threadIdx.x; idx < int64_t(d) * d; idx += few ? 16 : 1024) {
     int a = int(idx / d), b = int(idx % d);
     const T* ua = urows + int64_t(pick[a]) * n;
     const T* ub = urows + int64_t(pick[b]) * n;
     T s = T(0.0);
-    for (int k = 0; k < g; k++) s += ua[k] * conj_(ub[k]);
-    Md[idx] = T(a == b ? 1.0 : 0.0) - s;
+    for (int k = first; k < g; k += step) s += ua[k] * conj_(ub[k]);
+    s = total(s);
+    if (first == 0) Md[idx] = T(a == b ? 1.0 : 0.0) - s;
   }
   __syncthreads();
   // Cholesky Md = Rd^H Rd (upper), in place into Rd
@@ -771,11 +822,12 @@ __global__ __launch_bounds__(1024) void k_null_build(int64_t m, int n, const int
     T2[idx] = s;
   }
   __syncthreads();
-  for (int64_t idx = threadIdx.x; idx < int64_t(n) * d; idx += 1024) {
+  for (int64_t idx = few ? wv : threadIdx.x; idx < int64_t(n) * d; idx += few ? 16 : 1024) {
     int j = int(idx / d), b = int(idx % d);
     T s = T(0.0);
-    for (int k = 0; k < g; k++) s += W[int64_t(j) * ldw + k] * T2[int64_t(k) * d + b];
-    W[int64_t(j) * ldw + g + b] = -s;
+    for (int k = first; k < g; k += step) s += W[int64_t(j) * ldw + k] * T2[int64_t(k) * d + b];
+    s = total(s);
+    if (first == 0) W[int64_t(j) * ldw + g + b] = -s;
   }
 }
 
@@ -829,18 +881,25 @@ __global__ __launch_bounds__(256) void k_embed_pad(const cdouble* W, int ldw, in
   P[idx] = v;
 }
 
-// M <- M C, C = I - 1 1^T / n  (M n x n, column-major: M[i][j] = Hc[j * ld + i])
+// M <- M C, C = I - 1 1^T / n  (M n x n, column-major: M[i][j] = Hc[j * ld + i]); a
+// workgroup takes 16 rows, 16 threads sharing a row (one thread per row: 46 us at n = 256)
 template <class T>
 __global__ __launch_bounds__(256) void k_center_right(T* Hc, int ld, int n, int64_t zb = 0) {
   Hc = zoff(Hc, zb);
-  int i = blockIdx.x * 256 + threadIdx.x;
-  if (i >= n) return;
+  __shared__ T part[16][17];
+  const int r = threadIdx.x & 15, g = threadIdx.x >> 4, i = blockIdx.x * 16 + r;
+  T* row = Hc + (i < n ? i : 0);
   T s = T(0.0);
-#pragma unroll 16
-  for (int j = 0; j < n; j++) s += Hc[int64_t(j) * ld + i];  // loads ahead, sum in order
+#pragma unroll 8
+  for (int j = g; j < n; j += 16) s += row[int64_t(j) * ld];
+  part[r][g] = s;
+  __syncthreads();
+  s = T(0.0);
+  for (int k = 0; k < 16; k++) s += part[r][k];
   s = s * (1.0 / n);
-#pragma unroll 16
-  for (int j = 0; j < n; j++) Hc[int64_t(j) * ld + i] -= s;
+  if (i >= n) return;
+#pragma unroll 8
+  for (int j = g; j < n; j += 16) row[int64_t(j) * ld] -= s;
 }
 
 // mixed: Wr (real FP64 NB x NB, values of the rounded operand) -> T n x n
@@ -1255,7 +1314,7 @@ static int core_t(pc_ctx* ctx, const Plan& p, const void* A, int64_t lda, int ce
   // mixed path: the passes saw Y - a 1^T (a = row shift); Y C = (Y - a 1^T) C, so the
   // exact centring is M <- M C
   if (p.mixed && center)
-    hipLaunchKernelGGL((k_center_right<T>), dim3(nblk(n)), dim3(256), 0, st, b.Hc, n, n);
+    hipLaunchKernelGGL((k_center_right<T>), dim3(nblk(n, 16)), dim3(256), 0, st, b.Hc, n, n);
   hipLaunchKernelGGL((k_pad_identity<T>), dim3(1), dim3(256), 0, st, b.R2, n, n, b.rank);
   // R2i = R2^-1 is read first in W, after the Jacobi: it runs beside the
   // preconditioner and the Jacobi (no kernel between writes R2 or R2i)
@@ -1433,7 +1492,7 @@ static int core_batch_t(pc_ctx* ctx, const Plan& p, const pc_problem* pr, int64_
   hipLaunchKernelGGL((k_gemm_small<T>), gg, dim3(256), 0, st, 0, 0, n, n, n, T(1.0), b.R2, n, (const int*)nullptr,
                      b.R1h, n, (const int*)b.perm, T(0.0), b.Hc, n, 1, zb);
   if (p.mixed && center)
-    hipLaunchKernelGGL((k_center_right<T>), dim3(nblk(n), 1, z), dim3(256), 0, st, b.Hc, n, n, zb);
+    hipLaunchKernelGGL((k_center_right<T>), dim3(nblk(n, 16), 1, z), dim3(256), 0, st, b.Hc, n, n, zb);
   hipLaunchKernelGGL((k_pad_identity<T>), dim3(1, 1, z), dim3(256), 0, st, b.R2, n, n, b.rank, zb);
   run_trinv<T>(st, b.R2, n, b.R2i, nz, zb);
   launch_block_jacobi<T>(ctx, b.Hc, n, n, b.J, n, b.sig, b.jstate, b.jdstate, b.status,
