@@ -295,14 +295,13 @@ __global__ __launch_bounds__(kCholThreads) void k_chol_fast(const double* G, int
 // The pivot steps form one chain: largest diagonal, its row of A from L2, new row,
 // diagonals.  One wave per SIMD, thread t owning columns t + 256 c: with 16 waves
 // the chain's scalar work was issued four times per SIMD (2.0 us a step), with one
-// wave its LDS traffic and selections came one after the other (1.7 us).  A thread
-// reads its own columns of the panel while the pivot is being found, those of column
-// p by one LDS read, entry t on lane t, and lane reads, while A's row comes.  One
+// wave its LDS traffic and selections came one after the other (1.7 us).  The panel's
+// products run while A's row comes.  One
 // barrier per step, over which the waves exchange their largest diagonals.
 // The fold runs on MFMA and writes the Schur complement of the remaining columns
 // only, compacted (in increasing order) into the other of two buffers: a third of
-// the products that a fold of all columns does.  n = 256: 568 -> 310 us (1,800
-// cycles a step, a quarter of the time in the folds).
+// the products that a fold of all columns does.  n = 256: 568 -> 270 us (1,800
+// cycles a step, a fifth of the time in the folds).
 //
 // A, B: n x n workspaces.  R leaves with its columns in G's order (R[t][q], only
 // the columns unpivoted before row t's panel written); k_pchol_cols permutes them.
@@ -314,7 +313,7 @@ __global__ __launch_bounds__(kPcholThreads) void k_pchol_fast(const double* G, i
                                                               int* status) {
   using namespace dense;
   constexpr int NTH = kPcholThreads, NW = NTH / 64, N = NTH * C, LD = PW + 2;
-  __shared__ double P[N * LD];       // entry t of column q at P[q * LD + t]
+  __shared__ __attribute__((aligned(16))) double P[N * LD];  // entry t of column q at P[q * LD + t]
   __shared__ double dgs[N];          // diagonals, compacted
   __shared__ short id[N], al[N];     // column of a position; its position before the fold
   __shared__ short prm[N];           // the pivots
@@ -401,20 +400,6 @@ __global__ __launch_bounds__(kPcholThreads) void k_pchol_fast(const double* G, i
         bk[k] = cand_v[sl][k];
         pk[k] = cand_p[sl][k];
       }
-      // this thread's columns of the panel (zero from entry jj on) come from LDS while
-      // the pivot is being found; jd hides jj, or the compiler makes a loop of its own
-      // for each group of entries (32 KB of code)
-      int jd = jj;
-      asm volatile("" : "+s"(jd));
-      double pr[C][PW];
-#pragma unroll
-      for (int t0 = 0; t0 < PW; t0 += 8)
-        if (t0 < jd) {
-#pragma unroll
-          for (int t = t0; t < t0 + 8; t++)
-#pragma unroll
-            for (int c = 0; c < C; c++) pr[c][t] = P[(tid + NTH * c) * LD + t];
-        }
       double b = bk[0];
       int p = pk[0];
 #pragma unroll
@@ -425,7 +410,6 @@ __global__ __launch_bounds__(kPcholThreads) void k_pchol_fast(const double* G, i
       }
       p = __builtin_amdgcn_readfirstlane(p);
       if (__ballot(b > thr) == 0) break;
-      const double prow = P[p * LD + (l & (PW - 1))];
       double x[C], s[C][4];
 #pragma unroll
       for (int c = 0; c < C; c++) {
@@ -434,15 +418,25 @@ __global__ __launch_bounds__(kPcholThreads) void k_pchol_fast(const double* G, i
         s[c][0] = s[c][1] = s[c][2] = s[c][3] = 0.0;
       }
       const double y = rsqrt_f64(b), r = sqrt_from(b, y);
+      // The products of column p's panel entries (the same address in every lane) and this
+      // thread's (zero from entry jj on) run while A's row comes.  jd hides jj, or the
+      // compiler makes a loop of its own for each group of entries (32 KB of code).
+      int jd = jj;
+      asm volatile("" : "+s"(jd));
 #pragma unroll
       for (int t0 = 0; t0 < PW; t0 += 8)
         if (t0 < jd) {
+          double pp[8], pr[C][8];
 #pragma unroll
-          for (int t = t0; t < t0 + 8; t++) {
-            const double pt = lane_read_f64(prow, t);
+          for (int t = 0; t < 8; t++) {
+            pp[t] = P[p * LD + t0 + t];
 #pragma unroll
-            for (int c = 0; c < C; c++) s[c][t & 3] = fma(pt, pr[c][t], s[c][t & 3]);
+            for (int c = 0; c < C; c++) pr[c][t] = P[(tid + NTH * c) * LD + t0 + t];
           }
+#pragma unroll
+          for (int t = 0; t < 8; t++)
+#pragma unroll
+            for (int c = 0; c < C; c++) s[c][t & 3] = fma(pp[t], pr[c][t], s[c][t & 3]);
         }
       if (tid == 0) prm[k0 + jj] = short(p);  // as positions until the panel's end
 #pragma unroll

@@ -391,13 +391,33 @@ __global__ __launch_bounds__(256) void k_q1_rows(const TS* X, int64_t ldx, int n
   }
 }
 
-// D (n signs) from Q1 (n x n, overwritten by its shifted LU); one workgroup.
-// The shift makes every pivot at least 1 in modulus, so no pivoting is needed.
+// D (n signs) from Q1 (n x n; overwritten by its shifted LU unless that runs in LDS);
+// one workgroup.  The shift makes every pivot at least 1 in modulus, so no pivoting is
+// needed.  LDS copy: up to kSignsLds bytes of it (n = 64: 70 -> 17 us; in memory a step
+// waits for the step before it through the L2).
+constexpr size_t kSignsLds = 140 * 1024;
 template <class T>
-__global__ __launch_bounds__(1024) void k_lapack_signs(T* Q1, int n, T* D) {
+inline size_t signs_lds(int n) {
+  const size_t b = size_t(n) * (n + 1) * sizeof(T);
+  return b <= kSignsLds ? b : 0;
+}
+template <class T>
+__global__ __launch_bounds__(1024) void k_lapack_signs(T* Q1, int n, int in_lds, T* D) {
   constexpr double kReduced = 64 * 2.220446049250313e-16;
+  HIP_DYNAMIC_SHARED(char, signs_smem)
+  const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
+  T* A = Q1;
+  int ld = n;
+  if (in_lds) {
+    A = reinterpret_cast<T*>(signs_smem);
+    ld = n + 1;
+    for (int i = w; i < n; i += 16)
+      for (int j = l; j < n; j += 64) A[i * ld + j] = Q1[int64_t(i) * n + j];
+    __syncthreads();
+  }
   for (int k = 0; k < n; k++) {
-    const T a = Q1[int64_t(k) * n + k];
+    const T* rk = A + int64_t(k) * ld;
+    const T a = rk[k];
     const double re = real_(a);
     const T s = T(re >= 0.0 ? -1.0 : 1.0);
     if (threadIdx.x == 0) {
@@ -405,10 +425,10 @@ __global__ __launch_bounds__(1024) void k_lapack_signs(T* Q1, int n, T* D) {
       D[k] = reduced ? T(re >= 0.0 ? 1.0 : -1.0) : s;
     }
     const T ip = inv_(a - s);
-    const int w = n - k - 1;
-    for (int64_t idx = threadIdx.x; idx < int64_t(w) * w; idx += 1024) {
-      const int i = k + 1 + int(idx / w), j = k + 1 + int(idx % w);
-      Q1[int64_t(i) * n + j] -= Q1[int64_t(i) * n + k] * ip * Q1[int64_t(k) * n + j];
+    for (int i = k + 1 + w; i < n; i += 16) {
+      T* ri = A + int64_t(i) * ld;
+      const T f = ri[k] * ip;
+      for (int j = k + 1 + l; j < n; j += 64) ri[j] -= f * rk[j];
     }
     __syncthreads();
   }
@@ -1395,7 +1415,8 @@ static int core_t(pc_ctx* ctx, const Plan& p, const void* A, int64_t lda, int ce
     // LAPACK's signs (numpy.linalg.qr): D from the first n rows of Q, then
     // R = D R+, Q = Q+ D through W and the null fix; Q1 in tmp, D in G2
     launch_q1_rows<T>(st, p, A, lda, b);
-    hipLaunchKernelGGL((k_lapack_signs<T>), dim3(1), dim3(1024), 0, st, b.tmp, n, b.G2);
+    hipLaunchKernelGGL((k_lapack_signs<T>), dim3(1), dim3(1024), signs_lds<T>(n), st, b.tmp, n, int(signs_lds<T>(n) > 0),
+                       b.G2);
     hipLaunchKernelGGL((k_apply_signs<T>), dim3(nblk(nn)), dim3(256), 0, st, (const T*)b.G2, n, b.J, n, b.Wf, n,
                        (const int*)b.nnull, b.cnull);
     hipLaunchKernelGGL((k_store_r<T, typename VtType<T, ST>::type>), dim3(nblk(nn)), dim3(256), 0, st, b.J, n, n,
