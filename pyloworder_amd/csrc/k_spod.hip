@@ -109,28 +109,37 @@ __global__ __launch_bounds__(256) void k_spod_blocks(const float* __restrict__ X
   }
 }
 
-// Power-of-two nDFT: radix-2 Stockham FFT in LDS.  A workgroup owns one row
+constexpr int kFftPad = 4;  // complex values between the rows of blocks: other banks for the same frequency
+
+// Power-of-two nDFT >= 4: Stockham FFT in LDS.  A workgroup owns one row
 // pair and runs through the blocks in chunks of BC; rows a, b form one
 // complex sequence z = y_a + i y_b, and after the FFT Z the two real spectra
 // are
 //   Y_a[f] = (Z[f] + conj Z[N-f]) / 2,   Y_b[f] = (Z[f] - conj Z[N-f]) / 2i.
 // Stage with half-size m (m = 1, 2, ..., N/2), butterfly j < N/2, k = j mod m:
 //   a = A[j], b = A[j + N/2] w^(k N / 2m);  B[2j - k] = a + b, B[2j - k + m] = a - b.
-// Twiddles w^q = exp(-2 pi i q / N) come from the FP64-accurate tables.  The
+// Every stage reads and writes the sequence in LDS once, which is what bounds the kernel,
+// so two are taken at a time: butterflies j and j + N/4 of stage m feed 2j - k and
+// 2j - k + m of stage 2m, the same operations on four values in registers.  The first
+// two take the samples from the registers they were fetched into, and their twiddles
+// are 1 and -i; a last stage is left when log2 N is odd.  Twiddles
+// w^q = exp(-2 pi i q / N) come from the FP64-accurate tables.  The
 // spectra of a chunk are staged in LDS as [f][row][block], so that each
 // frequency's two rows leave as one contiguous run Q[f][ra][b0..b1),
 // Q[f][ra+1][b0..b1) (consecutive rows are adjacent in Q).
+// 200,000 x 2048, nDFT = 256: 3.85 ms with a pass over LDS per stage and divided
+// indices, now 2.2.
 __global__ __launch_bounds__(256) void k_spod_fft(const float* __restrict__ X, int64_t ldx, int64_t M,
                                                   const double* __restrict__ mean, const float* __restrict__ win,
                                                   const float* __restrict__ twc, const float* __restrict__ tws,
                                                   int nDFT, int logN, int step, int nBlks, int nf, int BC, int P,
                                                   const float* __restrict__ fscale, float2* __restrict__ Q) {
   extern __shared__ float2 fsm[];
-  const int N = nDFT, H = nDFT / 2;
-  float2* A = fsm;              // [P][N]: P blocks transformed side by side
-  float2* B = A + P * N;        // [P][N]
-  float2* tw = B + P * N;       // [N / 2]
-  float2* stg = tw + H;         // [nf][2][BC]
+  const int N = nDFT, Q4 = N >> 2, NS = N + kFftPad;
+  float2* A = fsm;              // [P][NS]: P blocks transformed side by side
+  float2* B = A + P * NS;       // [P][NS]
+  float2* tw = B + P * NS;      // [N / 2]
+  float2* stg = tw + 2 * Q4;    // [nf][2][BC]
   // Row pairs are split into 8 contiguous ranges, one per XCD (workgroup x
   // runs on XCD x mod 8), so neighbouring pairs, whose output runs share
   // cache lines, are written through the same L2.
@@ -140,34 +149,58 @@ __global__ __launch_bounds__(256) void k_spod_fft(const float* __restrict__ X, i
   const int64_t ra = pair * 2, rb = ra + 1;
   const bool va = ra < M, vb = rb < M;
   const double mua = (mean && va) ? mean[ra] : 0.0, mub = (mean && vb) ? mean[rb] : 0.0;
-  for (int q = threadIdx.x; q < H; q += 256) tw[q] = make_float2(twc[q], -tws[q]);
-  // Samples of the next pass are fetched into registers while the current
-  // pass is transformed (at most P N / 256 <= 8 per thread and row).
-  constexpr int EMAX = 8;
-  float xa[EMAX], xb[EMAX];
+  for (int q = threadIdx.x; q < 2 * Q4; q += 256) tw[q] = make_float2(twc[q], -tws[q]);
+  const float *rowa = X + (va ? ra : 0) * ldx, *rowb = X + (vb ? rb : 0) * ldx;
+  // Samples of the next pass are fetched into registers while the current pass is
+  // transformed: the four inputs of at most BF first butterflies per thread
+  constexpr int BF = 2;
+  float xa[BF][4], xb[BF][4];
+  const int lq = logN - 2;
   auto fetch = [&](int gb, int np) {
 #pragma unroll
-    for (int u = 0; u < EMAX; u++) {
-      const int e = threadIdx.x + u * 256;
-      if (e < np * N) {
-        const int pi = e / N, t = e - pi * N;
-        const int64_t t0 = int64_t(gb + pi) * step + t;
-        xa[u] = va ? X[ra * ldx + t0] : 0.0f;
-        xb[u] = vb ? X[rb * ldx + t0] : 0.0f;
+    for (int u = 0; u < BF; u++) {
+      const int jj = threadIdx.x + u * 256;
+      if (jj < np << lq) {
+        const int64_t t0 = int64_t(gb + (jj >> lq)) * step + (jj & (Q4 - 1));
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+          xa[u][r] = va ? rowa[t0 + r * Q4] : 0.0f;
+          xb[u][r] = vb ? rowb[t0 + r * Q4] : 0.0f;
+        }
       }
     }
   };
+  // which product of the two is fused is part of the result: a noise mode's phase shows it
+  auto mul = [](float2 w, float2 x) {
+    return make_float2(__builtin_fmaf(w.x, x.x, -(w.y * x.y)), __builtin_fmaf(w.x, x.y, w.y * x.x));
+  };
+  auto add = [](float2 x, float2 y) { return make_float2(x.x + y.x, x.y + y.y); };
+  auto sub = [](float2 x, float2 y) { return make_float2(x.x - y.x, x.y - y.y); };
   fetch(0, nBlks < P ? nBlks : P);
   for (int b0 = 0; b0 < nBlks; b0 += BC) {
     const int nb = nBlks - b0 < BC ? nBlks - b0 : BC;
     for (int bp = 0; bp < nb; bp += P) {
       const int np = nb - bp < P ? nb - bp : P;  // blocks in this pass
 #pragma unroll
-      for (int u = 0; u < EMAX; u++) {
-        const int e = threadIdx.x + u * 256;
-        if (e < np * N) {
-          const int t = e & (N - 1);
-          A[e] = make_float2(float(double(xa[u]) - mua) * win[t], float(double(xb[u]) - mub) * win[t]);
+      for (int u = 0; u < BF; u++) {
+        const int jj = threadIdx.x + u * 256;
+        if (jj < np << lq) {
+          const int j = jj & (Q4 - 1);
+          float2 x[4];
+#pragma unroll
+          for (int r = 0; r < 4; r++) {
+            const float wn = win[j + r * Q4];
+            x[r] = make_float2(float(double(xa[u][r]) - mua) * wn, float(double(xb[u][r]) - mub) * wn);
+            // rounded: the sums below must not contract with the window's products
+            asm volatile("" : "+v"(x[r].x), "+v"(x[r].y));
+          }
+          const float2 u0 = add(x[0], x[2]), u1 = sub(x[0], x[2]), v0 = add(x[1], x[3]), v = sub(x[1], x[3]);
+          const float2 v1 = make_float2(v.y, -v.x);  // -i v
+          float2* d = A + (jj >> lq) * NS + 4 * j;
+          d[0] = add(u0, v0);
+          d[1] = add(u1, v1);
+          d[2] = sub(u0, v0);
+          d[3] = sub(u1, v1);
         }
       }
       __syncthreads();
@@ -181,23 +214,42 @@ __global__ __launch_bounds__(256) void k_spod_fft(const float* __restrict__ X, i
       }
       float2* src = A;
       float2* dst = B;
-      for (int s = 0, m = 1; s < logN; s++, m <<= 1) {
-        const int tstride = N >> (s + 1);  // N / 2m
-        for (int jj = threadIdx.x; jj < np * H; jj += 256) {
-          const int pi = jj / H, j = jj - pi * H, k = j & (m - 1);
-          const float2* sp = src + pi * N;
-          float2* dp = dst + pi * N;
-          const float2 a = sp[j], bv = sp[j + H], w = tw[k * tstride];
-          const float2 wb = make_float2(w.x * bv.x - w.y * bv.y, w.x * bv.y + w.y * bv.x);
-          dp[2 * j - k] = make_float2(a.x + wb.x, a.y + wb.y);
-          dp[2 * j - k + m] = make_float2(a.x - wb.x, a.y - wb.y);
+      int lm = 2;
+      for (; lm + 2 <= logN; lm += 2) {
+        const int m = 1 << lm, ts = logN - 2 - lm;  // twiddle stride N / 4m
+        for (int jj = threadIdx.x; jj < np << lq; jj += 256) {
+          const int pi = jj >> lq, j = jj & (Q4 - 1), k = j & (m - 1);
+          const float2* sp = src + pi * NS + j;
+          const float2 x0 = sp[0], x1 = sp[Q4], w = tw[(2 * k) << ts];
+          const float2 x2 = mul(w, sp[2 * Q4]), x3 = mul(w, sp[3 * Q4]);
+          const float2 u0 = add(x0, x2), u1 = sub(x0, x2);
+          const float2 v0 = mul(tw[k << ts], add(x1, x3)), v1 = mul(tw[(k + m) << ts], sub(x1, x3));
+          float2* d = dst + pi * NS + 4 * (j - k) + k;
+          d[0] = add(u0, v0);
+          d[m] = add(u1, v1);
+          d[2 * m] = sub(u0, v0);
+          d[3 * m] = sub(u1, v1);
         }
         __syncthreads();
         float2* t = src; src = dst; dst = t;
       }
+      if (lm < logN) {
+        const int H = N >> 1;
+        for (int jj = threadIdx.x; jj < np * H; jj += 256) {
+          const int pi = jj >> (logN - 1), j = jj & (H - 1);
+          const float2 x0 = src[pi * NS + j], x1 = mul(tw[j], src[pi * NS + j + H]);
+          dst[pi * NS + j] = make_float2(x0.x + x1.x, x0.y + x1.y);
+          dst[pi * NS + j + H] = make_float2(x0.x - x1.x, x0.y - x1.y);
+        }
+        __syncthreads();
+        float2* t = src; src = dst; dst = t;
+      }
+      // the lanes run over a frequency's blocks, which are neighbours in the staging area
+      // (e < 2^14: the quotient is exact)
+      const float inv = 1.0f / float(np);
       for (int e = threadIdx.x; e < np * nf; e += 256) {
-        const int pi = e / nf, f = e - pi * nf, bi = bp + pi;
-        const float2 z = src[pi * N + f], zr = src[pi * N + ((N - f) & (N - 1))];
+        const int f = int((float(e) + 0.5f) * inv), pi = e - f * np, bi = bp + pi;
+        const float2 z = src[pi * NS + f], zr = src[pi * NS + ((N - f) & (N - 1))];
         const float sc = fscale[f];
         // Y_a = (z + conj zr) / 2,  Y_b = (z - conj zr) / 2i
         stg[(f * 2 + 0) * BC + bi] = make_float2(0.5f * (z.x + zr.x) * sc, 0.5f * (z.y - zr.y) * sc);
@@ -206,12 +258,15 @@ __global__ __launch_bounds__(256) void k_spod_fft(const float* __restrict__ X, i
       __syncthreads();  // A is reloaded by the next pass
     }
     // frequency f: rows ra, ra + 1 x blocks b0 .. b0 + nb, one contiguous run
-    // when both rows exist (Q[f][row][b] with row stride nBlks)
-    const int run = 2 * nb;
-    for (int idx = threadIdx.x; idx < nf * run; idx += 256) {
-      const int f = idx / run, e = idx - f * run, r = e / nb, bi = e - r * nb;
-      const int64_t row = ra + r;
-      if (row < M) Q[(int64_t(f) * M + row) * nBlks + b0 + bi] = stg[(f * 2 + r) * BC + bi];
+    // when both rows exist (Q[f][row][b] with row stride nBlks), by 32 or 64 lanes
+    const int run = vb ? 2 * nb : nb, sh = run <= 32 ? 5 : 6;
+    const int e0 = threadIdx.x & ((1 << sh) - 1);
+    for (int f = threadIdx.x >> sh; f < nf; f += 256 >> sh) {
+      float2* o = Q + (int64_t(f) * M + ra) * nBlks + b0;
+      for (int e = e0; e < run; e += 1 << sh) {
+        const int r = e >= nb, bi = e - (r ? nb : 0);
+        o[(r ? nBlks : 0) + bi] = stg[(f * 2 + r) * BC + bi];
+      }
     }
     __syncthreads();  // the staging area is refilled by the next chunk
   }
@@ -336,14 +391,15 @@ extern "C" int pc_spod_blocks(pc_ctx* ctx, const float* X, int64_t ldx, int64_t 
   int logN = 0;
   while ((int64_t(1) << logN) < nDFT) logN++;
   const bool pow2 = (int64_t(1) << logN) == nDFT;
-  // LDS of the FFT: A, B (P blocks of N complex each, P = 512 / N so that the
-  // 256 threads all have a butterfly), twiddles (N/2) and the staging of BC
-  // blocks' spectra (nf x 2 x BC complex), kept within 56 KB
-  if (pow2 && nDFT <= 2048) {
-    int64_t P = nDFT >= 512 ? 1 : 512 / nDFT;
+  // LDS of the FFT: A, B (P blocks of N complex each, P = 1024 / N so that the
+  // 256 threads all have two stages' butterflies of four values), twiddles (N / 2) and
+  // the staging of BC
+  // blocks' spectra (nf x 2 x BC complex), kept within 64 KB
+  if (pow2 && nDFT >= 4 && nDFT <= 2048) {
+    int64_t P = nDFT >= 1024 ? 1 : 1024 / nDFT;
     P = P > nBlks ? nBlks : P;
-    const int64_t fixed = (2 * P * nDFT + nDFT / 2) * int64_t(sizeof(float2));
-    int64_t bc = (57344 - fixed) / (nf * 2 * int64_t(sizeof(float2)));
+    const int64_t fixed = (2 * P * (nDFT + kFftPad) + nDFT / 2) * int64_t(sizeof(float2));
+    int64_t bc = (65536 - fixed) / (nf * 2 * int64_t(sizeof(float2)));
     bc = bc < 1 ? 1 : (bc > nBlks ? nBlks : bc);
     const size_t lds = size_t(fixed + nf * 2 * bc * int64_t(sizeof(float2)));
     hipLaunchKernelGGL(k_spod_fft, dim3(unsigned(ceil_div(M, 2))), dim3(256), lds, st, X, ldx, M,
