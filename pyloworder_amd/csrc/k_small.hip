@@ -71,10 +71,11 @@ PC_DEV double block_max(double v, double* sh) {
 // and 16 chunk lanes; lane k sums chunks k, k+16, ... in four interleaved
 // accumulators combined in a fixed order, then lane 0 adds the 16 lane sums in
 // order: the summation order depends only on (chunks, ld), so results are
-// deterministic.  Entry e is read and written only by its own workgroup.
+// deterministic.  Entry e is read and written only by its own workgroup.  G: the sums go
+// to the symmetric rows x rows matrix G instead (UPPER).
 template <bool UPPER>
 __global__ __launch_bounds__(1024) void k_reduce_slab(double* P, int chunks, int64_t pstride, int ld, int rows,
-                                                      int cols, int64_t zb = 0) {
+                                                      int cols, double* G, int64_t zb = 0) {
   P = zoff(P, zb);
   __shared__ double red[16][65];
   const int le = threadIdx.x & 63, k = threadIdx.x >> 6;
@@ -101,24 +102,13 @@ __global__ __launch_bounds__(1024) void k_reduce_slab(double* P, int chunks, int
     double t = 0.0;
 #pragma unroll
     for (int q = 0; q < 16; q++) t += red[q][le];
-    P[e] = t;
+    if (UPPER && G) {
+      G[int64_t(i) * rows + j] = t;
+      G[int64_t(j) * rows + i] = t;
+    } else {
+      P[e] = t;
+    }
   }
-}
-
-__global__ __launch_bounds__(256) void k_reduce_gram_real(const double* __restrict__ P, int chunks, int64_t pstride,
-                                                         int NB, int n, double* G, int ldg, int64_t zb = 0) {
-  P = zoff(P, zb);
-  G = zoff(G, zb);
-  int64_t idx = int64_t(blockIdx.x) * 256 + threadIdx.x;
-  int64_t tot = int64_t(n) * n;
-  if (idx >= tot) return;
-  int i = int(idx / n), j = int(idx % n);
-  if (i > j) return;
-  double s = 0.0;
-  const double* p = P + int64_t(i) * NB + j;
-  for (int c = 0; c < chunks; c++) s += p[c * pstride];
-  G[int64_t(i) * ldg + j] = s;
-  G[int64_t(j) * ldg + i] = s;
 }
 
 __global__ __launch_bounds__(256) void k_reduce_gram_cplx(const double* __restrict__ P, int chunks, int64_t pstride,

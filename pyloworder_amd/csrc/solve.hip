@@ -598,6 +598,7 @@ int64_t carve(WsCursor& c, const Plan& p, SmallBufs<T>& b, double** mean, double
 // ---------------------------------------------------------------------------
 // null completion kernels
 // ---------------------------------------------------------------------------
+constexpr int kLevRows = 4;
 // leverage of candidate rows: u_c = y_c W[:, :g] (g = n - nnull), lev_c = ||u_c||^2
 template <class T, class TS>
 __global__ __launch_bounds__(256) void k_null_lev(const TS* X, int64_t ldx, int64_t m, int n, int center,
@@ -612,38 +613,57 @@ __global__ __launch_bounds__(256) void k_null_lev(const TS* X, int64_t ldx, int6
   urows = zoff(urows, zb);
   int d = nnull[0];
   if (d == 0) return;
-  int c = blockIdx.x;
-  int64_t row = ncand >= m ? c : (int64_t(c) * m) / ncand;
-  HIP_DYNAMIC_SHARED(char, lev_smem)  // n values of T
-  T* yrow = reinterpret_cast<T*>(lev_smem);
-  for (int j = threadIdx.x; j < n; j += 256) {
-    T v = load_elem<T, TS>(X, row * ldx, j);
-    if (center == 3) {
-      v = v - load_elem<T, TS>(X, row * ldx, 0);  // mixed path: rows shifted by their first element
-    } else if (center) {
-      v = v - T(mean[row]);
-      if (center == 2) v = v * (1.0 / var[row]);
+  // kLevRows candidates per workgroup: W is read once for all of them (one each read n^2
+  // of it per row from the L2, 44 us at n = 256)
+  const int cand0 = blockIdx.x * kLevRows;
+  auto row_of = [&](int c) { return ncand >= m ? int64_t(c) : (int64_t(c) * m) / ncand; };
+  HIP_DYNAMIC_SHARED(char, lev_smem)  // kLevRows x n values of T
+  T* y = reinterpret_cast<T*>(lev_smem);
+#pragma unroll
+  for (int x = 0; x < kLevRows; x++) {
+    const int64_t row = row_of(cand0 + x < ncand ? cand0 + x : ncand - 1);
+    for (int j = threadIdx.x; j < n; j += 256) {
+      T v = load_elem<T, TS>(X, row * ldx, j);
+      if (center == 3) {
+        v = v - load_elem<T, TS>(X, row * ldx, 0);  // mixed path: rows shifted by their first element
+      } else if (center) {
+        v = v - T(mean[row]);
+        if (center == 2) v = v * (1.0 / var[row]);
+      }
+      y[x * n + j] = v;
     }
-    yrow[j] = v;
   }
   __syncthreads();
   int g = n - d;
-  double s = 0;
+  double s[kLevRows] = {};
   for (int k = threadIdx.x; k < n; k += 256) {
-    T u = T(0.0);
+    T u[kLevRows];
+#pragma unroll
+    for (int x = 0; x < kLevRows; x++) u[x] = T(0.0);
     if (k < g)
-      for (int j = 0; j < n; j++) u += yrow[j] * W[int64_t(j) * ldw + k];
-    urows[int64_t(c) * n + k] = u;
-    s += abs2_(u);
+#pragma unroll 8
+      for (int j = 0; j < n; j++) {
+        const T wj = W[int64_t(j) * ldw + k];
+#pragma unroll
+        for (int x = 0; x < kLevRows; x++) u[x] += y[x * n + j] * wj;
+      }
+#pragma unroll
+    for (int x = 0; x < kLevRows; x++) {
+      if (cand0 + x < ncand) urows[int64_t(cand0 + x) * n + k] = u[x];
+      s[x] += abs2_(u[x]);
+    }
   }
-  __shared__ double sh[256];
-  sh[threadIdx.x] = s;
+  __shared__ double sh[kLevRows][256];
+#pragma unroll
+  for (int x = 0; x < kLevRows; x++) sh[x][threadIdx.x] = s[x];
   __syncthreads();
   for (int o = 128; o > 0; o >>= 1) {
-    if (threadIdx.x < o) sh[threadIdx.x] += sh[threadIdx.x + o];
+    if (threadIdx.x < o)
+#pragma unroll
+      for (int x = 0; x < kLevRows; x++) sh[x][threadIdx.x] += sh[x][threadIdx.x + o];
     __syncthreads();
   }
-  if (threadIdx.x == 0) lev[c] = sh[0];
+  if (threadIdx.x < kLevRows && cand0 + int(threadIdx.x) < ncand) lev[cand0 + threadIdx.x] = sh[threadIdx.x][0];
 }
 
 
@@ -655,10 +675,10 @@ void launch_null_lev<double>(hipStream_t st, const Plan& p, const void* A, int64
                              const double* var, SmallBufs<double>& b, int ncand, int nz,
                              int64_t zb, int64_t zx) {
   if (p.dt == PC_F64)
-    hipLaunchKernelGGL((k_null_lev<double, double>), dim3(ncand, 1, nz), dim3(256), size_t(p.n) * sizeof(double), st, (const double*)A, lda, p.m, p.n,
+    hipLaunchKernelGGL((k_null_lev<double, double>), dim3(nblk(ncand, kLevRows), 1, nz), dim3(256), kLevRows * size_t(p.n) * sizeof(double), st, (const double*)A, lda, p.m, p.n,
                        center, mean, var, b.Wf, p.n, b.nnull, ncand, b.lev, b.urows, zb, zx);
   else
-    hipLaunchKernelGGL((k_null_lev<double, float>), dim3(ncand, 1, nz), dim3(256), size_t(p.n) * sizeof(double), st, (const float*)A, lda, p.m, p.n,
+    hipLaunchKernelGGL((k_null_lev<double, float>), dim3(nblk(ncand, kLevRows), 1, nz), dim3(256), kLevRows * size_t(p.n) * sizeof(double), st, (const float*)A, lda, p.m, p.n,
                        center, mean, var, b.Wf, p.n, b.nnull, ncand, b.lev, b.urows, zb, zx);
 }
 template <>
@@ -666,10 +686,10 @@ void launch_null_lev<cdouble>(hipStream_t st, const Plan& p, const void* A, int6
                               const double* var, SmallBufs<cdouble>& b, int ncand, int nz,
                               int64_t zb, int64_t zx) {
   if (p.dt == PC_C128)
-    hipLaunchKernelGGL((k_null_lev<cdouble, cdouble>), dim3(ncand, 1, nz), dim3(256), size_t(p.n) * sizeof(cdouble), st, (const cdouble*)A, lda, p.m,
+    hipLaunchKernelGGL((k_null_lev<cdouble, cdouble>), dim3(nblk(ncand, kLevRows), 1, nz), dim3(256), kLevRows * size_t(p.n) * sizeof(cdouble), st, (const cdouble*)A, lda, p.m,
                        p.n, center, mean, var, b.Wf, p.n, b.nnull, ncand, b.lev, b.urows, zb, zx);
   else
-    hipLaunchKernelGGL((k_null_lev<cdouble, cfloat>), dim3(ncand, 1, nz), dim3(256), size_t(p.n) * sizeof(cdouble), st, (const cfloat*)A, lda, p.m, p.n,
+    hipLaunchKernelGGL((k_null_lev<cdouble, cfloat>), dim3(nblk(ncand, kLevRows), 1, nz), dim3(256), kLevRows * size_t(p.n) * sizeof(cdouble), st, (const cfloat*)A, lda, p.m, p.n,
                        center, mean, var, b.Wf, p.n, b.nnull, ncand, b.lev, b.urows, zb, zx);
 }
 
@@ -1065,24 +1085,22 @@ static int launch_streams(pc_ctx* ctx, const Plan& p, const void* A, int64_t lda
 template <class T>
 static void reduce_gram(hipStream_t st, const Plan& p, const double* part, int nparts, T* G, int nz = 1,
                         int64_t zb = 0);
-// the chunk partials are summed in place into chunk 0 (k_reduce_slab), then
-// chunk 0 is unpacked into the symmetric / Hermitian n x n Gram
-static void reduce_slab(hipStream_t st, const Plan& p, const double* part, int nparts, int nz, int64_t zb) {
+// the chunk partials are summed into the symmetric n x n Gram, or in place into chunk 0
+// (k_reduce_slab), which is then folded into the Hermitian one
+static void reduce_slab(hipStream_t st, const Plan& p, const double* part, int nparts, double* G, int nz, int64_t zb) {
   const int64_t e = int64_t(p.NB) * p.NB;
   hipLaunchKernelGGL(k_reduce_slab<true>, dim3(unsigned(ceil_div(e, 64)), 1, nz), dim3(1024), 0, st,
-                     const_cast<double*>(part), nparts, e, p.NB, p.nr, p.nr, zb);
+                     const_cast<double*>(part), nparts, e, p.NB, p.nr, p.nr, G, zb);
 }
 template <>
 void reduce_gram<double>(hipStream_t st, const Plan& p, const double* part, int nparts, double* G, int nz,
                          int64_t zb) {
-  reduce_slab(st, p, part, nparts, nz, zb);
-  hipLaunchKernelGGL(k_reduce_gram_real, dim3(nblk(int64_t(p.n) * p.n), 1, nz), dim3(256), 0, st, part, 1,
-                     int64_t(p.NB) * p.NB, p.NB, p.n, G, p.n, zb);
+  reduce_slab(st, p, part, nparts, G, nz, zb);  // batched solves are complex only: nz = 1
 }
 template <>
 void reduce_gram<cdouble>(hipStream_t st, const Plan& p, const double* part, int nparts, cdouble* G, int nz,
                           int64_t zb) {
-  reduce_slab(st, p, part, nparts, nz, zb);
+  reduce_slab(st, p, part, nparts, nullptr, nz, zb);
   hipLaunchKernelGGL(k_reduce_gram_cplx, dim3(nblk(int64_t(p.n) * p.n), 1, nz), dim3(256), 0, st, part, 1,
                      int64_t(p.NB) * p.NB, p.NB, p.n, G, p.n, zb);
 }
