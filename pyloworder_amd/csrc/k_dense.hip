@@ -921,13 +921,15 @@ __global__ __launch_bounds__(256) void k_hqr_rq(int n, const double* __restrict_
 // The chain of a step is two lane reads and four FMAs (125 cycles): the row block
 // that holds r_i is known when the code is compiled and rows at or below i, which
 // nothing reads again, are updated with the others, so no selection or mask is in it.
+// rank: R's rows from rank[0] on are zero and count as the identity's.
 template <int C>
 __global__ __launch_bounds__(256) void k_trinv_cols(const double* __restrict__ R, int ldr, int n,
-                                                    double* __restrict__ W, int ldw) {
+                                                    const int* __restrict__ rank, double* __restrict__ W, int ldw) {
   constexpr int ST = C <= 4 ? 64 : 32, LD = ST + 1, PER = 64 / ST;
   __shared__ double Rs[64 * C * LD];
   const int jw = n - 1 - 4 * int(blockIdx.x);  // the workgroup's last column; the longest go first
   const int j = jw - int(threadIdx.x >> 6), l = threadIdx.x & 63;
+  const int rk0 = rank ? rank[0] : n;
   double r[C], w[C];
 #pragma unroll
   for (int q = 0; q < C; q++) {
@@ -940,7 +942,7 @@ __global__ __launch_bounds__(256) void k_trinv_cols(const double* __restrict__ R
     for (int h = PER - 1; h >= 0; h--) {
       const int c0 = 64 * g + ST * h;
       if (c0 > jw) continue;
-      // always whole stretches (a constant trip count): below row j (i > j) the
+      // eight steps at a time up to the workgroup's last column: below row j (i > j) the
       // right-hand side is zero and the diagonal counts as 1, so those steps do nothing
       const int cl = j - c0 < ST - 1 ? j - c0 : ST - 1;
       __syncthreads();  // the previous stretch has been read
@@ -967,21 +969,23 @@ __global__ __launch_bounds__(256) void k_trinv_cols(const double* __restrict__ R
       // step, q0 + (r - d q0) y (the last step of Newton-Markstein division),
       // so the division leaves the step's dependency chain.
       const int ld = l % ST;
-      const double dgl = ld <= cl ? Rs[(c0 + ld) * LD + ld] : 1.0;
+      const double dgl = ld <= cl && c0 + ld < rk0 ? Rs[(c0 + ld) * LD + ld] : 1.0;
       const double dl = 1.0 / dgl;
-#pragma unroll 8
-      for (int t = ST - 1; t >= 0; --t) {
-        double rk[C];
+      for (int t8 = min(jw - c0, ST - 1) & ~7; t8 >= 0; t8 -= 8) {
 #pragma unroll
-        for (int q = 0; q <= g; q++) rk[q] = Rs[(l + 64 * q) * LD + t];
-        const int tl = ST * h + t;  // the lane of row c0 + t
-        const double rt = dense::lane_read_f64(r[g], tl), d = dense::lane_read_f64(dgl, t),
-                     y = dense::lane_read_f64(dl, t);
-        const double q0 = rt * y;
-        const double wi = fma(fma(-d, q0, rt), y, q0);
-        w[g] = l == tl ? wi : w[g];
+        for (int t = t8 + 7; t >= t8; --t) {
+          double rk[C];
 #pragma unroll
-        for (int q = 0; q <= g; q++) r[q] = fma(-rk[q], wi, r[q]);
+          for (int q = 0; q <= g; q++) rk[q] = Rs[(l + 64 * q) * LD + t];
+          const int tl = ST * h + t;  // the lane of row c0 + t
+          const double rt = dense::lane_read_f64(r[g], tl), d = dense::lane_read_f64(dgl, t),
+                       y = dense::lane_read_f64(dl, t);
+          const double q0 = rt * y;
+          const double wi = fma(fma(-d, q0, rt), y, q0);
+          w[g] = l == tl ? wi : w[g];
+#pragma unroll
+          for (int q = 0; q <= g; q++) r[q] = fma(-rk[q], wi, r[q]);
+        }
       }
     }
   if (j < 0) return;

@@ -208,15 +208,19 @@ void run_chol_shift(hipStream_t st, const T* G, int n, double shift, T* R, int* 
   hipLaunchKernelGGL((k_chol_shift<T>), dim3(1, 1, nz), dim3(NT), 0, st, G, n, n, shift, R, n, status, zb,
                      (const int*)nullptr);
 }
+// rank: the rows of R from rank[0] on are zero and get a unit diagonal (in R, or in effect)
 template <class T>
-void run_trinv(hipStream_t st, const T* R, int n, T* W, int nz = 1, int64_t zb = 0) {
+__global__ void k_pad_identity(T* R, int ldr, int n, const int* rank, int64_t zb);
+template <class T>
+void run_trinv(hipStream_t st, T* R, int n, const int* rank, T* W, int nz = 1, int64_t zb = 0) {
   if constexpr (std::is_same<T, double>::value)
     if (use_fast<T>(n, nz)) {
       with_cols(n, [&](auto c) {
-        hipLaunchKernelGGL(k_trinv_cols<decltype(c)::value>, dim3(unsigned(ceil_div(n, 4))), dim3(256), 0, st, R, n, n, W, n);
+        hipLaunchKernelGGL(k_trinv_cols<decltype(c)::value>, dim3(unsigned(ceil_div(n, 4))), dim3(256), 0, st, (const T*)R, n, n, rank, W, n);
       });
       return;
     }
+  if (rank) hipLaunchKernelGGL((k_pad_identity<T>), dim3(1, 1, nz), dim3(256), 0, st, R, n, n, rank, zb);
   if (use_mw(n, nz)) {  // columns spread over the workgroups
     hipLaunchKernelGGL((k_trinv_upper<T>), dim3(unsigned(ceil_div(n, NT / 64))), dim3(NT), 0, st, R, n, n, W, n,
                        int64_t(0));
@@ -891,7 +895,7 @@ __global__ __launch_bounds__(256) void k_null_fix(const int* nnull, int64_t m, i
 
 // set unit diagonal on the rows >= rank (keeps R2 invertible)
 template <class T>
-__global__ void k_pad_identity(T* R, int ldr, int n, const int* rank, int64_t zb = 0) {
+__global__ void k_pad_identity(T* R, int ldr, int n, const int* rank, int64_t zb) {
   R = zoff(R, zb);
   rank = zoff(rank, zb);
   int r = rank[0];
@@ -1329,12 +1333,12 @@ static int core_t(pc_ctx* ctx, const Plan& p, const void* A, int64_t lda, int ce
   reduce_gram<T>(st, p, part, p.nparts, b.G1);
   // rank[1] / rank[2]: state words of the multi-workgroup factorisations
   run_chol_shift<T>(st, b.G1, n, p.mixed ? kShiftMx : kShiftF64, b.R1, b.status, 1, 0, b.Awk, b.dsc, b.rank + 2);
-  run_trinv<T>(st, b.R1, n, b.W1);
+  run_trinv<T>(st, b.R1, n, nullptr, b.W1);
   to_operand<T>(st, p, b.W1, n, b, false);
   if (p.mixed) rounded_back<T>(st, p, b, b.W1);  // W1 := the operand actually applied
   // (W1^-1 stays on the main stream: beside P2 its workgroups, with
   // 133 KB of LDS each, would take whole CUs from P2)
-  run_trinv<T>(st, b.W1, n, b.R1h);
+  run_trinv<T>(st, b.W1, n, nullptr, b.R1h);
   SideWork side(ctx, st);
   // ---- P2
   if (p.wide && !b.Zw) {  // FP64 storage: Z lives in U until P3 overwrites it
@@ -1353,10 +1357,9 @@ static int core_t(pc_ctx* ctx, const Plan& p, const void* A, int64_t lda, int ce
   // exact centring is M <- M C
   if (p.mixed && center)
     hipLaunchKernelGGL((k_center_right<T>), dim3(nblk(n, 16)), dim3(256), 0, st, b.Hc, n, n);
-  hipLaunchKernelGGL((k_pad_identity<T>), dim3(1), dim3(256), 0, st, b.R2, n, n, b.rank);
   // R2i = R2^-1 is read first in W, after the Jacobi: it runs beside the
   // preconditioner and the Jacobi (no kernel between writes R2 or R2i)
-  run_trinv<T>(side.fork(), b.R2, n, b.R2i);
+  run_trinv<T>(side.fork(), b.R2, n, b.rank, b.R2i);
   if (mode == CORE_RAND) {
     side.join();
     if constexpr (std::is_same<T, double>::value && std::is_same<ST, float>::value)
@@ -1519,10 +1522,10 @@ static int core_batch_t(pc_ctx* ctx, const Plan& p, const pc_problem* pr, int64_
   PC_CHECK(ctx, launch_streams<T>(ctx, p, pr[0].A, lda, center, mean, var, part, b, 1, pb));
   reduce_gram<T>(st, p, part, p.nparts, b.G1, nz, zb);
   run_chol_shift<T>(st, b.G1, n, p.mixed ? kShiftMx : kShiftF64, b.R1, b.status, nz, zb);
-  run_trinv<T>(st, b.R1, n, b.W1, nz, zb);
+  run_trinv<T>(st, b.R1, n, nullptr, b.W1, nz, zb);
   to_operand<T>(st, p, b.W1, n, b, false, nz, zb);
   if (p.mixed) rounded_back<T>(st, p, b, b.W1, nz, zb);
-  run_trinv<T>(st, b.W1, n, b.R1h, nz, zb);
+  run_trinv<T>(st, b.W1, n, nullptr, b.R1h, nz, zb);
   // ---- P2
   PC_CHECK(ctx, launch_streams<T>(ctx, p, pr[0].A, lda, center, mean, var, part, b, 2, pb));
   reduce_gram<T>(st, p, part, p.mixed ? p.chunks2 : p.chunks, b.G2, nz, zb);
@@ -1532,8 +1535,7 @@ static int core_batch_t(pc_ctx* ctx, const Plan& p, const pc_problem* pr, int64_
                      b.R1h, n, (const int*)b.perm, T(0.0), b.Hc, n, 1, zb);
   if (p.mixed && center)
     hipLaunchKernelGGL((k_center_right<T>), dim3(nblk(n, 16), 1, z), dim3(256), 0, st, b.Hc, n, n, zb);
-  hipLaunchKernelGGL((k_pad_identity<T>), dim3(1, 1, z), dim3(256), 0, st, b.R2, n, n, b.rank, zb);
-  run_trinv<T>(st, b.R2, n, b.R2i, nz, zb);
+  run_trinv<T>(st, b.R2, n, b.rank, b.R2i, nz, zb);
   launch_block_jacobi<T>(ctx, b.Hc, n, n, b.J, n, b.sig, b.jstate, b.jdstate, b.status,
                          p.mixed ? kJacTolMx : 0.0, nullptr, nullptr, nz, zb);
   hipLaunchKernelGGL(k_sort_desc, dim3(1, 1, z), dim3(1024), 0, st, b.sig, n, b.order, zb);
