@@ -31,7 +31,8 @@ namespace {
 
 constexpr int TR = 32;       // rows per tile
 constexpr int NTH = 512;     // threads per workgroup
-constexpr int NTG = 256;     // of a product
+// rows from which a product takes 64-row tiles: eight of them for each CU
+constexpr int64_t kTallProduct = 1 << 17;
 constexpr int NWV = NTH / 64;
 constexpr int PADD = 2;      // LDS row padding (doubles): rows 4 banks apart
 
@@ -245,14 +246,18 @@ __global__ __launch_bounds__(NTH) void k_zgram_f64(const TS* __restrict__ X, int
 }
 
 // Product C[m x nc] = Yc W, W (K rows up to a multiple of 16, zero beyond K; ld ldw).
-// 32-row tiles, the K columns in chunks of KC; blockIdx.y: slice of 256 columns.  Four
-// waves, two workgroups per CU: a wave's loads and stores complete in order, so W of
-// the next rows waits behind the next tile's rows and the last one's stores, and only
-// another workgroup fills that time.  Wave w forms both 16-row blocks of the column
-// blocks w + 4 i of the slice, so each element of W it loads feeds two products.
+// 16 NR-row tiles, the K columns in chunks of KC; blockIdx.y: slice of 256 columns.  A
+// wave's loads and stores complete in order, so W of the next rows waits behind the
+// next tile's rows and the last one's stores, and only other waves fill that time.
+// Wave w forms the NR 16-row blocks of the column blocks w + NW i of the slice, so each
+// element of W it loads from the L2 feeds NR products.  NR = 4 on eight waves, one
+// workgroup per CU, for tall inputs: half the traffic of W and half as many of those
+// waits per row (8M x 256 float64 62.1 -> 61.3 ms, 1M x 512 38.4 -> 37.2 ms for the
+// whole solves); NR = 2 on four waves, two workgroups per CU, where 64-row tiles would be
+// too few or the columns leave half of the waves idle.
 // upper: W is upper triangular with 16 x 16 blocks (block (kb, J) is zero for kb > J).
-template <class TS, class TO, int KC, bool VAR>
-__global__ __launch_bounds__(NTG) void k_gemm_f64(const TS* __restrict__ X, int64_t ldx, int64_t m, int K, int center,
+template <class TS, class TO, int KC, bool VAR, int NR, int NW>
+__global__ __launch_bounds__(64 * NW) void k_gemm_f64(const TS* __restrict__ X, int64_t ldx, int64_t m, int K, int center,
                                                   const double* mean_in, const double* var_in,
                                                   const double* __restrict__ W, int64_t ldw, int nc, int upper,
                                                   TO* __restrict__ C, int64_t ldc, int64_t zx, int64_t zb,
@@ -262,26 +267,26 @@ __global__ __launch_bounds__(NTG) void k_gemm_f64(const TS* __restrict__ X, int6
   var_in = zoff(var_in, zb);
   W = zoff(W, zb);
   C = zoff(C, zc);
-  constexpr int LD = KC + PADD;
-  __shared__ double S[TR * LD];
+  constexpr int LD = KC + PADD, TRG = 16 * NR, NI = 16 / NW, SH = NW == 8 ? 3 : 2;
+  __shared__ double S[TRG * LD];
   const int w = __builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6)), l = threadIdx.x & 63, kr = l >> 4, cc = l & 15;
   const int Jg = 16 * blockIdx.y + w;
   const int nkb = (K + 15) / 16, nch = (K + KC - 1) / KC;
   int nJ = 0;  // this wave's column blocks inside nc
 #pragma unroll
-  for (int i = 0; i < 4; i++) nJ += 16 * (Jg + 4 * i) < nc;
-  const int64_t ntl = ceil_div(m, TR);
-  RowStage<TS, TR, KC, VAR, NTG> st;
-  d4 acc[2][4];
+  for (int i = 0; i < NI; i++) nJ += 16 * (Jg + NW * i) < nc;
+  const int64_t ntl = ceil_div(m, TRG);
+  RowStage<TS, TRG, KC, VAR, 64 * NW> st;
+  d4 acc[NR][NI];
 #pragma unroll
-  for (int R = 0; R < 2; R++)
+  for (int R = 0; R < NR; R++)
 #pragma unroll
-    for (int i = 0; i < 4; i++) acc[R][i] = d4{0, 0, 0, 0};
+    for (int i = 0; i < NI; i++) acc[R][i] = d4{0, 0, 0, 0};
   int64_t t = blockIdx.x;
   int ch = 0;
-  if (t < ntl) st.fetch(X, ldx, m, K, t * TR, 0, center, mean_in, var_in);
+  if (t < ntl) st.fetch(X, ldx, m, K, t * TRG, 0, center, mean_in, var_in);
   while (t < ntl) {
-    st.template put<LD>(S, 0, m, K, t * TR, ch * KC, center, false, nullptr, nullptr);
+    st.template put<LD>(S, 0, m, K, t * TRG, ch * KC, center, false, nullptr, nullptr);
     const bool last = ch + 1 == nch;
     const int64_t tn = last ? t + gridDim.x : t;
     const int chn = last ? 0 : ch + 1;
@@ -291,21 +296,21 @@ __global__ __launch_bounds__(NTG) void k_gemm_f64(const TS* __restrict__ X, int6
     auto lo = [&](int kb) {
       if (!upper) return 0;
       const int d = kb0 + kb - Jg;
-      return d <= 0 ? 0 : (d + 3) >> 2;
+      return d <= 0 ? 0 : (d + NW - 1) >> SH;
     };
     // Unconditional (column blocks beyond the wave's last repeat it): were the loads
     // behind branches, their number would be unknown and the products of the current
     // rows would wait for the next ones'.
     auto load_w = [&](int kb, double (*b)[4]) {
 #pragma unroll
-      for (int i = 0; i < 4; i++)
+      for (int i = 0; i < NI; i++)
 #pragma unroll
         for (int kk = 0; kk < 4; kk++)
-          b[i][kk] = wl[int64_t(16 * kb + 4 * kk) * ldw + 64 * (i < nJ ? i : nJ - 1)];
+          b[i][kk] = wl[int64_t(16 * kb + 4 * kk) * ldw + 16 * NW * (i < nJ ? i : nJ - 1)];
     };
-    double wc[4][4], wn[4][4];
+    double wc[NI][4], wn[NI][4];
     if (nJ > 0) load_w(0, wc);
-    st.fetch(X, ldx, m, K, (tn < ntl ? tn : t) * TR, chn * KC, center, mean_in, var_in);
+    st.fetch(X, ldx, m, K, (tn < ntl ? tn : t) * TRG, chn * KC, center, mean_in, var_in);
     lds_barrier();
 #pragma unroll 1
     for (int kb = 0; nJ > 0 && kb < kb1; kb++) {
@@ -313,39 +318,39 @@ __global__ __launch_bounds__(NTG) void k_gemm_f64(const TS* __restrict__ X, int6
       if (from >= nJ) break;  // every later block is zero too
       load_w(kb + 1 < kb1 ? kb + 1 : kb, wn);
       const double* sr = S + cc * LD + 16 * kb + kr;
-      double x[2][4];
+      double x[NR][4];
 #pragma unroll
-      for (int R = 0; R < 2; R++)
+      for (int R = 0; R < NR; R++)
 #pragma unroll
         for (int kk = 0; kk < 4; kk++) x[R][kk] = sr[16 * R * LD + 4 * kk];
 #pragma unroll
-      for (int i = 0; i < 4; i++)
+      for (int i = 0; i < NI; i++)
         if (i < nJ && i >= from) {
 #pragma unroll
           for (int kk = 0; kk < 4; kk++)
 #pragma unroll
-            for (int R = 0; R < 2; R++) acc[R][i] = mfma64(x[R][kk], wc[i][kk], acc[R][i]);
+            for (int R = 0; R < NR; R++) acc[R][i] = mfma64(x[R][kk], wc[i][kk], acc[R][i]);
         }
 #pragma unroll
-      for (int i = 0; i < 4; i++)
+      for (int i = 0; i < NI; i++)
 #pragma unroll
         for (int kk = 0; kk < 4; kk++) wc[i][kk] = wn[i][kk];
     }
     if (last) {
-      TO* ct = C + (t * TR + kr) * ldc + 16 * Jg + cc;
-      const bool whole = (t + 1) * TR <= m && 16 * (Jg + 4 * (nJ - 1) + 1) <= nc;  // no edge in the wave's blocks
+      TO* ct = C + (t * TRG + kr) * ldc + 16 * Jg + cc;
+      const bool whole = (t + 1) * TRG <= m && 16 * (Jg + NW * (nJ - 1) + 1) <= nc;  // no edge in the wave's blocks
 #pragma unroll
-      for (int i = 0; i < 4; i++) {
-        const int col = 16 * (Jg + 4 * i) + cc;
+      for (int i = 0; i < NI; i++) {
+        const int col = 16 * (Jg + NW * i) + cc;
 #pragma unroll
-        for (int R = 0; R < 2; R++) {
+        for (int R = 0; R < NR; R++) {
           if (i < nJ && whole) {
 #pragma unroll
-            for (int r = 0; r < 4; r++) ct[(16 * R + 4 * r) * ldc + 64 * i] = TO(acc[R][i][r]);
+            for (int r = 0; r < 4; r++) ct[(16 * R + 4 * r) * ldc + 16 * NW * i] = TO(acc[R][i][r]);
           } else if (i < nJ) {
 #pragma unroll
             for (int r = 0; r < 4; r++)
-              if (t * TR + 16 * R + 4 * r + kr < m && col < nc) ct[(16 * R + 4 * r) * ldc + 64 * i] = TO(acc[R][i][r]);
+              if (t * TRG + 16 * R + 4 * r + kr < m && col < nc) ct[(16 * R + 4 * r) * ldc + 16 * NW * i] = TO(acc[R][i][r]);
           }
           acc[R][i] = d4{0, 0, 0, 0};
         }
@@ -514,9 +519,13 @@ static int launch_gemm_t(hipStream_t st, const TS* X, int64_t ldx, int64_t m, in
     if constexpr (KC > kDirectProduct) {
       with_var(center, [&](auto vc) {
         constexpr bool VAR = decltype(vc)::value;
-        hipLaunchKernelGGL((k_gemm_f64<TS, TO, KC, VAR>),
-                           dim3(unsigned(chunks), unsigned(ceil_div(nc, 256)), unsigned(bz.nz)), dim3(NTG), 0, st, X,
-                           ldx, m, n, center, mean_in, var_in, W, ldw, nc, upper, C, ldc, bz.zx, bz.zb, bz.zc);
+        const dim3 g(unsigned(chunks), unsigned(ceil_div(nc, 256)), unsigned(bz.nz));
+        if (nc > 128 && m >= kTallProduct)
+          hipLaunchKernelGGL((k_gemm_f64<TS, TO, KC, VAR, 4, 8>), g, dim3(512), 0, st, X, ldx, m, n, center, mean_in,
+                             var_in, W, ldw, nc, upper, C, ldc, bz.zx, bz.zb, bz.zc);
+        else
+          hipLaunchKernelGGL((k_gemm_f64<TS, TO, KC, VAR, 2, 4>), g, dim3(256), 0, st, X, ldx, m, n, center, mean_in,
+                             var_in, W, ldw, nc, upper, C, ldc, bz.zx, bz.zb, bz.zc);
       });
       return 0;
     }
