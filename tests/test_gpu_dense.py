@@ -76,3 +76,23 @@ def test_eig_sizes(n, kind):
     assert np.abs(np.linalg.norm(V, axis=0) - 1).max() <= 1e-13
     if kind == "rotations":
         assert np.abs(np.abs(w) - 1).max() <= tol and (np.abs(wi) > 0.1).sum() == 2 * (n // 2)
+
+
+@pytest.mark.parametrize("missing", [1, 2, 4, 5])
+@pytest.mark.parametrize("dtype", [np.float64, np.complex128])
+def test_few_null_directions(missing, dtype):
+    """Completion of U where a wave forms each sum (up to four directions) and where a thread does."""
+    rng = np.random.default_rng(missing)
+    n, m = 40, 300
+    k = n - missing
+
+    def orth(r, c):
+        z = rng.standard_normal((r, c)) + (1j * rng.standard_normal((r, c)) if dtype is np.complex128 else 0)
+        return np.linalg.qr(z)[0]
+
+    s = np.linspace(2.0, 1.0, k)
+    A = (orth(m, k) * s) @ orth(n, k).conj().T
+    U, S, VT = (x.cpu().numpy() for x in pl.math.tsqr_svd(torch.from_numpy(A).cuda()))
+    tol = 1e-13 * n
+    assert np.abs(S[:k] - s).max() <= tol and S[k:].max() <= tol
+    assert np.abs(U.conj().T @ U - np.eye(n)).max() <= tol and np.abs((U * S) @ VT - A).max() <= tol
