@@ -1,5 +1,5 @@
-// Small dense factorisations of wide problems (n > 256) spread over the GPU:
-// one launch per elimination step, the step's updates spread over many
+// Small dense factorisations of wide problems (real n > 512, complex n > 128) spread
+// over the GPU: one launch per elimination step, the step's updates spread over many
 // workgroups (one wave per row or column).  The single-workgroup kernels of
 // k_small.hip serialise every step on one CU, which costs seconds at
 // n = 1000; here a step costs one launch and its share of L2 bandwidth.
