@@ -561,7 +561,7 @@ int dxgram_t(hipStream_t st, const TS* A, int64_t lda, int p, const TS* B, int64
 
 }  // namespace
 
-// Row chunks of the direct Grams, from m and the columns alone; *tpc: turns of 32
+// Row chunks of the direct Grams (at least one: of no rows it writes zeros), from m and the columns alone; *tpc: turns of 32
 // rows (up to 32 columns, one wave per chunk) or of 128 (at most 512 chunks, two
 // workgroups per CU, of at least 256 rows: a 64-column slab is 32 KB to write and sum)
 int d64_gram_chunks(int64_t m, int n, int64_t* tpc) {
@@ -575,7 +575,7 @@ int d64_gram_chunks(int64_t m, int n, int64_t* tpc) {
     if (per < 2) per = 2;
   }
   *tpc = per;
-  return int(ceil_div(tiles, per));
+  return tiles < 1 ? 1 : int(ceil_div(tiles, per));
 }
 // Workgroups of the direct product: enough to fill the CUs at the LDS its W takes,
 // no more than there are turns of work.
@@ -585,7 +585,7 @@ int d64_gemm_chunks(int64_t m, int n, int nc) {
   const int64_t lds = int64_t(kb) * 8 * (nc <= 16 ? 16 : nc <= 32 ? 32 : nc <= 64 ? 64 : nc <= 128 || n > 64 ? 128 : 256);
   const int64_t fit = lds > 80 * 1024 ? 1 : lds > 40 * 1024 ? 2 : 4;
   const int64_t want = 256 * fit;
-  return int(turns < want ? turns : want);
+  return turns < 1 ? 1 : int(turns < want ? turns : want);
 }
 
 // row chunks of the direct cross products, turns of 128 rows

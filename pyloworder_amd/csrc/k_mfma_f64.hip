@@ -460,7 +460,7 @@ int f64_gram_chunks(int64_t m, int n, int64_t* tpc) {
   int64_t per = ceil_div(tiles, 512);
   if (per < 4) per = 4;
   *tpc = per;
-  return int(ceil_div(tiles, per));
+  return tiles < 1 ? 1 : int(ceil_div(tiles, per));
 }
 // cross products take the direct kernel when both operands are narrow
 int f64_xgram_chunks(int64_t m, int p, int q, int64_t* tpc) {
@@ -474,7 +474,7 @@ int f64_gemm_rows(int n) { return n > kDirectProduct ? TR : n > 64 ? 128 : 256; 
 int f64_gemm_chunks(int64_t m, int n, int nc) {
   if (n <= kDirectProduct) return d64_gemm_chunks(m, n, nc);
   const int64_t tiles = ceil_div(m, TR);
-  return int(tiles < 512 ? tiles : 512);
+  return tiles < 1 ? 1 : int(tiles < 512 ? tiles : 512);
 }
 
 // P1 / P2 launchers -----------------------------------------------------------
