@@ -109,9 +109,10 @@ __global__ __launch_bounds__(256) void k_spod_blocks(const float* __restrict__ X
   }
 }
 
-constexpr int kFftPad = 4;  // complex values between the rows of blocks: other banks for the same frequency
+// complex values between the rows of blocks: other banks for the same frequency
+constexpr int fft_pad(int64_t N) { return N > 2 ? 4 : 0; }
 
-// Power-of-two nDFT >= 4: Stockham FFT in LDS.  A workgroup owns one row
+// Power-of-two nDFT >= 2: Stockham FFT in LDS.  A workgroup owns one row
 // pair and runs through the blocks in chunks of BC; rows a, b form one
 // complex sequence z = y_a + i y_b, and after the FFT Z the two real spectra
 // are
@@ -122,24 +123,29 @@ constexpr int kFftPad = 4;  // complex values between the rows of blocks: other 
 // so two are taken at a time: butterflies j and j + N/4 of stage m feed 2j - k and
 // 2j - k + m of stage 2m, the same operations on four values in registers.  The first
 // two take the samples from the registers they were fetched into, and their twiddles
-// are 1 and -i; a last stage is left when log2 N is odd.  Twiddles
+// are 1 and -i; a last stage is left when log2 N is odd, and of N = 2 the first stage is
+// all there is (TWO; 20,000 x 1024 takes 5.2 ms in the direct kernel, whose workgroups
+// hold one block of a few rows, and 0.17 here).  Twiddles
 // w^q = exp(-2 pi i q / N) come from the FP64-accurate tables.  The
 // spectra of a chunk are staged in LDS as [f][row][block], so that each
 // frequency's two rows leave as one contiguous run Q[f][ra][b0..b1),
 // Q[f][ra+1][b0..b1) (consecutive rows are adjacent in Q).
 // 200,000 x 2048, nDFT = 256: 3.85 ms with a pass over LDS per stage and divided
 // indices, now 2.2.
+template <bool TWO>
 __global__ __launch_bounds__(256) void k_spod_fft(const float* __restrict__ X, int64_t ldx, int64_t M,
                                                   const double* __restrict__ mean, const float* __restrict__ win,
                                                   const float* __restrict__ twc, const float* __restrict__ tws,
                                                   int nDFT, int logN, int step, int nBlks, int nf, int BC, int P,
                                                   const float* __restrict__ fscale, float2* __restrict__ Q) {
   extern __shared__ float2 fsm[];
-  const int N = nDFT, Q4 = N >> 2, NS = N + kFftPad;
+  const int N = nDFT, NS = N + (TWO ? 0 : fft_pad(4));
+  constexpr int IN = TWO ? 2 : 4;  // inputs of a first butterfly, Q4 apart
+  const int Q4 = TWO ? 1 : N >> 2;
   float2* A = fsm;              // [P][NS]: P blocks transformed side by side
   float2* B = A + P * NS;       // [P][NS]
   float2* tw = B + P * NS;      // [N / 2]
-  float2* stg = tw + 2 * Q4;    // [nf][2][BC]
+  float2* stg = tw + (N >> 1);  // [nf][2][BC]
   // Row pairs are split into 8 contiguous ranges, one per XCD (workgroup x
   // runs on XCD x mod 8), so neighbouring pairs, whose output runs share
   // cache lines, are written through the same L2.
@@ -149,13 +155,13 @@ __global__ __launch_bounds__(256) void k_spod_fft(const float* __restrict__ X, i
   const int64_t ra = pair * 2, rb = ra + 1;
   const bool va = ra < M, vb = rb < M;
   const double mua = (mean && va) ? mean[ra] : 0.0, mub = (mean && vb) ? mean[rb] : 0.0;
-  for (int q = threadIdx.x; q < 2 * Q4; q += 256) tw[q] = make_float2(twc[q], -tws[q]);
+  for (int q = threadIdx.x; q < N >> 1; q += 256) tw[q] = make_float2(twc[q], -tws[q]);
   const float *rowa = X + (va ? ra : 0) * ldx, *rowb = X + (vb ? rb : 0) * ldx;
   // Samples of the next pass are fetched into registers while the current pass is
   // transformed: the four inputs of at most BF first butterflies per thread
   constexpr int BF = 2;
-  float xa[BF][4], xb[BF][4];
-  const int lq = logN - 2;
+  float xa[BF][IN], xb[BF][IN];
+  const int lq = TWO ? 0 : logN - 2;
   auto fetch = [&](int gb, int np) {
 #pragma unroll
     for (int u = 0; u < BF; u++) {
@@ -163,7 +169,7 @@ __global__ __launch_bounds__(256) void k_spod_fft(const float* __restrict__ X, i
       if (jj < np << lq) {
         const int64_t t0 = int64_t(gb + (jj >> lq)) * step + (jj & (Q4 - 1));
 #pragma unroll
-        for (int r = 0; r < 4; r++) {
+        for (int r = 0; r < IN; r++) {
           xa[u][r] = va ? rowa[t0 + r * Q4] : 0.0f;
           xb[u][r] = vb ? rowb[t0 + r * Q4] : 0.0f;
         }
@@ -186,21 +192,26 @@ __global__ __launch_bounds__(256) void k_spod_fft(const float* __restrict__ X, i
         const int jj = threadIdx.x + u * 256;
         if (jj < np << lq) {
           const int j = jj & (Q4 - 1);
-          float2 x[4];
+          float2 x[IN];
 #pragma unroll
-          for (int r = 0; r < 4; r++) {
+          for (int r = 0; r < IN; r++) {
             const float wn = win[j + r * Q4];
             x[r] = make_float2(float(double(xa[u][r]) - mua) * wn, float(double(xb[u][r]) - mub) * wn);
             // rounded: the sums below must not contract with the window's products
             asm volatile("" : "+v"(x[r].x), "+v"(x[r].y));
           }
-          const float2 u0 = add(x[0], x[2]), u1 = sub(x[0], x[2]), v0 = add(x[1], x[3]), v = sub(x[1], x[3]);
-          const float2 v1 = make_float2(v.y, -v.x);  // -i v
-          float2* d = A + (jj >> lq) * NS + 4 * j;
-          d[0] = add(u0, v0);
-          d[1] = add(u1, v1);
-          d[2] = sub(u0, v0);
-          d[3] = sub(u1, v1);
+          float2* d = A + (jj >> lq) * NS + IN * j;
+          if constexpr (TWO) {
+            d[0] = add(x[0], x[1]);
+            d[1] = sub(x[0], x[1]);
+          } else {
+            const float2 u0 = add(x[0], x[2]), u1 = sub(x[0], x[2]), v0 = add(x[1], x[3]), v = sub(x[1], x[3]);
+            const float2 v1 = make_float2(v.y, -v.x);  // -i v
+            d[0] = add(u0, v0);
+            d[1] = add(u1, v1);
+            d[2] = sub(u0, v0);
+            d[3] = sub(u1, v1);
+          }
         }
       }
       __syncthreads();
@@ -214,7 +225,7 @@ __global__ __launch_bounds__(256) void k_spod_fft(const float* __restrict__ X, i
       }
       float2* src = A;
       float2* dst = B;
-      int lm = 2;
+      int lm = TWO ? 1 : 2;
       for (; lm + 2 <= logN; lm += 2) {
         const int m = 1 << lm, ts = logN - 2 - lm;  // twiddle stride N / 4m
         for (int jj = threadIdx.x; jj < np << lq; jj += 256) {
@@ -395,14 +406,14 @@ extern "C" int pc_spod_blocks(pc_ctx* ctx, const float* X, int64_t ldx, int64_t 
   // 256 threads all have two stages' butterflies of four values), twiddles (N / 2) and
   // the staging of BC
   // blocks' spectra (nf x 2 x BC complex), kept within 64 KB
-  if (pow2 && nDFT >= 4 && nDFT <= 2048) {
+  if (pow2 && nDFT >= 2 && nDFT <= 2048) {
     int64_t P = nDFT >= 1024 ? 1 : 1024 / nDFT;
     P = P > nBlks ? nBlks : P;
-    const int64_t fixed = (2 * P * (nDFT + kFftPad) + nDFT / 2) * int64_t(sizeof(float2));
+    const int64_t fixed = (2 * P * (nDFT + fft_pad(nDFT)) + nDFT / 2) * int64_t(sizeof(float2));
     int64_t bc = (65536 - fixed) / (nf * 2 * int64_t(sizeof(float2)));
     bc = bc < 1 ? 1 : (bc > nBlks ? nBlks : bc);
     const size_t lds = size_t(fixed + nf * 2 * bc * int64_t(sizeof(float2)));
-    hipLaunchKernelGGL(k_spod_fft, dim3(unsigned(ceil_div(M, 2))), dim3(256), lds, st, X, ldx, M,
+    hipLaunchKernelGGL(nDFT == 2 ? k_spod_fft<true> : k_spod_fft<false>, dim3(unsigned(ceil_div(M, 2))), dim3(256), lds, st, X, ldx, M,
                        remove_mean ? mean : nullptr, win, twc, tws, int(nDFT), logN, int(step), int(nBlks), int(nf),
                        int(bc), int(P), fsc, (float2*)Q);
   }

@@ -22,3 +22,15 @@ def test_lengths(ndft, rows, blocks):
     Q, f, nb = pl.SPOD.blocks(X, t, ndft, nolap)
     assert nb == nbo == blocks and np.array_equal(f, fo) and Q.shape == Qo.shape
     assert np.abs(Q - Qo).max() <= 2e-6 * np.abs(Qo).max() * np.sqrt(Qo.shape[2])
+
+
+@pytest.mark.parametrize("rows,n", [(1, 2), (7, 300), (18, 1024), (5, 1999)])
+def test_length_two(rows, n):
+    """The shortest transform, y0 +- y1: one block to several chunks of them, same bounds."""
+    rng = np.random.default_rng(n)
+    t = 0.01 * np.arange(n)
+    X = (rng.standard_normal((rows, n)) + 50.0).astype(np.float32)
+    Qo, fo, nbo = oracle.spod_blocks(X.astype(np.float64), t, 2, 1)
+    Q, f, nb = pl.SPOD.blocks(X, t, 2, 1)
+    assert nb == nbo == n - 1 and np.array_equal(f, fo) and Q.shape == Qo.shape
+    assert np.abs(Q - Qo).max() <= 2e-6 * np.abs(Qo).max() * np.sqrt(Qo.shape[2])
