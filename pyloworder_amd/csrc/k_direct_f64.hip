@@ -27,6 +27,7 @@
 #include "common.hpp"
 #include "f64_common.hpp"
 #include "kernels.hpp"
+#include <algorithm>
 
 namespace {
 
@@ -228,10 +229,20 @@ PC_DEV void afrag_values(const TS* x, double* a, int n, bool rv, int center, dou
 // 4 V (st / V) + V g + st % V, column col0 + colmap(J, i); zero beyond n rows / ldw columns
 template <int KS, int NBL, int V, class Map>
 PC_DEV void stage_w(const double* __restrict__ W, int n, int ldw, int col0, double* Wl, Map colmap) {
-  for (int idx = threadIdx.x; idx < KS * NBL * 64; idx += DNT) {
-    const int lane = idx & 63, sj = idx >> 6, st = sj / NBL, J = sj - st * NBL;
-    const int k = 4 * V * (st / V) + V * (lane >> 4) + st % V, col = col0 + colmap(J, lane & 15);
-    Wl[idx] = k < n && col < ldw ? W[int64_t(k) * ldw + col] : 0.0;
+  constexpr int ALL = KS * NBL * 64, U = ALL / DNT < 16 ? (ALL + DNT - 1) / DNT : 16;
+  for (int i0 = threadIdx.x; i0 < ALL; i0 += U * DNT) {
+    double v[U];
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      const int idx = i0 + u * DNT, lane = idx & 63, sj = idx >> 6, st = sj / NBL, J = sj - st * NBL;
+      const int k = 4 * V * (st / V) + V * (lane >> 4) + st % V, col = col0 + colmap(J, lane & 15);
+      const bool in = idx < ALL && k < n && col < ldw;
+      v[u] = W[in ? int64_t(k) * ldw + col : 0];
+      v[u] = in ? v[u] : 0.0;
+    }
+#pragma unroll
+    for (int u = 0; u < U; u++)
+      if (ALL % (U * DNT) == 0 || i0 + u * DNT < ALL) Wl[i0 + u * DNT] = v[u];
   }
 }
 
@@ -324,30 +335,33 @@ __global__ __launch_bounds__(DNT) void k_dgemm_f64(const TS* __restrict__ X, int
   __shared__ double Wl[KS * nbl * 64];
   const int w = threadIdx.x >> 6, l = threadIdx.x & 63, i = l & 15, g = l >> 4;
   const int col0 = blockIdx.y * NCB;
-  stage_w<KS, nbl, V>(W, n, ldw, col0, Wl, [](int J, int j) { return 16 * CV * (J / CV) + CV * j + J % CV; });
   const int64_t step = int64_t(gridDim.x) * DNW * 16 * R;
   TS cur[R][KS] = {}, nxt[R][KS] = {};
   double mu[R] = {}, var[R], mu_n[R] = {}, var_n[R];
 #pragma unroll
   for (int q = 0; q < R; q++) var[q] = var_n[q] = 1.0;
-  auto load = [&](int64_t t, TS (*a)[KS], double* mu_, double* var_) {
+  auto load = [&](int64_t t, int n_, TS (*a)[KS], double* mu_, double* var_) {
 #pragma unroll
     for (int q = 0; q < R; q++) {
       const int64_t row = t + 16 * q + i, rc = row < m ? row : m - 1;
-      load_afrag<TS, KS, V>(X, ldx, n, row, m, a[q]);
+      load_afrag<TS, KS, V>(X, ldx, n_, row, m, a[q]);
       if (center) mu_[q] = mean_in[rc];
       if (center == 2) var_[q] = var_in[rc];
     }
   };
   int64_t t = (int64_t(blockIdx.x) * DNW + w) * 16 * R;
-  if (t < m) load(t, cur, mu, var);
+  if (t < m) load(t, n, cur, mu, var);
+  stage_w<KS, nbl, V>(W, n, ldw, col0, Wl, [](int J, int j) { return 16 * CV * (J / CV) + CV * j + J % CV; });
   __syncthreads();
   for (; t < m; t += step) {
-    if (t + step < m) load(t + step, nxt, mu_n, var_n);
+    // n anew each turn: the columns' clamps and masks, kept over the loop, spilled registers
+    int nn = n;
+    asm volatile("" : "+s"(nn));
+    if (t + step < m) load(t + step, nn, nxt, mu_n, var_n);
     double a[R][KS];
 #pragma unroll
     for (int q = 0; q < R; q++)
-      afrag_values<TS, KS, V>(cur[q], a[q], n, t + 16 * q + i < m, center, mu[q], var[q]);
+      afrag_values<TS, KS, V>(cur[q], a[q], nn, t + 16 * q + i < m, center, mu[q], var[q]);
 #pragma unroll 1
     for (int q0 = 0; q0 < nbl / CV; q0++) {
       if (col0 + 16 * CV * q0 >= nc) break;
@@ -356,18 +370,31 @@ __global__ __launch_bounds__(DNT) void k_dgemm_f64(const TS* __restrict__ X, int
       for (int q = 0; q < R; q++)
 #pragma unroll
         for (int u = 0; u < CV; u++) z[q][u] = d4{0, 0, 0, 0};
+      // X k-steps at a time, beyond 32 inputs their fragments read while the X before are
+      // multiplied (up to 32 HBM is the bound, and the registers keep rows in flight).  A
+      // branch round each step left every product waiting for its read: 500,000 x 128 by
+      // 128 x 128 float64 391 -> 315 us
+      constexpr int X = CV == 4 ? 2 : 4, AHEAD = KB > 32 ? 1 : 0;
       const double* wq = Wl + q0 * CV * 64 + l;
+      double b[1 + AHEAD][X][CV];
+      auto read = [&](int c) {
 #pragma unroll
-      for (int st = 0; st < KS; st++) {
-        if (4 * V * (st / V) < n) {
+        for (int x = 0; x < X; x++)
 #pragma unroll
-          for (int u = 0; u < CV; u++) {
-            const double b = wq[(st * nbl + u) * 64];
+          for (int u = 0; u < CV; u++) b[c & AHEAD][x][u] = wq[((X * c + x) * nbl + u) * 64];
+      };
+      if (AHEAD) read(0);
 #pragma unroll
-            for (int q = 0; q < R; q++) z[q][u] = mfma64(a[q][st], b, z[q][u]);
-          }
+      for (int c = 0; c < KS / X; c++)
+        if (16 * (X * c / 4) < n) {
+          if (!AHEAD || c + 1 < KS / X) read(c + AHEAD);
+#pragma unroll
+          for (int x = 0; x < X; x++)
+#pragma unroll
+            for (int u = 0; u < CV; u++)
+#pragma unroll
+              for (int q = 0; q < R; q++) z[q][u] = mfma64(a[q][X * c + x], b[c & AHEAD][x][u], z[q][u]);
         }
-      }
       const int col = col0 + 16 * CV * q0 + CV * i;
 #pragma unroll
       for (int q = 0; q < R; q++)
@@ -479,6 +506,37 @@ int with_vec(int v, F&& f) {
   return f(Int<1>{});
 }
 
+// K class, and row turns of the direct product over n inputs
+int gemm_k(int n) { return n <= 16 ? 16 : n <= 32 ? 32 : n <= 64 ? 64 : 128; }
+int64_t gemm_turns(int64_t m, int n) { return ceil_div(m, DNW * (n > 64 ? 16 : 32)); }
+// Workgroups per slice of s columns, one per CU: all slices side by side, or one after the
+// other where that is less work for the CU with the most of it (a last slice of few
+// columns leaves its workgroups idle beside the others).
+int64_t gemm_workgroups(int64_t turns, int nc, int s) {
+  const int64_t shared = std::max<int64_t>(1, 256 / ceil_div(nc, s));
+  return ceil_div(turns, 256) * nc < ceil_div(turns, shared) * s ? 256 : shared;
+}
+// Columns of W that a workgroup keeps in LDS: a power of two, at most 128 KB of it.  X is
+// read once per slice, so a tall product takes the widest; one of few rows takes the
+// narrowest of which every CU holds a workgroup at once (1024 x 128 by 128 x 256 float64:
+// 16 workgroups of 128 columns 44 us, 256 of 16 columns 20, where the call's launch is
+// what is left; 5000 rows: 36 us with 128, 23 with 64, 30 with 32, which take two rounds).
+int gemm_slice(int64_t m, int n, int nc) {
+  const int64_t turns = gemm_turns(m, n);
+  int most = n > 64 ? 128 : 256;
+  while (most > 16 && most / 2 >= nc) most /= 2;
+  auto slices = [&](int s) { return ceil_div(nc, s); };
+  if (turns * slices(most) > 256) {
+    // several turns each: half as many columns where that shortens the longest
+    // workgroup's work by a fifth and X, read once per slice, stays in the caches
+    auto work = [&](int s) { return ceil_div(turns, gemm_workgroups(turns, nc, s)) * s; };
+    const int half = most / 2;
+    return half >= 16 && 5 * work(half) <= 4 * work(most) && slices(half) * m * n * 8 <= (int64_t(128) << 20) ? half : most;
+  }
+  while (most > 16 && turns * slices(most / 2) <= 256) most /= 2;
+  return most;
+}
+
 template <class TS>
 int dgram_t(hipStream_t st, const TS* X, int64_t ldx, int64_t m, int n, int center, const double* mean_in,
             const double* var_in, double* mean_out, double* var_out, const double* W, int chunks, int64_t tpc,
@@ -526,10 +584,11 @@ int dgemm_t(hipStream_t st, const TS* X, int64_t ldx, int64_t m, int n, int cent
   };
   auto cols = [&](auto kc) {
     constexpr int KB = decltype(kc)::value;
-    if (nc <= 16) return go(kc, Int<16>{});
-    if (nc <= 32) return go(kc, Int<32>{});
-    if (nc <= 64) return go(kc, Int<64>{});
-    if (KB > 64 || nc <= 128) return go(kc, Int<128>{});
+    const int slice = gemm_slice(m, n, nc);
+    if (slice == 16) return go(kc, Int<16>{});
+    if (slice == 32) return go(kc, Int<32>{});
+    if (slice == 64) return go(kc, Int<64>{});
+    if (slice == 128) return go(kc, Int<128>{});
     if constexpr (KB <= 64) return go(kc, Int<256>{});
     return -1;
   };
@@ -577,15 +636,23 @@ int d64_gram_chunks(int64_t m, int n, int64_t* tpc) {
   *tpc = per;
   return tiles < 1 ? 1 : int(ceil_div(tiles, per));
 }
-// Workgroups of the direct product: enough to fill the CUs at the LDS its W takes,
-// no more than there are turns of work.
+// Workgroups of the direct product per column slice, no more than there are turns of work.
+// One per CU in all beyond 32 inputs, whose rows fill its registers: with more, waiting
+// for a CU, each took one or two turns with nothing loaded ahead and staged W for them
+// (250,000 x 64 by 64 x 64 float64: 977 workgroups 76 us, 256 workgroups 60).  Up to 32
+// inputs HBM bounds the pass, and as many as W's LDS allows keep more bytes in flight
+// (4M x 8 by 8 x 8: 137 us with one per CU, 107 with four), beyond 16 while each has four
+// turns (250,000 x 30 by 30 x 30: 33 us with one turn each, 27 with four).
 int d64_gemm_chunks(int64_t m, int n, int nc) {
-  const int64_t turns = ceil_div(m, DNW * (n > 64 ? 16 : 32));
-  const int kb = n <= 16 ? 16 : n <= 32 ? 32 : n <= 64 ? 64 : 128;
-  const int64_t lds = int64_t(kb) * 8 * (nc <= 16 ? 16 : nc <= 32 ? 32 : nc <= 64 ? 64 : nc <= 128 || n > 64 ? 128 : 256);
-  const int64_t fit = lds > 80 * 1024 ? 1 : lds > 40 * 1024 ? 2 : 4;
-  const int64_t want = 256 * fit;
-  return turns < 1 ? 1 : int(turns < want ? turns : want);
+  const int64_t turns = gemm_turns(m, n);
+  const int slice = gemm_slice(m, n, nc);
+  int64_t want = gemm_workgroups(turns, nc, slice);
+  if (n <= 32) {
+    const int64_t lds = int64_t(gemm_k(n)) * 8 * slice, fit = lds > 40 * 1024 ? 2 : 4;
+    const int64_t all = n <= 16 ? 256 * fit : std::min(256 * fit, std::max<int64_t>(256, ceil_div(turns, 4)));
+    want = std::max<int64_t>(1, all / ceil_div(nc, slice));
+  }
+  return turns < 1 ? 1 : int(std::min(turns, want));
 }
 
 // row chunks of the direct cross products, turns of 128 rows

@@ -1,0 +1,26 @@
+"""Products over at most 128 inputs at each way their rows and columns are dealt to workgroups: narrow slices of few
+rows, half slices, slices side by side and one after the other, W's staging in one part and in several, odd widths.
+Tolerances as in test_gpu_narrow.py: (K + 2) sqrt(K) 2^-53 for a product over K terms, 2^-24 more for float32 results.
+"""
+import numpy as np
+import pytest
+import torch
+
+import pyloworder_amd as pl
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
+@pytest.mark.parametrize("m,k,n", [(1024, 128, 256), (1100, 37, 19), (5003, 128, 999), (20011, 128, 256), (10007, 64, 131),
+                                   (60001, 100, 300), (60001, 101, 203), (70001, 16, 64), (70001, 30, 200),
+                                   (65537, 17, 16), (131073, 64, 64)])
+def test_products(m, k, n, dtype):
+    g = torch.Generator(device="cuda").manual_seed(m)
+    A = torch.randn((m, k), generator=g, device="cuda", dtype=dtype)
+    B = torch.randn((k, n), generator=g, device="cuda", dtype=dtype)
+    ref = A.double() @ B.double()
+    tol = (k + 2) * np.sqrt(k) * 2.0 ** -53 + (2.0 ** -24 if dtype == torch.float32 else 0.0)
+    for C in (pl.math.matmul(A, B), pl.POD.reconstruct(A, torch.ones(k, device="cuda", dtype=dtype), B)):
+        assert float((C.double() - ref).norm() / ref.norm()) <= tol
+        assert float((C.double() - ref).abs().max()) <= 8 * tol * float(ref.abs().max())
