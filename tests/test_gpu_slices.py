@@ -1,5 +1,6 @@
 """Products over at most 128 inputs at each way their rows and columns are dealt to workgroups: narrow slices of few
 rows, half slices, slices side by side and one after the other, W's staging in one part and in several, odd widths.
+Cross products around the numbers of chunks and of entries from which their slabs are summed otherwise.
 Tolerances as in test_gpu_narrow.py: (K + 2) sqrt(K) 2^-53 for a product over K terms, 2^-24 more for float32 results.
 """
 import numpy as np
@@ -24,3 +25,16 @@ def test_products(m, k, n, dtype):
     for C in (pl.math.matmul(A, B), pl.POD.reconstruct(A, torch.ones(k, device="cuda", dtype=dtype), B)):
         assert float((C.double() - ref).norm() / ref.norm()) <= tol
         assert float((C.double() - ref).abs().max()) <= 8 * tol * float(ref.abs().max())
+
+
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32, torch.complex128, torch.complex64])
+@pytest.mark.parametrize("m,k,n", [(200, 5, 3), (8192, 30, 30), (8193, 30, 30), (8193, 17, 64), (70000, 33, 20),
+                                   (9001, 70, 65), (9001, 256, 256), (9001, 257, 256)])
+def test_cross_products(m, k, n, dtype):
+    g = torch.Generator(device="cuda").manual_seed(m + k)
+    A = torch.randn((m, k), generator=g, device="cuda", dtype=dtype)
+    B = torch.randn((m, n), generator=g, device="cuda", dtype=dtype)
+    wide = torch.complex128 if dtype.is_complex else torch.float64
+    ref = A.to(wide).conj().t().contiguous() @ B.to(wide)
+    tol = (m + 2) * np.sqrt(m) * 2.0 ** -53 + (2.0 ** -24 if dtype in (torch.float32, torch.complex64) else 0.0)
+    assert float((pl.POD.project(A, B).to(wide) - ref).norm() / ref.norm()) <= 2 * tol
