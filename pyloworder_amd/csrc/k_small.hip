@@ -77,6 +77,7 @@ template <bool UPPER>
 __global__ __launch_bounds__(1024) void k_reduce_slab(double* P, int chunks, int64_t pstride, int ld, int rows,
                                                       int cols, double* G, int64_t zb = 0) {
   P = zoff(P, zb);
+  if (G) G = zoff(G, zb);
   __shared__ double red[16][65];
   const int le = threadIdx.x & 63, k = threadIdx.x >> 6;
   const int e = blockIdx.x * 64 + le;

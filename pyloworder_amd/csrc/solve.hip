@@ -1099,7 +1099,7 @@ static void reduce_slab(hipStream_t st, const Plan& p, const double* part, int n
 template <>
 void reduce_gram<double>(hipStream_t st, const Plan& p, const double* part, int nparts, double* G, int nz,
                          int64_t zb) {
-  reduce_slab(st, p, part, nparts, G, nz, zb);  // batched solves are complex only: nz = 1
+  reduce_slab(st, p, part, nparts, G, nz, zb);
 }
 template <>
 void reduce_gram<cdouble>(hipStream_t st, const Plan& p, const double* part, int nparts, cdouble* G, int nz,
