@@ -39,6 +39,9 @@ constexpr int DNW = DNT / 64;
 // workgroup about as much as 200 rows of 30 columns.)  Wider Grams have few chunks
 // of long rows, so 8 waves share one.
 constexpr int chunk_waves(int NB) { return NB <= 32 ? 1 : 8; }
+// Threads of those workgroups: with a chunk per wave, four of them, or a lone problem of
+// 1024 chunks has workgroups for half of the CUs only.
+constexpr int gram_threads(int NB) { return NB <= 32 ? 256 : DNT; }
 
 template <class TS, int V>
 PC_DEV void load_vec(const TS* p, TS* o) {
@@ -130,7 +133,7 @@ PC_DEV void load_rows(const TS* __restrict__ X, int64_t ldx, int n, int64_t base
 
 // P1: partial Gram of the (centred) rows of a chunk
 template <class TS, int NB, int V>
-__global__ __launch_bounds__(DNT) void k_dgram_f64(const TS* __restrict__ X, int64_t ldx, int64_t m, int n, int center,
+__global__ __launch_bounds__(gram_threads(NB)) void k_dgram_f64(const TS* __restrict__ X, int64_t ldx, int64_t m, int n, int center,
                                                    double* mean_out, double* var_out, int chunks, int64_t rpc,
                                                    double* __restrict__ part, int64_t zx, int64_t zb) {
   X = zoff(X, zx);
@@ -141,7 +144,7 @@ __global__ __launch_bounds__(DNT) void k_dgram_f64(const TS* __restrict__ X, int
   constexpr int WPC = chunk_waves(NB);
   __shared__ double red[WPC > 1 ? DNW * 2 * 256 : 1];
   const int w = threadIdx.x >> 6, l = threadIdx.x & 63, i = l & 15, g = l >> 4;
-  const int64_t chunk = int64_t(blockIdx.x) * (DNW / WPC) + w / WPC;
+  const int64_t chunk = int64_t(blockIdx.x) * (gram_threads(NB) / 64 / WPC) + w / WPC;
   if (WPC == 1 && chunk >= chunks) return;
   const int64_t row0 = chunk * rpc;
   const int64_t row1 = row0 + rpc < m ? row0 + rpc : m;
@@ -227,14 +230,14 @@ PC_DEV void afrag_values(const TS* x, double* a, int n, bool rv, int center, dou
 }
 // W (ld ldw) into LDS in B-fragment order: Wl[(st nbl + J) 64 + l] is row
 // 4 V (st / V) + V g + st % V, column col0 + colmap(J, i); zero beyond n rows / ldw columns
-template <int KS, int NBL, int V, class Map>
+template <int NTHR, int KS, int NBL, int V, class Map>
 PC_DEV void stage_w(const double* __restrict__ W, int n, int ldw, int col0, double* Wl, Map colmap) {
-  constexpr int ALL = KS * NBL * 64, U = ALL / DNT < 16 ? (ALL + DNT - 1) / DNT : 16;
-  for (int i0 = threadIdx.x; i0 < ALL; i0 += U * DNT) {
+  constexpr int ALL = KS * NBL * 64, U = ALL / NTHR < 16 ? (ALL + NTHR - 1) / NTHR : 16;
+  for (int i0 = threadIdx.x; i0 < ALL; i0 += U * NTHR) {
     double v[U];
 #pragma unroll
     for (int u = 0; u < U; u++) {
-      const int idx = i0 + u * DNT, lane = idx & 63, sj = idx >> 6, st = sj / NBL, J = sj - st * NBL;
+      const int idx = i0 + u * NTHR, lane = idx & 63, sj = idx >> 6, st = sj / NBL, J = sj - st * NBL;
       const int k = 4 * V * (st / V) + V * (lane >> 4) + st % V, col = col0 + colmap(J, lane & 15);
       const bool in = idx < ALL && k < n && col < ldw;
       v[u] = W[in ? int64_t(k) * ldw + col : 0];
@@ -242,14 +245,14 @@ PC_DEV void stage_w(const double* __restrict__ W, int n, int ldw, int col0, doub
     }
 #pragma unroll
     for (int u = 0; u < U; u++)
-      if (ALL % (U * DNT) == 0 || i0 + u * DNT < ALL) Wl[i0 + u * DNT] = v[u];
+      if (ALL % (U * NTHR) == 0 || i0 + u * NTHR < ALL) Wl[i0 + u * NTHR] = v[u];
   }
 }
 
 // P2: Z = Yc W in registers, then its Gram.  W is upper triangular: column block J
 // takes the k-steps below 16 (J + 1) only (the rest are exact zeros).
 template <class TS, int NB, int V>
-__global__ __launch_bounds__(DNT) void k_dzgram_f64(const TS* __restrict__ X, int64_t ldx, int64_t m, int n, int center,
+__global__ __launch_bounds__(gram_threads(NB)) void k_dzgram_f64(const TS* __restrict__ X, int64_t ldx, int64_t m, int n, int center,
                                                     const double* mean_in, const double* var_in,
                                                     const double* __restrict__ W, int chunks, int64_t rpc,
                                                     double* __restrict__ part, int64_t zx, int64_t zb) {
@@ -263,8 +266,8 @@ __global__ __launch_bounds__(DNT) void k_dzgram_f64(const TS* __restrict__ X, in
   constexpr int WL = KS * nb * 64, RL = WPC > 1 ? DNW * 2 * 256 : 1;
   __shared__ double sm[WL > RL ? WL : RL];  // W fragments, then the waves' partial Grams
   const int w = threadIdx.x >> 6, l = threadIdx.x & 63, i = l & 15;
-  stage_w<KS, nb, V>(W, n, NB, 0, sm, [](int J, int j) { return 16 * J + j; });
-  const int64_t chunk = int64_t(blockIdx.x) * (DNW / WPC) + w / WPC;
+  stage_w<gram_threads(NB), KS, nb, V>(W, n, NB, 0, sm, [](int J, int j) { return 16 * J + j; });
+  const int64_t chunk = int64_t(blockIdx.x) * (gram_threads(NB) / 64 / WPC) + w / WPC;
   const int64_t row0 = chunk * rpc;
   const int64_t row1 = WPC == 1 && chunk >= chunks ? row0 : row0 + rpc < m ? row0 + rpc : m;
   d4 acc[NBLK];
@@ -351,7 +354,7 @@ __global__ __launch_bounds__(DNT) void k_dgemm_f64(const TS* __restrict__ X, int
   };
   int64_t t = (int64_t(blockIdx.x) * DNW + w) * 16 * R;
   if (t < m) load(t, n, cur, mu, var);
-  stage_w<KS, nbl, V>(W, n, ldw, col0, Wl, [](int J, int j) { return 16 * CV * (J / CV) + CV * j + J % CV; });
+  stage_w<DNT, KS, nbl, V>(W, n, ldw, col0, Wl, [](int J, int j) { return 16 * CV * (J / CV) + CV * j + J % CV; });
   __syncthreads();
   for (; t < m; t += step) {
     // n anew each turn: the columns' clamps and masks, kept over the loop, spilled registers
@@ -544,7 +547,8 @@ int dgram_t(hipStream_t st, const TS* X, int64_t ldx, int64_t m, int n, int cent
   const int64_t rpc = tpc * (n <= 32 ? 32 : 128);
   return with_nb(n, [&](auto nbc) {
     constexpr int NB = decltype(nbc)::value;
-    const dim3 g(unsigned(ceil_div(chunks, DNW / chunk_waves(NB))), 1, unsigned(bz.nz));
+    constexpr int NTHR = gram_threads(NB);
+    const dim3 g(unsigned(ceil_div(chunks, NTHR / 64 / chunk_waves(NB))), 1, unsigned(bz.nz));
     // the Gram's V column blocks have to exist: 48 columns are three blocks; up to 32
     // columns Z's k-steps stay in ascending order
     const int vmax = W ? (NB <= 32 ? 1 : 4) : NB == 64 ? 4 : NB == 32 ? 2 : 1;
@@ -552,11 +556,11 @@ int dgram_t(hipStream_t st, const TS* X, int64_t ldx, int64_t m, int n, int cent
       constexpr int V = decltype(vc)::value;
       if (W) {
         if constexpr (NB > 32 || V == 1)
-          hipLaunchKernelGGL((k_dzgram_f64<TS, NB, V>), g, dim3(DNT), 0, st, X, ldx, m, n, center, mean_in, var_in, W,
+          hipLaunchKernelGGL((k_dzgram_f64<TS, NB, V>), g, dim3(NTHR), 0, st, X, ldx, m, n, center, mean_in, var_in, W,
                              chunks, rpc, part, bz.zx, bz.zb);
       } else {
         if constexpr ((NB / 16) % V == 0)
-          hipLaunchKernelGGL((k_dgram_f64<TS, NB, V>), g, dim3(DNT), 0, st, X, ldx, m, n, center, mean_out, var_out,
+          hipLaunchKernelGGL((k_dgram_f64<TS, NB, V>), g, dim3(NTHR), 0, st, X, ldx, m, n, center, mean_out, var_out,
                              chunks, rpc, part, bz.zx, bz.zb);
       }
       return 0;
@@ -620,14 +624,19 @@ int dxgram_t(hipStream_t st, const TS* A, int64_t lda, int p, const TS* B, int64
 
 }  // namespace
 
-// Row chunks of the direct Grams (at least one: of no rows it writes zeros), from m and the columns alone; *tpc: turns of 32
-// rows (up to 32 columns, one wave per chunk) or of 128 (at most 512 chunks, two
-// workgroups per CU, of at least 256 rows: a 64-column slab is 32 KB to write and sum)
+// Row chunks of the direct Grams (at least one: of no rows it writes zeros), from m and the
+// columns alone; *tpc: turns of 32 rows (up to 32 columns, one wave per chunk) or of 128
+// (at most 512 chunks, two workgroups per CU, of at least 256 rows: a 64-column slab is
+// 32 KB to write and sum).  One-wave chunks: 1024, which 129 problems at once fill the
+// chip with, more from 2^18 rows on, where a lone problem has rows enough for them
+// (4M x 8 float32 SVD with 1024, 2048, 4096: 587, 457, 414 us; 1M x 16: 314, 282, 285;
+// with workgroups of eight waves on half of the CUs 658 and 350).
 int d64_gram_chunks(int64_t m, int n, int64_t* tpc) {
   int64_t tiles, per;
   if (n <= 32) {
     tiles = ceil_div(m, 32);
-    per = ceil_div(tiles, stream_chunks(m, 32));
+    const int64_t most = m <= (1 << 18) ? 1024 : m <= (1 << 21) ? 2048 : 4096;
+    per = std::max<int64_t>(4, ceil_div(tiles, most));
   } else {
     tiles = ceil_div(m, 128);
     per = ceil_div(tiles, 512);

@@ -67,20 +67,22 @@ PC_DEV double block_max(double v, double* sh) {
 // Summation over chunks is in a fixed order (deterministic).
 // ---------------------------------------------------------------------------
 // Chunk sum of the partial slabs (row stride ld), in place into chunk 0, for the
-// entries i < rows, j < cols (UPPER: and i <= j).  A workgroup owns 64 consecutive entries
-// and 16 chunk lanes; lane k sums chunks k, k+16, ... in four interleaved
-// accumulators combined in a fixed order, then lane 0 adds the 16 lane sums in
+// entries i < rows, j < cols (UPPER: and i <= j).  A workgroup owns E consecutive entries
+// and L = 1024 / E chunk lanes; lane k sums chunks k, k + L, ... in four interleaved
+// accumulators combined in a fixed order, then lane 0 adds the L lane sums in
 // order: the summation order depends only on (chunks, ld), so results are
-// deterministic.  Entry e is read and written only by its own workgroup.  G: the sums go
+// deterministic.  E: 64, or 16 for slabs of at most 32 columns, which 64 entries each
+// spread over 4 to 16 workgroups only (1024 slabs of 32 x 32: 15 -> 9 us).  Entry e is read and written only by its own workgroup.  G: the sums go
 // to the symmetric rows x rows matrix G instead (UPPER).
-template <bool UPPER>
+template <bool UPPER, int E = 64>
 __global__ __launch_bounds__(1024) void k_reduce_slab(double* P, int chunks, int64_t pstride, int ld, int rows,
                                                       int cols, double* G, int64_t zb = 0) {
   P = zoff(P, zb);
   if (G) G = zoff(G, zb);
-  __shared__ double red[16][65];
-  const int le = threadIdx.x & 63, k = threadIdx.x >> 6;
-  const int e = blockIdx.x * 64 + le;
+  constexpr int L = 1024 / E;
+  __shared__ double red[L][E + 1];
+  const int le = threadIdx.x & (E - 1), k = threadIdx.x / E;
+  const int e = blockIdx.x * E + le;
   const int i = e / ld, j = e - i * ld;
   const bool use = i < rows && j < cols && (!UPPER || i <= j);
   double s = 0.0;
@@ -88,13 +90,13 @@ __global__ __launch_bounds__(1024) void k_reduce_slab(double* P, int chunks, int
     const double* p = P + e;
     double s0 = 0.0, s1 = 0.0, s2 = 0.0, s3 = 0.0;
     int c = k;
-    for (; c + 48 < chunks; c += 64) {
+    for (; c + 3 * L < chunks; c += 4 * L) {
       s0 += p[int64_t(c) * pstride];
-      s1 += p[int64_t(c + 16) * pstride];
-      s2 += p[int64_t(c + 32) * pstride];
-      s3 += p[int64_t(c + 48) * pstride];
+      s1 += p[int64_t(c + L) * pstride];
+      s2 += p[int64_t(c + 2 * L) * pstride];
+      s3 += p[int64_t(c + 3 * L) * pstride];
     }
-    for (; c < chunks; c += 16) s0 += p[int64_t(c) * pstride];
+    for (; c < chunks; c += L) s0 += p[int64_t(c) * pstride];
     s = (s0 + s1) + (s2 + s3);
   }
   red[k][le] = s;
@@ -102,7 +104,7 @@ __global__ __launch_bounds__(1024) void k_reduce_slab(double* P, int chunks, int
   if (k == 0 && use) {
     double t = 0.0;
 #pragma unroll
-    for (int q = 0; q < 16; q++) t += red[q][le];
+    for (int q = 0; q < L; q++) t += red[q][le];
     if (UPPER && G) {
       G[int64_t(i) * rows + j] = t;
       G[int64_t(j) * rows + i] = t;

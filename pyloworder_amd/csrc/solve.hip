@@ -1093,7 +1093,11 @@ static void reduce_gram(hipStream_t st, const Plan& p, const double* part, int n
 // (k_reduce_slab), which is then folded into the Hermitian one
 static void reduce_slab(hipStream_t st, const Plan& p, const double* part, int nparts, double* G, int nz, int64_t zb) {
   const int64_t e = int64_t(p.NB) * p.NB;
-  hipLaunchKernelGGL(k_reduce_slab<true>, dim3(unsigned(ceil_div(e, 64)), 1, nz), dim3(1024), 0, st,
+  if (p.NB <= 32)
+    hipLaunchKernelGGL((k_reduce_slab<true, 16>), dim3(unsigned(ceil_div(e, 16)), 1, nz), dim3(1024), 0, st,
+                       const_cast<double*>(part), nparts, e, p.NB, p.nr, p.nr, G, zb);
+  else
+    hipLaunchKernelGGL(k_reduce_slab<true>, dim3(unsigned(ceil_div(e, 64)), 1, nz), dim3(1024), 0, st,
                      const_cast<double*>(part), nparts, e, p.NB, p.nr, p.nr, G, zb);
 }
 template <>
