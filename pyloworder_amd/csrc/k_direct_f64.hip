@@ -626,21 +626,21 @@ int dxgram_t(hipStream_t st, const TS* A, int64_t lda, int p, const TS* B, int64
 
 // Row chunks of the direct Grams (at least one: of no rows it writes zeros), from m and the
 // columns alone; *tpc: turns of 32 rows (up to 32 columns, one wave per chunk) or of 128
-// (at most 512 chunks, two workgroups per CU, of at least 256 rows: a 64-column slab is
-// 32 KB to write and sum).  One-wave chunks: 1024, which 129 problems at once fill the
+// (at most 512 chunks, two workgroups per CU: a 64-column slab is 32 KB to write and sum).  One-wave chunks: 1024, which 129 problems at once fill the
 // chip with, more from 2^18 rows on, where a lone problem has rows enough for them
 // (4M x 8 float32 SVD with 1024, 2048, 4096: 587, 457, 414 us; 1M x 16: 314, 282, 285;
-// with workgroups of eight waves on half of the CUs 658 and 350).
+// with workgroups of eight waves on half of the CUs 658 and 350).  Few rows: one turn
+// each (P2 of 5000 x 32 with four turns 16 us, with one 6, of 5000 x 64 with two 17, with
+// one 11, the sum of the slabs the same).
 int d64_gram_chunks(int64_t m, int n, int64_t* tpc) {
   int64_t tiles, per;
   if (n <= 32) {
     tiles = ceil_div(m, 32);
     const int64_t most = m <= (1 << 18) ? 1024 : m <= (1 << 21) ? 2048 : 4096;
-    per = std::max<int64_t>(4, ceil_div(tiles, most));
+    per = std::max<int64_t>(1, ceil_div(tiles, most));
   } else {
     tiles = ceil_div(m, 128);
-    per = ceil_div(tiles, 512);
-    if (per < 2) per = 2;
+    per = std::max<int64_t>(1, ceil_div(tiles, 512));
   }
   *tpc = per;
   return tiles < 1 ? 1 : int(ceil_div(tiles, per));
