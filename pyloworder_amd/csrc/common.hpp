@@ -98,9 +98,9 @@ struct pc_ctx {
   // one sub-context per internal stream (own workspace and status words),
   // driven by its own host thread during a grouped solve
   pc_ctx* sub[kGroupStreams] = {};
-  // set on those sub-contexts: the small stage takes its one-launch kernels
-  // (same results), since launches, not one CU's step time, bound it when
-  // many solves share the GPU
+  // set on those sub-contexts: no side stream, and the Jacobi's test is read
+  // after each sweep, since the number of launches bounds a solve that
+  // shares the GPU with many others
   bool concurrent = false;
   // side stream (default priority) and fork / join events for the small
   // stage's off-path triangular inverses of a lone solve; created on first use

@@ -68,7 +68,7 @@ void jacobi_blocks(int n, int& b, int& nb2) {
 // n = 256).  Under stream capture no host read is possible, so every sweep is
 // queued; converged sweeps then return at once.
 struct SweepChecks {
-  static constexpr int kFirst = 8, kNext = 2;
+  static constexpr int kFirst = 8, kNext = 2, kEach = 4;
   pc_ctx* ctx;
   bool host;
   int next = kFirst;
@@ -77,11 +77,22 @@ struct SweepChecks {
     (void)hipStreamIsCapturing(c->stream, &cap);
     host = cap == hipStreamCaptureStatusNone;
   }
+  bool read(const int* flag) {
+    return hipMemcpyAsync(ctx->hflag + 8, flag, sizeof(int), hipMemcpyDeviceToHost, ctx->stream) == hipSuccess &&
+           hipStreamSynchronize(ctx->stream) == hipSuccess;
+  }
   bool converged(int s, const int* state) {
     if (!host || s != next) return false;
     next += kNext;
-    return hipMemcpyAsync(ctx->hflag + 8, state, sizeof(int), hipMemcpyDeviceToHost, ctx->stream) == hipSuccess &&
-           hipStreamSynchronize(ctx->stream) == hipSuccess && ctx->hflag[8];
+    return read(state) && ctx->hflag[8];
+  }
+  // Real members of a group: their test's result as soon as it is known, from sweep kEach
+  // on.  A lone solve's launches run ahead of the GPU, which a wait after each test would
+  // end; a group on many hardware queues is bound by the number of its launches (8 us
+  // each at 16 queues, however short), and a sweep that finds nothing to rotate is n / 16
+  // of them: 64 mixed problems of up to 256 columns 73.5 -> 70.4 ms, in FP64 141 -> 140.
+  bool nothing(int s, const int* state) {
+    return host && ctx->concurrent && s >= kEach && read(state + 1 + s) && !ctx->hflag[8];
   }
 };
 
@@ -101,7 +112,8 @@ void real_sweeps(pc_ctx* ctx, double* H, int ldh, int n, double* J, int ldj, int
   for (int s = 0; s < kBjacMaxSweeps && !chk.converged(s, state); s++) {
     hipLaunchKernelGGL(k_bjac_gram, dim3(nt * (nt + 1) / 2), dim3(256), 0, st, (const double*)H, ldh, n, nt, Ga, s,
                        state, (const double*)dstate, tol2);
-    for (int step = 0; step < nb2 - 1; step++) {
+    const int steps = chk.nothing(s, state) ? 1 : nb2 - 1;  // the first step sets the done flag
+    for (int step = 0; step < steps; step++) {
       auto launch = [&](auto mode, int wgs) {
         constexpr int M = decltype(mode)::value;
         if (step == 0)
@@ -119,6 +131,7 @@ void real_sweeps(pc_ctx* ctx, double* H, int ldh, int n, double* J, int ldj, int
       }
       std::swap(Ga, Gb);
     }
+    if (steps == 1) return;
   }
 }
 
