@@ -58,7 +58,10 @@ PC_DEV double row16_next(double x) {
 // about 1e-6); what has to hold to rounding is cs^2 + sn^2 = 1, and the FP64 step
 // (cs, sn) (1 + e / 2 + 3 e^2 / 8), e = 1 - cs^2 - sn^2, does that to e^3.  The test is
 // FP64.  (256 -> 150 cycles of a round's chain against FP64 estimates with Newton
-// steps.)  G's scale keeps d, c of any active pair far inside float's range.
+// steps.)  Against the angle in FP64 by square root and division, over 128 matrices each of
+// 16 to 100 columns and condition 1e10, 1e12 and 1e14: the same singular values to three
+// digits of their error, V orthogonal to 2e-15 to 4e-15 (2e-15 to 1e-14 with the other).
+// G's scale keeps d, c of any active pair far inside float's range.
 PC_DEV bool jac_active(double a, double b, double c, double negl, double tol2) {
   return a > negl && b > negl && c * c > tol2 * a * b;
 }
