@@ -2,8 +2,11 @@
 // counterpart of numpy.linalg.eig (LAPACK ?geev) used by the reference's
 // `eigen` (pyLOM/vmmath/maths.py:161-183) for the DMD operator.
 //
-// Algorithm (textbook: Wilkinson and Reinsch, Handbook for Automatic
-// Computation II; Golub and Van Loan, Matrix Computations, 7.4-7.6):
+// Algorithm (Wilkinson and Reinsch, Handbook for Automatic Computation II; Golub and
+// Van Loan, Matrix Computations, 7.4-7.6).  The iteration and the back substitution
+// follow EISPACK's orthes and hqr2 in the form of the public-domain JAMA package (NIST
+// and MathWorks), step by step and with its names, the exceptional shift after 30
+// iterations, which the two books do not have, included:
 //   1. Householder reduction to upper Hessenberg form, H = Z^T A Z, with Z
 //      accumulated;
 //   2. Francis implicit double-shift QR on H down to real Schur form
@@ -20,7 +23,7 @@
 // __host__ __device__; work arrays are the caller's.  The lanes L of one group run it
 // together: every scalar of the iteration is formed by all of them from the same
 // values, rows, columns and vectors are dealt to them, and sync() orders their
-// accesses.  Serial is one lane; on the GPU one wave, with the arrays in LDS where
+// accesses.  Serial is one lane, on the host; on the GPU one wave, with the arrays in LDS where
 // they fit (n is the truncated DMD rank, small): one thread on arrays in memory spent
 // its time on the latency of one access after the other, 1.6 ms at n = 12.
 #pragma once
