@@ -17,7 +17,7 @@
 // flight, W of the next 16 k-steps is loaded before the products of the current ones,
 // and NB comes in steps of 32 columns, not in powers of two.
 // Measured (MI355X; a large library product reaches 72.6 TFLOP/s): 8M x 256 float64
-// P1 11.3 -> 10.2 ms, P2 23.4 -> 22.9 (its 256-column form spills 40 registers), U = Y W
+// P1 11.3 -> 10.2 ms, P2 23.4 -> 22.9 (its 256-column form has 160 bytes a lane in scratch), U = Y W
 // 20.8 -> 20.9 (50 TFLOP/s; its cycles fell by a fifth and the clock from 2.24 to 2.07
 // GHz with them, so power is what is left);
 // 400,003 x 151 float32 (160 columns instead of 256) P1 0.77 -> 0.26, P2 1.53 -> 0.53,
@@ -292,7 +292,7 @@ __global__ __launch_bounds__(64 * NW) void k_gemm_f64(const TS* __restrict__ X, 
     const int chn = last ? 0 : ch + 1;
     const int kb0 = ch * (KC / 16), kb1 = nkb - kb0 < KC / 16 ? nkb - kb0 : KC / 16;
     const double* wl = W + int64_t(16 * kb0 + kr) * ldw + 16 * Jg + cc;
-    // a block of W's rows takes part in column block Jg + 4 i from lo(kb) on
+    // a block of W's rows takes part in column block Jg + NW i from lo(kb) on
     auto lo = [&](int kb) {
       if (!upper) return 0;
       const int d = kb0 + kb - Jg;
@@ -469,11 +469,15 @@ int f64_xgram_chunks(int64_t m, int p, int q, int64_t* tpc) {
   *tpc = ceil_div(ceil_div(m, TR), c);
   return c;
 }
-// rows of one turn of a product pass over n inputs, and its workgroups (two per CU)
-int f64_gemm_rows(int n) { return n > kDirectProduct ? TR : n > 64 ? 128 : 256; }
+// rows of one turn of a product pass over n inputs, and its workgroups: at most 512 of the
+// tiled kernel's (two per CU at a time, or one after the other with 64-row tiles)
+static bool gemm_tall(int64_t m, int nc) { return nc > 128 && m >= kTallProduct; }
+int f64_gemm_rows(int64_t m, int n, int nc) {
+  return n > kDirectProduct ? (gemm_tall(m, nc) ? 2 * TR : TR) : n > 64 ? 128 : 256;
+}
 int f64_gemm_chunks(int64_t m, int n, int nc) {
   if (n <= kDirectProduct) return d64_gemm_chunks(m, n, nc);
-  const int64_t tiles = ceil_div(m, TR);
+  const int64_t tiles = ceil_div(m, f64_gemm_rows(m, n, nc));
   return tiles < 1 ? 1 : int(tiles < 512 ? tiles : 512);
 }
 
@@ -520,7 +524,7 @@ static int launch_gemm_t(hipStream_t st, const TS* X, int64_t ldx, int64_t m, in
       with_var(center, [&](auto vc) {
         constexpr bool VAR = decltype(vc)::value;
         const dim3 g(unsigned(chunks), unsigned(ceil_div(nc, 256)), unsigned(bz.nz));
-        if (nc > 128 && m >= kTallProduct)
+        if (gemm_tall(m, nc))
           hipLaunchKernelGGL((k_gemm_f64<TS, TO, KC, VAR, 4, 8>), g, dim3(512), 0, st, X, ldx, m, n, center, mean_in,
                              var_in, W, ldw, nc, upper, C, ldc, bz.zx, bz.zb, bz.zc);
         else

@@ -9,7 +9,7 @@ int f64_xnb(int n);  // of a cross product's operand
 // per chunk), rows of a product's turn and its workgroups
 int f64_gram_chunks(int64_t m, int n, int64_t* tpc);
 int f64_xgram_chunks(int64_t m, int p, int q, int64_t* tpc);
-int f64_gemm_rows(int n);
+int f64_gemm_rows(int64_t m, int n, int nc);
 int f64_gemm_chunks(int64_t m, int n, int nc);
 // Batched streaming passes: nz problems in one launch (blockIdx.z), the input
 // moving by zx bytes, the workspace operands by zb and the output by zc.

@@ -526,7 +526,7 @@ int make_plan(pc_ctx* ctx, pc_dtype dt, int64_t m, int64_t n, int precision, Pla
     p.tr3 = mx2_tile_rows(p.nr);
   } else {
     p.NB = f64_nb(p.nr);
-    p.tr3 = f64_gemm_rows(p.nr);
+    p.tr3 = f64_gemm_rows(m, p.nr, p.nr);
   }
   p.wide = false;
   if (p.NB < 0 && p.mixed)
@@ -541,7 +541,7 @@ int make_plan(pc_ctx* ctx, pc_dtype dt, int64_t m, int64_t n, int precision, Pla
     p.wide = true;
     p.NB = int(round_up(p.nr, wide_stripe()));
     p.tr = wide_tile_rows();
-    p.tr3 = f64_gemm_rows(p.nr);
+    p.tr3 = f64_gemm_rows(m, p.nr, p.nr);
     const int64_t cap = std::max<int64_t>(1, kWideSlabBytes / (int64_t(p.NB) * p.NB * 8));
     p.chunks = int(std::min<int64_t>(stream_chunks(m, p.tr), cap));
     p.tpc = ceil_div(ceil_div(m, p.tr), p.chunks);
