@@ -410,24 +410,26 @@ __global__ __launch_bounds__(256) void k_q1_rows(const TS* X, int64_t ldx, int n
 
 // D (n signs) from Q1 (n x n; overwritten by its shifted LU unless that runs in LDS);
 // one workgroup.  The shift makes every pivot at least 1 in modulus, so no pivoting is
-// needed.  LDS copy: up to kSignsLds bytes of it (n = 64: 70 -> 17 us; in memory a step
-// waits for the step before it through the L2).
-constexpr size_t kSignsLds = 140 * 1024;
+// needed.  LDS copy: up to kSignsLds bytes of it (n = 64: 70 -> 40 us, 128: 373 -> 139; in
+// memory a step waits for the step before it through the L2).  In memory the trailing
+// block's elements are dealt to all threads up to kSignsFlat columns, a wave to a row
+// beyond, which reads the row's factor once (complex n = 128: 400 and 434 us, n = 200: 1340
+// and 1240; real n = 512: 20.7 and 14.1 ms).
+constexpr size_t kSignsLds = 160 * 1024;
+constexpr int kSignsFlat = 180;
 template <class T>
 inline size_t signs_lds(int n) {
   const size_t b = size_t(n) * (n + 1) * sizeof(T);
   return b <= kSignsLds ? b : 0;
 }
-template <class T>
-__global__ __launch_bounds__(1024) void k_lapack_signs(T* Q1, int n, int in_lds, T* D) {
+template <class T, bool LDS>
+__global__ __launch_bounds__(1024) void k_lapack_signs(T* Q1, int n, T* D) {
   constexpr double kReduced = 64 * 2.220446049250313e-16;
   HIP_DYNAMIC_SHARED(char, signs_smem)
   const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
-  T* A = Q1;
-  int ld = n;
-  if (in_lds) {
-    A = reinterpret_cast<T*>(signs_smem);
-    ld = n + 1;
+  T* A = LDS ? reinterpret_cast<T*>(signs_smem) : Q1;
+  const int ld = LDS ? n + 1 : n;
+  if constexpr (LDS) {
     for (int i = w; i < n; i += 16)
       for (int j = l; j < n; j += 64) A[i * ld + j] = Q1[int64_t(i) * n + j];
     __syncthreads();
@@ -442,13 +444,44 @@ __global__ __launch_bounds__(1024) void k_lapack_signs(T* Q1, int n, int in_lds,
       D[k] = reduced ? T(re >= 0.0 ? 1.0 : -1.0) : s;
     }
     const T ip = inv_(a - s);
-    for (int i = k + 1 + w; i < n; i += 16) {
-      T* ri = A + int64_t(i) * ld;
-      const T f = ri[k] * ip;
-      for (int j = k + 1 + l; j < n; j += 64) ri[j] -= f * rk[j];
+    if constexpr (LDS) {
+      for (int i = k + 1 + w; i < n; i += 16) {
+        T* ri = A + int64_t(i) * ld;
+        const T f = ri[k] * ip;
+        for (int j = k + 1 + l; j < n; j += 64) ri[j] -= f * rk[j];
+      }
+    } else if (n <= kSignsFlat) {
+      const int r = n - k - 1;
+      for (int e = threadIdx.x; e < r * r; e += 1024) {
+        const int i = k + 1 + e / r, j = k + 1 + e % r;
+        Q1[i * n + j] -= Q1[i * n + k] * ip * rk[j];
+      }
+    } else {
+      // four rows of a wave at a time, so that their loads go out together
+      for (int i0 = k + 1 + w; i0 < n; i0 += 64) {
+        T f[4];
+#pragma unroll
+        for (int x = 0; x < 4; x++) f[x] = Q1[int64_t(min(i0 + 16 * x, n - 1)) * n + k];
+        for (int j = k + 1 + l; j < n; j += 64) {
+          T v[4];
+          const T u = rk[j];
+#pragma unroll
+          for (int x = 0; x < 4; x++) v[x] = Q1[int64_t(min(i0 + 16 * x, n - 1)) * n + j];
+#pragma unroll
+          for (int x = 0; x < 4; x++)
+            if (i0 + 16 * x < n) Q1[int64_t(i0 + 16 * x) * n + j] = v[x] - f[x] * ip * u;
+        }
+      }
     }
     __syncthreads();
   }
+}
+
+template <class T>
+void run_lapack_signs(hipStream_t st, T* Q1, int n, T* D) {
+  const size_t lds = signs_lds<T>(n);
+  if (lds) hipLaunchKernelGGL((k_lapack_signs<T, true>), dim3(1), dim3(1024), lds, st, Q1, n, D);
+  else hipLaunchKernelGGL((k_lapack_signs<T, false>), dim3(1), dim3(1024), 0, st, Q1, n, D);
 }
 
 // R := D R (rows), W := W D (columns), null fix entries of column g + b by D_{g+b}
@@ -1453,8 +1486,7 @@ static int core_t(pc_ctx* ctx, const Plan& p, const void* A, int64_t lda, int ce
     // LAPACK's signs (numpy.linalg.qr): D from the first n rows of Q, then
     // R = D R+, Q = Q+ D through W and the null fix; Q1 in tmp, D in G2
     launch_q1_rows<T>(st, p, A, lda, b);
-    hipLaunchKernelGGL((k_lapack_signs<T>), dim3(1), dim3(1024), signs_lds<T>(n), st, b.tmp, n, int(signs_lds<T>(n) > 0),
-                       b.G2);
+    run_lapack_signs<T>(st, b.tmp, n, b.G2);
     hipLaunchKernelGGL((k_apply_signs<T>), dim3(nblk(nn)), dim3(256), 0, st, (const T*)b.G2, n, b.J, n, b.Wf, n,
                        (const int*)b.nnull, b.cnull);
     hipLaunchKernelGGL((k_store_r<T, typename VtType<T, ST>::type>), dim3(nblk(nn)), dim3(256), 0, st, b.J, n, n,

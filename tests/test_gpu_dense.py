@@ -96,3 +96,18 @@ def test_few_null_directions(missing, dtype):
     tol = 1e-13 * n
     assert np.abs(S[:k] - s).max() <= tol and S[k:].max() <= tol
     assert np.abs(U.conj().T @ U - np.eye(n)).max() <= tol and np.abs((U * S) @ VT - A).max() <= tol
+
+
+@pytest.mark.parametrize("dtype,n", [(np.float64, 142), (np.float64, 143), (np.float64, 180), (np.float64, 181),
+                                     (np.complex128, 100), (np.complex128, 101), (np.complex128, 181)])
+def test_qr_signs_at_the_forms_of_their_factorisation(dtype, n):
+    """R and Q as numpy.linalg.qr, signs and all, where the shifted LU leaves LDS and where its rows go to waves: 1e-9
+    of max |R|, 1e-8 for Q, as in test_tsqr_lapack_signs."""
+    rng = np.random.default_rng(n)
+    A = rng.standard_normal((700, n)).astype(dtype)
+    if np.iscomplexobj(A):
+        A = A + 1j * rng.standard_normal((700, n))
+    Q, R = pl.math.tsqr(A)
+    Qo, Ro = np.linalg.qr(A)
+    assert np.abs(R - Ro).max() <= 1e-9 * np.abs(Ro).max()
+    assert np.abs(Q - Qo).max() <= 1e-8
