@@ -33,15 +33,17 @@ namespace {
 
 constexpr int DNT = 512;        // 8 waves
 constexpr int DNW = DNT / 64;
-// Waves that share a row chunk of a Gram over NB columns, 16 rows each per turn.  Up
-// to 32 columns a chunk is one wave's: its rows are summed in ascending order and the
-// slab is written from registers.  (Summing 8 waves' parts through LDS costs a
-// workgroup about as much as 200 rows of 30 columns.)  Wider Grams have few chunks
-// of long rows, so 8 waves share one.
-constexpr int chunk_waves(int NB) { return NB <= 32 ? 1 : 8; }
-// Threads of those workgroups: with a chunk per wave, four of them, or a lone problem of
-// 1024 chunks has workgroups for half of the CUs only.
+// A row chunk of a Gram over more than 32 columns is a workgroup's of 8 waves, 16 rows
+// each per turn, which sum their parts through LDS; up to 32 columns one of 4 waves', or
+// a wave's of its own, whose slab is written from registers (chunk_waves).
 constexpr int gram_threads(int NB) { return NB <= 32 ? 256 : DNT; }
+// Waves of a chunk over at most 32 columns: 4, except from 2^17 to 2^18 rows, where the
+// 1024 chunks have 128 to 256 rows and the sum of a workgroup's 4 parts through LDS costs
+// the most beside them: 64 problems of 130,000 x 15 complex in one launch 2.63 ms with 4
+// waves a chunk, 2.49 with one.  From 2^18 on one wave a chunk leaves the chip half idle
+// (a lone 4M x 8 float32 SVD 587 us, with 4 waves 402), below 2^17 most of it (P2 of
+// 5000 x 32 23 us, now 12; 64 of 50,000 x 15 complex 1.47 and 1.46 ms).
+inline int chunk_waves(int64_t m) { return m > (1 << 17) && m <= (1 << 18) ? 1 : 4; }
 
 template <class TS, int V>
 PC_DEV void load_vec(const TS* p, TS* o) {
@@ -67,31 +69,33 @@ PC_DEV void store_vec(TO* p, const TO* o) {
   }
 }
 
-// Sum the NBLK accumulators of the 8 waves in wave order through red (two blocks
+// Sum the NBLK accumulators of NW waves in wave order through red (NW KB; NW / 4 blocks
 // at a time) and hand every entry (block, i, j, value) to `put`.
-template <int NBLK, class Put>
+template <int NBLK, int NW, class Put>
 PC_DEV void sum_waves(const d4* acc, double* red, Put put) {
+  constexpr int BP = NW / 4;  // blocks whose entries the threads of NW waves are
   const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
 #pragma unroll
-  for (int b0 = 0; b0 < NBLK; b0 += 2) {
+  for (int b0 = 0; b0 < NBLK; b0 += BP) {
     __syncthreads();
 #pragma unroll
-    for (int u = 0; u < 2; u++)
+    for (int u = 0; u < BP; u++)
       if (b0 + u < NBLK)
 #pragma unroll
-        for (int r = 0; r < 4; r++) red[(w * 2 + u) * 256 + r * 64 + l] = acc[b0 + u][r];
+        for (int r = 0; r < 4; r++) red[(w * BP + u) * 256 + r * 64 + l] = acc[b0 + u][r];
     __syncthreads();
     const int u = threadIdx.x >> 8, e = threadIdx.x & 255;
     if (b0 + u < NBLK) {
       double s = 0.0;
 #pragma unroll
-      for (int q = 0; q < DNW; q++) s += red[(q * 2 + u) * 256 + e];
+      for (int q = 0; q < NW; q++) s += red[(q * BP + u) * 256 + e];
       put(b0 + u, 4 * (e >> 6) + ((e >> 4) & 3), e & 15, s);
     }
   }
 }
+constexpr int red_size(int NW) { return NW * (NW / 4) * 256; }  // doubles
 
-// Upper blocks (I, J) of a chunk's Gram to `put`: from registers, or summed over its 8 waves
+// Upper blocks (I, J) of a chunk's Gram to `put`: from registers, or summed over its waves
 template <int nb, int WPC, class Put>
 PC_DEV void store_gram(const d4* acc, double* red, Put put) {
   constexpr int NBLK = nb * (nb + 1) / 2;
@@ -105,7 +109,7 @@ PC_DEV void store_gram(const d4* acc, double* red, Put put) {
 #pragma unroll
         for (int r = 0; r < 4; r++) put(I, J, 4 * r + (l >> 4), l & 15, acc[b][r]);
   } else {
-    sum_waves<NBLK>(acc, red, [&](int blk, int pi, int pj, double s) {
+    sum_waves<NBLK, WPC>(acc, red, [&](int blk, int pi, int pj, double s) {
       int I = 0, o = 0;
       while (o + nb - I <= blk) o += nb - I++;
       put(I, I + blk - o, pi, pj, s);
@@ -132,7 +136,7 @@ PC_DEV void load_rows(const TS* __restrict__ X, int64_t ldx, int n, int64_t base
 }
 
 // P1: partial Gram of the (centred) rows of a chunk
-template <class TS, int NB, int V>
+template <class TS, int NB, int V, int WPC>
 __global__ __launch_bounds__(gram_threads(NB)) void k_dgram_f64(const TS* __restrict__ X, int64_t ldx, int64_t m, int n, int center,
                                                    double* mean_out, double* var_out, int chunks, int64_t rpc,
                                                    double* __restrict__ part, int64_t zx, int64_t zb) {
@@ -141,8 +145,7 @@ __global__ __launch_bounds__(gram_threads(NB)) void k_dgram_f64(const TS* __rest
   var_out = zoff(var_out, zb);
   part = zoff(part, zb);
   constexpr int nb = NB / 16, NBLK = nb * (nb + 1) / 2;
-  constexpr int WPC = chunk_waves(NB);
-  __shared__ double red[WPC > 1 ? DNW * 2 * 256 : 1];
+  __shared__ double red[WPC > 1 ? red_size(WPC) : 1];
   const int w = threadIdx.x >> 6, l = threadIdx.x & 63, i = l & 15, g = l >> 4;
   const int64_t chunk = int64_t(blockIdx.x) * (gram_threads(NB) / 64 / WPC) + w / WPC;
   if (WPC == 1 && chunk >= chunks) return;
@@ -251,7 +254,7 @@ PC_DEV void stage_w(const double* __restrict__ W, int n, int ldw, int col0, doub
 
 // P2: Z = Yc W in registers, then its Gram.  W is upper triangular: column block J
 // takes the k-steps below 16 (J + 1) only (the rest are exact zeros).
-template <class TS, int NB, int V>
+template <class TS, int NB, int V, int WPC>
 __global__ __launch_bounds__(gram_threads(NB)) void k_dzgram_f64(const TS* __restrict__ X, int64_t ldx, int64_t m, int n, int center,
                                                     const double* mean_in, const double* var_in,
                                                     const double* __restrict__ W, int chunks, int64_t rpc,
@@ -262,8 +265,7 @@ __global__ __launch_bounds__(gram_threads(NB)) void k_dzgram_f64(const TS* __res
   W = zoff(W, zb);
   part = zoff(part, zb);
   constexpr int nb = NB / 16, NBLK = nb * (nb + 1) / 2, KS = NB / 4;
-  constexpr int WPC = chunk_waves(NB);
-  constexpr int WL = KS * nb * 64, RL = WPC > 1 ? DNW * 2 * 256 : 1;
+  constexpr int WL = KS * nb * 64, RL = WPC > 1 ? red_size(WPC) : 1;
   __shared__ double sm[WL > RL ? WL : RL];  // W fragments, then the waves' partial Grams
   const int w = threadIdx.x >> 6, l = threadIdx.x & 63, i = l & 15;
   stage_w<gram_threads(NB), KS, nb, V>(W, n, NB, 0, sm, [](int J, int j) { return 16 * J + j; });
@@ -429,7 +431,7 @@ __global__ __launch_bounds__(DNT) void k_dxgram_f64(const TS* __restrict__ A, in
   // k-steps per turn: current and next rows beside the accumulators in 256 registers
   constexpr int RS = (pb + qb) * int(sizeof(TS)) * 2 + NBLK * 8 > 200 ? 2 : 4;
   constexpr int unit = DNW * 4 * RS;
-  __shared__ double red[DNW * 2 * 256];
+  __shared__ double red[red_size(DNW)];
   const int w = threadIdx.x >> 6, l = threadIdx.x & 63, i = l & 15, g = l >> 4;
   const int64_t row0 = int64_t(blockIdx.x) * rpc;
   const int64_t row1 = row0 + rpc < m ? row0 + rpc : m;
@@ -474,7 +476,7 @@ __global__ __launch_bounds__(DNT) void k_dxgram_f64(const TS* __restrict__ A, in
     }
   }
   double* P = part + int64_t(blockIdx.x) * PB * QB;
-  sum_waves<NBLK>(acc, red, [&](int blk, int pi, int pj, double s) {
+  sum_waves<NBLK, DNW>(acc, red, [&](int blk, int pi, int pj, double s) {
     const int I = blk / qb, J = blk - I * qb;
     P[int64_t(16 * V * (I / V) + V * pi + I % V) * QB + 16 * V * (J / V) + V * pj + J % V] = s;
   });
@@ -544,25 +546,32 @@ template <class TS>
 int dgram_t(hipStream_t st, const TS* X, int64_t ldx, int64_t m, int n, int center, const double* mean_in,
             const double* var_in, double* mean_out, double* var_out, const double* W, int chunks, int64_t tpc,
             double* part, const PassBatch& bz) {
-  const int64_t rpc = tpc * (n <= 32 ? 32 : 128);
+  const int wpc = n > 32 ? DNW : chunk_waves(m);
+  const int64_t rpc = tpc * 32 * (wpc == 1 ? 1 : 4);
   return with_nb(n, [&](auto nbc) {
     constexpr int NB = decltype(nbc)::value;
     constexpr int NTHR = gram_threads(NB);
-    const dim3 g(unsigned(ceil_div(chunks, NTHR / 64 / chunk_waves(NB))), 1, unsigned(bz.nz));
+    const dim3 g(unsigned(ceil_div(chunks, NTHR / 64 / wpc)), 1, unsigned(bz.nz));
     // the Gram's V column blocks have to exist: 48 columns are three blocks; up to 32
     // columns Z's k-steps stay in ascending order
     const int vmax = W ? (NB <= 32 ? 1 : 4) : NB == 64 ? 4 : NB == 32 ? 2 : 1;
     return with_vec<TS>(vec_width<TS>(X, ldx, n, bz.zx, vmax), [&](auto vc) {
       constexpr int V = decltype(vc)::value;
-      if (W) {
-        if constexpr (NB > 32 || V == 1)
-          hipLaunchKernelGGL((k_dzgram_f64<TS, NB, V>), g, dim3(NTHR), 0, st, X, ldx, m, n, center, mean_in, var_in, W,
-                             chunks, rpc, part, bz.zx, bz.zb);
-      } else {
-        if constexpr ((NB / 16) % V == 0)
-          hipLaunchKernelGGL((k_dgram_f64<TS, NB, V>), g, dim3(NTHR), 0, st, X, ldx, m, n, center, mean_out, var_out,
-                             chunks, rpc, part, bz.zx, bz.zb);
-      }
+      auto go = [&](auto wc) {
+        constexpr int WPC = decltype(wc)::value;
+        if (W) {
+          if constexpr (NB > 32 || V == 1)
+            hipLaunchKernelGGL((k_dzgram_f64<TS, NB, V, WPC>), g, dim3(NTHR), 0, st, X, ldx, m, n, center, mean_in,
+                               var_in, W, chunks, rpc, part, bz.zx, bz.zb);
+        } else {
+          if constexpr ((NB / 16) % V == 0)
+            hipLaunchKernelGGL((k_dgram_f64<TS, NB, V, WPC>), g, dim3(NTHR), 0, st, X, ldx, m, n, center, mean_out,
+                               var_out, chunks, rpc, part, bz.zx, bz.zb);
+        }
+      };
+      if constexpr (NB > 32) go(Int<DNW>{});
+      else if (wpc == 1) go(Int<1>{});
+      else go(Int<4>{});
       return 0;
     });
   });
@@ -625,19 +634,16 @@ int dxgram_t(hipStream_t st, const TS* A, int64_t lda, int p, const TS* B, int64
 }  // namespace
 
 // Row chunks of the direct Grams (at least one: of no rows it writes zeros), from m and the
-// columns alone; *tpc: turns of 32 rows (up to 32 columns, one wave per chunk) or of 128
-// (at most 512 chunks, two workgroups per CU: a 64-column slab is 32 KB to write and sum).  One-wave chunks: 1024, which 129 problems at once fill the
-// chip with, more from 2^18 rows on, where a lone problem has rows enough for them
-// (4M x 8 float32 SVD with 1024, 2048, 4096: 587, 457, 414 us; 1M x 16: 314, 282, 285;
-// with workgroups of eight waves on half of the CUs 658 and 350).  Few rows: one turn
-// each (P2 of 5000 x 32 with four turns 16 us, with one 6, of 5000 x 64 with two 17, with
-// one 11, the sum of the slabs the same).
+// columns alone; *tpc: turns of 128 rows, or of 32 where a chunk is one wave's.  At most
+// 1024 up to 32 columns and 512 (two workgroups per CU) beyond, where a slab is 32 KB to
+// write and sum.  Few rows: one turn each (P2 of 5000 x 64 with two turns 17 us, with one
+// 11), two up to 32 columns, where many small problems may share a launch (64 of
+// 50,000 x 15 complex with one 1.53 ms, with two 1.46).
 int d64_gram_chunks(int64_t m, int n, int64_t* tpc) {
   int64_t tiles, per;
   if (n <= 32) {
-    tiles = ceil_div(m, 32);
-    const int64_t most = m <= (1 << 18) ? 1024 : m <= (1 << 21) ? 2048 : 4096;
-    per = std::max<int64_t>(1, ceil_div(tiles, most));
+    tiles = ceil_div(m, chunk_waves(m) == 1 ? 32 : 128);
+    per = std::max<int64_t>(2, ceil_div(tiles, 1024));
   } else {
     tiles = ceil_div(m, 128);
     per = std::max<int64_t>(1, ceil_div(tiles, 512));
