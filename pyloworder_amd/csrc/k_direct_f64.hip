@@ -37,13 +37,12 @@ constexpr int DNW = DNT / 64;
 // each per turn, which sum their parts through LDS; up to 32 columns one of 4 waves', or
 // a wave's of its own, whose slab is written from registers (chunk_waves).
 constexpr int gram_threads(int NB) { return NB <= 32 ? 256 : DNT; }
-// Waves of a chunk over at most 32 columns: 4, except from 2^17 to 2^18 rows, where the
-// 1024 chunks have 128 to 256 rows and the sum of a workgroup's 4 parts through LDS costs
-// the most beside them: 64 problems of 130,000 x 15 complex in one launch 2.63 ms with 4
-// waves a chunk, 2.49 with one.  From 2^18 on one wave a chunk leaves the chip half idle
-// (a lone 4M x 8 float32 SVD 587 us, with 4 waves 402), below 2^17 most of it (P2 of
-// 5000 x 32 23 us, now 12; 64 of 50,000 x 15 complex 1.47 and 1.46 ms).
-inline int chunk_waves(int64_t m) { return m > (1 << 17) && m <= (1 << 18) ? 1 : 4; }
+// Waves of a chunk over at most 32 columns.  Real ones: 4, since with one a lone problem
+// leaves the chip half idle or more (4M x 8 float32 SVD 587 us, with 4 waves 402; P2 of
+// 5000 x 32 23 and 12 us).  Complex ones, the blocks of a spectral POD, many in a launch:
+// one, its rows summed in ascending order, which fixes the phase that a noise mode's
+// vector has (64 of 130,000 x 15 in one launch 2.49 ms, with 4 waves a chunk 2.63).
+inline int chunk_waves(bool cplx) { return cplx ? 1 : 4; }
 
 template <class TS, int V>
 PC_DEV void load_vec(const TS* p, TS* o) {
@@ -546,7 +545,7 @@ template <class TS>
 int dgram_t(hipStream_t st, const TS* X, int64_t ldx, int64_t m, int n, int center, const double* mean_in,
             const double* var_in, double* mean_out, double* var_out, const double* W, int chunks, int64_t tpc,
             double* part, const PassBatch& bz) {
-  const int wpc = n > 32 ? DNW : chunk_waves(m);
+  const int wpc = n > 32 ? DNW : chunk_waves(bz.cplx);
   const int64_t rpc = tpc * 32 * (wpc == 1 ? 1 : 4);
   return with_nb(n, [&](auto nbc) {
     constexpr int NB = decltype(nbc)::value;
@@ -636,17 +635,16 @@ int dxgram_t(hipStream_t st, const TS* A, int64_t lda, int p, const TS* B, int64
 // Row chunks of the direct Grams (at least one: of no rows it writes zeros), from m and the
 // columns alone; *tpc: turns of 128 rows, or of 32 where a chunk is one wave's.  At most
 // 1024 up to 32 columns and 512 (two workgroups per CU) beyond, where a slab is 32 KB to
-// write and sum.  Few rows: one turn each (P2 of 5000 x 64 with two turns 17 us, with one
-// 11), two up to 32 columns, where many small problems may share a launch (64 of
-// 50,000 x 15 complex with one 1.53 ms, with two 1.46).
-int d64_gram_chunks(int64_t m, int n, int64_t* tpc) {
+// write and sum.  Few rows: as few turns as that gives (P2 of 5000 x 64 with two turns a
+// chunk 17 us, with one 11), for complex columns at least 128 and 256 rows a chunk.
+int d64_gram_chunks(int64_t m, int n, bool cplx, int64_t* tpc) {
   int64_t tiles, per;
-  if (n <= 32) {
-    tiles = ceil_div(m, chunk_waves(m) == 1 ? 32 : 128);
-    per = std::max<int64_t>(2, ceil_div(tiles, 1024));
+  if (n <= 32 && chunk_waves(cplx) == 1) {
+    tiles = ceil_div(m, 32);
+    per = ceil_div(tiles, stream_chunks(m, 32));
   } else {
     tiles = ceil_div(m, 128);
-    per = std::max<int64_t>(1, ceil_div(tiles, 512));
+    per = std::max<int64_t>(cplx ? 2 : 1, ceil_div(tiles, n <= 32 ? 1024 : 512));
   }
   *tpc = per;
   return tiles < 1 ? 1 : int(ceil_div(tiles, per));
@@ -671,7 +669,7 @@ int d64_gemm_chunks(int64_t m, int n, int nc) {
 }
 
 // row chunks of the direct cross products, turns of 128 rows
-int d64_xgram_chunks(int64_t m, int64_t* tpc) { return d64_gram_chunks(m, kDirectGram, tpc); }
+int d64_xgram_chunks(int64_t m, int64_t* tpc) { return d64_gram_chunks(m, kDirectGram, false, tpc); }
 
 int launch_d64_gram(hipStream_t st, pc_dtype dt, const void* X, int64_t ldx, int64_t m, int n, int center,
                     const double* mean_in, const double* var_in, double* mean_out, double* var_out, const double* W,

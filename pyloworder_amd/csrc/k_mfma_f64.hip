@@ -454,8 +454,8 @@ int f64_nb(int n) { return n <= 64 ? int(round_up(n < 1 ? 1 : n, 16)) : n <= 256
 int f64_xnb(int n) { return n <= 64 ? f64_nb(n) : n <= 128 ? 128 : n <= 256 ? 256 : -1; }
 // Row chunks of the Gram passes over n columns (k_direct_f64.hip up to 64): at most
 // 512, two per CU in turn, so that half the slabs of 1024 are written and summed
-int f64_gram_chunks(int64_t m, int n, int64_t* tpc) {
-  if (n <= kDirectGram) return d64_gram_chunks(m, n, tpc);
+int f64_gram_chunks(int64_t m, int n, bool cplx, int64_t* tpc) {
+  if (n <= kDirectGram) return d64_gram_chunks(m, n, cplx, tpc);
   const int64_t tiles = ceil_div(m, TR);
   int64_t per = ceil_div(tiles, 512);
   if (per < 4) per = 4;

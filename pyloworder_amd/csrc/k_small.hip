@@ -68,18 +68,18 @@ PC_DEV double block_max(double v, double* sh) {
 // ---------------------------------------------------------------------------
 // Chunk sum of the partial slabs (row stride ld), in place into chunk 0, for the
 // entries i < rows, j < cols (UPPER: and i <= j).  A workgroup owns E consecutive entries
-// and L = 1024 / E chunk lanes; lane k sums chunks k, k + L, ... in four interleaved
-// accumulators combined in a fixed order, then lane 0 adds the L lane sums in
-// order: the summation order depends only on (chunks, ld), so results are
-// deterministic.  E: 64, or 16 for slabs of at most 32 columns, which 64 entries each
-// spread over 4 to 16 workgroups only (1024 slabs of 32 x 32: 15 -> 9 us).  Entry e is read and written only by its own workgroup.  G: the sums go
-// to the symmetric rows x rows matrix G instead (UPPER).
-template <bool UPPER, int E = 64>
-__global__ __launch_bounds__(1024) void k_reduce_slab(double* P, int chunks, int64_t pstride, int ld, int rows,
+// and L chunk lanes; lane k sums chunks k, k + L, ... in four interleaved accumulators
+// combined in a fixed order, then lane 0 adds the L lane sums in order: the summation
+// order depends only on (chunks, L), so results are deterministic.  Entry e is read and
+// written only by its own workgroup.  64 entries and 16 lanes; 16 entries for slabs of at
+// most 32 columns, which 64 each spread over 4 to 16 workgroups only, and 64 lanes for real
+// ones (1024 slabs of 32 x 32: 15 -> 9 us).  G: the sums go to the symmetric rows x rows
+// matrix G instead (UPPER).
+template <bool UPPER, int E = 64, int L = 16>
+__global__ __launch_bounds__(E * L) void k_reduce_slab(double* P, int chunks, int64_t pstride, int ld, int rows,
                                                       int cols, double* G, int64_t zb = 0) {
   P = zoff(P, zb);
   if (G) G = zoff(G, zb);
-  constexpr int L = 1024 / E;
   __shared__ double red[L][E + 1];
   const int le = threadIdx.x & (E - 1), k = threadIdx.x / E;
   const int e = blockIdx.x * E + le;

@@ -7,15 +7,17 @@ int f64_nb(int n);
 int f64_xnb(int n);  // of a cross product's operand
 // partition of the passes, from the sizes alone: row chunks of a Gram (tpc: turns
 // per chunk), rows of a product's turn and its workgroups
-int f64_gram_chunks(int64_t m, int n, int64_t* tpc);
+int f64_gram_chunks(int64_t m, int n, bool cplx, int64_t* tpc);
 int f64_xgram_chunks(int64_t m, int p, int q, int64_t* tpc);
 int f64_gemm_rows(int64_t m, int n, int nc);
 int f64_gemm_chunks(int64_t m, int n, int nc);
 // Batched streaming passes: nz problems in one launch (blockIdx.z), the input
 // moving by zx bytes, the workspace operands by zb and the output by zc.
+// cplx: the columns are the interleaved parts of complex ones (a Gram's partition).
 struct PassBatch {
   int nz = 1;
   int64_t zx = 0, zb = 0, zc = 0;
+  bool cplx = false;
 };
 // W non-null: the second pass, Gram of Z = Y W, W (n x n, padded to f64_nb) upper
 // triangular: Z skips the products with its zero blocks
@@ -36,7 +38,7 @@ int launch_xgram_f64(hipStream_t st, pc_dtype dt, const void* A, int64_t lda, in
 // fragments fit one wave's registers), products of at most kDirectProduct inputs
 // (W fits one CU's LDS in slices of 128 columns)
 constexpr int kDirectGram = 64, kDirectProduct = 128;
-int d64_gram_chunks(int64_t m, int n, int64_t* tpc);
+int d64_gram_chunks(int64_t m, int n, bool cplx, int64_t* tpc);
 int d64_xgram_chunks(int64_t m, int64_t* tpc);
 int d64_gemm_chunks(int64_t m, int n, int nc);
 int launch_d64_gram(hipStream_t st, pc_dtype dt, const void* X, int64_t ldx, int64_t m, int n, int center,

@@ -586,7 +586,7 @@ int make_plan(pc_ctx* ctx, pc_dtype dt, int64_t m, int64_t n, int precision, Pla
     return PC_OK;
   }
   if (!p.mixed) {
-    p.chunks = f64_gram_chunks(m, p.nr, &p.tpc);
+    p.chunks = f64_gram_chunks(m, p.nr, p.cplx, &p.tpc);
     p.chunks3 = f64_gemm_chunks(m, p.nr, p.nr);
     p.tpc3 = ceil_div(ceil_div(m, p.tr3), p.chunks3);
     p.chunks2 = p.chunks;
@@ -1084,8 +1084,9 @@ struct CoreOut {
 
 template <class T>
 static int launch_streams(pc_ctx* ctx, const Plan& p, const void* A, int64_t lda, int center, double* mean,
-                          double* var, double* part, SmallBufs<T>& b, int pass, const PassBatch& bz = PassBatch()) {
+                          double* var, double* part, SmallBufs<T>& b, int pass, PassBatch bz = PassBatch()) {
   hipStream_t st = ctx->stream;
+  bz.cplx = p.cplx;
   int rc = 0;
   pc_dtype sdt = p.cplx ? (p.dt == PC_C64 ? PC_F32 : PC_F64) : p.dt;
   int64_t ldr = p.cplx ? 2 * lda : lda;
@@ -1139,12 +1140,13 @@ static void reduce_gram(hipStream_t st, const Plan& p, const double* part, int n
 // (k_reduce_slab), which is then folded into the Hermitian one
 static void reduce_slab(hipStream_t st, const Plan& p, const double* part, int nparts, double* G, int nz, int64_t zb) {
   const int64_t e = int64_t(p.NB) * p.NB;
-  if (p.NB <= 32)
-    hipLaunchKernelGGL((k_reduce_slab<true, 16>), dim3(unsigned(ceil_div(e, 16)), 1, nz), dim3(1024), 0, st,
+  auto go = [&](auto kernel, int E, int L) {
+    hipLaunchKernelGGL(kernel, dim3(unsigned(ceil_div(e, E)), 1, nz), dim3(unsigned(E * L)), 0, st,
                        const_cast<double*>(part), nparts, e, p.NB, p.nr, p.nr, G, zb);
-  else
-    hipLaunchKernelGGL(k_reduce_slab<true>, dim3(unsigned(ceil_div(e, 64)), 1, nz), dim3(1024), 0, st,
-                     const_cast<double*>(part), nparts, e, p.NB, p.nr, p.nr, G, zb);
+  };
+  if (p.NB > 32) go(k_reduce_slab<true>, 64, 16);
+  else if (p.cplx) go(k_reduce_slab<true, 16, 16>, 16, 16);
+  else go(k_reduce_slab<true, 16, 64>, 16, 64);
 }
 template <>
 void reduce_gram<double>(hipStream_t st, const Plan& p, const double* part, int nparts, double* G, int nz,
