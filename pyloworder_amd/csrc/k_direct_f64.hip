@@ -36,7 +36,9 @@ constexpr int DNW = DNT / 64;
 // A row chunk of a Gram over more than 32 columns is a workgroup's of 8 waves, 16 rows
 // each per turn, which sum their parts through LDS; up to 32 columns one of 4 waves', or
 // a wave's of its own, whose slab is written from registers (chunk_waves).
-constexpr int gram_threads(int NB) { return NB <= 32 ? 256 : DNT; }
+// Threads of a workgroup: up to 32 columns 256 (129 x 200,000 x 30 float32 P1 0.96 -> 0.91
+// ms), but 512 in a P2 of one wave a chunk, where the waves share one copy of W (1.80 -> 1.63).
+constexpr int gram_threads(int NB, int WPC, bool P2) { return NB <= 32 && !(P2 && WPC == 1) ? 256 : DNT; }
 // Waves of a chunk over at most 32 columns.  Real ones: 4, since with one a lone problem
 // leaves the chip half idle or more (4M x 8 float32 SVD 587 us, with 4 waves 402; P2 of
 // 5000 x 32 23 and 12 us).  Complex ones, the blocks of a spectral POD, many in a launch:
@@ -136,7 +138,7 @@ PC_DEV void load_rows(const TS* __restrict__ X, int64_t ldx, int n, int64_t base
 
 // P1: partial Gram of the (centred) rows of a chunk
 template <class TS, int NB, int V, int WPC>
-__global__ __launch_bounds__(gram_threads(NB)) void k_dgram_f64(const TS* __restrict__ X, int64_t ldx, int64_t m, int n, int center,
+__global__ __launch_bounds__(gram_threads(NB, WPC, false)) void k_dgram_f64(const TS* __restrict__ X, int64_t ldx, int64_t m, int n, int center,
                                                    double* mean_out, double* var_out, int chunks, int64_t rpc,
                                                    double* __restrict__ part, int64_t zx, int64_t zb) {
   X = zoff(X, zx);
@@ -146,7 +148,7 @@ __global__ __launch_bounds__(gram_threads(NB)) void k_dgram_f64(const TS* __rest
   constexpr int nb = NB / 16, NBLK = nb * (nb + 1) / 2;
   __shared__ double red[WPC > 1 ? red_size(WPC) : 1];
   const int w = threadIdx.x >> 6, l = threadIdx.x & 63, i = l & 15, g = l >> 4;
-  const int64_t chunk = int64_t(blockIdx.x) * (gram_threads(NB) / 64 / WPC) + w / WPC;
+  const int64_t chunk = int64_t(blockIdx.x) * (gram_threads(NB, WPC, false) / 64 / WPC) + w / WPC;
   if (WPC == 1 && chunk >= chunks) return;
   const int64_t row0 = chunk * rpc;
   const int64_t row1 = row0 + rpc < m ? row0 + rpc : m;
@@ -254,7 +256,7 @@ PC_DEV void stage_w(const double* __restrict__ W, int n, int ldw, int col0, doub
 // P2: Z = Yc W in registers, then its Gram.  W is upper triangular: column block J
 // takes the k-steps below 16 (J + 1) only (the rest are exact zeros).
 template <class TS, int NB, int V, int WPC>
-__global__ __launch_bounds__(gram_threads(NB)) void k_dzgram_f64(const TS* __restrict__ X, int64_t ldx, int64_t m, int n, int center,
+__global__ __launch_bounds__(gram_threads(NB, WPC, true)) void k_dzgram_f64(const TS* __restrict__ X, int64_t ldx, int64_t m, int n, int center,
                                                     const double* mean_in, const double* var_in,
                                                     const double* __restrict__ W, int chunks, int64_t rpc,
                                                     double* __restrict__ part, int64_t zx, int64_t zb) {
@@ -267,8 +269,8 @@ __global__ __launch_bounds__(gram_threads(NB)) void k_dzgram_f64(const TS* __res
   constexpr int WL = KS * nb * 64, RL = WPC > 1 ? red_size(WPC) : 1;
   __shared__ double sm[WL > RL ? WL : RL];  // W fragments, then the waves' partial Grams
   const int w = threadIdx.x >> 6, l = threadIdx.x & 63, i = l & 15;
-  stage_w<gram_threads(NB), KS, nb, V>(W, n, NB, 0, sm, [](int J, int j) { return 16 * J + j; });
-  const int64_t chunk = int64_t(blockIdx.x) * (gram_threads(NB) / 64 / WPC) + w / WPC;
+  stage_w<gram_threads(NB, WPC, true), KS, nb, V>(W, n, NB, 0, sm, [](int J, int j) { return 16 * J + j; });
+  const int64_t chunk = int64_t(blockIdx.x) * (gram_threads(NB, WPC, true) / 64 / WPC) + w / WPC;
   const int64_t row0 = chunk * rpc;
   const int64_t row1 = WPC == 1 && chunk >= chunks ? row0 : row0 + rpc < m ? row0 + rpc : m;
   d4 acc[NBLK];
@@ -549,22 +551,21 @@ int dgram_t(hipStream_t st, const TS* X, int64_t ldx, int64_t m, int n, int cent
   const int64_t rpc = tpc * 32 * (wpc == 1 ? 1 : 4);
   return with_nb(n, [&](auto nbc) {
     constexpr int NB = decltype(nbc)::value;
-    constexpr int NTHR = gram_threads(NB);
-    const dim3 g(unsigned(ceil_div(chunks, NTHR / 64 / wpc)), 1, unsigned(bz.nz));
     // the Gram's V column blocks have to exist: 48 columns are three blocks; up to 32
     // columns Z's k-steps stay in ascending order
     const int vmax = W ? (NB <= 32 ? 1 : 4) : NB == 64 ? 4 : NB == 32 ? 2 : 1;
     return with_vec<TS>(vec_width<TS>(X, ldx, n, bz.zx, vmax), [&](auto vc) {
       constexpr int V = decltype(vc)::value;
       auto go = [&](auto wc) {
-        constexpr int WPC = decltype(wc)::value;
+        constexpr int WPC = decltype(wc)::value, N1 = gram_threads(NB, WPC, false), N2 = gram_threads(NB, WPC, true);
+        const dim3 g(unsigned(ceil_div(chunks, (W ? N2 : N1) / 64 / WPC)), 1, unsigned(bz.nz));
         if (W) {
           if constexpr (NB > 32 || V == 1)
-            hipLaunchKernelGGL((k_dzgram_f64<TS, NB, V, WPC>), g, dim3(NTHR), 0, st, X, ldx, m, n, center, mean_in,
+            hipLaunchKernelGGL((k_dzgram_f64<TS, NB, V, WPC>), g, dim3(N2), 0, st, X, ldx, m, n, center, mean_in,
                                var_in, W, chunks, rpc, part, bz.zx, bz.zb);
         } else {
           if constexpr ((NB / 16) % V == 0)
-            hipLaunchKernelGGL((k_dgram_f64<TS, NB, V, WPC>), g, dim3(NTHR), 0, st, X, ldx, m, n, center, mean_out,
+            hipLaunchKernelGGL((k_dgram_f64<TS, NB, V, WPC>), g, dim3(N1), 0, st, X, ldx, m, n, center, mean_out,
                                var_out, chunks, rpc, part, bz.zx, bz.zb);
         }
       };
