@@ -377,10 +377,11 @@ __global__ __launch_bounds__(DNT) void k_dgemm_f64(const TS* __restrict__ X, int
 #pragma unroll
         for (int u = 0; u < CV; u++) z[q][u] = d4{0, 0, 0, 0};
       // X k-steps at a time, beyond 32 inputs their fragments read while the X before are
-      // multiplied (up to 32 HBM is the bound, and the registers keep rows in flight).  A
-      // branch round each step left every product waiting for its read: 500,000 x 128 by
-      // 128 x 128 float64 391 -> 315 us
-      constexpr int X = CV == 4 ? 2 : 4, AHEAD = KB > 32 ? 1 : 0;
+      // multiplied.  A branch round each step left every product waiting for its read:
+      // 500,000 x 128 by 128 x 128 float64 391 -> 315 us.  Up to 16, where a step is a quarter
+      // of the products and more, the steps beyond n stay out one load's width at a time
+      // (250,000 x 3 by 3 x 64 float32 21 us in fours, 16 so)
+      constexpr int AHEAD = KB > 32 ? 1 : 0, XM = CV == 4 ? 2 : 4, X = KB > 16 || V > XM ? XM : V;
       const double* wq = Wl + q0 * CV * 64 + l;
       double b[1 + AHEAD][X][CV];
       auto read = [&](int c) {
@@ -392,7 +393,7 @@ __global__ __launch_bounds__(DNT) void k_dgemm_f64(const TS* __restrict__ X, int
       if (AHEAD) read(0);
 #pragma unroll
       for (int c = 0; c < KS / X; c++)
-        if (16 * (X * c / 4) < n) {
+        if (4 * V * (X * c / V) < n) {
           if (!AHEAD || c + 1 < KS / X) read(c + AHEAD);
 #pragma unroll
           for (int x = 0; x < X; x++)
@@ -523,18 +524,22 @@ int64_t gemm_workgroups(int64_t turns, int nc, int s) {
   return ceil_div(turns, 256) * nc < ceil_div(turns, shared) * s ? 256 : shared;
 }
 // Columns of W that a workgroup keeps in LDS: a power of two, at most 128 KB of it.  X is
-// read once per slice, so a tall product takes the widest; one of few rows takes the
-// narrowest of which every CU holds a workgroup at once (1024 x 128 by 128 x 256 float64:
-// 16 workgroups of 128 columns 44 us, 256 of 16 columns 20, where the call's launch is
-// what is left; 5000 rows: 36 us with 128, 23 with 64, 30 with 32, which take two rounds).
-int gemm_slice(int64_t m, int n, int nc) {
-  const int64_t turns = gemm_turns(m, n);
+// read once per slice, and a slice writes only a part of each row, so a tall product takes
+// the widest (1.5M x 5 by 5 x 41 float64 in halves 285 us, whole 152); one of few rows (nz
+// problems together) takes the narrowest of which every CU holds a workgroup at once
+// (1024 x 128 by 128 x 256 float64: 16 workgroups of 128 columns 44 us, 256 of 16 columns
+// 20, where the call's launch is what is left; 5000 rows: 36 us with 128, 23 with 64, 30
+// with 32, which take two rounds).
+int gemm_slice(int64_t m, int n, int nc, int nz) {
+  const int64_t turns = gemm_turns(m, n) * nz;
   int most = n > 64 ? 128 : 256;
   while (most > 16 && most / 2 >= nc) most /= 2;
   auto slices = [&](int s) { return ceil_div(nc, s); };
   if (turns * slices(most) > 256) {
-    // several turns each: half as many columns where that shortens the longest
-    // workgroup's work by a fifth and X, read once per slice, stays in the caches
+    if (n <= 32) return most;
+    // several turns each, beyond 32 inputs, where the matrix units bound them: half as
+    // many columns where that shortens the longest workgroup's work by a fifth and X, read
+    // once per slice, stays in the caches
     auto work = [&](int s) { return ceil_div(turns, gemm_workgroups(turns, nc, s)) * s; };
     const int half = most / 2;
     return half >= 16 && 5 * work(half) <= 4 * work(most) && slices(half) * m * n * 8 <= (int64_t(128) << 20) ? half : most;
@@ -577,6 +582,17 @@ int dgram_t(hipStream_t st, const TS* X, int64_t ldx, int64_t m, int n, int cent
   });
 }
 
+// Unused LDS that keeps a direct product of up to 32 inputs alone on its CU: where C is
+// beyond the 256 MB cache and its rows, of more than a line, begin inside lines, a line that
+// two rows share is written to HBM twice unless the waves in flight are few (1.5M x 8 by
+// 8 x 41 float64 203 us with two workgroups a CU, 145 with one; by 8 x 60 268 and 228;
+// 700,000 x 8 by 8 x 41, C of 230 MB, 76 and 76).  Shorter rows, and rows of whole lines,
+// take the waves (4M x 8 by 8 x 20 float32 with one 1.3 times as long).
+inline size_t alone_lds(int kb, size_t wl, int64_t rows, int nc, int64_t ldc, size_t size) {
+  const int64_t pitch = ldc * int64_t(size);
+  const bool split = kb <= 32 && pitch > 128 && pitch % 128 != 0 && rows * nc * int64_t(size) > (int64_t(256) << 20);
+  return split && wl < 84 * 1024 ? 84 * 1024 - wl : 0;
+}
 template <class TS, class TO>
 int dgemm_t(hipStream_t st, const TS* X, int64_t ldx, int64_t m, int n, int center, const double* mean_in,
             const double* var_in, const double* W, int ldw, int nc, int chunks, TO* C, int64_t ldc,
@@ -587,9 +603,10 @@ int dgemm_t(hipStream_t st, const TS* X, int64_t ldx, int64_t m, int n, int cent
     return with_vec<TS>(vx, [&](auto v_) {
       return with_vec<TO>(NCB / 16 < vc ? NCB / 16 : vc, [&](auto c_) {
         constexpr int V = decltype(v_)::value, CV = decltype(c_)::value;
+        const size_t pad = alone_lds(KB, size_t(KB) * NCB * sizeof(double), m * bz.nz, nc, ldc, sizeof(TO));
         if constexpr ((NCB / 16) % CV == 0)
           hipLaunchKernelGGL((k_dgemm_f64<TS, TO, KB, NCB, V, CV>),
-                             dim3(unsigned(chunks), unsigned(ceil_div(nc, NCB)), unsigned(bz.nz)), dim3(DNT), 0, st, X,
+                             dim3(unsigned(chunks), unsigned(ceil_div(nc, NCB)), unsigned(bz.nz)), dim3(DNT), pad, st, X,
                              ldx, m, n, center, mean_in, var_in, W, ldw, nc, C, ldc, bz.zx, bz.zb, bz.zc);
         return 0;
       });
@@ -597,7 +614,7 @@ int dgemm_t(hipStream_t st, const TS* X, int64_t ldx, int64_t m, int n, int cent
   };
   auto cols = [&](auto kc) {
     constexpr int KB = decltype(kc)::value;
-    const int slice = gemm_slice(m, n, nc);
+    const int slice = gemm_slice(m, n, nc, bz.nz);
     if (slice == 16) return go(kc, Int<16>{});
     if (slice == 32) return go(kc, Int<32>{});
     if (slice == 64) return go(kc, Int<64>{});
@@ -659,7 +676,7 @@ int d64_gram_chunks(int64_t m, int n, bool cplx, int64_t* tpc) {
 // turns (250,000 x 30 by 30 x 30: 33 us with one turn each, 27 with four).
 int d64_gemm_chunks(int64_t m, int n, int nc) {
   const int64_t turns = gemm_turns(m, n);
-  const int slice = gemm_slice(m, n, nc);
+  const int slice = gemm_slice(m, n, nc, 1);
   int64_t want = gemm_workgroups(turns, nc, slice);
   if (n <= 32) {
     const int64_t lds = int64_t(gemm_k(n)) * 8 * slice, fit = lds > 40 * 1024 ? 2 : 4;

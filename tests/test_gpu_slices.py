@@ -27,6 +27,21 @@ def test_products(m, k, n, dtype):
         assert float((C.double() - ref).abs().max()) <= 8 * tol * float(ref.abs().max())
 
 
+@pytest.mark.parametrize("m,k,n,dtype", [(1100003, 3, 41, torch.float64), (900001, 30, 60, torch.float64),
+                                         (1100003, 13, 67, torch.float32), (700003, 16, 131, torch.float32),
+                                         (2200003, 5, 17, torch.float64)])
+def test_products_beyond_the_cache(m, k, n, dtype):
+    """Results of more than 256 MB, their rows on both sides of a line's length and no multiple of it."""
+    g = torch.Generator(device="cuda").manual_seed(n)
+    A = torch.randn((m, k), generator=g, device="cuda", dtype=dtype)
+    B = torch.randn((k, n), generator=g, device="cuda", dtype=dtype)
+    C = pl.math.matmul(A, B)
+    tol = (k + 2) * np.sqrt(k) * 2.0 ** -53 + (2.0 ** -24 if dtype == torch.float32 else 0.0)
+    for r in range(0, m, 1 << 18):
+        ref = A[r:r + (1 << 18)].double() @ B.double()
+        assert float((C[r:r + (1 << 18)].double() - ref).norm() / ref.norm()) <= tol
+
+
 @pytest.mark.parametrize("dtype", [torch.float64, torch.float32, torch.complex128, torch.complex64])
 @pytest.mark.parametrize("m,k,n", [(200, 5, 3), (8192, 30, 30), (8193, 30, 30), (8193, 17, 64), (70000, 33, 20),
                                    (9001, 70, 65), (9001, 256, 256), (9001, 257, 256)])
