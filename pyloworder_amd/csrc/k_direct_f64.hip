@@ -14,10 +14,10 @@
 //   - the D registers of Z = Y W are themselves such fragments of Z (register r is
 //     rows 4 r .. 4 r + 3), so P2's Gram takes them as they are.
 // Measured (MI355X) against LDS-staged 32-row tiles: 129 x 200,000 x 30 float32
-// (SPOD) P1 1.54 -> 0.91 ms, P2 2.78 -> 1.62 ms, U = Y W 2.47 -> 1.69 ms (3.7 TB/s);
-// 1M x 64 float64 P1 192 -> 132 us, P2 417 -> 222 us, product 279 -> 242 us (4.2 TB/s,
-// a copy reaches 4.7); 8M x 64 by 64 x 256 float32 (reconstruct) 6.46 -> 4.96 ms;
-// A^T B of 700,001 x 64 and x 48 float32 189 -> 108 us.
+// (SPOD) P1 1.54 -> 0.91 ms, P2 2.78 -> 1.65 ms, U = Y W 2.47 -> 1.39 ms (4.4 TB/s, a copy
+// reaches 4.7); 1M x 64 float64 P1 195 -> 144 us, P2 423 -> 228 us, product 282 -> 194 us;
+// 8M x 64 by 64 x 256 float32 (reconstruct) 7.19 -> 4.61 ms (57 TFLOP/s); A^T B of
+// 700,001 x 64 and x 48 float32 189 -> 109 us.
 //
 // Loads are V elements per lane (V = 1, 2, 4 by alignment).  In the Grams the V
 // elements go to V column blocks (block c V + e holds the physical columns
@@ -36,8 +36,9 @@ constexpr int DNW = DNT / 64;
 // A row chunk of a Gram over more than 32 columns is a workgroup's of 8 waves, 16 rows
 // each per turn, which sum their parts through LDS; up to 32 columns one of 4 waves', or
 // a wave's of its own, whose slab is written from registers (chunk_waves).
-// Threads of a workgroup: up to 32 columns 256 (129 x 200,000 x 30 float32 P1 0.96 -> 0.91
-// ms), but 512 in a P2 of one wave a chunk, where the waves share one copy of W (1.80 -> 1.63).
+// So a workgroup has 256 threads up to 32 columns (129 x 200,000 x 30 float32 P1 0.96 ->
+// 0.91 ms), but 512 in a P2 of one wave a chunk, where the waves share one copy of W (1.80
+// -> 1.65 ms).
 constexpr int gram_threads(int NB, int WPC, bool P2) { return NB <= 32 && !(P2 && WPC == 1) ? 256 : DNT; }
 // Waves of a chunk over at most 32 columns.  Real ones: 4, since with one a lone problem
 // leaves the chip half idle or more (4M x 8 float32 SVD 587 us, with 4 waves 402; P2 of

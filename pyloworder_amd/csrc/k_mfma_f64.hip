@@ -17,9 +17,9 @@
 // flight, W of the next 16 k-steps is loaded before the products of the current ones,
 // and NB comes in steps of 32 columns, not in powers of two.
 // Measured (MI355X; a large library product reaches 72.6 TFLOP/s): 8M x 256 float64
-// P1 11.3 -> 10.2 ms, P2 23.4 -> 22.9 (its 256-column form has 160 bytes a lane in scratch), U = Y W
-// 20.8 -> 20.9 (50 TFLOP/s; its cycles fell by a fifth and the clock from 2.24 to 2.07
-// GHz with them, so power is what is left);
+// P1 11.3 -> 10.4 ms, P2 23.4 -> 23.0 (its 256-column form has 160 bytes a lane in
+// scratch), U = Y W 20.8 -> 20.2 (52 TFLOP/s).  Counters: the matrix units are busy in 62
+// to 70 % of the cycles, which run at 2.1 to 2.4 GHz;
 // 400,003 x 151 float32 (160 columns instead of 256) P1 0.77 -> 0.26, P2 1.53 -> 0.53,
 // U 1.07 -> 0.55 ms; 1M x 512 float32 Z 13.8 -> 6.6 (its zero blocks skipped), U 13.9 ->
 // 9.9 ms.

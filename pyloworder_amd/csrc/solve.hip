@@ -663,8 +663,8 @@ __global__ __launch_bounds__(256) void k_null_lev(const TS* X, int64_t ldx, int6
   urows = zoff(urows, zb);
   int d = nnull[0];
   if (d == 0) return;
-  // kLevRows candidates per workgroup: W is read once for all of them (one each read n^2
-  // of it per row from the L2, 44 us at n = 256)
+  // kLevRows candidates per workgroup: W is read once for all of them (n = 256: one each
+  // 44 us, two 27, four 21, eight 30, with 128 workgroups; n = 64: 5.6 with two, 7.3, 11)
   const int cand0 = blockIdx.x * kLevRows;
   auto row_of = [&](int c) { return ncand >= m ? int64_t(c) : (int64_t(c) * m) / ncand; };
   HIP_DYNAMIC_SHARED(char, lev_smem)  // kLevRows x n values of T
@@ -791,7 +791,9 @@ __global__ __launch_bounds__(1024) void k_null_build(int64_t m, int n, const int
   __syncthreads();
   // the d candidates of the lowest leverage (ties by index).  Few, the usual case (row
   // centring leaves one null direction): the next one after the last pick, d times, and
-  // below one wave per sum; n = 256, d = 1: 118 -> 25 us.  Many: by their ranks.
+  // below one wave per sum; n = 256, d = 1: 116 -> 28 us.  Many: by their ranks.  In us by
+  // picks and by ranks at d = 4 and 8: n = 256 91 and 144, 211 and 213; n = 64 29 and 26,
+  // 53 and 35; n = 30 21 and 17, 40 and 22.
   const bool few = d <= 4;
   const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
   __shared__ double best_v[16];
